@@ -197,12 +197,14 @@ static bool dispatch_f32(cigemmHandle_t h, int64_t M, int64_t N, int64_t K, cons
     case CIGEMM_ALGO_SKINNY:
       return false;
     case CIGEMM_ALGO_MFMA_ANY:
-      return launch_mfma_any_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba);
+      return launch_tile_any_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba) ||
+             launch_mfma_any_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba);
     case CIGEMM_ALGO_GENERIC:
       launch_generic_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba);
       return true;
     default:
       if (!launch_f32_mfma(h, M, N, K, A, lda, B, ldb, C, ldc, ba) &&
+          !launch_tile_any_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba) &&
           !launch_mfma_any_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba))
         launch_generic_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba);
       return true;
@@ -244,13 +246,17 @@ static cigemmStatus_t gemm16(cigemmHandle_t h, const char* name, bool bf16, int6
     case CIGEMM_ALGO_SKINNY: ok = launch_skinny_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc); break;
     case CIGEMM_ALGO_TILE: ok = launch_16b_mfma(h, bf16, M, N, K, A, lda, B, ldb, C, ldc); break;
     case CIGEMM_ALGO_SMALL: ok = false; break;
-    case CIGEMM_ALGO_MFMA_ANY: ok = launch_mfma_any_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc); break;
+    case CIGEMM_ALGO_MFMA_ANY:
+      ok = launch_tile_any_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc) ||
+           launch_mfma_any_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc);
+      break;
     case CIGEMM_ALGO_GENERIC: launch_generic_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc); break;
     default:
       // decode shapes (M <= 32) first: they are bandwidth problems with their own kernel; what
       // neither that nor the tile kernel takes (odd N, unaligned rows) stays on the matrix cores
       if (!launch_skinny_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc) &&
           !launch_16b_mfma(h, bf16, M, N, K, A, lda, B, ldb, C, ldc) &&
+          !launch_tile_any_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc) &&
           !launch_mfma_any_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc))
         launch_generic_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc);
   }
@@ -281,12 +287,14 @@ static cigemmStatus_t gemm_i8(cigemmHandle_t h, const char* name, int64_t M, int
     case CIGEMM_ALGO_TILE: ok = launch_i8_mfma(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq); break;
     case CIGEMM_ALGO_SMALL: ok = false; break;
     case CIGEMM_ALGO_MFMA_ANY:
-      ok = launch_mfma_any_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq);
+      ok = launch_tile_any_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq) ||
+           launch_mfma_any_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq);
       break;
     case CIGEMM_ALGO_GENERIC: launch_generic_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq); break;
     default:
       if (!launch_skinny_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq) &&
           !launch_i8_mfma(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq) &&
+          !launch_tile_any_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq) &&
           !launch_mfma_any_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq))
         launch_generic_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq);
   }

@@ -58,8 +58,9 @@ cigemmStatus_t check_launch(cigemmContext* ctx, const char* what);
 // Name of a tile-kernel call from what the launcher recorded on the context, e.g.
 // "i8_mfma_192x256x64_w4_ring4_nk_dequant" (tile rows x 256 columns x k elements per stage,
 // waves per workgroup), "256+192" / "w4+w4" when two launches covered the columns.
+// `any`: "i8_mfma_any_192x256x64_...", the form that takes any alignment.
 void set_tile_kernel_name(cigemmContext* ctx, const char* dtype, int k_elems, const char* suffix,
-                          bool splitk);
+                          bool splitk, bool any = false);
 // Raises the dynamic-LDS limit of `kernel` to `bytes` once per device and template instance
 // (`done` = that instance's bit mask of devices already set).  A refusal is recorded on the
 // context and reported by check_launch; it returns false and the caller must not launch.
@@ -226,6 +227,17 @@ bool launch_mfma_any_f32(cigemmContext*, int64_t M, int64_t N, int64_t K, const 
                          int64_t lda, const float* B, int64_t ldb, float* C, int64_t ldc,
                          const BiasAct* ba);
 bool launch_mfma_any_i8(cigemmContext*, int64_t M, int64_t N, int64_t K, const int8_t* A,
+                        int64_t lda, const int8_t* B, int64_t ldb, bool b_nk, int32_t* C,
+                        int64_t ldc, const DequantArgs* dq);
+// gemm_any_tile.hip: the tile kernel at any alignment.  False for matrices narrower than one
+// 16-byte piece, for the accumulator dump and beyond the launch limits (nothing launched).
+bool launch_tile_any_16(cigemmContext*, bool bf16, int64_t M, int64_t N, int64_t K,
+                        const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb,
+                        uint16_t* C, int64_t ldc);
+bool launch_tile_any_f32(cigemmContext*, int64_t M, int64_t N, int64_t K, const float* A,
+                         int64_t lda, const float* B, int64_t ldb, float* C, int64_t ldc,
+                         const BiasAct* ba);
+bool launch_tile_any_i8(cigemmContext*, int64_t M, int64_t N, int64_t K, const int8_t* A,
                         int64_t lda, const int8_t* B, int64_t ldb, bool b_nk, int32_t* C,
                         int64_t ldc, const DequantArgs* dq);
 void launch_generic_16(cigemmContext*, bool bf16, int64_t M, int64_t N, int64_t K,

@@ -35,7 +35,7 @@ cigemmStatus_t check_launch(cigemmContext* ctx, const char* what) {
 }
 
 void set_tile_kernel_name(cigemmContext* ctx, const char* dtype, int k_elems, const char* suffix,
-                          bool splitk) {
+                          bool splitk, bool any) {
   char rows[24], waves[24];
   if (ctx->first_tile_rows) {
     snprintf(rows, sizeof(rows), "%d+%d", ctx->first_tile_rows, ctx->last_tile_rows);
@@ -44,8 +44,8 @@ void set_tile_kernel_name(cigemmContext* ctx, const char* dtype, int k_elems, co
     snprintf(rows, sizeof(rows), "%d", ctx->last_tile_rows);
     snprintf(waves, sizeof(waves), ctx->last_per_cu == 2 ? "w%dx2" : "w%d", ctx->last_waves);
   }
-  snprintf(ctx->kernel_name, sizeof(ctx->kernel_name), "%s_mfma_%sx256x%d_%s_ring%d%s%s", dtype,
-           rows, k_elems, waves, ctx->last_per_cu == 2 ? 3 : 4, suffix, splitk ? "_splitk" : "");
+  snprintf(ctx->kernel_name, sizeof(ctx->kernel_name), "%s_mfma_%s%sx256x%d_%s_ring%d%s%s", dtype,
+           any ? "any_" : "", rows, k_elems, waves, ctx->last_per_cu == 2 ? 3 : 4, suffix, splitk ? "_splitk" : "");
   ctx->last_kernel = ctx->kernel_name;
 }
 

@@ -2,6 +2,7 @@
 // accumulators of one output row (columns col..col+3) into output bits:
 //   load_row(row)            what the epilogue needs per output row (a scale), fetched once;
 //   load_cols(col)           what it needs for the four columns col..col+3 (scales, bias);
+//   load_col(col)            the same for one column, where col_t holds four floats;
 //   pack(rowv, colv, v0..v3) the 4 output elements as raw bits (u32x2 for 16-bit outputs,
 //                            u32x4 for 32-bit ones) from those; no memory is touched;
 //   pack(row, col, v0..v3)   the same with both fetched on the spot;
@@ -132,6 +133,41 @@ struct EpiBiasActF32x4 {
   }
 };
 
+// The same with both options chosen at run time and a bias of any alignment, for the tile kernel's
+// ANY form (load_col is all that reads the bias there).
+struct EpiBiasActAnyF32x4 {
+  float* C;
+  int64_t ldc;
+  const float* bias;
+  int relu;
+  static constexpr int OUT_BYTES = 4;
+  typedef EpiNothing row_t;
+  typedef f32x4 col_t;
+  __device__ __forceinline__ row_t load_row(int64_t) const { return row_t{}; }
+  __device__ __forceinline__ float load_col(int64_t c) const { return bias ? bias[c] : 0.0f; }
+  __device__ __forceinline__ u32x4 pack(row_t, col_t b, float v0, float v1, float v2,
+                                        float v3) const {
+    f32x4 v = {v0, v1, v2, v3};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (bias) v[e] = __fadd_rn(v[e], b[e]);
+      if (relu) v[e] = fmaxf(0.0f, v[e]);
+    }
+    return __builtin_bit_cast(u32x4, v);
+  }
+  __device__ __forceinline__ u32x4 pack(int64_t, int64_t, float v0, float v1, float v2,
+                                        float v3) const {
+    return pack(row_t{}, f32x4{0.0f, 0.0f, 0.0f, 0.0f}, v0, v1, v2, v3);
+  }
+  __device__ __forceinline__ char* out_row(int64_t r) const {
+    return reinterpret_cast<char*>(C + r * ldc);
+  }
+  __device__ __forceinline__ void side(int64_t, int64_t, float, float, float, float) const {}
+  EpiBiasActAnyF32x4 shift_cols(int64_t c0) const {
+    return EpiBiasActAnyF32x4{C + c0, ldc, bias ? bias + c0 : nullptr, relu};
+  }
+};
+
 struct EpiStoreI32x4 {
   int32_t* C;
   int64_t ldc;
@@ -184,6 +220,7 @@ struct EpiDequantX4 {
   __device__ __forceinline__ row_t row_from_word(float w) const { return w; }
   __device__ __forceinline__ col_t cols_from_word(float w) const { return f32x4{w, w, w, w}; }
   __device__ __forceinline__ row_t load_row(int64_t r) const { return sa[sa_vec ? r : 0]; }
+  __device__ __forceinline__ float load_col(int64_t c) const { return sb[sb_vec ? c : 0]; }
   __device__ __forceinline__ col_t load_cols(int64_t c) const {
     if (sb_vec) return *reinterpret_cast<const f32x4*>(sb + c);
     const float b0 = sb[0];

@@ -32,11 +32,24 @@ bool launch_f32_mfma(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const 
     // 512^3: 17 against 9; 960 x 3584 x 3584: 222 against 298).
     const bool one_round = ((M + 255) / 256) * ((N + tile::BN - 1) / tile::BN) <= cus;
     const bool long_k_split = tile_ok && K >= 2048 && one_round;
-    // What the tile kernel cannot take (B or C rows not 16-byte aligned, an odd N) and fills the
-    // chip with 128 x 128 tiles is left to the any-shape matrix-core kernel (4096 x 4095 x 4096:
-    // 109 against 63 TFLOP/s; at 1000^3, 64 such tiles, this kernel is 3x the faster one).
-    const double tiles128 = (double)((M + 127) / 128) * (double)((N + 127) / 128);
-    if (!tile_ok && tiles128 >= cus) return false;
+    // What the aligned tile kernel cannot take (B or C rows not 16-byte aligned, an odd N): the
+    // tile kernel's any-alignment form when it is estimated the faster.  Without 16-byte loads of
+    // B this kernel takes about 2 us + K x (13 ns for up to one resident round of tiles -- 7 where
+    // B is at most 1 MiB --, 7.8 ns per round beyond), at least 6.5 us; the tile kernel its plan's
+    // estimate + 4 us.  Both timed over M 8..4096, N 251..4095, K 64..4096 (112 shapes): 4096 x
+    // 4095 x 4096 2031 (this kernel) against 923 us, 64 x 1001 x 4096 55 against 21, 4096 x 251 x
+    // 1000 38 against 28; the other way 512 x 2047 x 336 13 against 21, 8 x 251 x 1000 9 against
+    // 15.  The rule takes the slower one on 4 of them, by 6-14 %.
+    if (!tile_ok && tile::tile_any_ok(M, N, K, 4, lda, ldb, true)) {
+      if (!one_round) return false;
+      double plan = 0;
+      tile::plan_small(cus, ctx->workspace ? ctx->ws_partial_bytes : 0, M,
+                       tile::partial_ld<true>(N), K * 4, 4, tile::STAGE_COST_KN32, K * 4 * N, &plan);
+      const double rounds = tiles32 / cus;
+      const double per_k = rounds > 1.7 ? 0.0078 * rounds : K * N <= (256 << 10) ? 0.007 : 0.013;
+      const double small_us = 2.0 + (double)K * per_k;
+      if (plan + 4.0 < (small_us > 6.5 ? small_us : 6.5)) return false;
+    }
     if (!tile_ok || (small_cost < tile_cost && !long_k_split)) {
       launch_f32_small(ctx, M, N, K, A, lda, B, ldb, C, ldc, ba);
       return true;

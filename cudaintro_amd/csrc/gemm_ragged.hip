@@ -1,8 +1,8 @@
-// Any-shape GEMM on the matrix cores, for the calls that the LDS-DMA tile kernel and the small
-// fp32 kernel cannot take (an odd N, rows or pointers that are not 16-byte aligned, a K whose bytes
-// are not a multiple of 16): the scalar any-shape kernel runs those at 30 (16-bit) to 45 (fp32)
-// TFLOP/s, far below the tile kernel, and the library this path replaces has no such cliff
-// (quantization/GEMM_bf16.cu:51-56 passes whatever m, n, k, lda, ldb it is given).
+// Any-shape GEMM on the matrix cores, for the calls that no form of the LDS-DMA tile kernel takes
+// (gemm_any_tile.hip serves odd sizes and unaligned rows): a K, or the N of a K x N operand, of
+// fewer than 16 bytes, leading dimensions beyond that kernel's 32-bit row offsets, and the int32
+// accumulator dump beside a dequantized output on unaligned rows.  The library this path replaces
+// takes whatever m, n, k, lda, ldb it is given (quantization/GEMM_bf16.cu:51-56).
 //
 // One 128 x 128 output tile per 256-thread workgroup, four waves of 64 x 64 (2 x 2 MFMA tiles
 // of 32 x 32), 64 bytes of k per step.  Operands are fetched in 16-byte pieces of a row, each
@@ -56,37 +56,9 @@ struct RaggedElem<4> {
   static constexpr int KN_PITCH = 544;  // [16 k][512 B], rows k and k + 4 half the banks apart
 };
 
-// One 16-byte piece = elements [col, col + CE) of row `row` of a row-major matrix with `rows`
-// rows of `cols` elements, zero outside the matrix, in two steps so that the load is one
-// unconditional instruction that can stay in flight while the previous step multiplies:
-// load_piece reads 16 bytes that lie inside the matrix whatever the piece (row clamped to the
-// last one; a piece that crosses the end of its row is replaced by the row's last 16 bytes),
-// trim_piece, applied when the value is needed, moves those down so that element `col` comes
-// first and zeroes what lies outside.  Needs cols >= CE.
-template <typename T>
-__device__ __forceinline__ u32x4 load_piece(const T* __restrict__ P, int64_t ld, int64_t row,
-                                            int64_t rows, int64_t col, int64_t cols) {
-  constexpr int CE = 16 / (int)sizeof(T);
-  const int64_t r = row < rows ? row : rows - 1;
-  const int64_t c = col + CE <= cols ? col : cols - CE;
-  u32x4 v;
-  __builtin_memcpy(&v, P + r * ld + c, 16);
-  return v;
-}
-template <typename T>
-__device__ __forceinline__ u32x4 trim_piece(u32x4 v, int64_t row, int64_t rows, int64_t col,
-                                            int64_t cols) {
-  constexpr int CE = 16 / (int)sizeof(T);
-  const bool inside = row < rows && col < cols;
-  const int s = col + CE > cols && inside ? (int)(col - (cols - CE)) * 8 * (int)sizeof(T) : 0;
-  const int s1 = s & 63;  // bits to move down: 0 <= s < 128
-  const uint64_t lo = v[0] | ((uint64_t)v[1] << 32), hi = v[2] | ((uint64_t)v[3] << 32);
-  const uint64_t lo1 = (lo >> s1) | ((hi << 1) << (63 - s1)), hi1 = hi >> s1;
-  const uint64_t lo2 = s >= 64 ? hi1 : lo1, hi2 = s >= 64 ? 0 : hi1;
-  const u32x4 r = {inside ? (uint32_t)lo2 : 0u, inside ? (uint32_t)(lo2 >> 32) : 0u,
-                   inside ? (uint32_t)hi2 : 0u, inside ? (uint32_t)(hi2 >> 32) : 0u};
-  return r;
-}
+// (16-byte pieces at any alignment: tile::load_piece / tile::trim_piece in mfma_tile.h)
+using tile::load_piece;
+using tile::trim_piece;
 // The same piece element by element, for a matrix narrower than a piece.
 template <typename T>
 __device__ __forceinline__ u32x4 fetch_piece_narrow(const T* __restrict__ P, int64_t ld,

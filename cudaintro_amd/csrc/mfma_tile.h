@@ -208,6 +208,7 @@ struct BTile<B_KN32> {
   static constexpr int NREADS = 16;
   typedef uint32_t piece_t;
   static __device__ __forceinline__ int swz(int k) { return ((k >> 2) & 1) << 3; }
+  static __device__ __forceinline__ int off(int k, int c) { return k * 1024 + ((c ^ swz(k)) << 4); }
   static __device__ __forceinline__ int dma_lds(int w, int i) { return (4 * w + i) * 1024; }
   static __device__ __forceinline__ int dma_k(int w, int i, int) { return 4 * w + i; }
   static __device__ __forceinline__ int64_t dma_src(int w, int i, int l, int64_t ld, int last) {
@@ -237,6 +238,53 @@ __device__ __forceinline__ typename BTile<MODE>::piece_t read_b_piece(const char
   else
     return BTile<MODE>::frag_half(sb, wn, idx >> 1, kk, idx & 1, l);
 }
+
+// ---- operand pieces at any alignment ----------------------------------------------------------
+// One 16-byte piece = elements [col, col + CE) of row `row` of a row-major matrix with `rows`
+// rows of `cols` elements, zero outside the matrix, in two steps so that the load is one
+// unconditional instruction that can stay in flight while other work is done:
+// load_piece reads 16 bytes that lie inside the matrix whatever the piece (row clamped to the
+// last one; a piece that crosses the end of its row is replaced by the row's last 16 bytes),
+// trim_piece, applied when the value is needed, moves those down so that element `col` comes
+// first and zeroes what lies outside.  Needs cols >= CE.
+template <typename T>
+__device__ __forceinline__ u32x4 load_piece(const T* __restrict__ P, int64_t ld, int64_t row,
+                                            int64_t rows, int64_t col, int64_t cols) {
+  constexpr int CE = 16 / (int)sizeof(T);
+  const int64_t r = row < rows ? row : rows - 1;
+  const int64_t c = col + CE <= cols ? col : cols - CE;
+  u32x4 v;
+  __builtin_memcpy(&v, P + r * ld + c, 16);
+  return v;
+}
+template <typename T>
+__device__ __forceinline__ u32x4 trim_piece(u32x4 v, int64_t row, int64_t rows, int64_t col,
+                                            int64_t cols) {
+  constexpr int CE = 16 / (int)sizeof(T);
+  const bool inside = row < rows && col < cols;
+  const int s = col + CE > cols && inside ? (int)(col - (cols - CE)) * 8 * (int)sizeof(T) : 0;
+  const int s1 = s & 63;  // bits to move down: 0 <= s < 128
+  const uint64_t lo = v[0] | ((uint64_t)v[1] << 32), hi = v[2] | ((uint64_t)v[3] << 32);
+  const uint64_t lo1 = (lo >> s1) | ((hi << 1) << (63 - s1)), hi1 = hi >> s1;
+  const uint64_t lo2 = s >= 64 ? hi1 : lo1, hi2 = s >= 64 ? 0 : hi1;
+  const u32x4 r = {inside ? (uint32_t)lo2 : 0u, inside ? (uint32_t)(lo2 >> 32) : 0u,
+                   inside ? (uint32_t)hi2 : 0u, inside ? (uint32_t)(hi2 >> 32) : 0u};
+  return r;
+}
+template <int ELEM_BYTES>
+struct ElemOf;
+template <>
+struct ElemOf<1> {
+  typedef uint8_t type;
+};
+template <>
+struct ElemOf<2> {
+  typedef uint16_t type;
+};
+template <>
+struct ElemOf<4> {
+  typedef uint32_t type;  // fp32, moved as bits
+};
 
 // ---- arithmetic traits ----------------------------------------------------------------------
 struct MathBF16 {
@@ -374,6 +422,23 @@ __device__ __forceinline__ Epi epilogue_of_split(const Epi& e, int) { return e; 
 __device__ __forceinline__ EpiPartialX4 epilogue_of_split(const EpiPartialX4& e, int split) {
   return EpiPartialX4{e.base + split * e.split_stride, e.ld, e.split_stride};
 }
+template <typename Epi>
+struct epi_is_partial : std::is_same<Epi, EpiPartialX4> {};
+
+// What an epilogue needs for the four columns col..col+3 when only their elements' alignment is
+// known and the quad may cross the last column (columns beyond it get the last one's value).
+template <typename Epi>
+__device__ __forceinline__ typename Epi::col_t load_cols_any(const Epi& epi, int64_t col,
+                                                             int64_t N) {
+  if constexpr (std::is_same<typename Epi::col_t, f32x4>::value) {
+    f32x4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = epi.load_col(col + e < N ? col + e : N - 1);
+    return v;
+  } else {
+    return typename Epi::col_t{};
+  }
+}
 
 // The epilogue of the tile kernels: accumulators -> output rows.
 // acc[i][j][4q+e] = C[m0 + wm*32*MT + 32i + l%32][n0 + wn*128 + 32j + 8q + 4g + e]: a lane
@@ -381,7 +446,10 @@ __device__ __forceinline__ EpiPartialX4 epilogue_of_split(const EpiPartialX4& e,
 // at a time in its own piece of the (now idle) LDS and writes it out as whole rows: every
 // store instruction then covers full 256- or 512-byte row segments.  Call it once every wave
 // of the workgroup has stopped reading the operand ring and no DMA is in flight.
-template <typename Math, int MT, int NW, int TILE_M, typename Epi>
+// ANY: N, the rows of C and the per-column operands have their elements' alignment only.  A whole
+// 16-byte piece still leaves with one (unaligned) store; only the piece that crosses the last
+// column is stored element by element, from the staged block.
+template <typename Math, int MT, int NW, int TILE_M, bool ANY = false, typename Epi>
 __device__ __forceinline__ void store_tile(const Epi& epi, typename Math::acc_t (&acc)[MT][4],
                                            char* lds, int w, int wm, int wn, int64_t m0,
                                            int64_t n0, int M, int N, float epi_row_word,
@@ -422,7 +490,10 @@ __device__ __forceinline__ void store_tile(const Epi& epi, typename Math::acc_t 
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int64_t col = n0 + wn * 128 + 32 * j + 8 * q + 4 * ge;
-        colv[j][q] = epi.load_cols(col < N ? col : N - 4);
+        if constexpr (ANY)
+          colv[j][q] = load_cols_any(epi, col, N);
+        else
+          colv[j][q] = epi.load_cols(col < N ? col : N - 4);
       }
   }
   // Store side of the staging: lane -> (row within a pass, 16-byte piece of the 128-column row).
@@ -470,7 +541,36 @@ __device__ __forceinline__ void store_tile(const Epi& epi, typename Math::acc_t 
                                              c16 * 16);
     __builtin_amdgcn_sched_barrier(0);
     char* dst0 = epi.out_row(row0 + lane_row) + (n0 + wn * 128) * OB + c16 * 16;
-    if (interior) {
+    if constexpr (ANY) {
+      constexpr int PE = 16 / OB;  // elements of a piece
+      typedef typename std::conditional<OB == 2, uint16_t, uint32_t>::type out_t;
+      const int inside = (int)(N - piece_col);  // elements of this lane's piece inside the row
+      // (uniform) streaming stores where C's rows are aligned all the same: plain ones evict the
+      // operands (bf16 4096 x 4096 x 4095 106 against 115 us).  On unaligned rows the plain ones
+      // are the better, the L2 joins the two halves of a line (int8 -> int32 4096 x 4095 x 2047
+      // 55 against 59 us).
+      const bool rows_aligned = (((intptr_t)epi.out_row(0) | row_step) & 15) == 0;
+#pragma unroll
+      for (int p = 0; p < NPASS; ++p)
+        if (row0 + p * ROWS_PER_PASS + lane_row < M && inside >= PE) {
+          char* dst = dst0 + p * ROWS_PER_PASS * row_step;
+          if (rows_aligned)
+            __builtin_nontemporal_store(v[p], reinterpret_cast<u32x4*>(dst));
+          else
+            __builtin_memcpy(dst, &v[p], 16);
+        }
+      if (inside > 0 && inside < PE) {
+#pragma unroll 1
+        for (int p = 0; p < NPASS; ++p) {
+          if (row0 + p * ROWS_PER_PASS + lane_row >= M) break;
+          const out_t* from = reinterpret_cast<const out_t*>(
+              scr + (p * ROWS_PER_PASS + lane_row) * ROW_STRIDE + c16 * 16);
+          out_t* to = reinterpret_cast<out_t*>(dst0 + p * ROWS_PER_PASS * row_step);
+#pragma unroll 1
+          for (int e = 0; e < inside; ++e) to[e] = from[e];
+        }
+      }
+    } else if (interior) {
 #pragma unroll
       for (int p = 0; p < NPASS; ++p)
         // streaming stores: C is not read again by this kernel and should not evict A / B
@@ -499,7 +599,26 @@ __device__ __forceinline__ void store_tile(const Epi& epi, typename Math::acc_t 
 // whole number of 64-byte stages whenever there is more than one range, so only the last
 // range can be shorter than the others or leave its last stage partly filled (the pieces
 // past its end are fetched as zeros).  k_total_bytes is a multiple of 16.
-template <typename Math, int BMODE, int NSTAGES, int MT, typename Epi, int WM = 2>
+//
+// ANY: any M, N, K and leading dimensions, every matrix at its elements' alignment (needs K, and
+// the N of a K x N operand, to fill at least one 16-byte piece).  The LDS-DMA takes a 16-byte
+// piece from any byte address, so the ring, the main loop and the fragment reads stay what they
+// are; what changes is
+//   * K: the last 1..64 bytes of k (of the last K range) are multiplied first, from pieces loaded
+//     through registers with every bound checked (load_piece / trim_piece) and written to the
+//     ring slots the prologue's DMA leaves empty, so that their latency passes under it.  The
+//     rest is whole stages, and the DMA never touches the last k row of a K x N operand: a last
+//     piece of a row that spills past column N then reads the next row and stays in the matrix;
+//   * the epilogue (store_tile<ANY>).
+// Measured against the kernel that served these calls before (mfma_any_kernel: one 64-byte step
+// in flight between two barriers, every piece trimmed) and against aligned sizes: bf16 4096 x 4095
+// x 4096 264 -> 115 us (4096^3: 98), 8191 x 8192 at M = 2048 523 -> 219, at M = 1 31.5 -> 26.5;
+// int8 N x K 2048 x 8191 x 8191 342 -> 161; fp32 4095 x 4097 x 4099 1493 -> 981 (4096^3: 905).
+// What is left of the difference: a piece that is not 16-byte aligned takes the address path twice
+// (10 % per stage where one 16-bit operand is misaligned, 40 % where both int8 ones are), and so
+// do the stores of unaligned rows (10 us per 64 MiB).
+template <typename Math, int BMODE, int NSTAGES, int MT, typename Epi, int WM = 2,
+          bool ANY = false>
 __global__ __launch_bounds__(128 * WM, 1) void mfma_tile_kernel(int M, int N, int tiles_m,
                                                            int tiles_n, int k_range_bytes,
                                                            int k_total_bytes,
@@ -512,7 +631,10 @@ __global__ __launch_bounds__(128 * WM, 1) void mfma_tile_kernel(int M, int N, in
   // blockIdx.y = K range (split-K launches only): each starts a_split_step / b_split_step
   // bytes after the one before; k_bytes = bytes of k in this one, KTS = its stages
   const int k_left = k_total_bytes - (int)blockIdx.y * k_range_bytes;
-  const int k_bytes = k_left < k_range_bytes ? k_left : k_range_bytes;
+  // (ANY: the last range leaves its last 1..64 bytes of k to the tail: tail_bytes)
+  const int range_bytes = k_left < k_range_bytes ? k_left : k_range_bytes;
+  const int tail_bytes = ANY && k_left <= k_range_bytes ? (range_bytes - 1) % KB + 1 : 0;
+  const int k_bytes = range_bytes - tail_bytes;
   const int KTS = (k_bytes + KB - 1) / KB;
   const Epi epi = epilogue_of_split(epi_all, (int)blockIdx.y);
   A += blockIdx.y * a_split_step;
@@ -748,14 +870,79 @@ __global__ __launch_bounds__(128 * WM, 1) void mfma_tile_kernel(int M, int N, in
   // prologue, in the order the main loop keeps -- single B stages: B[0], A pair 0, B[1], B[2],
   // A pair 1; B pairs: B pair 0, A pair 0, B pair 1, A pair 1 -- then stage 0 landed and the
   // first fragments in registers
+  // (ANY with B pairs: the tail borrows the slots of the second pairs, which follow it; a K of at
+  // most 64 bytes is all tail)
+  auto prologue_first = [&]() {
 #pragma unroll
-  for (int d = 0; d < DMA_B + DMA_A; ++d) dma_piece(0, 0, 0, d, drain_t{});
-  if (!BPAIR) {
+    for (int d = 0; d < DMA_B + DMA_A; ++d) dma_piece(0, 0, 0, d, drain_t{});
+    if (!BPAIR) {
 #pragma unroll
-    for (int d = 0; d < DMA_B; ++d) dma_piece(1, 1, 0, d, drain_t{});
+      for (int d = 0; d < DMA_B; ++d) dma_piece(1, 1, 0, d, drain_t{});
+    }
+  };
+  auto prologue_second = [&]() {
+#pragma unroll
+    for (int d = 0; d < DMA_B + DMA_A; ++d) dma_piece(2, BPAIR ? 1 : 2, 1, d, drain_t{});
+  };
+  if constexpr (ANY) {
+    if (KTS > 0) prologue_first();
+    if (!BPAIR && KTS > 0) prologue_second();
+    if (tail_bytes > 0) {
+      constexpr int THREADS = 64 * NW, CE = 16 / Math::ELEM_BYTES;
+      constexpr int PA = TILE_M * 4 / THREADS, PB = 1024 / THREADS;
+      constexpr int KN_CHUNKS = 16 * Math::ELEM_BYTES;  // 16-byte pieces of a K x N tile row
+      constexpr int B_SLOT = BPAIR ? 1 : NSTAGES - 1;
+      constexpr int B_SLOT_AT = B_SLOT * (BPAIR ? BPAIR_BYTES : OPERAND_BYTES);
+      typedef typename ElemOf<Math::ELEM_BYTES>::type elem_t;
+      const elem_t* Ae = reinterpret_cast<const elem_t*>(A);
+      const elem_t* Be = reinterpret_cast<const elem_t*>(B);
+      const int64_t lda_e = lda / Math::ELEM_BYTES, ldb_e = ldb / Math::ELEM_BYTES;
+      const int64_t k0 = k_bytes / Math::ELEM_BYTES, k_end = range_bytes / Math::ELEM_BYTES;
+      u32x4 ta[PA], tb[PB];
+#pragma unroll
+      for (int i = 0; i < PA; ++i) {
+        const int c = t + THREADS * i;
+        ta[i] = load_piece(Ae, lda_e, m0 + (c >> 2), M, k0 + (c & 3) * CE, k_end);
+      }
+#pragma unroll
+      for (int i = 0; i < PB; ++i) {
+        const int c = t + THREADS * i;
+        if constexpr (BPAIR)
+          tb[i] = load_piece(Be, ldb_e, n0 + (c >> 2), N, k0 + (c & 3) * CE, k_end);
+        else
+          tb[i] = load_piece(Be, ldb_e, k0 + c / KN_CHUNKS, k_end, n0 + (c % KN_CHUNKS) * CE, N);
+      }
+#pragma unroll
+      for (int i = 0; i < PA; ++i) {
+        const int c = t + THREADS * i;
+        *reinterpret_cast<u32x4*>(lds + B_RING + 2 * APAIR_BYTES + pair_off(c >> 2, c & 3)) =
+            trim_piece<elem_t>(ta[i], m0 + (c >> 2), M, k0 + (c & 3) * CE, k_end);
+      }
+#pragma unroll
+      for (int i = 0; i < PB; ++i) {
+        const int c = t + THREADS * i;
+        if constexpr (BPAIR)
+          *reinterpret_cast<u32x4*>(lds + B_SLOT_AT + pair_off(c >> 2, c & 3)) =
+              trim_piece<elem_t>(tb[i], n0 + (c >> 2), N, k0 + (c & 3) * CE, k_end);
+        else
+          *reinterpret_cast<u32x4*>(lds + B_SLOT_AT + BT::off(c / KN_CHUNKS, c % KN_CHUNKS)) =
+              trim_piece<elem_t>(tb[i], k0 + c / KN_CHUNKS, k_end, n0 + (c % KN_CHUNKS) * CE, N);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk) {
+#pragma unroll
+        for (int r = 0; r < NREAD; ++r) read_piece(f0, B_SLOT, 2, 0, kk, r);
+#pragma unroll
+        for (int m = 0; m < NMFMA; ++m) mfma_piece(f0, m);
+      }
+      if (BPAIR) __syncthreads();
+    }
+    if (BPAIR && KTS > 0) prologue_second();
+  } else {
+    prologue_first();
+    prologue_second();
   }
-#pragma unroll
-  for (int d = 0; d < DMA_B + DMA_A; ++d) dma_piece(2, BPAIR ? 1 : 2, 1, d, drain_t{});
   wait_vmcnt(std::integral_constant<int, BPAIR ? DMA_B + DMA_A : 2 * DMA_B + DMA_A>{});
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
@@ -926,8 +1113,16 @@ __global__ __launch_bounds__(128 * WM, 1) void mfma_tile_kernel(int M, int N, in
   stamp(2);
 
   // ---- epilogue -----------------------------------------------------------------------------
-  store_tile<Math, MT, NW, TILE_M>(epi, acc, lds, w, wm, wn, m0, n0, M, N, epi_row_word,
-                                   epi_col_word);
+  // (the rows of a partial matrix are whole aligned pieces whatever N is)
+  if constexpr (ANY && !epi_is_partial<Epi>::value)
+    store_tile<Math, MT, NW, TILE_M, true>(epi, acc, lds, w, wm, wn, m0, n0, M, N, epi_row_word,
+                                           epi_col_word);
+  else if constexpr (ANY)
+    store_tile<Math, MT, NW, TILE_M>(epi, acc, lds, w, wm, wn, m0, n0, M, (int)epi.ld,
+                                     epi_row_word, epi_col_word);
+  else
+    store_tile<Math, MT, NW, TILE_M>(epi, acc, lds, w, wm, wn, m0, n0, M, N, epi_row_word,
+                                     epi_col_word);
   if constexpr (epi_profiled<Epi>::value) {
     // the epilogue ends when this wave's stores have been acknowledged
     wait_vmcnt(std::integral_constant<int, 0>{});
@@ -938,7 +1133,7 @@ __global__ __launch_bounds__(128 * WM, 1) void mfma_tile_kernel(int M, int N, in
 constexpr int DEFAULT_STAGES = 4;
 
 // `splits` must be a value k_ranges() returned for this K (1 = the whole of K in one range).
-template <typename Math, int BMODE, int MT, typename Epi, int WM = 2>
+template <typename Math, int BMODE, int MT, typename Epi, int WM = 2, bool ANY = false>
 void launch_tile_mt(cigemmContext* ctx, int64_t M, int64_t N, int64_t K_bytes, const void* A,
                     int64_t lda_bytes, const void* B, int64_t ldb_bytes, const Epi& epi,
                     int splits = 1) {
@@ -947,7 +1142,7 @@ void launch_tile_mt(cigemmContext* ctx, int64_t M, int64_t N, int64_t K_bytes, c
   constexpr int RING_BYTES = NSTAGES * OPERAND_BYTES + 3 * (TILE_M * 128);
   constexpr int STAGING_BYTES = 2 * WM * 32 * (128 * Epi::OUT_BYTES + 16);   // epilogue, per wave
   constexpr int LDS_BYTES = RING_BYTES > STAGING_BYTES ? RING_BYTES : STAGING_BYTES;
-  auto kern = mfma_tile_kernel<Math, BMODE, NSTAGES, MT, Epi, WM>;
+  auto kern = mfma_tile_kernel<Math, BMODE, NSTAGES, MT, Epi, WM, ANY>;
   static std::atomic<uint64_t> lds_set{0};  // one per template instance
   if (!ensure_dynamic_lds(ctx, (const void*)kern, LDS_BYTES, lds_set)) return;
   const int tiles_m = (int)((M + TILE_M - 1) / TILE_M), tiles_n = (int)((N + BN - 1) / BN);
@@ -967,17 +1162,45 @@ void launch_tile_mt(cigemmContext* ctx, int64_t M, int64_t N, int64_t K_bytes, c
                      static_cast<const char*>(B), ldb_bytes, epi, a_step, b_step);
 }
 
+// Four columns of one output row at any N and alignment: packed as the tile kernel packs them,
+// stored as one unaligned piece, or element by element when the quad crosses the last column.
+template <typename Epi, typename Scalar>
+__device__ __forceinline__ void store_quad_any(const Epi& epi, int64_t r, int64_t c, int64_t N,
+                                               const Scalar (&v)[4]) {
+  const auto p = epi.pack(epi.load_row(r), load_cols_any(epi, c, N), v[0], v[1], v[2], v[3]);
+  char* to = epi.out_row(r) + c * Epi::OUT_BYTES;
+  if (c + 4 <= N) {
+    __builtin_memcpy(to, &p, sizeof(p));
+  } else {
+#pragma unroll
+    for (int e = 0; e < 3; ++e)
+      if (c + e < N) {
+        if constexpr (Epi::OUT_BYTES == 2)
+          reinterpret_cast<uint16_t*>(to)[e] = (uint16_t)(p[e / 2] >> (16 * (e & 1)));
+        else
+          reinterpret_cast<uint32_t*>(to)[e] = p[e];
+      }
+  }
+}
+
+// Row pitch, in elements, of the partial matrices: N, or (ANY) the next multiple of a cache line.
+template <bool ANY>
+constexpr int64_t partial_ld(int64_t N) {
+  return ANY ? (N + 31) / 32 * 32 : N;
+}
+
 // Second half of a split-K GEMM: sums the `splits` partial matrices in split order (the
 // result does not depend on timing) and applies the real epilogue, four columns per lane.
-template <typename Scalar, typename Epi>
+template <typename Scalar, typename Epi, bool ANY = false>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(int M, int N, int splits,
                                                             const uint32_t* __restrict__ part,
                                                             int64_t split_stride, Epi epi) {
-  const int64_t quads_per_row = N / 4, quads = (int64_t)M * quads_per_row;
+  const int64_t quads_per_row = ((int64_t)N + 3) / 4, quads = (int64_t)M * quads_per_row;
+  const int64_t part_ld = partial_ld<ANY>(N);
   for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < quads;
        q += (int64_t)gridDim.x * 256) {
     const int64_t r = q / quads_per_row, c = (q % quads_per_row) * 4;
-    const uint32_t* p = part + r * N + c;
+    const uint32_t* p = part + r * part_ld + c;
     // (element-wise: a bit cast applied directly to a vector element misreads it)
     auto as_scalar = [](uint32_t bits) { return __builtin_bit_cast(Scalar, bits); };
     // (up to seven splits are read before the first add waits for one: the loop is otherwise
@@ -1004,7 +1227,10 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(int M, int N, int sp
           }
         }
     }
-    epi(r, c, sum[0], sum[1], sum[2], sum[3]);
+    if constexpr (ANY)
+      store_quad_any(epi, r, c, N, sum);
+    else
+      epi(r, c, sum[0], sum[1], sum[2], sum[3]);
   }
 }
 
@@ -1033,69 +1259,70 @@ struct epi_register_heavy<E, typename std::enable_if<E::REGISTER_HEAVY>::type> :
 // bench's data: bf16 8192^3 -0.1..+0.3 % for four waves, int8 N x K 8192^3 +-0.3 %, bf16 4096^3
 // (one round) +1.1 %, int8 N x K 4096^3 -> int32 +6.8 %; only N x K int8 weights with a 16-bit
 // output keep the eight waves (2048 x 11008 x 4096 at M = 1024, one round: 44.0 against 44.8 us).
-template <typename Math, int BMODE, typename Epi>
+template <typename Math, int BMODE, bool ANY = false, typename Epi>
 void launch_tile_256(cigemmContext* ctx, int64_t M, int64_t N, int64_t K_bytes, const void* A,
                      int64_t lda_bytes, const void* B, int64_t ldb_bytes, const Epi& epi,
                      int splits = 1) {
   if constexpr (BMODE == B_NK && Epi::OUT_BYTES == 2 && !epi_register_heavy<Epi>::value)
-    launch_tile_mt<Math, BMODE, 2, Epi, 4>(ctx, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, epi,
+    launch_tile_mt<Math, BMODE, 2, Epi, 4, ANY>(ctx, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, epi,
                                            splits);
   else
-    launch_tile_mt<Math, BMODE, 4, Epi, 2>(ctx, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, epi,
+    launch_tile_mt<Math, BMODE, 4, Epi, 2, ANY>(ctx, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, epi,
                                            splits);
 }
 
 // The 128-row tile has the same two forms (four waves of 64 x 128, eight of 32 x 128); with
 // N x K int8 weights the second is 9 % faster (2048 x 11008 x 4096: 108 -> 98 us), with K x N
 // operands 2 % slower (their transposing fragment reads are twice as many instructions).
-template <typename Math, int BMODE, typename Epi>
+template <typename Math, int BMODE, bool ANY = false, typename Epi>
 void launch_tile_128(cigemmContext* ctx, int64_t M, int64_t N, int64_t K_bytes, const void* A,
                      int64_t lda_bytes, const void* B, int64_t ldb_bytes, const Epi& epi,
                      int splits = 1) {
   if constexpr (BMODE == B_NK && !epi_register_heavy<Epi>::value)
-    launch_tile_mt<Math, BMODE, 1, Epi, 4>(ctx, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, epi,
+    launch_tile_mt<Math, BMODE, 1, Epi, 4, ANY>(ctx, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, epi,
                                            splits);
   else
-    launch_tile_mt<Math, BMODE, 2, Epi, 2>(ctx, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, epi,
+    launch_tile_mt<Math, BMODE, 2, Epi, 2, ANY>(ctx, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, epi,
                                            splits);
 }
 
-template <typename Math, int BMODE, typename Epi>
+template <typename Math, int BMODE, bool ANY = false, typename Epi>
 void launch_tile_any_mt(cigemmContext* ctx, int mt, int64_t M, int64_t N, int64_t K_bytes,
                         const void* A, int64_t lda_bytes, const void* B, int64_t ldb_bytes,
                         const Epi& epi, int splits = 1) {
   if (mt == 4)
-    launch_tile_256<Math, BMODE>(ctx, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, epi, splits);
+    launch_tile_256<Math, BMODE, ANY>(ctx, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, epi, splits);
   else if (mt == 3)
-    launch_tile_mt<Math, BMODE, 3>(ctx, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, epi, splits);
+    launch_tile_mt<Math, BMODE, 3, Epi, 2, ANY>(ctx, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, epi, splits);
   else if (mt == 2)
-    launch_tile_128<Math, BMODE>(ctx, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, epi, splits);
+    launch_tile_128<Math, BMODE, ANY>(ctx, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, epi, splits);
   else
-    launch_tile_mt<Math, BMODE, 1>(ctx, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, epi, splits);
+    launch_tile_mt<Math, BMODE, 1, Epi, 2, ANY>(ctx, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, epi, splits);
 }
 
 // Runs one plan: tiles of 64*mt rows; with more than one K range the ranges go over
 // blockIdx.y, partial sums to the workspace, then one reduction launch with the real epilogue.
 // Returns true when it ran as such a pair of launches.
-template <typename Math, int BMODE, typename Epi>
+template <typename Math, int BMODE, bool ANY = false, typename Epi>
 bool run_tile_plan(cigemmContext* ctx, int mt, int splits, int64_t M, int64_t N, int64_t K_bytes,
                    const void* A, int64_t lda_bytes, const void* B, int64_t ldb_bytes,
                    const Epi& epi) {
   if (splits <= 1) {
-    launch_tile_any_mt<Math, BMODE>(ctx, mt, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, epi);
+    launch_tile_any_mt<Math, BMODE, ANY>(ctx, mt, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, epi);
     return false;
   }
   typedef typename Math::scalar_t scalar_t;
   const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
   uint32_t* ws = static_cast<uint32_t*>(ctx->workspace);
-  const EpiPartialX4 part{ws, N, M * N};
-  launch_tile_any_mt<Math, BMODE>(ctx, mt, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, part,
+  const int64_t ld = partial_ld<ANY>(N);
+  const EpiPartialX4 part{ws, ld, M * ld};
+  launch_tile_any_mt<Math, BMODE, ANY>(ctx, mt, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, part,
                                   splits);
-  const int64_t quads = M * (N / 4);
+  const int64_t quads = M * ((N + 3) / 4);
   const unsigned grid = (unsigned)((quads + 255) / 256 < 4 * (int64_t)cus ? (quads + 255) / 256
                                                                           : 4 * (int64_t)cus);
-  hipLaunchKernelGGL((splitk_reduce_kernel<scalar_t, Epi>), dim3(grid), dim3(256), 0, ctx->stream,
-                     (int)M, (int)N, ctx->last_k_splits, ws, M * N, epi);
+  hipLaunchKernelGGL((splitk_reduce_kernel<scalar_t, Epi, ANY>), dim3(grid), dim3(256), 0, ctx->stream,
+                     (int)M, (int)N, ctx->last_k_splits, ws, M * ld, epi);
   return true;
 }
 
@@ -1104,7 +1331,7 @@ bool run_tile_plan(cigemmContext* ctx, int mt, int splits, int64_t M, int64_t N,
 // columns with a second launch of shorter tiles.  Epi::shift_cols(c) returns the epilogue of
 // the sub-problem starting at column c.
 // Returns true when the problem was run as a split-K pair of launches.
-template <typename Math, int BMODE, typename Epi>
+template <typename Math, int BMODE, bool ANY = false, typename Epi>
 bool launch_tile(cigemmContext* ctx, int64_t M, int64_t N, int64_t K_bytes, const void* A,
                  int64_t lda_bytes, const void* B, int64_t ldb_bytes, const Epi& epi) {
   const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
@@ -1114,9 +1341,9 @@ bool launch_tile(cigemmContext* ctx, int64_t M, int64_t N, int64_t K_bytes, cons
     int64_t range_stages = 0;
     int sp = k_ranges(K_bytes, ctx->force_tile_splits, &range_stages);
     if (sp > 1 && (!ctx->workspace ||
-                   (size_t)sp * (size_t)M * (size_t)N * 4 > ctx->ws_partial_bytes))
+                   (size_t)sp * (size_t)M * (size_t)partial_ld<ANY>(N) * 4 > ctx->ws_partial_bytes))
       sp = 1;
-    return run_tile_plan<Math, BMODE>(ctx, ctx->force_tile_mt, sp, M, N, K_bytes, A, lda_bytes, B,
+    return run_tile_plan<Math, BMODE, ANY>(ctx, ctx->force_tile_mt, sp, M, N, K_bytes, A, lda_bytes, B,
                                       ldb_bytes, epi);
   }
   double single = 0;
@@ -1126,9 +1353,9 @@ bool launch_tile(cigemmContext* ctx, int64_t M, int64_t N, int64_t K_bytes, cons
     // At most one round of 256-row tiles: pick the tile height and the number of K ranges
     // together.
     const SmallPlan plan =
-        plan_small(cus, ctx->workspace ? ctx->ws_partial_bytes : 0, M, N, K_bytes, Epi::OUT_BYTES,
+        plan_small(cus, ctx->workspace ? ctx->ws_partial_bytes : 0, M, partial_ld<ANY>(N), K_bytes, Epi::OUT_BYTES,
                    stage_cost<Math, BMODE>(), K_bytes * N);
-    return run_tile_plan<Math, BMODE>(ctx, plan.mt, plan.splits, M, N, K_bytes, A, lda_bytes, B,
+    return run_tile_plan<Math, BMODE, ANY>(ctx, plan.mt, plan.splits, M, N, K_bytes, A, lda_bytes, B,
                                       ldb_bytes, epi);
   }
   {
@@ -1151,19 +1378,19 @@ bool launch_tile(cigemmContext* ctx, int64_t M, int64_t N, int64_t K_bytes, cons
         // two rounds against 256 tiles of 256 rows + 176 of 128 rows, alternating in one process:
         // 85.3 against 86.0 us)
         if (tile_plan_cost(M, n1, 4, cus, units) + rest < single * 0.97) {
-          launch_tile_256<Math, BMODE>(ctx, M, n1, K_bytes, A, lda_bytes, B, ldb_bytes, epi);
+          launch_tile_256<Math, BMODE, ANY>(ctx, M, n1, K_bytes, A, lda_bytes, B, ldb_bytes, epi);
           const int rows1 = ctx->last_tile_rows, waves1 = ctx->last_waves;
           const char* B2 = static_cast<const char*>(B) +
                            (BMODE == B_NK ? n1 * ldb_bytes : n1 * Math::ELEM_BYTES);
           bool split = false;
           if (tiles_m * ((n2 + BN - 1) / BN) <= cus) {
             const SmallPlan plan =
-                plan_small(cus, ctx->workspace ? ctx->ws_partial_bytes : 0, M, n2, K_bytes,
+                plan_small(cus, ctx->workspace ? ctx->ws_partial_bytes : 0, M, partial_ld<ANY>(n2), K_bytes,
                            Epi::OUT_BYTES, stage_cost<Math, BMODE>(), K_bytes * n2);
-            split = run_tile_plan<Math, BMODE>(ctx, plan.mt, plan.splits, M, n2, K_bytes, A,
+            split = run_tile_plan<Math, BMODE, ANY>(ctx, plan.mt, plan.splits, M, n2, K_bytes, A,
                                                lda_bytes, B2, ldb_bytes, epi.shift_cols(n1));
           } else {
-            launch_tile_any_mt<Math, BMODE>(ctx, mt2, M, n2, K_bytes, A, lda_bytes, B2, ldb_bytes,
+            launch_tile_any_mt<Math, BMODE, ANY>(ctx, mt2, M, n2, K_bytes, A, lda_bytes, B2, ldb_bytes,
                                             epi.shift_cols(n1));
           }
           ctx->first_tile_rows = rows1;
@@ -1173,7 +1400,7 @@ bool launch_tile(cigemmContext* ctx, int64_t M, int64_t N, int64_t K_bytes, cons
       }
     }
   }
-  launch_tile_any_mt<Math, BMODE>(ctx, mt, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, epi);
+  launch_tile_any_mt<Math, BMODE, ANY>(ctx, mt, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, epi);
   return false;
 }
 
@@ -1193,6 +1420,16 @@ inline bool tile_shape_ok(int64_t M, int64_t N, int64_t K, int elem, const void*
   if (((M + 63) / 64) * ((N + BN - 1) / BN) > 2147483647LL) return false;
   if (lda * elem * 256 >= (1LL << 31) || ldb * elem * 256 >= (1LL << 31)) return false;
   return true;
+}
+
+// The gate of the ANY form: sizes only.  One 16-byte piece must fit a row of either operand (and a
+// column of k); the launch-size and 32-bit offset limits are those above.
+inline bool tile_any_ok(int64_t M, int64_t N, int64_t K, int elem, int64_t lda, int64_t ldb,
+                        bool b_kn) {
+  if (M <= 0 || N <= 0 || K * elem < 16 || (b_kn && N * elem < 16)) return false;
+  if (M > 2147483647LL - 255 || N > 2147483647LL - 255 || K * elem > 2147483647LL) return false;
+  if (((M + 63) / 64) * ((N + BN - 1) / BN) > 2147483647LL) return false;
+  return lda * elem * 256 < (1LL << 31) && ldb * elem * 256 < (1LL << 31);
 }
 
 // The int8 tile kernels' gate: the shape gate above plus what their epilogues store in 16-byte

@@ -98,9 +98,11 @@ inline double plan_us(int64_t M, int64_t N, int64_t K_bytes, int out_bytes, Stag
   return us;
 }
 
-// `partial_bytes` = room for partial sums (0: no split plans).
+// `partial_bytes` = room for partial sums (0: no split plans).  `est_us`, if given, receives the
+// estimate of the plan returned.
 inline SmallPlan plan_small(int cus, size_t partial_bytes, int64_t M, int64_t N, int64_t K_bytes,
-                            int out_bytes, StageCost sc, int64_t b_bytes) {
+                            int out_bytes, StageCost sc, int64_t b_bytes,
+                            double* est_us = nullptr) {
   const bool streamed = b_bytes > (16LL << 20);
   if (cus <= 0) cus = 256;
   SmallPlan best{0, 1};
@@ -126,6 +128,7 @@ inline SmallPlan plan_small(int cus, size_t partial_bytes, int64_t M, int64_t N,
       }
     }
   }
+  if (est_us) *est_us = best_us;
   return best;
 }
 

@@ -148,9 +148,9 @@ typedef enum cigemmAlgo {
                               K x N); M <= 64 for K x N weights of at least 4096 x 2048 in
                               whole 128-column slabs */
   CIGEMM_ALGO_SMALL = 3,   /* fp32 32x32 tile per workgroup, k split over the waves */
-  CIGEMM_ALGO_MFMA_ANY = 4 /* 128x128 MFMA tiles fed by bounds-checked loads and stores at element
-                              alignment: any shape, leading dimension and alignment, every type.
-                              DEFAULT uses it for what the families above do not take */
+  CIGEMM_ALGO_MFMA_ANY = 4 /* MFMA tiles at element alignment: any shape, leading dimension and
+                              alignment, every type.  DEFAULT uses it for what the families
+                              above do not take */
 } cigemmAlgo_t;
 CIGEMM_API cigemmStatus_t cigemmSetAlgo(cigemmHandle_t handle, cigemmAlgo_t algo);
 CIGEMM_API cigemmStatus_t cigemmGetAlgo(cigemmHandle_t handle, cigemmAlgo_t* algo);

@@ -1,0 +1,80 @@
+"""The tile kernel at any alignment, at the sizes where it can go wrong: every tile height, K
+around its 64-byte stages (all of K in the separately multiplied tail, one stage, an odd and an
+even number of them, a tail of one element up to a whole stage), one and several K ranges (a last
+range that is only tail among them), edge and interior tiles, every operand off by an element.
+Operand values are small integers and halves, so every sum is exact and the comparison is bit for
+bit; the padding around the operands is NaN (127 for int8), the output sits in a sentinel-filled
+buffer."""
+import numpy as np
+import pytest
+
+import cudaintro_amd as ci
+from cudaintro_amd import probe
+from gpu_util import bits
+from test_gpu_mfma_any import VALS, embed
+
+pytestmark = pytest.mark.gpu
+M, N = 300, 521
+BYTES = {"bf16": 2, "f16": 2, "f32": 4, "i8_kn": 1, "i8_nk": 1}
+
+
+def sizes_of_k(eb):
+    stage = 64 // eb
+    return [16 // eb, stage, stage + 1, 2 * stage, 2 * stage + 1, 13 * stage + 3, 25 * stage - 1]
+
+
+@pytest.mark.parametrize("rows", [256, 192, 128, 64])
+@pytest.mark.parametrize("kind", list(BYTES))
+def test_tile_any(handle, torch_gpu, oracle, rng, kind, rows):
+    torch = torch_gpu
+    int8 = kind.startswith("i8")
+    layout = ci.B_NK if kind == "i8_nk" else ci.B_KN
+    for K in sizes_of_k(BYTES[kind]):
+        if int8:
+            A = rng.integers(-127, 128, size=(M, K), dtype=np.int8)
+            B = rng.integers(-127, 128, size=(N, K) if layout == ci.B_NK else (K, N), dtype=np.int8)
+            dt, odt, pad, ref = torch.int8, torch.int32, 127, oracle.gemm_i8_i32(A, B, b_is_nk=layout == ci.B_NK)
+        else:
+            A, B = rng.choice(VALS, size=(M, K)), rng.choice(VALS, size=(K, N))
+            ref = oracle.gemm_f32(A, B)
+            dt = odt = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[kind]
+            pad = float("nan")
+            narrow = {"bf16": oracle.f32_to_bf16, "f16": oracle.f32_to_f16}.get(kind)
+            if narrow:
+                A, B, ref = narrow(A).view(np.int16), narrow(B).view(np.int16), narrow(ref)
+        _, a = embed(torch, A, dt, 1, 3, pad)
+        _, b = embed(torch, B, dt, 3, 1, pad)
+        flat, out = embed(torch, np.zeros((M, N), np.int32).astype(np.int16 if odt.itemsize == 2 else np.int32),
+                          odt, 1, 5, 0)
+        guard = np.ones(flat.numel(), bool)
+        for i in range(M):
+            guard[1 + i * (N + 5): 1 + i * (N + 5) + N] = False
+        host = lambda t: bits(torch, t) if t.element_size() == 2 else t.contiguous().cpu().numpy()  # noqa: E731
+        for ranges in (1, 3):
+            flat.fill_(7)
+            sentinel = host(flat)[0]
+            probe.force_tile_plan(handle, rows, ranges)
+            try:
+                with handle.algo(ci.ALGO_MFMA_ANY):
+                    if int8:
+                        handle.gemm_i8_i32(a, b, layout, out=out)
+                    else:
+                        getattr(handle, "gemm_" + kind)(a, b, out=out)
+                    assert f"_mfma_any_{rows}x256" in handle.last_kernel, handle.last_kernel
+                    np.testing.assert_array_equal(host(out), ref, err_msg=f"K={K} ranges={ranges}")
+                    assert (host(flat)[guard] == sentinel).all()
+                    if int8:
+                        sa = rng.uniform(1e-3, 5e-2, M).astype(np.float32)
+                        sb = rng.uniform(1e-3, 5e-2, N).astype(np.float32)
+                        for name, ot in (("f32", ci.OUT_F32), ("bf16", ci.OUT_BF16)):
+                            y = handle.gemm_i8_dequant(a, b, torch.from_numpy(sa).cuda(),
+                                                       torch.from_numpy(sb).cuda(), layout, ot)
+                            np.testing.assert_array_equal(
+                                host(y), oracle.dequant(ref, sa, sb, out_dtype=name, sa_per_row=True,
+                                                        sb_per_col=True))
+                    elif kind == "f32":
+                        bias = rng.choice(VALS, size=N)
+                        y = handle.linear_f32(a, b, torch.from_numpy(bias).cuda(), ci.ACT_RELU)
+                        np.testing.assert_array_equal(host(y), oracle.linear_f32(A, B, bias, True))
+            finally:
+                probe.force_tile_plan(handle, 0)
