@@ -146,57 +146,99 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(int64_t cols,
   }
 }
 
-// The same for rows of whole 16-byte pieces (cols a multiple of 4, aligned rows) of up to
-// 1024 * CHUNKS columns: a lane keeps its CHUNKS pieces of the row in registers, so the row is
-// read once, as 16-byte loads, and written as packed 4-byte stores.  Same arithmetic per
-// element as the kernel above (the maximum does not depend on the order it is taken in).
-template <int CHUNKS>
-__global__ __launch_bounds__(256) void quantize_rows_vec_kernel(int64_t cols,
-                                                                const float* __restrict__ x,
-                                                                int64_t ldx,
-                                                                int8_t* __restrict__ q,
-                                                                int64_t ldq,
-                                                                float* __restrict__ scale) {
-  __shared__ float red[4];
+// The same for rows of up to 16384 columns, of any length and alignment: THREADS lanes keep their
+// CHUNKS 16-byte pieces of the row in registers, so the row is read once.  Same bytes per element
+// as the kernel above (the maximum does not depend on the order it is taken in).
+//
+// The correctly rounded quotient costs about ten instructions an element, several of them at a
+// quarter of the rate, and with one row per workgroup it starts only when the whole row has
+// arrived.  So the quotient is first estimated as t = x * (1/s): both roundings together put t
+// within 127 * 2^-22 = 3.1e-5 of the correctly rounded quotient, so the two round to the same
+// whole number unless t lies that close to a half.  Pieces with an element within 1e-4 of a half,
+// or a NaN, are divided (one wave of 64 pieces in twenty).  s outside 2^-100..2^100, where 1/s
+// or t could leave the normal range, is divided throughout.
+//
+// Bound: HBM (8192 x 8192 in 58.8 us = 5.7 TB/s of 5 bytes an element).  Before, rows that are not
+// whole aligned 16-byte pieces were read twice, element by element, and every element was divided:
+// 8192 x 8190 130.6 -> 59.1 us, 2048 x 4095 14.2 -> 7.5; whole pieces 2048 x 4096 7.9 -> 7.1,
+// 512 x 16384 8.8 -> 8.0.
+template <int THREADS, int CHUNKS>
+__global__ __launch_bounds__(THREADS) void quantize_rows_vec_kernel(int cols,
+                                                                    const float* __restrict__ x,
+                                                                    int64_t ldx,
+                                                                    int8_t* __restrict__ q,
+                                                                    int64_t ldq,
+                                                                    float* __restrict__ scale) {
+  constexpr int WAVES = THREADS / 64;
+  __shared__ float red[WAVES];
   const int64_t row = blockIdx.x;
-  const f32x4* xr = reinterpret_cast<const f32x4*>(x + row * ldx);
-  uint32_t* qr = reinterpret_cast<uint32_t*>(q + row * ldq);
-  const int nquad = (int)(cols >> 2);
+  const float* xr = x + row * ldx;
+  int8_t* qr = q + row * ldq;
   f32x4 v[CHUNKS];
   float amax = 0.0f;
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c) {
-    const int i = threadIdx.x + 256 * c;
-    v[c] = i < nquad ? xr[i] : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    const int j = 4 * ((int)threadIdx.x + THREADS * c);
+    v[c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    if (j + 4 <= cols) {
+      __builtin_memcpy(&v[c], xr + j, 16);  // rows need not be 16-byte aligned
+    } else {
+#pragma unroll
+      for (int e = 0; e < 3; ++e)
+        if (j + e < cols) v[c][e] = xr[j + e];
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c)
 #pragma unroll
     for (int e = 0; e < 4; ++e) amax = fmaxf(amax, fabsf(v[c][e]));
-  }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = amax;
   __syncthreads();
-  amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  amax = red[0];
+#pragma unroll
+  for (int w = 1; w < WAVES; ++w) amax = fmaxf(amax, red[w]);
   const float s = amax > 0.0f ? __fdiv_rn(amax, 127.0f) : 1.0f;
   if (threadIdx.x == 0) scale[row] = s;
+  const bool estimate = s >= 0x1p-100f && s <= 0x1p100f;
+  const float inv = __fdiv_rn(1.0f, s);
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c) {
-    const int i = threadIdx.x + 256 * c;
+    float r[4];
+    bool sure = estimate;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float t = v[c][e] * inv;
+      r[e] = rintf(t);
+      sure = sure && fabsf(t - r[e]) <= 0.4999f;
+    }
+    if (!sure) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) r[e] = rintf(__fdiv_rn(v[c][e], s));  // ties to even
+    }
     uint32_t packed = 0;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      float r = rintf(__fdiv_rn(v[c][e], s));  // ties to even
-      r = fminf(fmaxf(r, -127.0f), 127.0f);
-      packed |= ((uint32_t)(int)r & 0xffu) << (8 * e);
+      r[e] = fminf(fmaxf(r[e], -127.0f), 127.0f);
+      packed |= ((uint32_t)(int)r[e] & 0xffu) << (8 * e);
     }
-    if (i < nquad) qr[i] = packed;
+    const int j = 4 * ((int)threadIdx.x + THREADS * c);
+    if (j + 4 <= cols) {
+      __builtin_memcpy(qr + j, &packed, 4);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 3; ++e)
+        if (j + e < cols) qr[j + e] = (int8_t)(packed >> (8 * e));
+    }
   }
 }
 
-template <int CHUNKS>
+template <int THREADS, int CHUNKS>
 void launch_quantize_vec(cigemmContext* ctx, int64_t rows, int64_t cols, const float* x,
                          int64_t ldx, int8_t* q, int64_t ldq, float* scale) {
-  hipLaunchKernelGGL((quantize_rows_vec_kernel<CHUNKS>), dim3((unsigned)rows), dim3(256), 0,
-                     ctx->stream, cols, x, ldx, q, ldq, scale);
+  hipLaunchKernelGGL((quantize_rows_vec_kernel<THREADS, CHUNKS>), dim3((unsigned)rows),
+                     dim3(THREADS), 0, ctx->stream, (int)cols, x, ldx, q, ldq, scale);
 }
 
 }  // namespace
@@ -263,21 +305,28 @@ cigemmStatus_t cigemm_quantize_rows_i8(cigemmHandle_t h, int64_t rows, int64_t c
     return fail(h, CIGEMM_STATUS_INVALID_VALUE, "cigemm_quantize_rows_i8: ld < cols");
   if (rows > 2147483647LL)
     return fail(h, CIGEMM_STATUS_NOT_SUPPORTED, "cigemm_quantize_rows_i8: rows > 2^31-1");
-  const bool pieces = cols > 0 && cols % 4 == 0 && ldx % 4 == 0 && ldq % 4 == 0 &&
-                      ((uintptr_t)x & 15) == 0 && ((uintptr_t)q & 3) == 0 && cols <= 16384;
-  if (pieces && cols <= 1024)
-    launch_quantize_vec<1>(h, rows, cols, x, ldx, q, ldq, scale);
-  else if (pieces && cols <= 2048)
-    launch_quantize_vec<2>(h, rows, cols, x, ldx, q, ldq, scale);
-  else if (pieces && cols <= 4096)
-    launch_quantize_vec<4>(h, rows, cols, x, ldx, q, ldq, scale);
-  else if (pieces && cols <= 8192)
-    launch_quantize_vec<8>(h, rows, cols, x, ldx, q, ldq, scale);
-  else if (pieces)
-    launch_quantize_vec<16>(h, rows, cols, x, ldx, q, ldq, scale);
-  else
+  // Up to one row per compute unit, all the lanes a workgroup can have work on a row (a chain of
+  // one or two loads and as many pieces to convert per lane); with more rows than that several
+  // 256-lane workgroups share a unit and hide each other's waits.  (The quantizer and the int8
+  // product of an 8 x 8192 decode step together: 15.1 -> 14.6 us.)
+  const bool wide = rows <= (h->num_cus > 0 ? h->num_cus : 256);
+  if (cols > 16384)
     hipLaunchKernelGGL(quantize_rows_kernel, dim3((unsigned)rows), dim3(256), 0, h->stream, cols,
                        x, ldx, q, ldq, scale);
+  else if (cols <= 1024)
+    launch_quantize_vec<256, 1>(h, rows, cols, x, ldx, q, ldq, scale);
+  else if (cols <= 2048)
+    wide ? launch_quantize_vec<512, 1>(h, rows, cols, x, ldx, q, ldq, scale)
+         : launch_quantize_vec<256, 2>(h, rows, cols, x, ldx, q, ldq, scale);
+  else if (cols <= 4096)
+    wide ? launch_quantize_vec<1024, 1>(h, rows, cols, x, ldx, q, ldq, scale)
+         : launch_quantize_vec<256, 4>(h, rows, cols, x, ldx, q, ldq, scale);
+  else if (cols <= 8192)
+    wide ? launch_quantize_vec<1024, 2>(h, rows, cols, x, ldx, q, ldq, scale)
+         : launch_quantize_vec<256, 8>(h, rows, cols, x, ldx, q, ldq, scale);
+  else
+    wide ? launch_quantize_vec<1024, 4>(h, rows, cols, x, ldx, q, ldq, scale)
+         : launch_quantize_vec<256, 16>(h, rows, cols, x, ldx, q, ldq, scale);
   return check_launch(h, "cigemm_quantize_rows_i8");
 }
 

@@ -84,8 +84,8 @@ def test_quantize_rows(handle, torch_gpu, oracle, rng, shape):
 
 @pytest.mark.parametrize("pad", [4, 1])
 def test_quantize_rows_of_a_wider_matrix(handle, torch_gpu, oracle, rng, pad):
-    """Rows with a leading dimension above the column count: a multiple of 4 keeps the
-    16-byte-piece kernel, any other falls back to the element-wise one; same bits."""
+    """Rows with a leading dimension above the column count: rows that stay 16-byte
+    aligned and rows that do not; same bits."""
     rows, cols = 33, 1024
     wide = rng.normal(size=(rows, cols + pad)).astype(np.float32) * 3
     xd = torch_gpu.from_numpy(wide).cuda()[:, :cols]
@@ -93,3 +93,36 @@ def test_quantize_rows_of_a_wider_matrix(handle, torch_gpu, oracle, rng, pad):
     qe, se = oracle.quantize_rows_i8(np.ascontiguousarray(wide[:, :cols]))
     np.testing.assert_array_equal(s.cpu().numpy(), se)
     np.testing.assert_array_equal(q.cpu().numpy(), qe)
+
+
+@pytest.mark.parametrize("shape", [(1, 1025), (300, 1027), (2, 2049), (257, 2047), (5, 4097),
+                                   (300, 4099), (260, 8193), (2, 16383), (260, 16381),
+                                   (2, 16385)])
+@pytest.mark.parametrize("scale", [1.0, 1e-36, 1e-41, 1e36])  # 127e36 is still finite
+def test_quantize_rows_close_to_halves(handle, torch_gpu, oracle, rng, shape, scale):
+    """Quotients on a half and one or two ulp beside it, where an estimated quotient can round to
+    the other side; rows of any length, one piece or several per lane, packed and with an odd
+    leading dimension; scales inside and outside the range the quotients are estimated in."""
+    rows, cols = shape
+    step = np.float32(scale) if scale > 1e-38 else np.float32(2.0 ** -136)  # a denormal step
+    x = (rng.integers(-127, 127, size=shape).astype(np.float32) + np.float32(0.5)) * step
+    ulps = rng.integers(-2, 3, size=shape)
+    for _ in range(2):
+        x = np.where(ulps > 0, np.nextafter(x, np.float32(np.inf)), x)
+        x = np.where(ulps < 0, np.nextafter(x, np.float32(-np.inf)), x)
+        ulps -= np.sign(ulps)
+    x[:, -1] = 127 * step  # the row's maximum is its last, ragged element
+    x = x.astype(np.float32)
+    qe, se = oracle.quantize_rows_i8(x)
+    xw = np.full((rows, cols + 3), np.inf, dtype=np.float32)  # the padding is not read
+    xw[:, :cols] = x
+    q, s = handle.quantize_rows_i8(torch_gpu.from_numpy(x).cuda())
+    np.testing.assert_array_equal(s.cpu().numpy(), se)
+    np.testing.assert_array_equal(q.cpu().numpy(), qe)
+    qw = torch_gpu.full((rows, cols + 5), 99, dtype=torch_gpu.int8, device="cuda")
+    sw = torch_gpu.empty(rows, dtype=torch_gpu.float32, device="cuda")
+    handle.quantize_rows_i8(torch_gpu.from_numpy(xw).cuda()[:, :cols], out=(qw[:, :cols], sw))
+    got = qw.cpu().numpy()
+    np.testing.assert_array_equal(sw.cpu().numpy(), se)
+    np.testing.assert_array_equal(got[:, :cols], qe)
+    assert (got[:, cols:] == 99).all()
