@@ -258,6 +258,8 @@ bool launch_f32_mfma(cigemmContext*, int64_t M, int64_t N, int64_t K, const floa
                      const BiasAct* ba = nullptr);
 // gemm_f32_small.hip: 32x32 tile per workgroup, k split over the waves.
 bool f32_small_shape_ok(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda);
+// any K, any alignment of A: the sizes alone
+bool f32_small_any_ok(int64_t M, int64_t N, int64_t K);
 void launch_f32_small(cigemmContext*, int64_t M, int64_t N, int64_t K, const float* A,
                       int64_t lda, const float* B, int64_t ldb, float* C, int64_t ldc,
                       const BiasAct* ba = nullptr);

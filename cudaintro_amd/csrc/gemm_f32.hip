@@ -18,7 +18,13 @@ bool launch_f32_mfma(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const 
                      int64_t lda, const float* B, int64_t ldb, float* C, int64_t ldc,
                      const BiasAct* ba) {
   const bool tile_ok = f32_tile_ok(M, N, K, A, lda, B, ldb, C, ldc, ba);
-  if (f32_small_shape_ok(M, N, K, A, lda)) {
+  // A K that is no multiple of 8, or unaligned rows of A: the same choice (the small kernel's
+  // last k block and its loads of A take them), where the tile kernel's any-alignment form is the
+  // other side of it.  Against that form alone: 2 x 192 x 725 14.2 -> 7.1 us; against the aligned
+  // tile kernel: 512 x 512 x 508 16.2 -> 6.4.
+  const bool small_ok = f32_small_shape_ok(M, N, K, A, lda);
+  const bool any_ok = tile::tile_any_ok(M, N, K, 4, lda, ldb, true);
+  if (small_ok || (any_ok && f32_small_any_ok(M, N, K))) {
     // Both costs in units of a quarter of one 256x256 tile's time per unit of k: the tile
     // plan's own figure against 0.115 per resident round of 32x32 tiles (2048^3: tile kernel
     // 157 us, small kernel 225 us; 1024^3: 74 us against 33 us; 512^3: 38 us against 8 us).
@@ -40,7 +46,7 @@ bool launch_f32_mfma(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const 
     // 4095 x 4096 2031 (this kernel) against 923 us, 64 x 1001 x 4096 55 against 21, 4096 x 251 x
     // 1000 38 against 28; the other way 512 x 2047 x 336 13 against 21, 8 x 251 x 1000 9 against
     // 15.  The rule takes the slower one on 4 of them, by 6-14 %.
-    if (!tile_ok && tile::tile_any_ok(M, N, K, 4, lda, ldb, true)) {
+    if (!tile_ok && any_ok) {
       if (!one_round) return false;
       double plan = 0;
       tile::plan_small(cus, ctx->workspace ? ctx->ws_partial_bytes : 0, M,

@@ -15,7 +15,8 @@
 // columns have a form of their own below.
 //
 // Ragged M and N: loads past the edge re-read the last valid row / column, stores are
-// masked.  K must be a multiple of 8 and A's rows 16-byte aligned.
+// masked.  Any K and any alignment: A's 16-byte loads take any row address, the last K % 8 of k
+// are loaded element by element by the wave that has the last share.
 #include "common.h"
 
 namespace cig {
@@ -60,7 +61,8 @@ __global__ __launch_bounds__(256) void f32_small_kernel(int M, int N, int K, int
   const float* bvp = B + (8 * (int64_t)b0 + (l >> 3)) * ldb + vq;
   // one 8-deep k block: fragments in, four MFMAs
   auto block = [&](int b) {
-    const f32x4 a = *reinterpret_cast<const f32x4*>(ap);
+    f32x4 a;
+    __builtin_memcpy(&a, ap, 16);  // A's rows need not be 16-byte aligned
     float x0, x1, x2, x3;
     if constexpr (BVEC) {
       float(*st)[BSTG_LD] = bstg[w][b & 1];
@@ -89,6 +91,18 @@ __global__ __launch_bounds__(256) void f32_small_kernel(int M, int N, int K, int
     }
   }
   for (; b < b1; ++b) block(b);
+  if (w == 3 && (K & 7)) {
+    // the last K % 8 of k: elements past the end are zero in both fragments
+    const int k0 = 8 * nblk + 4 * h;
+    const float* at = A + (int64_t)row * lda + k0;
+    const float* bt = B + (int64_t)k0 * ldb + col;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float av = 0.0f, bv = 0.0f;
+      if (k0 + e < K) av = at[e], bv = bt[e * ldb];
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(bv, av, acc, 0, 0, 0);
+    }
+  }
 
   // acc[4q+e] is C[m0 + r][n0 + 8q + 4h + e].
 #pragma unroll
@@ -258,9 +272,16 @@ void launch_f32_narrow(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, cons
 
 }  // namespace
 
+static bool a_rows_aligned(const float* A, int64_t lda) {
+  return lda % 4 == 0 && (reinterpret_cast<uintptr_t>(A) & 15) == 0;
+}
+
 bool f32_small_shape_ok(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda) {
-  if (M <= 0 || N <= 0 || K <= 0 || K % 8) return false;
-  if (lda % 4 || (reinterpret_cast<uintptr_t>(A) & 15)) return false;
+  return K % 8 == 0 && a_rows_aligned(A, lda) && f32_small_any_ok(M, N, K);
+}
+
+bool f32_small_any_ok(int64_t M, int64_t N, int64_t K) {
+  if (M <= 0 || N <= 0 || K <= 0) return false;
   if (M > (1 << 24) || N > (1 << 24) || K > (1 << 24)) return false;
   const int64_t tiles = ((M + ST - 1) / ST) * ((N + ST - 1) / ST);
   return tiles <= 0x7fffffff;
@@ -273,7 +294,7 @@ void launch_f32_small(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const
   const bool relu = ba && ba->relu;
   // narrow outputs with a k share per wave that fits the registers
   const int64_t nb_wave = (K / 16 + 3) / 4;
-  if (N <= NT && K % 16 == 0 && nb_wave <= 32 && M >= 64) {
+  if (N <= NT && K % 16 == 0 && a_rows_aligned(A, lda) && nb_wave <= 32 && M >= 64) {
     if (nb_wave <= 8)
       launch_f32_narrow<8>(ctx, M, N, K, A, lda, B, ldb, C, ldc, bias, relu);
     else if (nb_wave <= 16)
@@ -302,7 +323,11 @@ void launch_f32_small(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const
     if (relu) CIG_SMALL(false, true); else CIG_SMALL(false, false);
   }
 #undef CIG_SMALL
-  ctx->last_kernel = ba ? "f32_mfma_small_32x32_ksplit4_bias_act" : "f32_mfma_small_32x32_ksplit4";
+  if (!f32_small_shape_ok(M, N, K, A, lda))
+    ctx->last_kernel =
+        ba ? "f32_mfma_any_small_32x32_ksplit4_bias_act" : "f32_mfma_any_small_32x32_ksplit4";
+  else
+    ctx->last_kernel = ba ? "f32_mfma_small_32x32_ksplit4_bias_act" : "f32_mfma_small_32x32_ksplit4";
 }
 
 }  // namespace cig
