@@ -91,6 +91,7 @@ cigemmStatus_t cigemmCreate(cigemmHandle_t* handle) {
   ctx->ws_dirty = 0;
   ctx->force_tile_mt = 0;
   ctx->force_tile_splits = 0;
+  ctx->force_any_kernel = ANY_BY_SHAPE;
   ctx->workspace = nullptr;
   if (hipMalloc(&ctx->workspace,
                 ctx->ws_partial_bytes + ctx->ws_counter_bytes + ctx->ws_swap_bytes) != hipSuccess ||
@@ -197,6 +198,12 @@ static bool dispatch_f32(cigemmHandle_t h, int64_t M, int64_t N, int64_t K, cons
     case CIGEMM_ALGO_SKINNY:
       return false;
     case CIGEMM_ALGO_MFMA_ANY:
+      if (h->force_any_kernel == ANY_F32_SMALL && f32_small_any_ok(M, N, K)) {
+        launch_f32_small(h, M, N, K, A, lda, B, ldb, C, ldc, ba);
+        return true;
+      }
+      if (h->force_any_kernel == ANY_REGISTER_STAGED)
+        return launch_mfma_any_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba);
       return launch_tile_any_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba) ||
              launch_mfma_any_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba);
     case CIGEMM_ALGO_GENERIC:
@@ -247,7 +254,8 @@ static cigemmStatus_t gemm16(cigemmHandle_t h, const char* name, bool bf16, int6
     case CIGEMM_ALGO_TILE: ok = launch_16b_mfma(h, bf16, M, N, K, A, lda, B, ldb, C, ldc); break;
     case CIGEMM_ALGO_SMALL: ok = false; break;
     case CIGEMM_ALGO_MFMA_ANY:
-      ok = launch_tile_any_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc) ||
+      ok = (h->force_any_kernel != ANY_REGISTER_STAGED &&
+            launch_tile_any_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc)) ||
            launch_mfma_any_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc);
       break;
     case CIGEMM_ALGO_GENERIC: launch_generic_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc); break;
@@ -287,7 +295,8 @@ static cigemmStatus_t gemm_i8(cigemmHandle_t h, const char* name, int64_t M, int
     case CIGEMM_ALGO_TILE: ok = launch_i8_mfma(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq); break;
     case CIGEMM_ALGO_SMALL: ok = false; break;
     case CIGEMM_ALGO_MFMA_ANY:
-      ok = launch_tile_any_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq) ||
+      ok = (h->force_any_kernel != ANY_REGISTER_STAGED &&
+            launch_tile_any_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq)) ||
            launch_mfma_any_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq);
       break;
     case CIGEMM_ALGO_GENERIC: launch_generic_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq); break;

@@ -44,10 +44,16 @@ struct cigemmContext {
   // in place of its own plan; 0 = the launcher chooses.
   int force_tile_mt;
   int force_tile_splits;
+  // Test aid, set through the probe library only: which kernel serves a call that
+  // CIGEMM_ALGO_MFMA_ANY selects: AnyKernel.
+  int force_any_kernel;
   char last_error[256];
 };
 
 constexpr uint32_t kCtxMagic = 0xC16E3350u;
+// ANY_BY_SHAPE: the tile kernel's any-alignment form, or, for what that form does not take, the
+// register-staged kernel.  The others impose one kernel (ANY_F32_SMALL: fp32 calls only).
+enum AnyKernel { ANY_BY_SHAPE = 0, ANY_REGISTER_STAGED = 1, ANY_F32_SMALL = 2 };
 
 namespace cig {
 

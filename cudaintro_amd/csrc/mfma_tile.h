@@ -246,7 +246,10 @@ __device__ __forceinline__ typename BTile<MODE>::piece_t read_b_piece(const char
 // load_piece reads 16 bytes that lie inside the matrix whatever the piece (row clamped to the
 // last one; a piece that crosses the end of its row is replaced by the row's last 16 bytes),
 // trim_piece, applied when the value is needed, moves those down so that element `col` comes
-// first and zeroes what lies outside.  Needs cols >= CE.
+// first and zeroes what lies outside.  Needs CE elements of the same row up to column `cols`: cols >=
+// CE, or, for a sub-problem that starts inside a wider matrix (the second launch of launch_tile,
+// whose columns start at a multiple of 256; a K range but the first, which starts at a multiple of
+// 128 bytes), at least CE elements of the row in front of the sub-problem's first column.
 template <typename T>
 __device__ __forceinline__ u32x4 load_piece(const T* __restrict__ P, int64_t ld, int64_t row,
                                             int64_t rows, int64_t col, int64_t cols) {
@@ -1380,6 +1383,8 @@ bool launch_tile(cigemmContext* ctx, int64_t M, int64_t N, int64_t K_bytes, cons
         if (tile_plan_cost(M, n1, 4, cus, units) + rest < single * 0.97) {
           launch_tile_256<Math, BMODE, ANY>(ctx, M, n1, K_bytes, A, lda_bytes, B, ldb_bytes, epi);
           const int rows1 = ctx->last_tile_rows, waves1 = ctx->last_waves;
+          // (n2 may be less than a 16-byte piece; load_piece then reads from the n1 >= 256 columns
+          // in front)
           const char* B2 = static_cast<const char*>(B) +
                            (BMODE == B_NK ? n1 * ldb_bytes : n1 * Math::ELEM_BYTES);
           bool split = false;

@@ -5,6 +5,7 @@ Not part of the drop-in library.  ``bench.py`` and the probe tests load it besid
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes as C
 import os
 
@@ -30,6 +31,7 @@ SIGNATURES = {
                                                   _vp, _ci, _vp, _ci, _i64, _vp, _i64]),
     "cigemm_probe_dirty_workspace": (_ci, [_vp, _ci, C.c_uint32, _ci]),
     "cigemm_probe_force_tile_plan": (_ci, [_vp, _ci, _ci]),
+    "cigemm_probe_force_any_kernel": (_ci, [_vp, _ci]),
 }
 
 
@@ -164,3 +166,20 @@ def force_tile_plan(h: Handle, tile_rows: int, k_ranges: int = 1):
     choice back to the library."""
     _check(h, load_library().cigemm_probe_force_tile_plan(h.raw, tile_rows, k_ranges),
            "cigemm_probe_force_tile_plan")
+
+
+ANY_BY_SHAPE, ANY_REGISTER_STAGED, ANY_F32_SMALL = 0, 1, 2
+
+
+@contextlib.contextmanager
+def any_kernel(h: Handle, kernel: int):
+    """Context manager: ``with any_kernel(h, ANY_REGISTER_STAGED): ...`` runs the handle's calls
+    under ``ALGO_MFMA_ANY`` on that kernel."""
+    def choose(k):
+        _check(h, load_library().cigemm_probe_force_any_kernel(h.raw, k), "cigemm_probe_force_any_kernel")
+    choose(kernel)
+    try:
+        with h.algo(cigemm.ALGO_MFMA_ANY):
+            yield
+    finally:
+        choose(ANY_BY_SHAPE)

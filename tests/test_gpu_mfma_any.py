@@ -1,12 +1,17 @@
-"""The any-shape matrix-core kernel (CIGEMM_ALGO_MFMA_ANY): 16-bit and int8 calls with an odd N
+"""The any-shape matrix-core kernels (CIGEMM_ALGO_MFMA_ANY: the tile kernel's any-alignment form,
+the register-staged kernel for what that form does not take): 16-bit and int8 calls with an odd N
 or K, leading dimensions and pointers with no alignment beyond the element's, matrices smaller
 than a tile.  int8 bit for bit against the CPU loop, 16-bit bit for bit on exact-arithmetic
 inputs and within the K-scaled bound on normal ones; the padding around every operand is NaN
 (127 for int8) and the output sits inside a sentinel-filled buffer."""
+import re
+from contextlib import contextmanager
+
 import numpy as np
 import pytest
 
 import cudaintro_amd as ci
+from cudaintro_amd import probe
 from gpu_util import bits, error_bound_16
 
 pytestmark = pytest.mark.gpu
@@ -17,6 +22,33 @@ SHAPES = [(1, 1, 1), (3, 5, 7), (64, 63, 64), (129, 131, 67), (300, 257, 1000), 
           # few tiles and a long K: run as K ranges into the workspace plus a reduction launch
           (1, 2047, 2050), (16, 1000, 4097), (130, 257, 3001)]
 SPLIT = {(1, 2047, 2050), (16, 1000, 4097), (130, 257, 3001), (260, 4, 2049), (300, 257, 1000)}
+
+
+def is_register_staged(name):
+    return re.search(r"_mfma_any_128x128x", name) is not None
+
+
+def is_tile_form(name):
+    return re.search(r"_mfma_any_[0-9+]+x256x", name) is not None
+
+
+def too_narrow(N, K, elem, kn):
+    """Fewer than 16 bytes of K, or of the N of a K x N operand: the tile kernel's form refuses."""
+    return K * elem < 16 or (kn and N * elem < 16)
+
+
+@contextmanager
+def choice(handle, how):
+    """How the kernel is chosen: "staged" (imposed), "any" (ALGO_MFMA_ANY) or "default"."""
+    if how == "staged":
+        with probe.any_kernel(handle, probe.ANY_REGISTER_STAGED):
+            yield
+    else:
+        with handle.algo(ci.ALGO_MFMA_ANY if how == "any" else ci.ALGO_DEFAULT):
+            yield
+
+
+CHOICES = ["staged", "any", "default"]
 
 
 def embed(torch, a, dtype, off, pad, fill):
@@ -50,11 +82,12 @@ def test_any_shape_16bit(handle, torch_gpu, oracle, rng, kind, M, N, K):
         _, b = embed(torch, Bb.view(npv), tdt, 3, 1, float("nan"))
         flat, out = embed(torch, np.zeros((M, N), npv), tdt, 1, 5, 0.0)
         flat.fill_(3.0)
-        for algo in (ci.ALGO_MFMA_ANY, ci.ALGO_DEFAULT):
+        for how in CHOICES:
             flat.fill_(3.0)
-            with handle.algo(algo):
+            with choice(handle, how):
                 fn(a, b, out=out)
-            assert "mfma_any" in handle.last_kernel, handle.last_kernel
+            staged = how == "staged" or too_narrow(N, K, 2, True)
+            assert (is_register_staged if staged else is_tile_form)(handle.last_kernel), handle.last_kernel
             assert handle.last_kernel.endswith("_splitk") == ((M, N, K) in SPLIT), handle.last_kernel
             got = bits(torch, out)
             if exact:
@@ -83,11 +116,12 @@ def test_any_shape_int8(handle, torch_gpu, oracle, rng, layout, M, N, K):
     flat, out = embed(torch, np.zeros((M, N), np.int32), torch.int32, 1, 3, -9)
     sa = rng.uniform(1e-3, 5e-2, M).astype(np.float32)
     sb = rng.uniform(1e-3, 5e-2, N).astype(np.float32)
-    for algo in (ci.ALGO_MFMA_ANY, ci.ALGO_DEFAULT):
+    for how in CHOICES:
         flat.fill_(-9)
-        with handle.algo(algo):
+        with choice(handle, how):
             handle.gemm_i8_i32(a, b, layout, out=out)
-            assert "mfma_any" in handle.last_kernel, handle.last_kernel
+            staged = how == "staged" or too_narrow(N, K, 1, not nk)
+            assert (is_register_staged if staged else is_tile_form)(handle.last_kernel), handle.last_kernel
             np.testing.assert_array_equal(out.cpu().numpy(), acc_ref)
             f = flat.cpu().numpy()
             guard = np.ones(f.shape, bool)
@@ -97,7 +131,8 @@ def test_any_shape_int8(handle, torch_gpu, oracle, rng, layout, M, N, K):
             for out_type, ot in (("f32", ci.OUT_F32), ("bf16", ci.OUT_BF16)):
                 y, acc = handle.gemm_i8_dequant(a, b, torch.from_numpy(sa).cuda(), torch.from_numpy(sb).cuda(),
                                                 layout, ot, dump_acc=True)
-                assert "mfma_any" in handle.last_kernel and "dequant" in handle.last_kernel
+                # (the accumulator dump on unaligned rows is the register-staged kernel's)
+                assert is_register_staged(handle.last_kernel) and "dequant" in handle.last_kernel
                 np.testing.assert_array_equal(acc.cpu().numpy(), acc_ref)
                 expect = oracle.dequant(acc_ref, sa, sb, out_dtype=out_type, sa_per_row=True, sb_per_col=True)
                 got = bits(torch, y) if out_type == "bf16" else y.cpu().numpy()
@@ -119,17 +154,23 @@ def test_any_shape_f32(handle, torch_gpu, oracle, rng, M, N, K):
         _, a = embed(torch, A, torch.float32, 1, 3, float("nan"))
         _, b = embed(torch, B, torch.float32, 3, 1, float("nan"))
         flat, out = embed(torch, np.zeros((M, N), np.float32), torch.float32, 1, 5, 0.0)
-        for algo in (ci.ALGO_MFMA_ANY, ci.ALGO_DEFAULT):
+        for how in CHOICES:
             for with_bias in (False, True):
                 flat.fill_(3.0)
-                with handle.algo(algo):
+                with choice(handle, how):
                     if with_bias:
                         handle.linear_f32(a, b, torch.from_numpy(bias).cuda(), ci.ACT_RELU, out=out)
                         cpu = oracle.linear_f32(A, B, bias, True)
                     else:
                         handle.gemm_f32(a, b, out=out)
                         cpu = oracle.gemm_f32(A, B)
-                assert "f32_mfma_any" in handle.last_kernel, handle.last_kernel
+                if how == "staged" or too_narrow(N, K, 4, True):
+                    assert is_register_staged(handle.last_kernel), handle.last_kernel
+                    if how == "staged" and (M, N, K) in SPLIT:
+                        assert handle.last_kernel.endswith("_splitk"), handle.last_kernel
+                else:
+                    assert is_tile_form(handle.last_kernel) or (
+                        how == "default" and "f32_mfma_any_small" in handle.last_kernel), handle.last_kernel
                 got = out.cpu().numpy()
                 if exact:
                     np.testing.assert_array_equal(got, cpu)
@@ -143,6 +184,25 @@ def test_any_shape_f32(handle, torch_gpu, oracle, rng, M, N, K):
                 for i in range(M):
                     guard[1 + i * (N + 5): 1 + i * (N + 5) + N] = False
                 assert (f[guard] == 3.0).all()
+
+
+@pytest.mark.parametrize("kind", ["bf16", "f16", "f32"])
+def test_leading_dimension_beyond_the_tile_kernels_offsets(handle, torch_gpu, oracle, rng, kind):
+    """256 rows of A span 2 GiB and more: the tile kernel's 32-bit row offsets do not reach, the
+    call stays on the register-staged kernel without being asked to."""
+    torch = torch_gpu
+    M, N, K = 3, 137, 75
+    A, B = rng.choice(VALS, size=(M, K)), rng.choice(VALS, size=(K, N))
+    ref = oracle.gemm_f32(A, B)
+    dt = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[kind]
+    ld = (1 << 31) // 256 // dt.itemsize + 1
+    flat = torch.full((M * ld,), float("nan"), dtype=dt, device="cuda")
+    a = flat.view(M, ld)[:, 1:K + 1]
+    a.copy_(torch.from_numpy(A).cuda())
+    _, b = embed(torch, B, torch.float32, 0, 0, float("nan"))
+    out = getattr(handle, "gemm_" + kind)(a, b.to(dt).contiguous())
+    assert is_register_staged(handle.last_kernel), handle.last_kernel
+    np.testing.assert_array_equal(out.float().cpu().numpy(), torch.from_numpy(ref).to(dt).float().numpy())
 
 
 def test_any_shape_kernel_is_the_fallback_not_the_first_choice(handle, torch_gpu):

@@ -5,6 +5,8 @@ range that is only tail among them), edge and interior tiles, every operand off 
 Operand values are small integers and halves, so every sum is exact and the comparison is bit for
 bit; the padding around the operands is NaN (127 for int8), the output sits in a sentinel-filled
 buffer."""
+import re
+
 import numpy as np
 import pytest
 
@@ -78,3 +80,61 @@ def test_tile_any(handle, torch_gpu, oracle, rng, kind, rows):
                         np.testing.assert_array_equal(host(y), oracle.linear_f32(A, B, bias, True))
             finally:
                 probe.force_tile_plan(handle, 0)
+
+
+# Columns left over by the full rounds of 256-row tiles: fewer than a 16-byte piece (the second
+# launch then covers columns that are narrower than one piece), one piece, more than one tile.
+@pytest.mark.parametrize("rest", ["one", "piece - 1", "piece", "tile + 1"])
+@pytest.mark.parametrize("kind", list(BYTES))
+def test_two_launches(handle, torch_gpu, rng, kind, rest):
+    """The two-launch plan on unaligned rows: 16 x 16 tiles of 256 rows, the rest of the columns as
+    a second launch with its own plan (of one K range for the short K, several where the planner
+    splits the long one), so that output, bias and per-column scales start at a column of their own.
+    Reference: torch in 64 bits, on operands whose sums are exact in 32."""
+    torch = torch_gpu
+    eb = BYTES[kind]
+    m = 4095
+    n = 4096 + {"one": 1, "piece - 1": max(2, 16 // eb - 1), "piece": 16 // eb, "tile + 1": 257}[rest]
+    int8 = eb == 1
+    layout = ci.B_NK if kind == "i8_nk" else ci.B_KN
+    dt = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}.get(kind, torch.int8)
+    odt = torch.int32 if int8 else dt
+    for K in (16 // eb + 1, 1025):
+        def operand(r, c, off, pad):
+            src = rng.integers(-127, 128, size=(r, c), dtype=np.int8) if int8 else rng.choice(VALS, size=(r, c))
+            flat = torch.full((off + r * (c + pad) + 3,), 127 if int8 else float("nan"), dtype=dt, device="cuda")
+            view = flat[off: off + r * (c + pad)].view(r, c + pad)[:, :c]
+            view.copy_(torch.from_numpy(src).cuda())
+            return view
+        a = operand(m, K, 1, 2)
+        b = operand(n, K, 3, 1) if kind == "i8_nk" else operand(K, n, 3, 2)
+        ref = a.double() @ (b.t() if kind == "i8_nk" else b).double().contiguous()
+        flat = torch.full((1 + m * (n + 3),), 7, dtype=odt, device="cuda")
+        out = flat[1:].view(m, n + 3)[:, :n]
+
+        def check(want, name=""):
+            assert re.search(r"_mfma_any_256\+\d+x256x", handle.last_kernel), handle.last_kernel
+            assert torch.equal(out, want), (K, name, (out != want).nonzero()[:4].tolist())
+            out.fill_(7)
+            assert bool((flat == 7).all()), "a store outside the output"
+
+        with handle.algo(ci.ALGO_MFMA_ANY):
+            if not int8:
+                getattr(handle, "gemm_" + kind)(a, b, out=out)
+                check(ref.to(odt))
+                if kind == "f32":
+                    bias = torch.from_numpy(rng.choice(VALS, size=n + 1)).cuda()[1:]
+                    handle.linear_f32(a, b, bias, ci.ACT_RELU, out=out)
+                    check(torch.relu(ref + bias.double()).to(odt), "bias + ReLU")
+            else:
+                handle.gemm_i8_i32(a, b, layout, out=out)
+                check(ref.to(odt))
+                # scales that are powers of two: the product is exact, whatever its order
+                sa = torch.from_numpy(np.ldexp(np.float32(1), rng.integers(-6, 1, size=m)).astype(np.float32)).cuda()
+                sb = torch.from_numpy(np.ldexp(np.float32(1), rng.integers(-6, 1, size=n + 1)).astype(np.float32)).cuda()[1:]
+                scaled = ref * sa.double()[:, None] * sb.double()[None, :]
+                for ot, t in ((ci.OUT_F32, torch.float32), (ci.OUT_BF16, torch.bfloat16)):
+                    flat = torch.full((1 + m * (n + 3),), 7, dtype=t, device="cuda")
+                    out = flat[1:].view(m, n + 3)[:, :n]
+                    handle.gemm_i8_dequant(a, b, sa, sb, layout, ot, out=out)
+                    check(scaled.to(torch.float32).to(t), t)
