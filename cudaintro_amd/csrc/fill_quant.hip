@@ -162,60 +162,74 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(int64_t cols,
 // whole aligned 16-byte pieces were read twice, element by element, and every element was divided:
 // 8192 x 8190 130.6 -> 59.1 us, 2048 x 4095 14.2 -> 7.5; whole pieces 2048 x 4096 7.9 -> 7.1,
 // 512 x 16384 8.8 -> 8.0.
-template <int THREADS, int CHUNKS>
-__global__ __launch_bounds__(THREADS) void quantize_rows_vec_kernel(int cols,
-                                                                    const float* __restrict__ x,
-                                                                    int64_t ldx,
-                                                                    int8_t* __restrict__ q,
-                                                                    int64_t ldq,
-                                                                    float* __restrict__ scale) {
+//
+// ROWS = 4: one wave per row, four rows per workgroup, for short rows.  A whole workgroup per row
+// is mostly idle lanes there and pays for its launch, a barrier and the two divisions of the scale
+// with every one of its waves: 97677 x 41 73.1 -> 25.9 us (49.0 when such rows were read twice,
+// element by element), 143947 x 60 98.2 -> 33.6 (73.1), 17659 x 476 14.8 -> 7.9 (13.0), 61668 x 963
+// 77.4 -> 43.8 (142.7).
+template <int THREADS, int CHUNKS, int ROWS>
+__global__ __launch_bounds__(THREADS * ROWS) void quantize_rows_vec_kernel(
+    int64_t rows, int cols, const float* __restrict__ x, int64_t ldx, int8_t* __restrict__ q,
+    int64_t ldq, float* __restrict__ scale) {
+  static_assert(ROWS == 1 || THREADS == 64, "rows share a workgroup by whole waves");
   constexpr int WAVES = THREADS / 64;
   __shared__ float red[WAVES];
-  const int64_t row = blockIdx.x;
+  const int t = ROWS > 1 ? (int)threadIdx.x & 63 : (int)threadIdx.x;
+  const int64_t row =
+      (int64_t)blockIdx.x * ROWS + (ROWS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0);
+  if (ROWS > 1 && row >= rows) return;  // (the whole wave)
   const float* xr = x + row * ldx;
   int8_t* qr = q + row * ldq;
-  f32x4 v[CHUNKS];
+  // Lane t has pieces t, t + THREADS, ...; the last cols % 4 elements are a piece of their own, on
+  // the last lane, so that the loads of whole pieces carry no branch and are in flight together,
+  // and pieces beyond the row's end cost nothing (1744 x 8296 17.2 -> 13.1 us, 2199 x 9236 21.1 ->
+  // 17.0 with a branch for a ragged piece around every load and all 16 chunks quantized).
+  const int tail = (t == THREADS - 1) ? cols & 3 : 0, tail_at = cols & ~3;
+  f32x4 v[CHUNKS], vt = {0.0f, 0.0f, 0.0f, 0.0f};
   float amax = 0.0f;
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c) {
-    const int j = 4 * ((int)threadIdx.x + THREADS * c);
+    const int j = 4 * (t + THREADS * c);
     v[c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    if (j + 4 <= cols) {
-      __builtin_memcpy(&v[c], xr + j, 16);  // rows need not be 16-byte aligned
-    } else {
+    if (j + 4 <= cols) __builtin_memcpy(&v[c], xr + j, 16);  // rows need not be 16-byte aligned
+  }
+  if (tail) {
 #pragma unroll
-      for (int e = 0; e < 3; ++e)
-        if (j + e < cols) v[c][e] = xr[j + e];
-    }
+    for (int e = 0; e < 3; ++e)
+      if (e < tail) vt[e] = xr[tail_at + e];
   }
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c)
 #pragma unroll
     for (int e = 0; e < 4; ++e) amax = fmaxf(amax, fabsf(v[c][e]));
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = amax;
-  __syncthreads();
-  amax = red[0];
+  for (int e = 0; e < 3; ++e) amax = fmaxf(amax, fabsf(vt[e]));
 #pragma unroll
-  for (int w = 1; w < WAVES; ++w) amax = fmaxf(amax, red[w]);
+  for (int off = 32; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
+  if constexpr (WAVES > 1) {
+    if ((t & 63) == 0) red[t >> 6] = amax;
+    __syncthreads();
+    amax = red[0];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) amax = fmaxf(amax, red[w]);
+  }
   const float s = amax > 0.0f ? __fdiv_rn(amax, 127.0f) : 1.0f;
-  if (threadIdx.x == 0) scale[row] = s;
+  if (t == 0) scale[row] = s;
   const bool estimate = s >= 0x1p-100f && s <= 0x1p100f;
   const float inv = __fdiv_rn(1.0f, s);
-#pragma unroll
-  for (int c = 0; c < CHUNKS; ++c) {
+  auto quantize_piece = [&](const f32x4& x4) {
     float r[4];
     bool sure = estimate;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const float t = v[c][e] * inv;
-      r[e] = rintf(t);
-      sure = sure && fabsf(t - r[e]) <= 0.4999f;
+      const float est = x4[e] * inv;
+      r[e] = rintf(est);
+      sure = sure && fabsf(est - r[e]) <= 0.4999f;
     }
     if (!sure) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) r[e] = rintf(__fdiv_rn(v[c][e], s));  // ties to even
+      for (int e = 0; e < 4; ++e) r[e] = rintf(__fdiv_rn(x4[e], s));  // ties to even
     }
     uint32_t packed = 0;
 #pragma unroll
@@ -223,22 +237,30 @@ __global__ __launch_bounds__(THREADS) void quantize_rows_vec_kernel(int cols,
       r[e] = fminf(fmaxf(r[e], -127.0f), 127.0f);
       packed |= ((uint32_t)(int)r[e] & 0xffu) << (8 * e);
     }
-    const int j = 4 * ((int)threadIdx.x + THREADS * c);
-    if (j + 4 <= cols) {
-      __builtin_memcpy(qr + j, &packed, 4);
-    } else {
+    return packed;
+  };
 #pragma unroll
-      for (int e = 0; e < 3; ++e)
-        if (j + e < cols) qr[j + e] = (int8_t)(packed >> (8 * e));
+  for (int c = 0; c < CHUNKS; ++c) {
+    const int j = 4 * (t + THREADS * c);
+    if (j + 4 <= cols) {
+      const uint32_t packed = quantize_piece(v[c]);
+      __builtin_memcpy(qr + j, &packed, 4);
     }
+  }
+  if (tail) {
+    const uint32_t packed = quantize_piece(vt);
+#pragma unroll
+    for (int e = 0; e < 3; ++e)
+      if (e < tail) qr[tail_at + e] = (int8_t)(packed >> (8 * e));
   }
 }
 
-template <int THREADS, int CHUNKS>
+template <int THREADS, int CHUNKS, int ROWS = 1>
 void launch_quantize_vec(cigemmContext* ctx, int64_t rows, int64_t cols, const float* x,
                          int64_t ldx, int8_t* q, int64_t ldq, float* scale) {
-  hipLaunchKernelGGL((quantize_rows_vec_kernel<THREADS, CHUNKS>), dim3((unsigned)rows),
-                     dim3(THREADS), 0, ctx->stream, (int)cols, x, ldx, q, ldq, scale);
+  hipLaunchKernelGGL((quantize_rows_vec_kernel<THREADS, CHUNKS, ROWS>),
+                     dim3((unsigned)((rows + ROWS - 1) / ROWS)), dim3(THREADS * ROWS), 0,
+                     ctx->stream, rows, (int)cols, x, ldx, q, ldq, scale);
 }
 
 }  // namespace
@@ -308,11 +330,19 @@ cigemmStatus_t cigemm_quantize_rows_i8(cigemmHandle_t h, int64_t rows, int64_t c
   // Up to one row per compute unit, all the lanes a workgroup can have work on a row (a chain of
   // one or two loads and as many pieces to convert per lane); with more rows than that several
   // 256-lane workgroups share a unit and hide each other's waits.  (The quantizer and the int8
-  // product of an 8 x 8192 decode step together: 15.1 -> 14.6 us.)
+  // product of an 8 x 8192 decode step together: 15.1 -> 14.6 us.)  A row of up to 256
+  // columns is one piece per lane of a wave whatever their number; one of up to 1024 is a wave's
+  // work when there are more rows than units to spread over.
   const bool wide = rows <= (h->num_cus > 0 ? h->num_cus : 256);
   if (cols > 16384)
     hipLaunchKernelGGL(quantize_rows_kernel, dim3((unsigned)rows), dim3(256), 0, h->stream, cols,
                        x, ldx, q, ldq, scale);
+  else if (cols <= 256)
+    launch_quantize_vec<64, 1, 4>(h, rows, cols, x, ldx, q, ldq, scale);
+  else if (cols <= 512 && !wide)
+    launch_quantize_vec<64, 2, 4>(h, rows, cols, x, ldx, q, ldq, scale);
+  else if (cols <= 1024 && !wide)
+    launch_quantize_vec<64, 4, 4>(h, rows, cols, x, ldx, q, ldq, scale);
   else if (cols <= 1024)
     launch_quantize_vec<256, 1>(h, rows, cols, x, ldx, q, ldq, scale);
   else if (cols <= 2048)

@@ -97,7 +97,10 @@ def test_quantize_rows_of_a_wider_matrix(handle, torch_gpu, oracle, rng, pad):
 
 @pytest.mark.parametrize("shape", [(1, 1025), (300, 1027), (2, 2049), (257, 2047), (5, 4097),
                                    (300, 4099), (260, 8193), (2, 16383), (260, 16381),
-                                   (2, 16385)])
+                                   (2, 16385),
+                                   # a wave per row, rows that leave the last workgroup part full
+                                   (5, 1), (301, 3), (302, 255), (3, 256), (303, 257), (301, 510),
+                                   (301, 513), (259, 1023), (258, 1024), (256, 1023)])
 @pytest.mark.parametrize("scale", [1.0, 1e-36, 1e-41, 1e36])  # 127e36 is still finite
 def test_quantize_rows_close_to_halves(handle, torch_gpu, oracle, rng, shape, scale):
     """Quotients on a half and one or two ulp beside it, where an estimated quotient can round to
