@@ -82,6 +82,36 @@ def test_tile_any(handle, torch_gpu, oracle, rng, kind, rows):
                 probe.force_tile_plan(handle, 0)
 
 
+@pytest.mark.parametrize("kind", list(BYTES))
+def test_every_width_of_the_last_piece(handle, torch_gpu, oracle, rng, kind):
+    """Rows that end with 0 to 7 elements of a 16-byte piece, 16- and 32-bit outputs, the next row
+    directly behind them."""
+    torch = torch_gpu
+    int8 = kind.startswith("i8")
+    layout = ci.B_NK if kind == "i8_nk" else ci.B_KN
+    m, K = 70, 75
+    for n in range(264, 272):
+        if int8:
+            A = rng.integers(-127, 128, size=(m, K), dtype=np.int8)
+            B = rng.integers(-127, 128, size=(n, K) if layout == ci.B_NK else (K, n), dtype=np.int8)
+            acc = oracle.gemm_i8_i32(A, B, b_is_nk=layout == ci.B_NK)
+            sa, sb = (rng.uniform(1e-3, 5e-2, k).astype(np.float32) for k in (m, n))
+            a, b, da, db = (torch.from_numpy(v).cuda() for v in (A, B, sa, sb))
+            with handle.algo(ci.ALGO_MFMA_ANY):
+                np.testing.assert_array_equal(handle.gemm_i8_i32(a, b, layout).cpu().numpy(), acc)
+                y = handle.gemm_i8_dequant(a, b, da, db, layout, ci.OUT_BF16)
+            assert "_mfma_any_64x256" in handle.last_kernel, handle.last_kernel
+            np.testing.assert_array_equal(bits(torch, y), oracle.dequant(acc, sa, sb, out_dtype="bf16",
+                                                                         sa_per_row=True, sb_per_col=True))
+            continue
+        A, B = rng.choice(VALS, size=(m, K)), rng.choice(VALS, size=(K, n))
+        dt = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[kind]
+        with handle.algo(ci.ALGO_MFMA_ANY):
+            y = getattr(handle, "gemm_" + kind)(torch.from_numpy(A).cuda().to(dt), torch.from_numpy(B).cuda().to(dt))
+        assert "_mfma_any_64x256" in handle.last_kernel, handle.last_kernel
+        assert torch.equal(y.cpu(), torch.from_numpy(oracle.gemm_f32(A, B)).to(dt)), n
+
+
 # Columns left over by the full rounds of 256-row tiles: fewer than a 16-byte piece (the second
 # launch then covers columns that are narrower than one piece), one piece, more than one tile.
 @pytest.mark.parametrize("rest", ["one", "piece - 1", "piece", "tile + 1"])
