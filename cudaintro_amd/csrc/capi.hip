@@ -4,6 +4,7 @@
 #include <cstdlib>
 #include <new>
 
+#include "any_plan.h"
 #include "common.h"
 
 namespace cig {
@@ -182,8 +183,88 @@ static cigemmStatus_t algo_refused(cigemmHandle_t h, const char* name) {
               "%s: the selected kernel family (algo %d) does not take this call", name, h->algo);
 }
 
-// fp32 dispatch.  DEFAULT: one of the two aligned MFMA kernels when the shape allows, else the
-// any-shape MFMA kernel (the scalar kernel only if its tile grid does not fit a launch).
+// The kernel of a call that no aligned kernel takes, by the estimates of any_plan.h or as the
+// measurement library imposes it, and the tile form's plan if one was made.  `small_us` < 0: the
+// small kernel is no choice.
+struct AnyChoice {
+  AnyKernel kernel;
+  tile::SmallPlan plan;
+};
+static AnyChoice choose_any(cigemmHandle_t h, const any::Cost& cost, const any::Problem& p,
+                            bool tile_ok, double small_us) {
+  AnyChoice best{ANY_REGISTER_STAGED, tile::SmallPlan{0, 1}};
+  if (h->algo == CIGEMM_ALGO_MFMA_ANY && h->force_any_kernel != ANY_BY_SHAPE) {
+    best.kernel = (AnyKernel)h->force_any_kernel;
+    return best;
+  }
+  if (tile_ok && h->force_tile_mt) {  // a plan of the tile kernel is imposed
+    best.kernel = ANY_TILE;
+    return best;
+  }
+  const int cus = h->num_cus > 0 ? h->num_cus : 256;
+  const size_t room = h->workspace ? h->ws_partial_bytes : 0;
+  double best_us = any::staged_us(cost, p, cus, room);
+  if (tile_ok) {
+    const tile::SmallPlan plan = any::tile_plan(cost, p, cus, room);
+    const double us = any::tile_us(cost, p, cus, room, plan);
+    if (us < best_us) {
+      best_us = us;
+      best = AnyChoice{ANY_TILE, plan};
+    }
+  }
+  if (small_us >= 0.0 && small_us < best_us) best.kernel = ANY_F32_SMALL;
+  return best;
+}
+
+static bool rows_apart(const void* p, int64_t ld_bytes) {
+  return (((uintptr_t)p | (uintptr_t)ld_bytes) & 3) != 0;
+}
+
+static bool any_f32(cigemmHandle_t h, int64_t M, int64_t N, int64_t K, const float* A, int64_t lda,
+                    const float* B, int64_t ldb, float* C, int64_t ldc, const BiasAct* ba) {
+  const bool small_ok = f32_small_any_ok(M, N, K);
+  // (CIGEMM_ALGO_MFMA_ANY chooses among the tile kernels)
+  const double small_us =
+      small_ok && h->algo != CIGEMM_ALGO_MFMA_ANY
+          ? any::f32_small_us(M, N, K, h->num_cus > 0 ? h->num_cus : 256, f32_small_b16(N, B, ldb),
+                              f32_small_is_narrow(M, N, K, A, lda))
+          : -1.0;
+  const AnyChoice c = choose_any(h, any::COST_F32, any::Problem{M, N, K * 4, 4, 4, false, false, false},
+                                 any::tile_ok(M, N, K, 4, lda, ldb, true), small_us);
+  if (c.kernel == ANY_F32_SMALL && small_ok) {
+    launch_f32_small(h, M, N, K, A, lda, B, ldb, C, ldc, ba);
+    return true;
+  }
+  return (c.kernel != ANY_REGISTER_STAGED &&
+          launch_tile_any_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba, c.plan)) ||
+         launch_mfma_any_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba);
+}
+
+static bool any_16(cigemmHandle_t h, bool bf16, int64_t M, int64_t N, int64_t K, const uint16_t* A,
+                   int64_t lda, const uint16_t* B, int64_t ldb, uint16_t* C, int64_t ldc) {
+  const AnyChoice c = choose_any(h, any::COST_16, any::Problem{M, N, K * 2, 2, 2, false, rows_apart(A, lda * 2), rows_apart(B, ldb * 2)},
+                                 any::tile_ok(M, N, K, 2, lda, ldb, true), -1.0);
+  return (c.kernel != ANY_REGISTER_STAGED &&
+          launch_tile_any_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc, c.plan)) ||
+         launch_mfma_any_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc);
+}
+
+static bool any_i8(cigemmHandle_t h, int64_t M, int64_t N, int64_t K, const int8_t* A, int64_t lda,
+                   const int8_t* B, int64_t ldb, bool b_nk, int32_t* C, int64_t ldc,
+                   const DequantArgs* dq) {
+  const any::Problem p{M, N, K, 1, dq && dq->out_bf16 ? 2 : 4, dq != nullptr,
+                       rows_apart(A, lda), rows_apart(B, ldb)};
+  // (the accumulator dump is the register-staged kernel's)
+  const AnyChoice c = choose_any(h, b_nk ? any::COST_I8_NK : any::COST_I8_KN, p,
+                                 any::tile_ok(M, N, K, 1, lda, ldb, !b_nk) && !(dq && dq->acc_out),
+                                 -1.0);
+  return (c.kernel != ANY_REGISTER_STAGED &&
+          launch_tile_any_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq, c.plan)) ||
+         launch_mfma_any_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq);
+}
+
+// fp32 dispatch.  DEFAULT: one of the two aligned MFMA kernels when the shape allows, else one of
+// those that take any (the scalar kernel only if no tile grid fits a launch).
 // Returns false when a selected family refuses the call.
 static bool dispatch_f32(cigemmHandle_t h, int64_t M, int64_t N, int64_t K, const float* A,
                          int64_t lda, const float* B, int64_t ldb, float* C, int64_t ldc,
@@ -198,21 +279,13 @@ static bool dispatch_f32(cigemmHandle_t h, int64_t M, int64_t N, int64_t K, cons
     case CIGEMM_ALGO_SKINNY:
       return false;
     case CIGEMM_ALGO_MFMA_ANY:
-      if (h->force_any_kernel == ANY_F32_SMALL && f32_small_any_ok(M, N, K)) {
-        launch_f32_small(h, M, N, K, A, lda, B, ldb, C, ldc, ba);
-        return true;
-      }
-      if (h->force_any_kernel == ANY_REGISTER_STAGED)
-        return launch_mfma_any_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba);
-      return launch_tile_any_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba) ||
-             launch_mfma_any_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba);
+      return any_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba);
     case CIGEMM_ALGO_GENERIC:
       launch_generic_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba);
       return true;
     default:
       if (!launch_f32_mfma(h, M, N, K, A, lda, B, ldb, C, ldc, ba) &&
-          !launch_tile_any_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba) &&
-          !launch_mfma_any_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba))
+          !any_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba))
         launch_generic_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba);
       return true;
   }
@@ -254,9 +327,7 @@ static cigemmStatus_t gemm16(cigemmHandle_t h, const char* name, bool bf16, int6
     case CIGEMM_ALGO_TILE: ok = launch_16b_mfma(h, bf16, M, N, K, A, lda, B, ldb, C, ldc); break;
     case CIGEMM_ALGO_SMALL: ok = false; break;
     case CIGEMM_ALGO_MFMA_ANY:
-      ok = (h->force_any_kernel != ANY_REGISTER_STAGED &&
-            launch_tile_any_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc)) ||
-           launch_mfma_any_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc);
+      ok = any_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc);
       break;
     case CIGEMM_ALGO_GENERIC: launch_generic_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc); break;
     default:
@@ -264,8 +335,7 @@ static cigemmStatus_t gemm16(cigemmHandle_t h, const char* name, bool bf16, int6
       // neither that nor the tile kernel takes (odd N, unaligned rows) stays on the matrix cores
       if (!launch_skinny_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc) &&
           !launch_16b_mfma(h, bf16, M, N, K, A, lda, B, ldb, C, ldc) &&
-          !launch_tile_any_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc) &&
-          !launch_mfma_any_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc))
+          !any_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc))
         launch_generic_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc);
   }
   if (!ok) return algo_refused(h, name);
@@ -295,16 +365,13 @@ static cigemmStatus_t gemm_i8(cigemmHandle_t h, const char* name, int64_t M, int
     case CIGEMM_ALGO_TILE: ok = launch_i8_mfma(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq); break;
     case CIGEMM_ALGO_SMALL: ok = false; break;
     case CIGEMM_ALGO_MFMA_ANY:
-      ok = (h->force_any_kernel != ANY_REGISTER_STAGED &&
-            launch_tile_any_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq)) ||
-           launch_mfma_any_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq);
+      ok = any_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq);
       break;
     case CIGEMM_ALGO_GENERIC: launch_generic_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq); break;
     default:
       if (!launch_skinny_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq) &&
           !launch_i8_mfma(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq) &&
-          !launch_tile_any_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq) &&
-          !launch_mfma_any_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq))
+          !any_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq))
         launch_generic_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq);
   }
   if (!ok) return algo_refused(h, name);

@@ -10,6 +10,7 @@
 #include <cstring>
 
 #include "cigemm.h"
+#include "tile_plan.h"
 
 struct cigemmContext {
   uint32_t magic;
@@ -51,9 +52,9 @@ struct cigemmContext {
 };
 
 constexpr uint32_t kCtxMagic = 0xC16E3350u;
-// ANY_BY_SHAPE: the tile kernel's any-alignment form, or, for what that form does not take, the
-// register-staged kernel.  The others impose one kernel (ANY_F32_SMALL: fp32 calls only).
-enum AnyKernel { ANY_BY_SHAPE = 0, ANY_REGISTER_STAGED = 1, ANY_F32_SMALL = 2 };
+// ANY_BY_SHAPE: what any_plan.h estimates to be the faster.  The others impose one kernel where it
+// takes the call (ANY_F32_SMALL: fp32 calls only).
+enum AnyKernel { ANY_BY_SHAPE = 0, ANY_REGISTER_STAGED = 1, ANY_F32_SMALL = 2, ANY_TILE = 3 };
 
 namespace cig {
 
@@ -224,8 +225,8 @@ struct DequantArgs {
 void launch_generic_f32(cigemmContext*, int64_t M, int64_t N, int64_t K, const float* A,
                         int64_t lda, const float* B, int64_t ldb, float* C, int64_t ldc,
                         const BiasAct* ba = nullptr);
-// gemm_ragged.hip: any shape, any alignment, on the matrix cores.  False when
-// the tile grid does not fit a launch (nothing launched).
+// gemm_ragged.hip: any shape, any alignment, on the matrix cores, operands staged through registers.
+// False when the tile grid does not fit a launch (nothing launched).
 bool launch_mfma_any_16(cigemmContext*, bool bf16, int64_t M, int64_t N, int64_t K,
                         const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb,
                         uint16_t* C, int64_t ldc);
@@ -237,15 +238,16 @@ bool launch_mfma_any_i8(cigemmContext*, int64_t M, int64_t N, int64_t K, const i
                         int64_t ldc, const DequantArgs* dq);
 // gemm_any_tile.hip: the tile kernel at any alignment.  False for matrices narrower than one
 // 16-byte piece, for the accumulator dump and beyond the launch limits (nothing launched).
+// `plan`: made already (any_plan.h), or mt = 0.
 bool launch_tile_any_16(cigemmContext*, bool bf16, int64_t M, int64_t N, int64_t K,
                         const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb,
-                        uint16_t* C, int64_t ldc);
+                        uint16_t* C, int64_t ldc, tile::SmallPlan plan);
 bool launch_tile_any_f32(cigemmContext*, int64_t M, int64_t N, int64_t K, const float* A,
                          int64_t lda, const float* B, int64_t ldb, float* C, int64_t ldc,
-                         const BiasAct* ba);
+                         const BiasAct* ba, tile::SmallPlan plan);
 bool launch_tile_any_i8(cigemmContext*, int64_t M, int64_t N, int64_t K, const int8_t* A,
                         int64_t lda, const int8_t* B, int64_t ldb, bool b_nk, int32_t* C,
-                        int64_t ldc, const DequantArgs* dq);
+                        int64_t ldc, const DequantArgs* dq, tile::SmallPlan plan);
 void launch_generic_16(cigemmContext*, bool bf16, int64_t M, int64_t N, int64_t K,
                        const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb,
                        uint16_t* C, int64_t ldc);
@@ -266,6 +268,9 @@ bool launch_f32_mfma(cigemmContext*, int64_t M, int64_t N, int64_t K, const floa
 bool f32_small_shape_ok(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda);
 // any K, any alignment of A: the sizes alone
 bool f32_small_any_ok(int64_t M, int64_t N, int64_t K);
+// the 16 x 16 form's calls; B's rows loaded in 16-byte pieces
+bool f32_small_is_narrow(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda);
+bool f32_small_b16(int64_t N, const float* B, int64_t ldb);
 void launch_f32_small(cigemmContext*, int64_t M, int64_t N, int64_t K, const float* A,
                       int64_t lda, const float* B, int64_t ldb, float* C, int64_t ldc,
                       const BiasAct* ba = nullptr);

@@ -17,18 +17,15 @@ static bool f32_tile_ok(int64_t M, int64_t N, int64_t K, const float* A, int64_t
 bool launch_f32_mfma(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const float* A,
                      int64_t lda, const float* B, int64_t ldb, float* C, int64_t ldc,
                      const BiasAct* ba) {
-  const bool tile_ok = f32_tile_ok(M, N, K, A, lda, B, ldb, C, ldc, ba);
-  // A K that is no multiple of 8, or unaligned rows of A: the same choice (the small kernel's
-  // last k block and its loads of A take them), where the tile kernel's any-alignment form is the
-  // other side of it.  Against that form alone: 2 x 192 x 725 14.2 -> 7.1 us; against the aligned
-  // tile kernel: 512 x 512 x 508 16.2 -> 6.4.
-  const bool small_ok = f32_small_shape_ok(M, N, K, A, lda);
-  const bool any_ok = tile::tile_any_ok(M, N, K, 4, lda, ldb, true);
-  if (small_ok || (any_ok && f32_small_any_ok(M, N, K))) {
+  if (!f32_tile_ok(M, N, K, A, lda, B, ldb, C, ldc, ba)) return false;
+  const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+  const bool one_round = ((M + 255) / 256) * ((N + tile::BN - 1) / tile::BN) <= cus;
+  bool small = false;
+  // (a K that is no multiple of 8: the same choice)
+  if (f32_small_any_ok(M, N, K)) {
     // Both costs in units of a quarter of one 256x256 tile's time per unit of k: the tile
     // plan's own figure against 0.115 per resident round of 32x32 tiles (2048^3: tile kernel
     // 157 us, small kernel 225 us; 1024^3: 74 us against 33 us; 512^3: 38 us against 8 us).
-    const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
     double tile_cost = 0;
     tile::best_mt(M, N, cus, &tile_cost);
     const double tiles32 = (double)((M + 31) / 32) * (double)((N + 31) / 32);
@@ -36,32 +33,11 @@ bool launch_f32_mfma(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const 
     // With a long K the tile kernel wins whenever its tiles fit one round: it can split K over
     // the idle compute units (512 x 512 x 4096: 33 us against 55 us; 1024^3: 31 against 32;
     // 512^3: 17 against 9; 960 x 3584 x 3584: 222 against 298).
-    const bool one_round = ((M + 255) / 256) * ((N + tile::BN - 1) / tile::BN) <= cus;
-    const bool long_k_split = tile_ok && K >= 2048 && one_round;
-    // What the aligned tile kernel cannot take (B or C rows not 16-byte aligned, an odd N): the
-    // tile kernel's any-alignment form when it is estimated the faster.  Without 16-byte loads of
-    // B this kernel takes about 2 us + K x (13 ns for up to one resident round of tiles -- 7 where
-    // B is at most 1 MiB --, 7.8 ns per round beyond), at least 6.5 us; the tile kernel its plan's
-    // estimate + 4 us.  Both timed over M 8..4096, N 251..4095, K 64..4096 (112 shapes): 4096 x
-    // 4095 x 4096 2031 (this kernel) against 923 us, 64 x 1001 x 4096 55 against 21, 4096 x 251 x
-    // 1000 38 against 28; the other way 512 x 2047 x 336 13 against 21, 8 x 251 x 1000 9 against
-    // 15.  The rule takes the slower one on 4 of them, by 6-14 %.
-    if (!tile_ok && any_ok) {
-      if (!one_round) return false;
-      double plan = 0;
-      tile::plan_small(cus, ctx->workspace ? ctx->ws_partial_bytes : 0, M,
-                       tile::partial_ld<true>(N), K * 4, 4, tile::STAGE_COST_KN32, K * 4 * N, &plan);
-      const double rounds = tiles32 / cus;
-      const double per_k = rounds > 1.7 ? 0.0078 * rounds : K * N <= (256 << 10) ? 0.007 : 0.013;
-      const double small_us = 2.0 + (double)K * per_k;
-      if (plan + 4.0 < (small_us > 6.5 ? small_us : 6.5)) return false;
-    }
-    if (!tile_ok || (small_cost < tile_cost && !long_k_split)) {
-      launch_f32_small(ctx, M, N, K, A, lda, B, ldb, C, ldc, ba);
-      return true;
-    }
+    small = small_cost < tile_cost && !(K >= 2048 && one_round);
   }
-  return tile_ok && launch_f32_tile(ctx, M, N, K, A, lda, B, ldb, C, ldc, ba);
+  if (!small) return launch_f32_tile(ctx, M, N, K, A, lda, B, ldb, C, ldc, ba);
+  launch_f32_small(ctx, M, N, K, A, lda, B, ldb, C, ldc, ba);
+  return true;
 }
 
 bool launch_f32_tile(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const float* A,

@@ -287,14 +287,23 @@ bool f32_small_any_ok(int64_t M, int64_t N, int64_t K) {
   return tiles <= 0x7fffffff;
 }
 
+bool f32_small_is_narrow(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda) {
+  // a k share per wave that fits the registers
+  return N <= NT && K % 16 == 0 && a_rows_aligned(A, lda) && (K / 16 + 3) / 4 <= 32 && M >= 64;
+}
+
+bool f32_small_b16(int64_t N, const float* B, int64_t ldb) {
+  // every quad of columns whole and aligned
+  return N % 4 == 0 && ldb % 4 == 0 && (reinterpret_cast<uintptr_t>(B) & 15) == 0;
+}
+
 void launch_f32_small(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const float* A,
                       int64_t lda, const float* B, int64_t ldb, float* C, int64_t ldc,
                       const BiasAct* ba) {
   const float* bias = ba ? ba->bias : nullptr;
   const bool relu = ba && ba->relu;
-  // narrow outputs with a k share per wave that fits the registers
-  const int64_t nb_wave = (K / 16 + 3) / 4;
-  if (N <= NT && K % 16 == 0 && a_rows_aligned(A, lda) && nb_wave <= 32 && M >= 64) {
+  if (f32_small_is_narrow(M, N, K, A, lda)) {
+    const int64_t nb_wave = (K / 16 + 3) / 4;
     if (nb_wave <= 8)
       launch_f32_narrow<8>(ctx, M, N, K, A, lda, B, ldb, C, ldc, bias, relu);
     else if (nb_wave <= 16)
@@ -306,8 +315,7 @@ void launch_f32_small(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const
   }
   const int tiles_m = (int)((M + ST - 1) / ST), tiles_n = (int)((N + ST - 1) / ST);
   const dim3 grid((unsigned)(tiles_m * (int64_t)tiles_n)), block(256);
-  // 16-byte loads of B's rows: every quad of columns whole and aligned
-  const bool bvec = N % 4 == 0 && ldb % 4 == 0 && (reinterpret_cast<uintptr_t>(B) & 15) == 0;
+  const bool bvec = f32_small_b16(N, B, ldb);
 #define CIG_SMALL(HB, RL)                                                                        \
   do {                                                                                           \
     if (bvec)                                                                                    \

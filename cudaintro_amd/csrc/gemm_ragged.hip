@@ -1,8 +1,9 @@
-// Any-shape GEMM on the matrix cores, for the calls that no form of the LDS-DMA tile kernel takes
-// (gemm_any_tile.hip serves odd sizes and unaligned rows): a K, or the N of a K x N operand, of
-// fewer than 16 bytes, leading dimensions beyond that kernel's 32-bit row offsets, and the int32
-// accumulator dump beside a dequantized output on unaligned rows.  The library this path replaces
-// takes whatever m, n, k, lda, ldb it is given (quantization/GEMM_bf16.cu:51-56).
+// Any-shape GEMM on the matrix cores, for unaligned calls of few tiles, narrow outputs or a short K,
+// where it is the faster (any_plan.h), and for those that no form of the LDS-DMA tile kernel takes: a
+// K, or the N of a K x N operand, of fewer than 16 bytes, leading dimensions beyond that kernel's
+// 32-bit row offsets, and the int32 accumulator dump beside a dequantized output on unaligned rows.
+// The library this path replaces takes whatever m, n, k, lda, ldb it is given
+// (quantization/GEMM_bf16.cu:51-56).
 //
 // One 128 x 128 output tile per 256-thread workgroup, four waves of 64 x 64 (2 x 2 MFMA tiles
 // of 32 x 32), 64 bytes of k per step.  Operands are fetched in 16-byte pieces of a row, each
@@ -28,6 +29,7 @@
 // K-scaled bound as the tile kernel's; fp32 (v_mfma_f32_32x32x2_f32: true fp32 products and sums)
 // within the same scaled 1e-5 tolerance of the CPU loop as the fp32 tile kernel's.  Only the
 // scalar kernel (CIGEMM_ALGO_GENERIC) reproduces the CPU loop's fp32 bits.
+#include "any_plan.h"
 #include "common.h"
 #include "mfma_tile.h"
 
@@ -301,23 +303,6 @@ __global__ __launch_bounds__(256) void mfma_any_kernel(int64_t M, int64_t N, int
     }
 }
 
-// K ranges for a problem of few tiles (a decode or small-batch shape that no aligned kernel
-// takes): about three workgroups per compute unit are resident, so enough ranges to fill those
-// places, each of at least four steps, at most 16, partials within the workspace.  N = 8191,
-// K = 8192, M = 1 (64 tiles): 255 us unsplit.
-template <typename Math>
-int any_splits(const cigemmContext* ctx, int64_t M, int64_t N, int64_t K, int64_t tiles) {
-  constexpr int KE = RK / Math::ELEM_BYTES;
-  const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
-  if (!ctx->workspace || tiles * 2 > 3 * (int64_t)cus) return 1;  // fewer than two ranges fit
-  const int64_t steps = (K + KE - 1) / KE;
-  int64_t s = 3 * (int64_t)cus / tiles;
-  if (s > 16) s = 16;
-  if (s > steps / 4) s = steps / 4;
-  while (s > 1 && (size_t)s * (size_t)M * (size_t)N * 4 > ctx->ws_partial_bytes) --s;
-  return s < 1 ? 1 : (int)s;
-}
-
 // Returns the number of K ranges the problem was run in.
 template <typename Math, bool B_NK, typename Epi>
 int launch_any(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const void* A, int64_t lda,
@@ -326,11 +311,11 @@ int launch_any(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const void* 
   constexpr int KE = RK / Math::ELEM_BYTES;
   const int tiles_m = (int)((M + RT - 1) / RT), tiles_n = (int)((N + RT - 1) / RT);
   const int64_t tiles = (int64_t)tiles_m * tiles_n;
-  int splits = any_splits<Math>(ctx, M, N, K, tiles);
-  // steps per range, rounded up; ranges that would start past K are dropped
-  const int64_t steps = (K + KE - 1) / KE;
-  const int64_t k_range = splits > 1 ? (steps + splits - 1) / splits * KE : (K > 0 ? K : 1);
-  if (splits > 1) splits = (int)((K + k_range - 1) / k_range);
+  const any::Problem shape{M, N, K * Math::ELEM_BYTES, Math::ELEM_BYTES, 4, false, false, false};
+  int64_t steps = 0;  // per range
+  const int splits = any::staged_ranges(shape, ctx->num_cus > 0 ? ctx->num_cus : 256,
+                                        ctx->workspace ? ctx->ws_partial_bytes : 0, &steps);
+  const int64_t k_range = splits > 1 ? steps * KE : (K > 0 ? K : 1);
   if (splits <= 1) {
     hipLaunchKernelGGL((mfma_any_kernel<Math, B_NK, Epi>), dim3((unsigned)tiles), dim3(256), 0,
                        ctx->stream, M, N, K, A, lda, B, ldb, epi, tiles_m, tiles_n, k_range);

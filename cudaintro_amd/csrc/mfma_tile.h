@@ -1350,10 +1350,12 @@ bool run_tile_plan(cigemmContext* ctx, int mt, int splits, int64_t M, int64_t N,
 // chip idle, covers the columns of the full rounds with 256-row tiles and the remaining
 // columns with a second launch of shorter tiles.  Epi::shift_cols(c) returns the epilogue of
 // the sub-problem starting at column c.
+// `known`: the plan for a problem of at most one round where the caller has made it already.
 // Returns true when the problem was run as a split-K pair of launches.
 template <typename Math, int BMODE, bool ANY = false, typename Epi>
 bool launch_tile(cigemmContext* ctx, int64_t M, int64_t N, int64_t K_bytes, const void* A,
-                 int64_t lda_bytes, const void* B, int64_t ldb_bytes, const Epi& epi) {
+                 int64_t lda_bytes, const void* B, int64_t ldb_bytes, const Epi& epi,
+                 SmallPlan known = SmallPlan{0, 1}) {
   const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
   if (ctx->force_tile_mt >= 1 && ctx->force_tile_mt <= 4) {
     // a plan imposed through the measurement library: as asked, but for K ranges the
@@ -1366,64 +1368,44 @@ bool launch_tile(cigemmContext* ctx, int64_t M, int64_t N, int64_t K_bytes, cons
     return run_tile_plan<Math, BMODE, ANY>(ctx, ctx->force_tile_mt, sp, M, N, K_bytes, A, lda_bytes, B,
                                       ldb_bytes, epi);
   }
-  double single = 0;
-  constexpr TileUnits units = BMODE == B_KN32 ? TILE_UNITS_F32 : TILE_UNITS;
-  const int mt = best_mt(M, N, cus, &single, units);
   if (((M + BM - 1) / BM) * ((N + BN - 1) / BN) <= cus) {
     // At most one round of 256-row tiles: pick the tile height and the number of K ranges
     // together.
     const SmallPlan plan =
-        plan_small(cus, ctx->workspace ? ctx->ws_partial_bytes : 0, M, partial_ld<ANY>(N), K_bytes, Epi::OUT_BYTES,
-                   stage_cost<Math, BMODE>(), K_bytes * N);
+        known.mt ? known
+                 : plan_small(cus, ctx->workspace ? ctx->ws_partial_bytes : 0, M,
+                              partial_ld<ANY>(N), K_bytes, Epi::OUT_BYTES,
+                              stage_cost<Math, BMODE>(), K_bytes * N);
     return run_tile_plan<Math, BMODE, ANY>(ctx, plan.mt, plan.splits, M, N, K_bytes, A, lda_bytes, B,
                                       ldb_bytes, epi);
   }
-  {
-    // Several rounds.  When the tiles of the last round would leave much of the chip idle: the
-    // columns that fill whole rounds of 256-row tiles first, the remaining columns as a second,
-    // separately planned launch (which may split K).  Measured over 80 shapes with 5..24 row
-    // tiles (M = 1280..6144, N = 4096..14336; bf16 and int8 N x K), the two launches issued from
-    // the host: where this rule takes them +3..+22 % (1536 x 11008 x 4096 bf16 143 -> 117 us,
-    // 3584 x 14336 x 4096 347 -> 314), at worst -3 %; the shapes it leaves alone would lose up
-    // to 7 %.
-    const int64_t tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-    if (tiles_m * tiles_n > cus && tiles_m <= cus) {
-      const int64_t cols_per_round = cus / tiles_m;
-      const int64_t full_cols = (tiles_n / cols_per_round) * cols_per_round;
-      if (full_cols > 0 && full_cols < tiles_n) {
-        const int64_t n1 = full_cols * BN, n2 = N - n1;
-        double rest = 0;
-        const int mt2 = best_mt(M, n2, cus, &rest, units);
-        // (a tie stays with the single launch: int8 2048 x 11008 x 4096, 473 tiles of 192 rows in
-        // two rounds against 256 tiles of 256 rows + 176 of 128 rows, alternating in one process:
-        // 85.3 against 86.0 us)
-        if (tile_plan_cost(M, n1, 4, cus, units) + rest < single * 0.97) {
-          launch_tile_256<Math, BMODE, ANY>(ctx, M, n1, K_bytes, A, lda_bytes, B, ldb_bytes, epi);
-          const int rows1 = ctx->last_tile_rows, waves1 = ctx->last_waves;
-          // (n2 may be less than a 16-byte piece; load_piece then reads from the n1 >= 256 columns
-          // in front)
-          const char* B2 = static_cast<const char*>(B) +
-                           (BMODE == B_NK ? n1 * ldb_bytes : n1 * Math::ELEM_BYTES);
-          bool split = false;
-          if (tiles_m * ((n2 + BN - 1) / BN) <= cus) {
-            const SmallPlan plan =
-                plan_small(cus, ctx->workspace ? ctx->ws_partial_bytes : 0, M, partial_ld<ANY>(n2), K_bytes,
-                           Epi::OUT_BYTES, stage_cost<Math, BMODE>(), K_bytes * n2);
-            split = run_tile_plan<Math, BMODE, ANY>(ctx, plan.mt, plan.splits, M, n2, K_bytes, A,
-                                               lda_bytes, B2, ldb_bytes, epi.shift_cols(n1));
-          } else {
-            launch_tile_any_mt<Math, BMODE, ANY>(ctx, mt2, M, n2, K_bytes, A, lda_bytes, B2, ldb_bytes,
-                                            epi.shift_cols(n1));
-          }
-          ctx->first_tile_rows = rows1;
-          ctx->first_waves = waves1;
-          return split;
-        }
-      }
-    }
+  constexpr TileUnits units = BMODE == B_KN32 ? TILE_UNITS_F32 : TILE_UNITS;
+  const RoundsPlan rounds = plan_rounds(M, N, cus, units);
+  const int64_t n1 = rounds.first_cols, n2 = N - n1;
+  if (n1 == 0) {
+    launch_tile_any_mt<Math, BMODE, ANY>(ctx, rounds.mt, M, N, K_bytes, A, lda_bytes, B, ldb_bytes,
+                                         epi);
+    return false;
   }
-  launch_tile_any_mt<Math, BMODE, ANY>(ctx, mt, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, epi);
-  return false;
+  launch_tile_256<Math, BMODE, ANY>(ctx, M, n1, K_bytes, A, lda_bytes, B, ldb_bytes, epi);
+  const int rows1 = ctx->last_tile_rows, waves1 = ctx->last_waves;
+  // (n2 may be less than a 16-byte piece; load_piece then reads from the n1 >= 256 columns in front)
+  const char* B2 =
+      static_cast<const char*>(B) + (BMODE == B_NK ? n1 * ldb_bytes : n1 * Math::ELEM_BYTES);
+  bool split = false;
+  if ((M + BM - 1) / BM * ((n2 + BN - 1) / BN) <= cus) {
+    const SmallPlan plan =
+        plan_small(cus, ctx->workspace ? ctx->ws_partial_bytes : 0, M, partial_ld<ANY>(n2), K_bytes,
+                   Epi::OUT_BYTES, stage_cost<Math, BMODE>(), K_bytes * n2);
+    split = run_tile_plan<Math, BMODE, ANY>(ctx, plan.mt, plan.splits, M, n2, K_bytes, A, lda_bytes,
+                                            B2, ldb_bytes, epi.shift_cols(n1));
+  } else {
+    launch_tile_any_mt<Math, BMODE, ANY>(ctx, rounds.mt, M, n2, K_bytes, A, lda_bytes, B2, ldb_bytes,
+                                         epi.shift_cols(n1));
+  }
+  ctx->first_tile_rows = rows1;
+  ctx->first_waves = waves1;
+  return split;
 }
 
 // Shape / alignment gate shared by the families (sizes in elements, elem = bytes each;
@@ -1442,16 +1424,6 @@ inline bool tile_shape_ok(int64_t M, int64_t N, int64_t K, int elem, const void*
   if (((M + 63) / 64) * ((N + BN - 1) / BN) > 2147483647LL) return false;
   if (lda * elem * 256 >= (1LL << 31) || ldb * elem * 256 >= (1LL << 31)) return false;
   return true;
-}
-
-// The gate of the ANY form: sizes only.  One 16-byte piece must fit a row of either operand (and a
-// column of k); the launch-size and 32-bit offset limits are those above.
-inline bool tile_any_ok(int64_t M, int64_t N, int64_t K, int elem, int64_t lda, int64_t ldb,
-                        bool b_kn) {
-  if (M <= 0 || N <= 0 || K * elem < 16 || (b_kn && N * elem < 16)) return false;
-  if (M > 2147483647LL - 255 || N > 2147483647LL - 255 || K * elem > 2147483647LL) return false;
-  if (((M + 63) / 64) * ((N + BN - 1) / BN) > 2147483647LL) return false;
-  return lda * elem * 256 < (1LL << 31) && ldb * elem * 256 < (1LL << 31);
 }
 
 // The int8 tile kernels' gate: the shape gate above plus what their epilogues store in 16-byte

@@ -476,7 +476,7 @@ extern "C" cigemmStatus_t cigemm_probe_force_tile_plan(cigemmHandle_t h, int til
 
 extern "C" cigemmStatus_t cigemm_probe_force_any_kernel(cigemmHandle_t h, int kernel) {
   if (!h || h->magic != kCtxMagic) return CIGEMM_STATUS_NOT_INITIALIZED;
-  if (kernel < ANY_BY_SHAPE || kernel > ANY_F32_SMALL)
+  if (kernel < ANY_BY_SHAPE || kernel > ANY_TILE)
     return fail(h, CIGEMM_STATUS_INVALID_VALUE, "cigemm_probe_force_any_kernel: kernel %d", kernel);
   h->force_any_kernel = kernel;
   return CIGEMM_STATUS_SUCCESS;

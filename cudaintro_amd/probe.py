@@ -168,7 +168,7 @@ def force_tile_plan(h: Handle, tile_rows: int, k_ranges: int = 1):
            "cigemm_probe_force_tile_plan")
 
 
-ANY_BY_SHAPE, ANY_REGISTER_STAGED, ANY_F32_SMALL = 0, 1, 2
+ANY_BY_SHAPE, ANY_REGISTER_STAGED, ANY_F32_SMALL, ANY_TILE = 0, 1, 2, 3
 
 
 @contextlib.contextmanager

@@ -133,10 +133,10 @@ CIGEMM_API cigemmStatus_t cigemm_probe_dirty_workspace(cigemmHandle_t handle, in
 CIGEMM_API cigemmStatus_t cigemm_probe_force_tile_plan(cigemmHandle_t handle, int tile_rows,
                                                        int k_ranges);
 
-/* Test aid: which kernel serves the handle's calls under CIGEMM_ALGO_MFMA_ANY.  0 = by shape: the
- * tile kernel's any-alignment form and, for what that form does not take, the register-staged
- * kernel; 1 = the register-staged kernel for everything; 2 = fp32 calls on the small kernel (32x32
- * tiles), which takes any K and alignment.  The other algorithms choose as ever. */
+/* Test aid: which kernel serves the handle's calls under CIGEMM_ALGO_MFMA_ANY, where it takes them.
+ * 0 = by shape, as the library chooses; 1 = the register-staged kernel; 2 = fp32 calls on the small
+ * kernel (32x32 tiles), which takes any K and alignment; 3 = the tile kernel's any-alignment form.
+ * The other algorithms choose as ever. */
 CIGEMM_API cigemmStatus_t cigemm_probe_force_any_kernel(cigemmHandle_t handle, int kernel);
 
 #ifdef __cplusplus

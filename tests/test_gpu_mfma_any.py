@@ -1,5 +1,5 @@
-"""The any-shape matrix-core kernels (CIGEMM_ALGO_MFMA_ANY: the tile kernel's any-alignment form,
-the register-staged kernel for what that form does not take): 16-bit and int8 calls with an odd N
+"""The any-shape matrix-core kernels (CIGEMM_ALGO_MFMA_ANY: the tile kernel's any-alignment form and
+the register-staged kernel, each by itself and as the library chooses): 16-bit and int8 calls with an odd N
 or K, leading dimensions and pointers with no alignment beyond the element's, matrices smaller
 than a tile.  int8 bit for bit against the CPU loop, 16-bit bit for bit on exact-arithmetic
 inputs and within the K-scaled bound on normal ones; the padding around every operand is NaN
@@ -39,16 +39,25 @@ def too_narrow(N, K, elem, kn):
 
 @contextmanager
 def choice(handle, how):
-    """How the kernel is chosen: "staged" (imposed), "any" (ALGO_MFMA_ANY) or "default"."""
-    if how == "staged":
-        with probe.any_kernel(handle, probe.ANY_REGISTER_STAGED):
+    """How the kernel is chosen: "staged", "tile" (imposed), "any" (ALGO_MFMA_ANY) or "default"."""
+    if how in ("staged", "tile"):
+        with probe.any_kernel(handle, probe.ANY_TILE if how == "tile" else probe.ANY_REGISTER_STAGED):
             yield
     else:
         with handle.algo(ci.ALGO_MFMA_ANY if how == "any" else ci.ALGO_DEFAULT):
             yield
 
 
-CHOICES = ["staged", "any", "default"]
+CHOICES = ["staged", "tile", "any", "default"]
+
+
+def check_family(how, name, N, K, elem, kn):
+    if how == "staged" or too_narrow(N, K, elem, kn):
+        assert is_register_staged(name), name
+    elif how == "tile":
+        assert is_tile_form(name), name
+    else:
+        assert "_mfma_any_" in name, name
 
 
 def embed(torch, a, dtype, off, pad, fill):
@@ -86,8 +95,7 @@ def test_any_shape_16bit(handle, torch_gpu, oracle, rng, kind, M, N, K):
             flat.fill_(3.0)
             with choice(handle, how):
                 fn(a, b, out=out)
-            staged = how == "staged" or too_narrow(N, K, 2, True)
-            assert (is_register_staged if staged else is_tile_form)(handle.last_kernel), handle.last_kernel
+            check_family(how, handle.last_kernel, N, K, 2, True)
             assert handle.last_kernel.endswith("_splitk") == ((M, N, K) in SPLIT), handle.last_kernel
             got = bits(torch, out)
             if exact:
@@ -120,8 +128,7 @@ def test_any_shape_int8(handle, torch_gpu, oracle, rng, layout, M, N, K):
         flat.fill_(-9)
         with choice(handle, how):
             handle.gemm_i8_i32(a, b, layout, out=out)
-            staged = how == "staged" or too_narrow(N, K, 1, not nk)
-            assert (is_register_staged if staged else is_tile_form)(handle.last_kernel), handle.last_kernel
+            check_family(how, handle.last_kernel, N, K, 1, not nk)
             np.testing.assert_array_equal(out.cpu().numpy(), acc_ref)
             f = flat.cpu().numpy()
             guard = np.ones(f.shape, bool)
@@ -164,13 +171,12 @@ def test_any_shape_f32(handle, torch_gpu, oracle, rng, M, N, K):
                     else:
                         handle.gemm_f32(a, b, out=out)
                         cpu = oracle.gemm_f32(A, B)
-                if how == "staged" or too_narrow(N, K, 4, True):
-                    assert is_register_staged(handle.last_kernel), handle.last_kernel
-                    if how == "staged" and (M, N, K) in SPLIT:
-                        assert handle.last_kernel.endswith("_splitk"), handle.last_kernel
+                if how == "default" and "f32_mfma_any_small" in handle.last_kernel:
+                    pass     # (the small kernel takes any fp32 call)
                 else:
-                    assert is_tile_form(handle.last_kernel) or (
-                        how == "default" and "f32_mfma_any_small" in handle.last_kernel), handle.last_kernel
+                    check_family(how, handle.last_kernel, N, K, 4, True)
+                if how == "staged" and (M, N, K) in SPLIT:
+                    assert handle.last_kernel.endswith("_splitk"), handle.last_kernel
                 got = out.cpu().numpy()
                 if exact:
                     np.testing.assert_array_equal(got, cpu)
@@ -200,9 +206,47 @@ def test_leading_dimension_beyond_the_tile_kernels_offsets(handle, torch_gpu, or
     a = flat.view(M, ld)[:, 1:K + 1]
     a.copy_(torch.from_numpy(A).cuda())
     _, b = embed(torch, B, torch.float32, 0, 0, float("nan"))
-    out = getattr(handle, "gemm_" + kind)(a, b.to(dt).contiguous())
+    with handle.algo(ci.ALGO_MFMA_ANY):     # (by itself an fp32 call this small goes to the small kernel)
+        out = getattr(handle, "gemm_" + kind)(a, b.to(dt).contiguous())
     assert is_register_staged(handle.last_kernel), handle.last_kernel
     np.testing.assert_array_equal(out.float().cpu().numpy(), torch.from_numpy(ref).to(dt).float().numpy())
+
+
+def test_wide_rows_of_b_leave_a_large_fp32_call_to_the_register_staged_kernel(handle, torch_gpu, oracle, rng):
+    """256 rows of B span 2 GiB: not the tile kernel's; A's rows are aligned and K a multiple of 8, so
+    the small kernel takes the call, but 4096 tiles of 32 x 32 are not where it is the faster."""
+    torch = torch_gpu
+    M, N, K = 2048, 2047, 64
+    A, B = rng.choice(VALS, size=(M, K)), rng.choice(VALS, size=(K, N))
+    flat = torch.full((K * ((1 << 21) + 1),), float("nan"), dtype=torch.float32, device="cuda")
+    b = flat.view(K, (1 << 21) + 1)[:, :N]
+    b.copy_(torch.from_numpy(B).cuda())
+    out = handle.gemm_f32(torch.from_numpy(A).cuda(), b)
+    assert is_register_staged(handle.last_kernel), handle.last_kernel
+    np.testing.assert_array_equal(out.cpu().numpy(), oracle.gemm_f32(A, B))
+
+
+def test_choice_by_shape(handle, torch_gpu):
+    """Which of the kernels that take any alignment serves a call, where their times differ by a
+    factor (any_plan.h): narrow outputs and short K stay off the 256-column tiles."""
+    torch = torch_gpu
+    def kernel_for(kind, M, N, K):
+        dt = {"bf16": torch.bfloat16, "f32": torch.float32, "i8nk": torch.int8}[kind]
+        a = torch.zeros((M, K), dtype=dt, device="cuda")
+        if kind == "i8nk":
+            handle.gemm_i8_i32(a, torch.zeros((N, K), dtype=dt, device="cuda"), ci.B_NK)
+        else:
+            getattr(handle, "gemm_" + kind)(a, torch.zeros((K, N), dtype=dt, device="cuda"))
+        return handle.last_kernel
+    assert is_tile_form(kernel_for("bf16", 4096, 4095, 1024))
+    assert is_tile_form(kernel_for("f32", 2049, 2047, 1025))
+    assert is_tile_form(kernel_for("i8nk", 2048, 2047, 4097))
+    assert is_register_staged(kernel_for("i8nk", 4456, 7, 1575))
+    assert is_register_staged(kernel_for("bf16", 33, 11, 741))
+    assert is_register_staged(kernel_for("bf16", 171960, 25, 257))
+    # an output layer of 10 columns keeps its 16-column form beyond one round of 256-row tiles
+    assert kernel_for("f32", 65536, 10, 512) == kernel_for("f32", 70000, 10, 512) == "f32_mfma_small_16x16_ksplit4"
+    assert "small" in kernel_for("f32", 1000, 3, 77)        # narrower than a 16-byte piece, K odd
 
 
 def test_any_shape_kernel_is_the_fallback_not_the_first_choice(handle, torch_gpu):

@@ -97,7 +97,7 @@ def test_every_width_of_the_last_piece(handle, torch_gpu, oracle, rng, kind):
             acc = oracle.gemm_i8_i32(A, B, b_is_nk=layout == ci.B_NK)
             sa, sb = (rng.uniform(1e-3, 5e-2, k).astype(np.float32) for k in (m, n))
             a, b, da, db = (torch.from_numpy(v).cuda() for v in (A, B, sa, sb))
-            with handle.algo(ci.ALGO_MFMA_ANY):
+            with probe.any_kernel(handle, probe.ANY_TILE):
                 np.testing.assert_array_equal(handle.gemm_i8_i32(a, b, layout).cpu().numpy(), acc)
                 y = handle.gemm_i8_dequant(a, b, da, db, layout, ci.OUT_BF16)
             assert "_mfma_any_64x256" in handle.last_kernel, handle.last_kernel
@@ -106,7 +106,7 @@ def test_every_width_of_the_last_piece(handle, torch_gpu, oracle, rng, kind):
             continue
         A, B = rng.choice(VALS, size=(m, K)), rng.choice(VALS, size=(K, n))
         dt = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[kind]
-        with handle.algo(ci.ALGO_MFMA_ANY):
+        with probe.any_kernel(handle, probe.ANY_TILE):
             y = getattr(handle, "gemm_" + kind)(torch.from_numpy(A).cuda().to(dt), torch.from_numpy(B).cuda().to(dt))
         assert "_mfma_any_64x256" in handle.last_kernel, handle.last_kernel
         assert torch.equal(y.cpu(), torch.from_numpy(oracle.gemm_f32(A, B)).to(dt)), n
@@ -148,7 +148,7 @@ def test_two_launches(handle, torch_gpu, rng, kind, rest):
             out.fill_(7)
             assert bool((flat == 7).all()), "a store outside the output"
 
-        with handle.algo(ci.ALGO_MFMA_ANY):
+        with probe.any_kernel(handle, probe.ANY_TILE):
             if not int8:
                 getattr(handle, "gemm_" + kind)(a, b, out=out)
                 check(ref.to(odt))
