@@ -2,6 +2,7 @@
 // accumulation): the shared LDS-tiled MFMA kernel with the fp32 fragment plumbing, plain or
 // with the linear layer's bias + activation epilogue; or, when 256-column tiles would leave
 // most of the chip idle or N is too ragged for them, the 32x32 k-split kernel.
+#include "any_plan.h"
 #include "epilogues.h"
 #include "mfma_tile.h"
 
@@ -21,8 +22,7 @@ bool launch_f32_mfma(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const 
   const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
   const bool one_round = ((M + 255) / 256) * ((N + tile::BN - 1) / tile::BN) <= cus;
   bool small = false;
-  // (a K that is no multiple of 8: the same choice)
-  if (f32_small_any_ok(M, N, K)) {
+  if (f32_small_shape_ok(M, N, K, A, lda)) {
     // Both costs in units of a quarter of one 256x256 tile's time per unit of k: the tile
     // plan's own figure against 0.115 per resident round of 32x32 tiles (2048^3: tile kernel
     // 157 us, small kernel 225 us; 1024^3: 74 us against 33 us; 512^3: 38 us against 8 us).
@@ -34,6 +34,25 @@ bool launch_f32_mfma(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const 
     // the idle compute units (512 x 512 x 4096: 33 us against 55 us; 1024^3: 31 against 32;
     // 512^3: 17 against 9; 960 x 3584 x 3584: 222 against 298).
     small = small_cost < tile_cost && !(K >= 2048 && one_round);
+  } else if (f32_small_any_ok(M, N, K)) {
+    // A K of whole 16-byte pieces that is no multiple of 8: by the small kernel's estimate against
+    // the planner's + 4 us, or against what the launches of several rounds are estimated at.  Over
+    // 300 sizes 0.5 % slower than the faster of the two on average; the tile kernel throughout 38 %,
+    // the comparison above 1.8 %: 3837 x 808 x 1588 144 us on the small kernel against 100, 78 x 1900
+    // x 1972 25.6 against 19.9.
+    const size_t room = ctx->workspace ? ctx->ws_partial_bytes : 0;
+    double tile_us = 0;
+    if (one_round) {
+      tile::plan_small(cus, room, M, N, K * 4, 4, tile::STAGE_COST_KN32, K * 4 * N, &tile_us);
+      tile_us += 4.0;
+    } else {
+      tile_us = any::tile_us(any::COST_F32, any::Problem{M, N, K * 4, 4, 4, false, false, false}, cus,
+                             room, tile::SmallPlan{0, 1});
+      // (that is the any-alignment form; a K of one stage is a single trip here, there a tail and a
+      // loop: 81708 x 356 x 12 38.3 us, estimated 48.0, small kernel 54.4)
+      if (K <= 16) tile_us *= 0.73;
+    }
+    small = any::f32_small_us(M, N, K, cus, f32_small_b16(N, B, ldb), false) < tile_us;
   }
   if (!small) return launch_f32_tile(ctx, M, N, K, A, lda, B, ldb, C, ldc, ba);
   launch_f32_small(ctx, M, N, K, A, lda, B, ldb, C, ldc, ba);

@@ -247,6 +247,9 @@ def test_choice_by_shape(handle, torch_gpu):
     # an output layer of 10 columns keeps its 16-column form beyond one round of 256-row tiles
     assert kernel_for("f32", 65536, 10, 512) == kernel_for("f32", 70000, 10, 512) == "f32_mfma_small_16x16_ksplit4"
     assert "small" in kernel_for("f32", 1000, 3, 77)        # narrower than a 16-byte piece, K odd
+    # K a multiple of 4 but not of 8, all aligned
+    assert "small" in kernel_for("f32", 512, 512, 508)
+    assert "_mfma_any" not in kernel_for("f32", 3837, 808, 1588)
 
 
 def test_any_shape_kernel_is_the_fallback_not_the_first_choice(handle, torch_gpu):
