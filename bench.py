@@ -681,7 +681,7 @@ def main():
                                                    "kernel": handle.last_kernel}
             del a, b, c
         # shapes no aligned kernel takes (odd N: rows of B and C at every 2-byte alignment; odd K:
-        # rows of A): the any-shape matrix-core kernel, and the scalar kernel it took them from
+        # rows of A): the kernel for any alignment, and the scalar kernel
         for (Mx, Nx, Kx) in ((4096, 4095, 4096), (4096, 4096, 4095)):
             a_b, b_b = wl.normal_16bit(Mx, Nx, Kx, seed=2, kind="bf16")
             a, b = dev16(torch, a_b, "bf16"), dev16(torch, b_b, "bf16")

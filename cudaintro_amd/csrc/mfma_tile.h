@@ -632,7 +632,7 @@ __device__ __forceinline__ void store_tile(const Epi& epi, typename Math::acc_t 
 //   * the epilogue (store_tile<ANY>).
 // Measured against the kernel that served these calls before (mfma_any_kernel: one 64-byte step
 // in flight between two barriers, every piece trimmed) and against aligned sizes: bf16 4096 x 4095
-// x 4096 264 -> 115 us (4096^3: 98), 8191 x 8192 at M = 2048 523 -> 219, at M = 1 31.5 -> 26.5;
+// x 4096 264 -> 112 us (4096^3: 104), 8191 x 8192 at M = 2048 523 -> 219, at M = 1 31.5 -> 26.5;
 // int8 N x K 2048 x 8191 x 8191 342 -> 161; fp32 4095 x 4097 x 4099 1493 -> 981 (4096^3: 905).
 // What is left of the difference: a piece that is not 16-byte aligned takes the address path twice
 // (10 % per stage where one 16-bit operand is misaligned, 40 % where both int8 ones are), and so

@@ -149,8 +149,9 @@ typedef enum cigemmAlgo {
                               whole 128-column slabs */
   CIGEMM_ALGO_SMALL = 3,   /* fp32 32x32 tile per workgroup, k split over the waves */
   CIGEMM_ALGO_MFMA_ANY = 4 /* MFMA tiles at element alignment: any shape, leading dimension and
-                              alignment, every type.  DEFAULT uses it for what the families
-                              above do not take */
+                              alignment, every type, on the one of two kernels estimated to be the
+                              faster.  DEFAULT uses it (fp32: or the small kernel at any K and
+                              alignment) for what the families above do not take */
 } cigemmAlgo_t;
 CIGEMM_API cigemmStatus_t cigemmSetAlgo(cigemmHandle_t handle, cigemmAlgo_t algo);
 CIGEMM_API cigemmStatus_t cigemmGetAlgo(cigemmHandle_t handle, cigemmAlgo_t* algo);

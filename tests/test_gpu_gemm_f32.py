@@ -1,4 +1,6 @@
 """fp32 GEMM through the C ABI against the reference CPU GEMM (oracle)."""
+import re
+
 import numpy as np
 import pytest
 
@@ -241,7 +243,7 @@ def test_narrow_kernel_weights_inside_a_wider_matrix(handle, torch_gpu, oracle, 
 
 def test_default_choice_by_shape(handle, torch_gpu):
     """Small problems and narrow outputs go to the 32x32 kernel, large ones to 256-column
-    tiles, what neither takes to the any-shape matrix-core kernel."""
+    tiles, unaligned ones to the small kernel or to the tile kernel's any-alignment form."""
     torch = torch_gpu
     def kernel_for(M, N, K):
         handle.gemm_f32(torch.zeros((M, K), device="cuda"), torch.zeros((K, N), device="cuda"))
@@ -255,7 +257,8 @@ def test_default_choice_by_shape(handle, torch_gpu):
     assert "x256x16_w" in kernel_for(20000, 512, 784)
     assert kernel_for(512, 512, 4096).endswith("_splitk")      # long K: tile kernel, K split
     assert kernel_for(256, 1024, 8192).endswith("_splitk")
-    assert "mfma_any" in kernel_for(77, 91, 300)
+    assert kernel_for(77, 91, 300) == "f32_mfma_any_small_32x32_ksplit4"
+    assert re.match(r"f32_mfma_any_[0-9+]+x256x16_w4_ring4", kernel_for(2049, 2047, 1025))
 
 
 def test_all_kernels_agree_on_exact_inputs(handle, torch_gpu, oracle, rng):
