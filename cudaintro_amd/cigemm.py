@@ -138,6 +138,15 @@ def gemm_bf16_static(A, B, out=None, stream=None):
     return out
 
 
+def _mat(t):
+    """(rows, columns, leading dimension) of a matrix whose rows are contiguous."""
+    s = t.stride()
+    assert len(s) == 2
+    rows, cols = t.shape
+    assert cols <= 1 or s[1] == 1, "rows must be contiguous"
+    return rows, cols, s[0] if rows > 1 else max(cols, s[0], 1)
+
+
 class Handle:
     """Owns one ``cigemmHandle_t`` bound to the current device and to torch's current stream."""
 
@@ -149,6 +158,8 @@ class Handle:
             raise CigemmError(st, "", "cigemmCreate")
         self._h = h
         torch = _torch()
+        self._f32, self._bf16, self._f16, self._i8 = (torch.float32, torch.bfloat16, torch.float16,
+                                                      torch.int8)
         s = torch.cuda.current_stream() if stream is None else stream
         self.set_stream(s.cuda_stream)
 
@@ -224,45 +235,47 @@ class Handle:
     # -- GEMMs ------------------------------------------------------------------------------
     @staticmethod
     def _ld(t):
-        assert t.dim() == 2 and (t.shape[1] <= 1 or t.stride(1) == 1), "rows must be contiguous"
-        return t.stride(0) if t.shape[0] > 1 else max(t.shape[1], t.stride(0), 1)
+        return _mat(t)[2]
 
-    def _gemm(self, fn, A, B, out, out_dtype):
-        torch = _torch()
-        M, K = A.shape
-        K2, N = B.shape
+    # A small product takes as long as the host needs to issue it (fp32 512^3: 6.55 us a call, 5.80
+    # since), so each call asks a tensor for its shape, strides and address once and looks nothing
+    # else up.
+    def _gemm(self, fn, name, A, B, out, out_dtype):
+        M, K, lda = _mat(A)
+        K2, N, ldb = _mat(B)
         assert K == K2
         if out is None:
-            out = torch.empty((M, N), dtype=out_dtype, device=A.device)
-        st = getattr(self.lib, fn)(self._h, M, N, K, A.data_ptr(), self._ld(A), B.data_ptr(),
-                                   self._ld(B), out.data_ptr(), self._ld(out))
-        self._check(st, fn)
+            out = _torch().empty((M, N), dtype=out_dtype, device=A.device)
+        st = fn(self._h, M, N, K, A.data_ptr(), lda, B.data_ptr(), ldb, out.data_ptr(), _mat(out)[2])
+        if st:
+            self._check(st, name)
         return out
 
     def gemm_f32(self, A, B, out=None):
-        torch = _torch()
-        assert A.dtype == torch.float32 and B.dtype == torch.float32
-        return self._gemm("cigemm_gemm_f32", A, B, out, torch.float32)
+        f32 = self._f32
+        assert A.dtype == f32 and B.dtype == f32
+        return self._gemm(self.lib.cigemm_gemm_f32, "cigemm_gemm_f32", A, B, out, f32)
 
     def linear_f32(self, X, W, bias=None, act=ACT_NONE, out=None):
         """out = act(bias + X @ W) with W stored K x N (input-major)."""
-        torch = _torch()
-        assert X.dtype == torch.float32 and W.dtype == torch.float32
-        M, K = X.shape
-        K2, N = W.shape
-        assert K == K2 and (bias is None or (bias.dtype == torch.float32 and bias.numel() == N))
+        f32 = self._f32
+        assert X.dtype == f32 and W.dtype == f32
+        M, K, ldx = _mat(X)
+        K2, N, ldw = _mat(W)
+        assert K == K2 and (bias is None or (bias.dtype == f32 and bias.numel() == N))
         if out is None:
-            out = torch.empty((M, N), dtype=torch.float32, device=X.device)
-        st = self.lib.cigemm_linear_f32(self._h, M, N, K, X.data_ptr(), self._ld(X), W.data_ptr(),
-                                        self._ld(W), bias.data_ptr() if bias is not None else None,
-                                        act, out.data_ptr(), self._ld(out))
-        self._check(st, "cigemm_linear_f32")
+            out = _torch().empty((M, N), dtype=f32, device=X.device)
+        st = self.lib.cigemm_linear_f32(self._h, M, N, K, X.data_ptr(), ldx, W.data_ptr(), ldw,
+                                        bias.data_ptr() if bias is not None else None, act,
+                                        out.data_ptr(), _mat(out)[2])
+        if st:
+            self._check(st, "cigemm_linear_f32")
         return out
 
     def gemm_f16(self, A, B, out=None):
-        torch = _torch()
-        assert A.dtype == torch.float16 and B.dtype == torch.float16
-        return self._gemm("cigemm_gemm_f16", A, B, out, torch.float16)
+        f16 = self._f16
+        assert A.dtype == f16 and B.dtype == f16
+        return self._gemm(self.lib.cigemm_gemm_f16, "cigemm_gemm_f16", A, B, out, f16)
 
     # -- study kernels (TileProgramming demo) -------------------------------------------------
     def matrixMulTiled(self, A, B):
@@ -289,45 +302,53 @@ class Handle:
         return Cm
 
     def gemm_bf16(self, A, B, out=None):
-        torch = _torch()
-        assert A.dtype == torch.bfloat16 and B.dtype == torch.bfloat16
-        return self._gemm("cigemm_gemm_bf16", A, B, out, torch.bfloat16)
+        bf16 = self._bf16
+        assert A.dtype == bf16 and B.dtype == bf16
+        return self._gemm(self.lib.cigemm_gemm_bf16, "cigemm_gemm_bf16", A, B, out, bf16)
 
     def gemm_i8_i32(self, A, B, b_layout=B_KN, out=None):
-        torch = _torch()
-        assert A.dtype == torch.int8 and B.dtype == torch.int8
-        M, K = A.shape
-        N = B.shape[0] if b_layout == B_NK else B.shape[1]
-        assert (B.shape[1] if b_layout == B_NK else B.shape[0]) == K
+        assert A.dtype == self._i8 and B.dtype == self._i8
+        M, K, lda = _mat(A)
+        K2, N, ldb = _mat(B)
+        if b_layout == B_NK:
+            K2, N = N, K2
+        assert K == K2
         if out is None:
+            torch = _torch()
             out = torch.empty((M, N), dtype=torch.int32, device=A.device)
-        st = self.lib.cigemm_gemm_i8_i32(self._h, M, N, K, A.data_ptr(), self._ld(A),
-                                         B.data_ptr(), self._ld(B), b_layout, out.data_ptr(),
-                                         self._ld(out))
-        self._check(st, "cigemm_gemm_i8_i32")
+        st = self.lib.cigemm_gemm_i8_i32(self._h, M, N, K, A.data_ptr(), lda, B.data_ptr(), ldb,
+                                         b_layout, out.data_ptr(), _mat(out)[2])
+        if st:
+            self._check(st, "cigemm_gemm_i8_i32")
         return out
 
     def gemm_i8_dequant(self, A, B, scale_a, scale_b, b_layout=B_KN, out_type=OUT_F32, out=None,
                         dump_acc=False):
         """Returns ``out`` or ``(out, acc)`` when ``dump_acc``.  A scale tensor with one
         element is per-tensor, otherwise per-row (A) / per-column (B)."""
-        torch = _torch()
-        M, K = A.shape
-        N = B.shape[0] if b_layout == B_NK else B.shape[1]
-        assert (B.shape[1] if b_layout == B_NK else B.shape[0]) == K
-        assert scale_a.dtype == torch.float32 and scale_b.dtype == torch.float32
-        assert scale_a.numel() in (1, M) and scale_b.numel() in (1, N)
-        ma = SCALE_VECTOR if scale_a.numel() == M and M > 1 else SCALE_TENSOR
-        mb = SCALE_VECTOR if scale_b.numel() == N and N > 1 else SCALE_TENSOR
+        f32 = self._f32
+        M, K, lda = _mat(A)
+        K2, N, ldb = _mat(B)
+        if b_layout == B_NK:
+            K2, N = N, K2
+        assert K == K2
+        assert scale_a.dtype == f32 and scale_b.dtype == f32
+        na, nb = scale_a.numel(), scale_b.numel()
+        assert (na == 1 or na == M) and (nb == 1 or nb == N)
         if out is None:
-            out = torch.empty((M, N), device=A.device,
-                              dtype=torch.bfloat16 if out_type == OUT_BF16 else torch.float32)
-        acc = torch.empty((M, N), dtype=torch.int32, device=A.device) if dump_acc else None
+            out = _torch().empty((M, N), device=A.device,
+                                 dtype=self._bf16 if out_type == OUT_BF16 else f32)
+        acc = None
+        if dump_acc:
+            torch = _torch()
+            acc = torch.empty((M, N), dtype=torch.int32, device=A.device)
         st = self.lib.cigemm_gemm_i8_dequant(
-            self._h, M, N, K, A.data_ptr(), self._ld(A), B.data_ptr(), self._ld(B), b_layout,
-            scale_a.data_ptr(), ma, scale_b.data_ptr(), mb, out.data_ptr(), out_type,
-            self._ld(out), acc.data_ptr() if dump_acc else None, N if dump_acc else 0)
-        self._check(st, "cigemm_gemm_i8_dequant")
+            self._h, M, N, K, A.data_ptr(), lda, B.data_ptr(), ldb, b_layout, scale_a.data_ptr(),
+            SCALE_VECTOR if na > 1 else SCALE_TENSOR, scale_b.data_ptr(),
+            SCALE_VECTOR if nb > 1 else SCALE_TENSOR, out.data_ptr(), out_type, _mat(out)[2],
+            acc.data_ptr() if dump_acc else None, N if dump_acc else 0)
+        if st:
+            self._check(st, "cigemm_gemm_i8_dequant")
         return (out, acc) if dump_acc else out
 
     # -- generators / quantizer ---------------------------------------------------------------
@@ -342,16 +363,17 @@ class Handle:
         return out
 
     def quantize_rows_i8(self, x, out=None):
-        torch = _torch()
-        assert x.dtype == torch.float32 and x.dim() == 2
-        rows, cols = x.shape
+        assert x.dtype == self._f32 and x.dim() == 2
+        rows, cols, ldx = _mat(x)
         if out is None:
+            torch = _torch()
             q = torch.empty((rows, cols), dtype=torch.int8, device=x.device)
             s = torch.empty((rows,), dtype=torch.float32, device=x.device)
         else:
             q, s = out
-            assert q.dtype == torch.int8 and q.shape == x.shape and s.dtype == torch.float32
-        st = self.lib.cigemm_quantize_rows_i8(self._h, rows, cols, x.data_ptr(), self._ld(x),
-                                              q.data_ptr(), self._ld(q), s.data_ptr())
-        self._check(st, "cigemm_quantize_rows_i8")
+            assert q.dtype == self._i8 and q.shape == x.shape and s.dtype == self._f32
+        st = self.lib.cigemm_quantize_rows_i8(self._h, rows, cols, x.data_ptr(), ldx, q.data_ptr(),
+                                              _mat(q)[2], s.data_ptr())
+        if st:
+            self._check(st, "cigemm_quantize_rows_i8")
         return q, s
