@@ -59,6 +59,10 @@ constexpr Cost COST_I8_NK{
     tile::STAGE_COST_NK8, tile::TILE_UNITS};
 
 inline int64_t div_up(int64_t a, int64_t b) { return (a + b - 1) / b; }
+// (see Problem::a_apart)
+inline bool rows_apart(const void* p, int64_t ld_bytes) {
+  return (((uintptr_t)p | (uintptr_t)ld_bytes) & 3) != 0;
+}
 inline double at_most(double v, double top) { return v < top ? v : top; }
 
 // What the tile form takes: sizes only.  One 16-byte piece must fit a row of either operand (and a
@@ -141,6 +145,22 @@ inline double staged_us(const Cost& c, const Problem& p, int cus, size_t partial
   if (sp > 1) us += c.s_reduce + c.s_reduce_mb * mn * (4 * sp + p.out_bytes);
   if (p.dequant) us += (sp > 1 ? 0.0 : c.s_dequant * rows) + c.s_dequant_mb * mn;
   return us;
+}
+
+// What the tile kernel or the register-staged kernel is estimated to take, whichever serves the call;
+// `aligned`: the tile kernel's aligned form does (the same terms rank it: rms error 12..14 % over
+// 250 aligned calls).
+inline double other_us(const Cost& c, const Problem& p, bool aligned, int cus, size_t partial_bytes) {
+  if (aligned) {
+    tile::SmallPlan plan{0, 1};
+    if (div_up(p.M, tile::BM) * div_up(p.N, tile::BN) <= cus)
+      plan = tile::plan_small(cus, partial_bytes, p.M, p.N, p.K_bytes, p.out_bytes, c.sc,
+                              p.K_bytes * p.N);
+    return tile_us(c, p, cus, partial_bytes, plan);
+  }
+  const double staged = staged_us(c, p, cus, partial_bytes);
+  const double tile = tile_us(c, p, cus, partial_bytes, tile_plan(c, p, cus, partial_bytes));
+  return staged < tile ? staged : tile;
 }
 
 // The small fp32 kernel: 32 x 32 tiles, K walked by four waves, so a chain of loads whose price

@@ -92,6 +92,7 @@ cigemmStatus_t cigemmCreate(cigemmHandle_t* handle) {
   ctx->ws_dirty = 0;
   ctx->force_tile_mt = 0;
   ctx->force_tile_splits = 0;
+  ctx->force_kwaves = 0;
   ctx->force_any_kernel = ANY_BY_SHAPE;
   ctx->workspace = nullptr;
   if (hipMalloc(&ctx->workspace,
@@ -216,10 +217,6 @@ static AnyChoice choose_any(cigemmHandle_t h, const any::Cost& cost, const any::
   return best;
 }
 
-static bool rows_apart(const void* p, int64_t ld_bytes) {
-  return (((uintptr_t)p | (uintptr_t)ld_bytes) & 3) != 0;
-}
-
 static bool any_f32(cigemmHandle_t h, int64_t M, int64_t N, int64_t K, const float* A, int64_t lda,
                     const float* B, int64_t ldb, float* C, int64_t ldc, const BiasAct* ba) {
   const bool small_ok = f32_small_any_ok(M, N, K);
@@ -242,7 +239,7 @@ static bool any_f32(cigemmHandle_t h, int64_t M, int64_t N, int64_t K, const flo
 
 static bool any_16(cigemmHandle_t h, bool bf16, int64_t M, int64_t N, int64_t K, const uint16_t* A,
                    int64_t lda, const uint16_t* B, int64_t ldb, uint16_t* C, int64_t ldc) {
-  const AnyChoice c = choose_any(h, any::COST_16, any::Problem{M, N, K * 2, 2, 2, false, rows_apart(A, lda * 2), rows_apart(B, ldb * 2)},
+  const AnyChoice c = choose_any(h, any::COST_16, any::Problem{M, N, K * 2, 2, 2, false, any::rows_apart(A, lda * 2), any::rows_apart(B, ldb * 2)},
                                  any::tile_ok(M, N, K, 2, lda, ldb, true), -1.0);
   return (c.kernel != ANY_REGISTER_STAGED &&
           launch_tile_any_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc, c.plan)) ||
@@ -253,7 +250,7 @@ static bool any_i8(cigemmHandle_t h, int64_t M, int64_t N, int64_t K, const int8
                    const int8_t* B, int64_t ldb, bool b_nk, int32_t* C, int64_t ldc,
                    const DequantArgs* dq) {
   const any::Problem p{M, N, K, 1, dq && dq->out_bf16 ? 2 : 4, dq != nullptr,
-                       rows_apart(A, lda), rows_apart(B, ldb)};
+                       any::rows_apart(A, lda), any::rows_apart(B, ldb)};
   // (the accumulator dump is the register-staged kernel's)
   const AnyChoice c = choose_any(h, b_nk ? any::COST_I8_NK : any::COST_I8_KN, p,
                                  any::tile_ok(M, N, K, 1, lda, ldb, !b_nk) && !(dq && dq->acc_out),
@@ -334,6 +331,7 @@ static cigemmStatus_t gemm16(cigemmHandle_t h, const char* name, bool bf16, int6
       // decode shapes (M <= 32) first: they are bandwidth problems with their own kernel; what
       // neither that nor the tile kernel takes (odd N, unaligned rows) stays on the matrix cores
       if (!launch_skinny_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc) &&
+          !launch_kwaves_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc) &&
           !launch_16b_mfma(h, bf16, M, N, K, A, lda, B, ldb, C, ldc) &&
           !any_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc))
         launch_generic_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc);
@@ -370,6 +368,7 @@ static cigemmStatus_t gemm_i8(cigemmHandle_t h, const char* name, int64_t M, int
     case CIGEMM_ALGO_GENERIC: launch_generic_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq); break;
     default:
       if (!launch_skinny_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq) &&
+          !launch_kwaves_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq) &&
           !launch_i8_mfma(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq) &&
           !any_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq))
         launch_generic_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq);

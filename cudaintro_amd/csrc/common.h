@@ -45,6 +45,9 @@ struct cigemmContext {
   // in place of its own plan; 0 = the launcher chooses.
   int force_tile_mt;
   int force_tile_splits;
+  // The same for the kernel of small outputs: the K ranges imposed on every call it takes, -1 keeps
+  // it out of every call, 0 = the library chooses.
+  int force_kwaves;
   // Test aid, set through the probe library only: which kernel serves a call that
   // CIGEMM_ALGO_MFMA_ANY selects: AnyKernel.
   int force_any_kernel;
@@ -248,6 +251,13 @@ bool launch_tile_any_f32(cigemmContext*, int64_t M, int64_t N, int64_t K, const 
 bool launch_tile_any_i8(cigemmContext*, int64_t M, int64_t N, int64_t K, const int8_t* A,
                         int64_t lda, const int8_t* B, int64_t ldb, bool b_nk, int32_t* C,
                         int64_t ldc, const DequantArgs* dq, tile::SmallPlan plan);
+// gemm_kwaves.hip: 32 x 64 tiles, k shared out to the waves; any size and alignment.  False, with
+// nothing launched, where another kernel is estimated to be faster.
+bool launch_kwaves_16(cigemmContext*, bool bf16, int64_t M, int64_t N, int64_t K, const uint16_t* A,
+                      int64_t lda, const uint16_t* B, int64_t ldb, uint16_t* C, int64_t ldc);
+bool launch_kwaves_i8(cigemmContext*, int64_t M, int64_t N, int64_t K, const int8_t* A, int64_t lda,
+                      const int8_t* B, int64_t ldb, bool b_nk, int32_t* C, int64_t ldc,
+                      const DequantArgs* dq);
 void launch_generic_16(cigemmContext*, bool bf16, int64_t M, int64_t N, int64_t K,
                        const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb,
                        uint16_t* C, int64_t ldc);
@@ -275,6 +285,8 @@ void launch_f32_small(cigemmContext*, int64_t M, int64_t N, int64_t K, const flo
                       int64_t lda, const float* B, int64_t ldb, float* C, int64_t ldc,
                       const BiasAct* ba = nullptr);
 // gemm_16b.hip
+bool tile_16_ok(int64_t M, int64_t N, int64_t K, const uint16_t* A, int64_t lda, const uint16_t* B,
+                int64_t ldb, const uint16_t* C, int64_t ldc);
 bool launch_16b_mfma(cigemmContext*, bool bf16, int64_t M, int64_t N, int64_t K,
                      const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb,
                      uint16_t* C, int64_t ldc);

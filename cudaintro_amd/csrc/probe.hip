@@ -474,6 +474,14 @@ extern "C" cigemmStatus_t cigemm_probe_force_tile_plan(cigemmHandle_t h, int til
   return CIGEMM_STATUS_SUCCESS;
 }
 
+extern "C" cigemmStatus_t cigemm_probe_force_kwaves_plan(cigemmHandle_t h, int k_ranges) {
+  if (!h || h->magic != kCtxMagic) return CIGEMM_STATUS_NOT_INITIALIZED;
+  if (k_ranges < -1 || k_ranges > 64)
+    return fail(h, CIGEMM_STATUS_INVALID_VALUE, "cigemm_probe_force_kwaves_plan: k_ranges %d", k_ranges);
+  h->force_kwaves = k_ranges;
+  return CIGEMM_STATUS_SUCCESS;
+}
+
 extern "C" cigemmStatus_t cigemm_probe_force_any_kernel(cigemmHandle_t h, int kernel) {
   if (!h || h->magic != kCtxMagic) return CIGEMM_STATUS_NOT_INITIALIZED;
   if (kernel < ANY_BY_SHAPE || kernel > ANY_TILE)

@@ -31,6 +31,7 @@ SIGNATURES = {
                                                   _vp, _ci, _vp, _ci, _i64, _vp, _i64]),
     "cigemm_probe_dirty_workspace": (_ci, [_vp, _ci, C.c_uint32, _ci]),
     "cigemm_probe_force_tile_plan": (_ci, [_vp, _ci, _ci]),
+    "cigemm_probe_force_kwaves_plan": (_ci, [_vp, _ci]),
     "cigemm_probe_force_any_kernel": (_ci, [_vp, _ci]),
 }
 
@@ -166,6 +167,13 @@ def force_tile_plan(h: Handle, tile_rows: int, k_ranges: int = 1):
     choice back to the library."""
     _check(h, load_library().cigemm_probe_force_tile_plan(h.raw, tile_rows, k_ranges),
            "cigemm_probe_force_tile_plan")
+
+
+def force_kwaves_plan(h: Handle, k_ranges: int):
+    """The same for the kernel of small outputs: its K ranges; -1 keeps it out of the handle's calls, 0
+    hands the choice back."""
+    _check(h, load_library().cigemm_probe_force_kwaves_plan(h.raw, k_ranges),
+           "cigemm_probe_force_kwaves_plan")
 
 
 ANY_BY_SHAPE, ANY_REGISTER_STAGED, ANY_F32_SMALL, ANY_TILE = 0, 1, 2, 3

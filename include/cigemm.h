@@ -124,13 +124,15 @@ CIGEMM_API int cigemmGetVersion(void);
  * "<type>_mfma_<tile rows>x256x<k per stage>_w<waves per workgroup>_ring4[_kn|_nk][_dequant]
  * [_bias_act][_splitk]", e.g. "bf16_mfma_256x256x32_w4_ring4", "i8_mfma_256+192x256x64_w8+w4_
  * ring4_nk_dequant" when two launches of different tile heights covered the columns (a
- * "_splitk" after such a name: the second launch ran as K ranges plus a reduction).  Valid
- * until the next GEMM call on the handle. */
+ * "_splitk" after such a name: the second launch ran as K ranges plus a reduction); the kernel of
+ * small outputs "<type>_mfma_[any_]kwaves_32x64x<k per piece>_w4[_kn|_nk][_dequant]_splitk" (k is
+ * always split, over its four waves at least).  Valid until the next GEMM call on the handle. */
 CIGEMM_API const char* cigemmGetLastKernelName(cigemmHandle_t handle);
 
 /* Plan of the last successful GEMM call on this handle, for tests and profiles: rows of the
- * output tile (256, 192, 128 or 64; with two launches, of the second) and number of K ranges
- * when the LDS-tiled matrix-core kernel ran, 0 and 0 when another family did.  Either pointer
+ * output tile (256, 192, 128 or 64; with two launches, of the second; 32 for the kernel of small
+ * outputs) and number of K ranges (one workgroup each) when the LDS-tiled matrix-core kernel or the
+ * kernel of small outputs ran, 0 and 0 when another family did.  Either pointer
  * may be null.  No counterpart in the reference: cuBLAS does not report its heuristics'
  * choice (quantization/GEMM_bf16.cu:51-56). */
 CIGEMM_API cigemmStatus_t cigemmGetLastPlan(cigemmHandle_t handle, int* tile_rows, int* k_splits);

@@ -133,6 +133,11 @@ CIGEMM_API cigemmStatus_t cigemm_probe_dirty_workspace(cigemmHandle_t handle, in
 CIGEMM_API cigemmStatus_t cigemm_probe_force_tile_plan(cigemmHandle_t handle, int tile_rows,
                                                        int k_ranges);
 
+/* The same for the kernel of small outputs (32 x 64 tiles): the number of K ranges of the handle's
+ * following calls under CIGEMM_ALGO_DEFAULT (those it takes).  -1 keeps the kernel out of them, 0
+ * hands the choice back to the library. */
+CIGEMM_API cigemmStatus_t cigemm_probe_force_kwaves_plan(cigemmHandle_t handle, int k_ranges);
+
 /* Test aid: which kernel serves the handle's calls under CIGEMM_ALGO_MFMA_ANY, where it takes them.
  * 0 = by shape, as the library chooses; 1 = the register-staged kernel; 2 = fp32 calls on the small
  * kernel (32x32 tiles), which takes any K and alignment; 3 = the tile kernel's any-alignment form.

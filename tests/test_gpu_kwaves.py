@@ -1,0 +1,91 @@
+"""The kernel of small outputs (32 x 64 tiles, k shared out to four waves, K ranges joined inside the
+kernel) at the sizes where it can go wrong: M and N around its tiles, K around its 128-byte pieces (all
+of K in the separately multiplied tail, fewer pieces than waves, more than its slots hold, a tail of one
+element up to a whole piece, in every wave), one and several K ranges, aligned and unaligned operands.  Operand
+values are small integers and halves, so every sum is exact in any order and the comparison is bit for
+bit; the padding around the operands is NaN (127 for int8), the output sits in a sentinel-filled
+buffer.  Every call runs twice: the second finds the workspace as the first left it."""
+import numpy as np
+import pytest
+
+import cudaintro_amd as ci
+from cudaintro_amd import probe
+from gpu_util import bits
+from test_gpu_mfma_any import VALS, embed
+
+pytestmark = pytest.mark.gpu
+BYTES = {"bf16": 2, "f16": 2, "i8_kn": 1, "i8_nk": 1}
+SHAPES = [  # M, N, aligned
+    (33, 136, True), (129, 260, True), (200, 384, True), (65, 64, True),
+    (64, 127, False), (130, 193, False), (257, 33, False),
+]
+
+
+def sizes_of_k(eb, aligned):
+    stage, piece = 128 // eb, 16 // eb
+    if aligned:
+        return [piece, stage, 3 * stage, 5 * stage, 6 * stage, 15 * stage + 3 * piece]
+    return [piece, stage + 1, 4 * stage + 1, 7 * stage - 1, 14 * stage]
+
+
+@pytest.mark.parametrize("kind", list(BYTES))
+def test_kwaves(handle, torch_gpu, oracle, rng, kind):
+    torch = torch_gpu
+    int8 = kind.startswith("i8")
+    layout = ci.B_NK if kind == "i8_nk" else ci.B_KN
+    host = lambda t: bits(torch, t) if t.element_size() == 2 else t.contiguous().cpu().numpy()  # noqa: E731
+    for M, N, aligned in SHAPES:
+        for K in sizes_of_k(BYTES[kind], aligned):
+            if int8:
+                A = rng.integers(-127, 128, size=(M, K), dtype=np.int8)
+                B = rng.integers(-127, 128, size=(N, K) if layout == ci.B_NK else (K, N), dtype=np.int8)
+                ref = oracle.gemm_i8_i32(A, B, b_is_nk=layout == ci.B_NK)
+                dt, odt, pad = torch.int8, torch.int32, 127
+            else:
+                A, B = rng.choice(VALS, size=(M, K)), rng.choice(VALS, size=(K, N))
+                ref = oracle.gemm_f32(A, B)
+                dt = odt = {"bf16": torch.bfloat16, "f16": torch.float16}[kind]
+                pad = float("nan")
+                narrow = {"bf16": oracle.f32_to_bf16, "f16": oracle.f32_to_f16}[kind]
+                A, B, ref = narrow(A).view(np.int16), narrow(B).view(np.int16), narrow(ref)
+            # rows of whole 16-byte pieces at offset 0, or everything off by an element
+            step = 16 // BYTES[kind]
+            off, fill = (0, lambda c, e: -c % e) if aligned else (1, lambda c, e: 3)
+            _, a = embed(torch, A, dt, off, fill(A.shape[1], step), pad)
+            _, b = embed(torch, B, dt, off, fill(B.shape[1], step), pad)
+            po = fill(N, 16 // odt.itemsize)
+            flat, out = embed(torch, np.zeros((M, N), np.int32).astype(np.int16 if odt.itemsize == 2 else np.int32),
+                              odt, off, po, 0)
+            guard = np.ones(flat.numel(), bool)
+            for i in range(M):
+                guard[off + i * (N + po): off + i * (N + po) + N] = False
+            for ranges in (1, 2, 3, 5):
+                probe.force_kwaves_plan(handle, ranges)
+                try:
+                    for _ in range(2):
+                        flat.fill_(7)
+                        sentinel = host(flat)[0]
+                        if int8:
+                            handle.gemm_i8_i32(a, b, layout, out=out)
+                        else:
+                            getattr(handle, "gemm_" + kind)(a, b, out=out)
+                        assert "kwaves_32x64" in handle.last_kernel, handle.last_kernel
+                        what = f"{handle.last_kernel} {handle.last_plan} M={M} N={N} K={K}"
+                        np.testing.assert_array_equal(host(out), ref, err_msg=what)
+                        assert (host(flat)[guard] == sentinel).all(), what
+                    if int8:
+                        sa = rng.uniform(1e-3, 5e-2, M).astype(np.float32)
+                        sb = rng.uniform(1e-3, 5e-2, N).astype(np.float32)
+                        for name, ot in (("f32", ci.OUT_F32), ("bf16", ci.OUT_BF16)):
+                            y = handle.gemm_i8_dequant(a, b, torch.from_numpy(sa).cuda(),
+                                                       torch.from_numpy(sb).cuda(), layout, ot)
+                            assert "kwaves_32x64" in handle.last_kernel, handle.last_kernel
+                            np.testing.assert_array_equal(
+                                host(y), oracle.dequant(ref, sa, sb, out_dtype=name, sa_per_row=M > 1,
+                                                        sb_per_col=True), err_msg=what)
+                            y = handle.gemm_i8_dequant(a, b, torch.from_numpy(sa[:1]).cuda(),
+                                                       torch.from_numpy(sb[:1]).cuda(), layout, ot)
+                            np.testing.assert_array_equal(
+                                host(y), oracle.dequant(ref, sa[:1], sb[:1], out_dtype=name), err_msg=what)
+                finally:
+                    probe.force_kwaves_plan(handle, 0)
