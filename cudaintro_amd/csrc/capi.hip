@@ -90,7 +90,7 @@ cigemmStatus_t cigemmCreate(cigemmHandle_t* handle) {
   ctx->ws_counter_bytes = (size_t)64 << 10;
   ctx->ws_swap_bytes = (size_t)8 << 20;  // 128 bytes per column: N <= 65536
   ctx->ws_dirty = 0;
-  ctx->force_tile_mt = 0;
+  ctx->force_tile_rows = 0;
   ctx->force_tile_splits = 0;
   ctx->force_kwaves = 0;
   ctx->force_any_kernel = ANY_BY_SHAPE;
@@ -198,7 +198,7 @@ static AnyChoice choose_any(cigemmHandle_t h, const any::Cost& cost, const any::
     best.kernel = (AnyKernel)h->force_any_kernel;
     return best;
   }
-  if (tile_ok && h->force_tile_mt) {  // a plan of the tile kernel is imposed
+  if (tile_ok && h->force_tile_rows) {  // a plan of the tile kernel is imposed
     best.kernel = ANY_TILE;
     return best;
   }

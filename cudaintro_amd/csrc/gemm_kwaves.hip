@@ -421,7 +421,7 @@ Plan plan_of(cigemmContext* ctx, bool ok, const Cost& cost, const any::Cost& oth
     return fits(p.M, p.N, imposed, room, ctx->ws_counter_bytes) ? imposed : Plan{1};
   }
   // (a plan of another kernel is imposed)
-  if (ctx->force_tile_mt) return Plan{0};
+  if (ctx->force_tile_rows) return Plan{0};
   return choose(cost, other, p, is_whole(p.K_bytes, p.N * p.elem, b_nk), aligned,
                 ctx->num_cus > 0 ? ctx->num_cus : 256, room, ctx->ws_counter_bytes);
 }

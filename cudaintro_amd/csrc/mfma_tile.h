@@ -205,7 +205,6 @@ struct BTile<B_KN8> : HalfPieces {
 // k+4, which the swizzle moves 128 bytes apart.
 template <>
 struct BTile<B_KN32> {
-  static constexpr int NREADS = 16;
   typedef uint32_t piece_t;
   static __device__ __forceinline__ int swz(int k) { return ((k >> 2) & 1) << 3; }
   static __device__ __forceinline__ int off(int k, int c) { return k * 1024 + ((c ^ swz(k)) << 4); }
@@ -216,16 +215,12 @@ struct BTile<B_KN32> {
     const int c = l ^ swz(k);
     return (int64_t)k * ld + ((c < last ? c : last) << 4);
   }
-  // read idx (0..15) of k-step kk: element e = idx/4 of the fragment of column tile j = idx%4
-  static __device__ __forceinline__ piece_t read(const char* sb, int wn, int idx, int kk, int l) {
-    const int e = idx >> 2, j = idx & 3;
+  // element e (0..3) of k-step kk of the fragment of the 32 columns from n0
+  static __device__ __forceinline__ piece_t read(const char* sb, int n0, int e, int kk, int l) {
     const int k = 8 * kk + 4 * (l >> 5) + e;
-    const int n = wn * 128 + 32 * j + (l & 31);
+    const int n = n0 + (l & 31);
     return *reinterpret_cast<const uint32_t*>(sb + k * 1024 + (((n >> 2) ^ swz(k)) << 4) +
                                               (n & 3) * 4);
-  }
-  static __device__ __forceinline__ float bfrag(const piece_t (&b)[NREADS], int j, int sub) {
-    return __builtin_bit_cast(float, b[4 * sub + j]);
   }
 };
 
@@ -233,10 +228,7 @@ struct BTile<B_KN32> {
 template <int MODE>
 __device__ __forceinline__ typename BTile<MODE>::piece_t read_b_piece(const char* sb, int wn,
                                                                       int idx, int kk, int l) {
-  if constexpr (MODE == B_KN32)
-    return BTile<MODE>::read(sb, wn, idx, kk, l);
-  else
-    return BTile<MODE>::frag_half(sb, wn, idx >> 1, kk, idx & 1, l);
+  return BTile<MODE>::frag_half(sb, wn, idx >> 1, kk, idx & 1, l);
 }
 
 // ---- operand pieces at any alignment ----------------------------------------------------------
@@ -444,16 +436,16 @@ __device__ __forceinline__ typename Epi::col_t load_cols_any(const Epi& epi, int
 }
 
 // The epilogue of the tile kernels: accumulators -> output rows.
-// acc[i][j][4q+e] = C[m0 + wm*32*MT + 32i + l%32][n0 + wn*128 + 32j + 8q + 4g + e]: a lane
-// holds short pieces of 32 different rows.  Each wave stages one 32-row x 128-column block
+// acc[i][j][4q+e] = C[m0 + wm*32*MT + 32i + l%32][n0 + wn*32*NT + 32j + 8q + 4g + e]: a lane
+// holds short pieces of 32 different rows.  Each wave stages one 32-row x 32 NT-column block
 // at a time in its own piece of the (now idle) LDS and writes it out as whole rows: every
-// store instruction then covers full 256- or 512-byte row segments.  Call it once every wave
+// store instruction then covers full row segments (NT = 4: 256 or 512 bytes).  Call it once every wave
 // of the workgroup has stopped reading the operand ring and no DMA is in flight.
 // ANY: N, the rows of C and the per-column operands have their elements' alignment only.  A whole
 // 16-byte piece still leaves with one (unaligned) store; the piece that crosses the last column
 // with one store per power of two of its elements.
-template <typename Math, int MT, int NW, int TILE_M, bool ANY = false, typename Epi>
-__device__ __forceinline__ void store_tile(const Epi& epi, typename Math::acc_t (&acc)[MT][4],
+template <typename Math, int MT, int NW, int TILE_M, bool ANY = false, int NT = 4, typename Epi>
+__device__ __forceinline__ void store_tile(const Epi& epi, typename Math::acc_t (&acc)[MT][NT],
                                            char* lds, int w, int wm, int wn, int64_t m0,
                                            int64_t n0, int M, int N, float epi_row_word,
                                            float epi_col_word) {
@@ -465,7 +457,7 @@ __device__ __forceinline__ void store_tile(const Epi& epi, typename Math::acc_t 
   le &= 63;
   const int ge = le >> 5;
   constexpr int OB = Epi::OUT_BYTES;
-  constexpr int ROW_BYTES = 128 * OB;
+  constexpr int ROW_BYTES = 32 * NT * OB;
   constexpr int ROW_STRIDE = ROW_BYTES + 16;
   constexpr int LANES_PER_ROW = ROW_BYTES / 16;
   constexpr int ROWS_PER_PASS = 64 / LANES_PER_ROW;
@@ -476,12 +468,12 @@ __device__ __forceinline__ void store_tile(const Epi& epi, typename Math::acc_t 
                             acc[0][0][0])) packed_t;
   // What the epilogue needs per column quad (scales, bias) is the same for every row tile:
   // fetched once, up front, so that no load latency sits between the accumulator reads.
-  typename Epi::col_t colv[4][4];
+  typename Epi::col_t colv[NT][4];
   bool cols_done = false;
   if constexpr (epi_has_uniform_mode<Epi>::value) {
     if (epi.col_uniform()) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < NT; ++j)
 #pragma unroll
         for (int q = 0; q < 4; ++q) colv[j][q] = epi.cols_from_word(epi_col_word);
       cols_done = true;
@@ -489,22 +481,22 @@ __device__ __forceinline__ void store_tile(const Epi& epi, typename Math::acc_t 
   }
   if (!cols_done) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < NT; ++j)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int64_t col = n0 + wn * 128 + 32 * j + 8 * q + 4 * ge;
+        const int64_t col = n0 + wn * (32 * NT) + 32 * j + 8 * q + 4 * ge;
         if constexpr (ANY)
           colv[j][q] = load_cols_any(epi, col, N);
         else
           colv[j][q] = epi.load_cols(col < N ? col : N - 4);
       }
   }
-  // Store side of the staging: lane -> (row within a pass, 16-byte piece of the 128-column row).
+  // Store side of the staging: lane -> (row within a pass, 16-byte piece of the block's row).
   // N is a multiple of 4: a piece of 32-bit outputs is in or out as a whole, one of 16-bit
   // outputs may be half inside (then its first 8 bytes are stored).
   constexpr int NPASS = 32 / ROWS_PER_PASS;
   const int lane_row = le / LANES_PER_ROW, c16 = le % LANES_PER_ROW;
-  const int64_t piece_col = n0 + wn * 128 + c16 * (16 / OB);
+  const int64_t piece_col = n0 + wn * (32 * NT) + c16 * (16 / OB);
   const bool piece_in = piece_col < N;
   const bool piece_half = OB == 2 && piece_col + 8 > N;
   const int64_t row_step = (intptr_t)epi.out_row(1) - (intptr_t)epi.out_row(0);  // bytes per row
@@ -521,11 +513,11 @@ __device__ __forceinline__ void store_tile(const Epi& epi, typename Math::acc_t 
     else
       rowv = epi.load_row(row_c);
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < NT; ++j)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int c = 32 * j + 8 * q + 4 * ge;
-        const int64_t col = n0 + wn * 128 + c;
+        const int64_t col = n0 + wn * (32 * NT) + c;
         const bool col_ok = col < N;  // N is a multiple of 4: a quad is in or out as a whole
         *reinterpret_cast<packed_t*>(scr + (le & 31) * ROW_STRIDE + c * OB) =
             epi.pack(rowv, colv[j][q], acc[i][j][4 * q + 0], acc[i][j][4 * q + 1],
@@ -543,7 +535,7 @@ __device__ __forceinline__ void store_tile(const Epi& epi, typename Math::acc_t 
       v[p] = *reinterpret_cast<const u32x4*>(scr + (p * ROWS_PER_PASS + lane_row) * ROW_STRIDE +
                                              c16 * 16);
     __builtin_amdgcn_sched_barrier(0);
-    char* dst0 = epi.out_row(row0 + lane_row) + (n0 + wn * 128) * OB + c16 * 16;
+    char* dst0 = epi.out_row(row0 + lane_row) + (n0 + wn * (32 * NT)) * OB + c16 * 16;
     if constexpr (ANY) {
       constexpr int PE = 16 / OB;  // elements of a piece
       const int inside = (int)(N - piece_col);  // elements of this lane's piece inside the row
@@ -637,9 +629,15 @@ __device__ __forceinline__ void store_tile(const Epi& epi, typename Math::acc_t 
 // What is left of the difference: a piece that is not 16-byte aligned takes the address path twice
 // (10 % per stage where one 16-bit operand is misaligned, 40 % where both int8 ones are), and so
 // do the stores of unaligned rows (10 us per 64 MiB).
+//
+// NT = 4: WM x 2 waves of 32 MT x 128.  NT = 2 (fp32): one row of four waves, 32 MT x 64 each, so that
+// the tile height is any multiple of 32: its matrix instructions take 64 cycles, so what the waves
+// read twice from LDS costs nothing (fewer reads per matrix instruction in all), and a height that
+// fits is worth more than anything in the main loop (20000 x 512 x 784: 250 tiles of 160 rows on 256
+// units in place of 210 of 192).
 template <typename Math, int BMODE, int NSTAGES, int MT, typename Epi, int WM = 2,
-          bool ANY = false>
-__global__ __launch_bounds__(128 * WM, 1) void mfma_tile_kernel(int M, int N, int tiles_m,
+          bool ANY = false, int NT = 4>
+__global__ __launch_bounds__(WM * (512 / NT), 1) void mfma_tile_kernel(int M, int N, int tiles_m,
                                                            int tiles_n, int k_range_bytes,
                                                            int k_total_bytes,
                                                            const char* __restrict__ A,
@@ -662,7 +660,8 @@ __global__ __launch_bounds__(128 * WM, 1) void mfma_tile_kernel(int M, int N, in
   typedef typename Math::acc_t acc_t;
   typedef BTile<BMODE> BT;
   constexpr int DIST = NSTAGES - 1;  // stages in flight ahead of the one being multiplied
-  constexpr int NW = 2 * WM;             // waves: WM rows of 2
+  constexpr int WN = 8 / NT, NW = WM * WN;  // waves: WM rows of WN
+  static_assert(NT == 4 || (NT == 2 && BMODE == B_KN32), "other column counts: fp32 only");
   constexpr int TILE_M = 32 * MT * WM;   // rows of the macro tile
   static_assert(NSTAGES == 4, "the wait counts below assume three stages in flight");
   // N x K weights are row-major like A: they too are fetched as whole 128-byte lines, a pair
@@ -670,6 +669,8 @@ __global__ __launch_bounds__(128 * WM, 1) void mfma_tile_kernel(int M, int N, in
   // single stages the K x N layouts use).
   constexpr bool BPAIR = BMODE == B_NK;
   constexpr int DMA_A = TILE_M / 8 / NW;        // per wave and stage pair: A instructions of 1 KiB
+  // (K x N: issued in two halves, the first in the pair's even stage)
+  constexpr int DMA_A0 = (DMA_A + 1) / 2, DMA_A1 = DMA_A / 2;
   // per wave: B instructions per stage pair (N x K weights) / per stage
   constexpr int DMA_B = (BPAIR ? 32 : 16) / NW;
   constexpr int BPAIR_BYTES = 256 * 128;
@@ -680,7 +681,7 @@ __global__ __launch_bounds__(128 * WM, 1) void mfma_tile_kernel(int M, int N, in
   const int t = threadIdx.x;
   const int l = t & 63;
   const int w = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int wm = w >> 1, wn = w & 1;
+  const int wm = w / WN, wn = w % WN;
   auto stamp = [&](int point) {
     if constexpr (epi_profiled<Epi>::value) {
       if (threadIdx.x == 0) {
@@ -826,11 +827,12 @@ __global__ __launch_bounds__(128 * WM, 1) void mfma_tile_kernel(int M, int N, in
 
   // One k-step's operands: MT A fragments (16 B each) and the pieces of the 4 B fragments.
   // N x K pairs: one 16-byte read per B fragment, kept behind the A fragments in Frags::a
-  constexpr int NREAD_B = BPAIR ? 4 : BT::NREADS;
+  constexpr bool FLOATS = BMODE == B_KN32;
+  constexpr int NPIECES = FLOATS ? 4 * NT : 8;         // pieces of the NT B fragments of a k-step
+  constexpr int NREAD_B = BPAIR ? 4 : NPIECES;
   constexpr int NREAD = MT + NREAD_B;                  // LDS reads per k-step
-  constexpr int NMFMA = 4 * MT * Math::SUBSTEPS;       // MFMAs per k-step
+  constexpr int NMFMA = NT * MT * Math::SUBSTEPS;      // MFMAs per k-step
   constexpr int READS_PER_SLOT = (NREAD + NMFMA - 1) / NMFMA;
-  static_assert(DMA_A % 2 == 0, "an A pair is issued in two halves");
   // DMA instruction d of the NDMA a k-step issues goes into MFMA slot d * NMFMA / NDMA: spread
   // evenly over the k-step.  The four waves leave the barrier together, and a compute unit's one
   // address path takes about 16 cycles per 1 KiB instruction: issued back to back, one per
@@ -843,7 +845,7 @@ __global__ __launch_bounds__(128 * WM, 1) void mfma_tile_kernel(int M, int N, in
   };
   struct Frags {
     u32x4 a[BPAIR ? MT + 4 : MT];
-    typename BT::piece_t b[BPAIR ? 1 : BT::NREADS];
+    typename BT::piece_t b[BPAIR ? 1 : NPIECES];
   };
   // LDS read r of k-step kk of the stage in ring slot `slot`: first the A fragments, then B.
   // `par` = parity of the stage: which half of the pair's 128-byte rows.
@@ -853,16 +855,19 @@ __global__ __launch_bounds__(128 * WM, 1) void mfma_tile_kernel(int M, int N, in
           lds + B_RING + pslot * APAIR_BYTES + pair_off(a_frag_row + 32 * r, 4 * par + 2 * kk + g));
     else if constexpr (BPAIR) {
       f.a[r] = BT::frag_pair(lds + slot * BPAIR_BYTES, wn, r - MT, par, kk, l);
+    } else if constexpr (FLOATS) {  // (element outermost)
+      f.b[r - MT] = BT::read(lds + slot * OPERAND_BYTES, wn * 32 * NT + 32 * ((r - MT) % NT),
+                             (r - MT) / NT, kk, l);
     } else {
       f.b[r - MT] = read_b_piece<BMODE>(lds + slot * OPERAND_BYTES, wn, r - MT, kk, l);
     }
   };
 
-  acc_t acc[MT][4];
+  acc_t acc[MT][NT];
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < NT; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0;
 
@@ -871,10 +876,13 @@ __global__ __launch_bounds__(128 * WM, 1) void mfma_tile_kernel(int M, int N, in
   // run up for even j and down for odd j, so that every MFMA shares one source operand with
   // the one before it (measured: 0.3-0.6 % less time at 8192^3 with one wave per SIMD).
   auto mfma_piece = [&](const Frags& f, int m) {
-    const int sub = m / (4 * MT), j = (m % (4 * MT)) / MT;
+    const int sub = m / (NT * MT), j = (m % (NT * MT)) / MT;
     const int i = (j & 1) ? MT - 1 - m % MT : m % MT;
     if constexpr (BPAIR)
       acc[i][j] = Math::mfma(f.a[MT + j], Math::afrag(f.a[i], sub), acc[i][j]);
+    else if constexpr (FLOATS)
+      acc[i][j] = Math::mfma(__builtin_bit_cast(float, f.b[NT * sub + j]), Math::afrag(f.a[i], sub),
+                             acc[i][j]);
     else
       acc[i][j] = Math::mfma(BT::bfrag(f.b, j, sub), Math::afrag(f.a[i], sub), acc[i][j]);
   };
@@ -909,7 +917,7 @@ __global__ __launch_bounds__(128 * WM, 1) void mfma_tile_kernel(int M, int N, in
     if (!BPAIR && KTS > 0) prologue_second();
     if (tail_bytes > 0) {
       constexpr int THREADS = 64 * NW, CE = 16 / Math::ELEM_BYTES;
-      constexpr int PA = TILE_M * 4 / THREADS, PB = 1024 / THREADS;
+      constexpr int PA = (TILE_M * 4 + THREADS - 1) / THREADS, PB = 1024 / THREADS;
       constexpr int KN_CHUNKS = 16 * Math::ELEM_BYTES;  // 16-byte pieces of a K x N tile row
       constexpr int B_SLOT = BPAIR ? 1 : NSTAGES - 1;
       constexpr int B_SLOT_AT = B_SLOT * (BPAIR ? BPAIR_BYTES : OPERAND_BYTES);
@@ -935,8 +943,9 @@ __global__ __launch_bounds__(128 * WM, 1) void mfma_tile_kernel(int M, int N, in
 #pragma unroll
       for (int i = 0; i < PA; ++i) {
         const int c = t + THREADS * i;
-        *reinterpret_cast<u32x4*>(lds + B_RING + 2 * APAIR_BYTES + pair_off(c >> 2, c & 3)) =
-            trim_piece<elem_t>(ta[i], m0 + (c >> 2), M, k0 + (c & 3) * CE, k_end);
+        if (TILE_M * 4 % THREADS == 0 || c < TILE_M * 4)
+          *reinterpret_cast<u32x4*>(lds + B_RING + 2 * APAIR_BYTES + pair_off(c >> 2, c & 3)) =
+              trim_piece<elem_t>(ta[i], m0 + (c >> 2), M, k0 + (c & 3) * CE, k_end);
       }
 #pragma unroll
       for (int i = 0; i < PB; ++i) {
@@ -993,7 +1002,7 @@ __global__ __launch_bounds__(128 * WM, 1) void mfma_tile_kernel(int M, int N, in
     constexpr int PAR = decltype(par_const)::value;
     constexpr int PHASE = decltype(phase_const)::value;
     static_assert(PHASE < 0 || (PHASE & 1) == PAR, "the phase fixes the parity");
-    constexpr int NDMA = BPAIR ? (PAR ? DMA_B : DMA_A) : DMA_B + DMA_A / 2;
+    constexpr int NDMA = BPAIR ? (PAR ? DMA_B : DMA_A) : DMA_B + (PAR ? DMA_A1 : DMA_A0);
     int slot_c = slot, next_slot_c = next_slot, dma_slot_c = dma_slot;
     int pslot_c = pslot, next_pslot_c = next_pslot, dma_pslot_c = dma_pslot;
     if constexpr (PHASE >= 0) {
@@ -1025,7 +1034,7 @@ __global__ __launch_bounds__(128 * WM, 1) void mfma_tile_kernel(int M, int N, in
       // stage s+1 landed for this wave.  Still in flight, in issue order after what stage
       // s+1 needs: even s: the first half of the A pair (s+2, s+3), B[s+2] and its second
       // half; odd s: B[s+2] and the first half of the A pair (s+3, s+4).
-      wait_vmcnt(std::integral_constant<int, PAR ? DMA_B + DMA_A / 2 : DMA_B + DMA_A>{});
+      wait_vmcnt(std::integral_constant<int, PAR ? DMA_B + DMA_A0 : DMA_B + DMA_A>{});
     }
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
@@ -1052,7 +1061,7 @@ __global__ __launch_bounds__(128 * WM, 1) void mfma_tile_kernel(int M, int N, in
             // half of the A pair the DMA is filling: stages s+4, s+5 seen from an even stage,
             // s+3, s+4 from the odd stage after it
             dma_piece(PAR ? s + DIST : s + DIST + 1, dma_slot_c, dma_pslot_c,
-                      d + (PAR ? DMA_A / 2 : 0), steady_const);
+                      d + (PAR ? DMA_A0 : 0), steady_const);
           }
         }
       }
@@ -1135,14 +1144,14 @@ __global__ __launch_bounds__(128 * WM, 1) void mfma_tile_kernel(int M, int N, in
   // ---- epilogue -----------------------------------------------------------------------------
   // (the rows of a partial matrix are whole aligned pieces whatever N is)
   if constexpr (ANY && !epi_is_partial<Epi>::value)
-    store_tile<Math, MT, NW, TILE_M, true>(epi, acc, lds, w, wm, wn, m0, n0, M, N, epi_row_word,
-                                           epi_col_word);
+    store_tile<Math, MT, NW, TILE_M, true, NT>(epi, acc, lds, w, wm, wn, m0, n0, M, N, epi_row_word,
+                                               epi_col_word);
   else if constexpr (ANY)
-    store_tile<Math, MT, NW, TILE_M>(epi, acc, lds, w, wm, wn, m0, n0, M, (int)epi.ld,
-                                     epi_row_word, epi_col_word);
+    store_tile<Math, MT, NW, TILE_M, false, NT>(epi, acc, lds, w, wm, wn, m0, n0, M, (int)epi.ld,
+                                                epi_row_word, epi_col_word);
   else
-    store_tile<Math, MT, NW, TILE_M>(epi, acc, lds, w, wm, wn, m0, n0, M, N, epi_row_word,
-                                     epi_col_word);
+    store_tile<Math, MT, NW, TILE_M, false, NT>(epi, acc, lds, w, wm, wn, m0, n0, M, N, epi_row_word,
+                                                epi_col_word);
   if constexpr (epi_profiled<Epi>::value) {
     // the epilogue ends when this wave's stores have been acknowledged
     wait_vmcnt(std::integral_constant<int, 0>{});
@@ -1153,16 +1162,17 @@ __global__ __launch_bounds__(128 * WM, 1) void mfma_tile_kernel(int M, int N, in
 constexpr int DEFAULT_STAGES = 4;
 
 // `splits` must be a value k_ranges() returned for this K (1 = the whole of K in one range).
-template <typename Math, int BMODE, int MT, typename Epi, int WM = 2, bool ANY = false>
+template <typename Math, int BMODE, int MT, typename Epi, int WM = 2, bool ANY = false, int NT = 4>
 void launch_tile_mt(cigemmContext* ctx, int64_t M, int64_t N, int64_t K_bytes, const void* A,
                     int64_t lda_bytes, const void* B, int64_t ldb_bytes, const Epi& epi,
                     int splits = 1) {
   constexpr int NSTAGES = DEFAULT_STAGES;
   constexpr int TILE_M = 32 * MT * WM;
   constexpr int RING_BYTES = NSTAGES * OPERAND_BYTES + 3 * (TILE_M * 128);
-  constexpr int STAGING_BYTES = 2 * WM * 32 * (128 * Epi::OUT_BYTES + 16);   // epilogue, per wave
+  constexpr int NW = WM * (8 / NT);
+  constexpr int STAGING_BYTES = NW * 32 * (32 * NT * Epi::OUT_BYTES + 16);   // epilogue, per wave
   constexpr int LDS_BYTES = RING_BYTES > STAGING_BYTES ? RING_BYTES : STAGING_BYTES;
-  auto kern = mfma_tile_kernel<Math, BMODE, NSTAGES, MT, Epi, WM, ANY>;
+  auto kern = mfma_tile_kernel<Math, BMODE, NSTAGES, MT, Epi, WM, ANY, NT>;
   static std::atomic<uint64_t> lds_set{0};  // one per template instance
   if (!ensure_dynamic_lds(ctx, (const void*)kern, LDS_BYTES, lds_set)) return;
   const int tiles_m = (int)((M + TILE_M - 1) / TILE_M), tiles_n = (int)((N + BN - 1) / BN);
@@ -1170,13 +1180,13 @@ void launch_tile_mt(cigemmContext* ctx, int64_t M, int64_t N, int64_t K_bytes, c
   splits = k_ranges(K_bytes, splits, &range_stages);
   ctx->last_tile_rows = TILE_M;
   ctx->last_k_splits = splits;
-  ctx->last_waves = 2 * WM;
+  ctx->last_waves = NW;
   ctx->last_per_cu = 1;
   const int64_t range_bytes = splits > 1 ? range_stages * KB : K_bytes;
   const int64_t a_step = range_stages * KB;
   const int64_t b_step =
       BMODE == B_NK ? range_stages * KB : range_stages * (KB / Math::ELEM_BYTES) * ldb_bytes;
-  hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n), (unsigned)splits), dim3(128 * WM),
+  hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n), (unsigned)splits), dim3(64 * NW),
                      LDS_BYTES, ctx->stream, (int)M, (int)N, tiles_m, tiles_n, (int)range_bytes,
                      (int)K_bytes, static_cast<const char*>(A), lda_bytes,
                      static_cast<const char*>(B), ldb_bytes, epi, a_step, b_step);
@@ -1306,29 +1316,40 @@ void launch_tile_128(cigemmContext* ctx, int64_t M, int64_t N, int64_t K_bytes, 
                                            splits);
 }
 
+// Tiles of `rows` rows: fp32 64 and any greater multiple of 32, the others multiples of 64.
 template <typename Math, int BMODE, bool ANY = false, typename Epi>
-void launch_tile_any_mt(cigemmContext* ctx, int mt, int64_t M, int64_t N, int64_t K_bytes,
-                        const void* A, int64_t lda_bytes, const void* B, int64_t ldb_bytes,
-                        const Epi& epi, int splits = 1) {
-  if (mt == 4)
+void launch_tile_rows(cigemmContext* ctx, int rows, int64_t M, int64_t N, int64_t K_bytes,
+                      const void* A, int64_t lda_bytes, const void* B, int64_t ldb_bytes,
+                      const Epi& epi, int splits = 1) {
+  if constexpr (BMODE == B_KN32) {
+#define CIG_ROWS(H)                                                                                 \
+  case H:                                                                                           \
+    return launch_tile_mt<Math, BMODE, H, Epi, 1, ANY, 2>(ctx, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, \
+                                                          epi, splits)
+    switch (rows / 32) {
+      CIG_ROWS(2); CIG_ROWS(3); CIG_ROWS(4); CIG_ROWS(5); CIG_ROWS(6); CIG_ROWS(7);
+      default: CIG_ROWS(8);
+    }
+#undef CIG_ROWS
+  } else if (rows == 256)
     launch_tile_256<Math, BMODE, ANY>(ctx, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, epi, splits);
-  else if (mt == 3)
+  else if (rows == 192)
     launch_tile_mt<Math, BMODE, 3, Epi, 2, ANY>(ctx, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, epi, splits);
-  else if (mt == 2)
+  else if (rows == 128)
     launch_tile_128<Math, BMODE, ANY>(ctx, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, epi, splits);
   else
     launch_tile_mt<Math, BMODE, 1, Epi, 2, ANY>(ctx, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, epi, splits);
 }
 
-// Runs one plan: tiles of 64*mt rows; with more than one K range the ranges go over
+// Runs one plan: tiles of `rows` rows; with more than one K range the ranges go over
 // blockIdx.y, partial sums to the workspace, then one reduction launch with the real epilogue.
 // Returns true when it ran as such a pair of launches.
 template <typename Math, int BMODE, bool ANY = false, typename Epi>
-bool run_tile_plan(cigemmContext* ctx, int mt, int splits, int64_t M, int64_t N, int64_t K_bytes,
+bool run_tile_plan(cigemmContext* ctx, int rows, int splits, int64_t M, int64_t N, int64_t K_bytes,
                    const void* A, int64_t lda_bytes, const void* B, int64_t ldb_bytes,
                    const Epi& epi) {
   if (splits <= 1) {
-    launch_tile_any_mt<Math, BMODE, ANY>(ctx, mt, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, epi);
+    launch_tile_rows<Math, BMODE, ANY>(ctx, rows, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, epi);
     return false;
   }
   typedef typename Math::scalar_t scalar_t;
@@ -1336,7 +1357,7 @@ bool run_tile_plan(cigemmContext* ctx, int mt, int splits, int64_t M, int64_t N,
   uint32_t* ws = static_cast<uint32_t*>(ctx->workspace);
   const int64_t ld = partial_ld<ANY>(N);
   const EpiPartialX4 part{ws, ld, M * ld};
-  launch_tile_any_mt<Math, BMODE, ANY>(ctx, mt, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, part,
+  launch_tile_rows<Math, BMODE, ANY>(ctx, rows, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, part,
                                   splits);
   const int64_t quads = M * ((N + 3) / 4);
   const unsigned grid = (unsigned)((quads + 255) / 256 < 4 * (int64_t)cus ? (quads + 255) / 256
@@ -1357,7 +1378,7 @@ bool launch_tile(cigemmContext* ctx, int64_t M, int64_t N, int64_t K_bytes, cons
                  int64_t lda_bytes, const void* B, int64_t ldb_bytes, const Epi& epi,
                  SmallPlan known = SmallPlan{0, 1}) {
   const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
-  if (ctx->force_tile_mt >= 1 && ctx->force_tile_mt <= 4) {
+  if (ctx->force_tile_rows > 0) {
     // a plan imposed through the measurement library: as asked, but for K ranges the
     // workspace cannot hold
     int64_t range_stages = 0;
@@ -1365,29 +1386,45 @@ bool launch_tile(cigemmContext* ctx, int64_t M, int64_t N, int64_t K_bytes, cons
     if (sp > 1 && (!ctx->workspace ||
                    (size_t)sp * (size_t)M * (size_t)partial_ld<ANY>(N) * 4 > ctx->ws_partial_bytes))
       sp = 1;
-    return run_tile_plan<Math, BMODE, ANY>(ctx, ctx->force_tile_mt, sp, M, N, K_bytes, A, lda_bytes, B,
+    const int rows =
+        BMODE == B_KN32 ? ctx->force_tile_rows : (ctx->force_tile_rows + 63) / 64 * 64;
+    return run_tile_plan<Math, BMODE, ANY>(ctx, rows, sp, M, N, K_bytes, A, lda_bytes, B,
                                       ldb_bytes, epi);
   }
+  const size_t room = ctx->workspace ? ctx->ws_partial_bytes : 0;
+  // rows of a small plan's tiles: fp32 may do better with a height between
+  auto rows_of = [&](const SmallPlan& plan, int64_t n) {
+    if constexpr (BMODE == B_KN32)
+      return plan_small_rows32(cus, M, partial_ld<ANY>(n), K_bytes, Epi::OUT_BYTES,
+                               stage_cost<Math, BMODE>(), K_bytes * n, plan);
+    else
+      return 64 * plan.mt;
+  };
   if (((M + BM - 1) / BM) * ((N + BN - 1) / BN) <= cus) {
     // At most one round of 256-row tiles: pick the tile height and the number of K ranges
     // together.
     const SmallPlan plan =
         known.mt ? known
-                 : plan_small(cus, ctx->workspace ? ctx->ws_partial_bytes : 0, M,
+                 : plan_small(cus, room, M,
                               partial_ld<ANY>(N), K_bytes, Epi::OUT_BYTES,
                               stage_cost<Math, BMODE>(), K_bytes * N);
-    return run_tile_plan<Math, BMODE, ANY>(ctx, plan.mt, plan.splits, M, N, K_bytes, A, lda_bytes, B,
+    return run_tile_plan<Math, BMODE, ANY>(ctx, rows_of(plan, N), plan.splits, M, N, K_bytes, A, lda_bytes, B,
                                       ldb_bytes, epi);
   }
-  constexpr TileUnits units = BMODE == B_KN32 ? TILE_UNITS_F32 : TILE_UNITS;
-  const RoundsPlan rounds = plan_rounds(M, N, cus, units);
+  RoundsPlan rounds;
+  int rows = 0;
+  if constexpr (BMODE == B_KN32) {
+    rounds = plan_rounds32(M, N, cus, &rows);
+  } else {
+    rounds = plan_rounds(M, N, cus, TILE_UNITS);
+    rows = 64 * rounds.mt;
+  }
   const int64_t n1 = rounds.first_cols, n2 = N - n1;
   if (n1 == 0) {
-    launch_tile_any_mt<Math, BMODE, ANY>(ctx, rounds.mt, M, N, K_bytes, A, lda_bytes, B, ldb_bytes,
-                                         epi);
+    launch_tile_rows<Math, BMODE, ANY>(ctx, rows, M, N, K_bytes, A, lda_bytes, B, ldb_bytes, epi);
     return false;
   }
-  launch_tile_256<Math, BMODE, ANY>(ctx, M, n1, K_bytes, A, lda_bytes, B, ldb_bytes, epi);
+  launch_tile_rows<Math, BMODE, ANY>(ctx, 256, M, n1, K_bytes, A, lda_bytes, B, ldb_bytes, epi);
   const int rows1 = ctx->last_tile_rows, waves1 = ctx->last_waves;
   // (n2 may be less than a 16-byte piece; load_piece then reads from the n1 >= 256 columns in front)
   const char* B2 =
@@ -1395,13 +1432,13 @@ bool launch_tile(cigemmContext* ctx, int64_t M, int64_t N, int64_t K_bytes, cons
   bool split = false;
   if ((M + BM - 1) / BM * ((n2 + BN - 1) / BN) <= cus) {
     const SmallPlan plan =
-        plan_small(cus, ctx->workspace ? ctx->ws_partial_bytes : 0, M, partial_ld<ANY>(n2), K_bytes,
+        plan_small(cus, room, M, partial_ld<ANY>(n2), K_bytes,
                    Epi::OUT_BYTES, stage_cost<Math, BMODE>(), K_bytes * n2);
-    split = run_tile_plan<Math, BMODE, ANY>(ctx, plan.mt, plan.splits, M, n2, K_bytes, A, lda_bytes,
+    split = run_tile_plan<Math, BMODE, ANY>(ctx, rows_of(plan, n2), plan.splits, M, n2, K_bytes, A, lda_bytes,
                                             B2, ldb_bytes, epi.shift_cols(n1));
   } else {
-    launch_tile_any_mt<Math, BMODE, ANY>(ctx, rounds.mt, M, n2, K_bytes, A, lda_bytes, B2, ldb_bytes,
-                                         epi.shift_cols(n1));
+    launch_tile_rows<Math, BMODE, ANY>(ctx, 64 * rounds.mt, M, n2, K_bytes, A, lda_bytes, B2, ldb_bytes,
+                                       epi.shift_cols(n1));
   }
   ctx->first_tile_rows = rows1;
   ctx->first_waves = waves1;

@@ -463,13 +463,13 @@ extern "C" cigemmStatus_t cigemm_probe_force_tile_plan(cigemmHandle_t h, int til
   const char* name = "cigemm_probe_force_tile_plan";
   if (!h || h->magic != kCtxMagic) return CIGEMM_STATUS_NOT_INITIALIZED;
   if (tile_rows == 0) {
-    h->force_tile_mt = h->force_tile_splits = 0;
+    h->force_tile_rows = h->force_tile_splits = 0;
     return CIGEMM_STATUS_SUCCESS;
   }
-  if (tile_rows % 64 || tile_rows < 64 || tile_rows > 256 || k_ranges < 1 || k_ranges > 64)
+  if (tile_rows % 32 || tile_rows < 64 || tile_rows > 256 || k_ranges < 1 || k_ranges > 64)
     return fail(h, CIGEMM_STATUS_INVALID_VALUE, "%s: tile_rows %d, k_ranges %d", name, tile_rows,
                 k_ranges);
-  h->force_tile_mt = tile_rows / 64;
+  h->force_tile_rows = tile_rows;
   h->force_tile_splits = k_ranges;
   return CIGEMM_STATUS_SUCCESS;
 }

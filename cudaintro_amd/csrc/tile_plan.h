@@ -71,12 +71,13 @@ struct PlanCost {
   static constexpr int MIN_RANGE_STAGES = 8;
   static constexpr int MAX_ROUNDS_SPLIT = 3;
 };
-inline double plan_us(int64_t M, int64_t N, int64_t K_bytes, int out_bytes, StageCost sc,
-                      bool streamed, int cus, int mt, int sp, int64_t range_stages) {
-  const int64_t tiles = ((M + 64 * mt - 1) / (64 * mt)) * ((N + BN - 1) / BN);
+// The estimate for tiles of `rows` rows.
+inline double plan_us_rows(int64_t M, int64_t N, int64_t K_bytes, int out_bytes, StageCost sc,
+                           bool streamed, int cus, int rows, int sp, int64_t range_stages) {
+  const int64_t tiles = ((M + rows - 1) / rows) * ((N + BN - 1) / BN);
   const int64_t wgs = tiles * sp, full = wgs / cus, rem = wgs % cus;
   const double stage =
-      (streamed ? sc.fixed_us : sc.fixed_us * PlanCost::RESIDENT_FIXED) + sc.per_64_rows_us * mt;
+      (streamed ? sc.fixed_us : sc.fixed_us * PlanCost::RESIDENT_FIXED) + sc.per_64_rows_us * rows / 64;
   const double mn = (double)M * (double)N;
   const double hbm_bytes = (double)(N + M) * (double)K_bytes +
                            PlanCost::PARTIAL_WEIGHT * (sp > 1 ? sp * mn * 4.0 : mn * out_bytes);
@@ -96,6 +97,11 @@ inline double plan_us(int64_t M, int64_t N, int64_t K_bytes, int out_bytes, Stag
     us += reduce > 4.75 ? reduce : 4.75;
   }
   return us;
+}
+
+inline double plan_us(int64_t M, int64_t N, int64_t K_bytes, int out_bytes, StageCost sc,
+                      bool streamed, int cus, int mt, int sp, int64_t range_stages) {
+  return plan_us_rows(M, N, K_bytes, out_bytes, sc, streamed, cus, 64 * mt, sp, range_stages);
 }
 
 // `partial_bytes` = room for partial sums (0: no split plans).  `est_us`, if given, receives the
@@ -129,6 +135,26 @@ inline SmallPlan plan_small(int cus, size_t partial_bytes, int64_t M, int64_t N,
     }
   }
   if (est_us) *est_us = best_us;
+  return best;
+}
+
+// fp32, whose tiles may have any multiple of 32 rows: the height for `plan`'s number of K ranges that
+// the same estimate likes best, among the plan's own and all that lie between the multiples of 64.
+// (96 x 4096 x 4096: 96 rows in place of 128.)
+inline int plan_small_rows32(int cus, int64_t M, int64_t N, int64_t K_bytes,
+                             int out_bytes, StageCost sc, int64_t b_bytes, SmallPlan plan) {
+  const bool streamed = b_bytes > (16LL << 20);
+  if (cus <= 0) cus = 256;
+  int64_t range_stages = 0;
+  const int sp = k_ranges(K_bytes, plan.splits, &range_stages);
+  int best = 64 * plan.mt;
+  double best_us = plan_us_rows(M, N, K_bytes, out_bytes, sc, streamed, cus, best, sp, range_stages);
+  for (int rows : {96, 160, 224}) {
+    if (rows - 32 >= M) break;  // a lower height already covers M
+    const double us =
+        plan_us_rows(M, N, K_bytes, out_bytes, sc, streamed, cus, rows, sp, range_stages);
+    if (us < best_us) best_us = us, best = rows;
+  }
   return best;
 }
 
@@ -196,6 +222,35 @@ inline RoundsPlan plan_rounds(int64_t M, int64_t N, int cus, TileUnits units) {
   // against 86.0 us)
   if (tile_plan_cost(M, n1, 4, cus, units) + rest < single * 0.97) r = RoundsPlan{mt2, n1};
   return r;
+}
+
+// fp32: the same with every multiple of 32 rows (but 32) for the single launch, whose height goes to
+// *rows; the second launch, which may split K, priced by the share of the chip its 64-row tiles take
+// (4095 x 4097 x 4099: 17th column of tiles 63 us + 5 for the reduction, a quarter of a 64-row round
+// is 60).  us before -> here: 20000 x 512 x 784 143.5 (210 tiles of 192 rows) -> 130.3 (250 of 160, one
+// round), 3000^3 503 (192) -> 422 (160), 7000 x 4096 x 4096 1604 (64) -> 1588 (224).
+inline RoundsPlan plan_rounds32(int64_t M, int64_t N, int cus, int* rows) {
+  constexpr TileUnits u = TILE_UNITS_F32;
+  const int64_t tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+  double best = 1e30;
+  for (int r = 256; r >= 64; r -= 32) {
+    const int64_t tiles = (M + r - 1) / r * tiles_n;
+    const double cost = (double)((tiles + cus - 1) / cus) * (u.fixed + u.per_64_rows * r / 64);
+    if (cost < best) best = cost, *rows = r;
+  }
+  if (tiles_m > cus) return RoundsPlan{*rows / 64, 0};
+  const int64_t cols_per_round = cus / tiles_m;
+  const int64_t full_cols = tiles_n / cols_per_round * cols_per_round;
+  if (full_cols <= 0 || full_cols >= tiles_n) return RoundsPlan{*rows / 64, 0};
+  double rest = 0;
+  const int mt2 = best_mt(M, N - full_cols * BN, cus, &rest, u);
+  if (tiles_m * (tiles_n - full_cols) <= cus) {
+    const double share =
+        0.05 + (double)((M + 63) / 64 * (tiles_n - full_cols)) / cus * tile_cost_units(1, u);
+    if (share < rest) rest = share;
+  }
+  if (tile_plan_cost(M, full_cols * BN, 4, cus, u) + rest < best) return RoundsPlan{mt2, full_cols * BN};
+  return RoundsPlan{*rows / 64, 0};
 }
 
 }  // namespace tile

@@ -125,7 +125,8 @@ CIGEMM_API cigemmStatus_t cigemm_probe_dirty_workspace(cigemmHandle_t handle, in
                                                        uint32_t value, int mark_dirty);
 
 /* Planner evidence: imposes the tile kernel's plan on the handle's following GEMM calls (those
- * the tile kernel serves): output tiles of `tile_rows` rows (64, 128, 192 or 256) over
+ * the tile kernel serves): output tiles of `tile_rows` rows (64, 128, 192 or 256; fp32 also 96, 160
+ * or 224, which the other types round up) over
  * `k_ranges` ranges of K (1 = unsplit; rounded to ranges of an even number of 64-byte stages;
  * run unsplit when the handle's workspace cannot hold the partial sums).  tile_rows = 0 hands
  * the choice back to the library.  cigemmGetLastPlan() reports what ran.  Results are those of
