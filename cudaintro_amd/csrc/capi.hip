@@ -281,7 +281,8 @@ static bool dispatch_f32(cigemmHandle_t h, int64_t M, int64_t N, int64_t K, cons
       launch_generic_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba);
       return true;
     default:
-      if (!launch_f32_mfma(h, M, N, K, A, lda, B, ldb, C, ldc, ba) &&
+      if (!launch_kwaves_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba) &&
+          !launch_f32_mfma(h, M, N, K, A, lda, B, ldb, C, ldc, ba) &&
           !any_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba))
         launch_generic_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba);
       return true;

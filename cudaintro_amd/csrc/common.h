@@ -255,6 +255,8 @@ bool launch_tile_any_i8(cigemmContext*, int64_t M, int64_t N, int64_t K, const i
 // nothing launched, where another kernel is estimated to be faster.
 bool launch_kwaves_16(cigemmContext*, bool bf16, int64_t M, int64_t N, int64_t K, const uint16_t* A,
                       int64_t lda, const uint16_t* B, int64_t ldb, uint16_t* C, int64_t ldc);
+bool launch_kwaves_f32(cigemmContext*, int64_t M, int64_t N, int64_t K, const float* A, int64_t lda,
+                       const float* B, int64_t ldb, float* C, int64_t ldc, const BiasAct* ba);
 bool launch_kwaves_i8(cigemmContext*, int64_t M, int64_t N, int64_t K, const int8_t* A, int64_t lda,
                       const int8_t* B, int64_t ldb, bool b_nk, int32_t* C, int64_t ldc,
                       const DequantArgs* dq);
@@ -271,6 +273,10 @@ void launch_generic_i8(cigemmContext*, int64_t M, int64_t N, int64_t K, const in
 bool launch_f32_tile(cigemmContext*, int64_t M, int64_t N, int64_t K, const float* A,
                      int64_t lda, const float* B, int64_t ldb, float* C, int64_t ldc,
                      const BiasAct* ba = nullptr);
+// what the call is estimated to take on the kernel that DEFAULT would choose without gemm_kwaves.hip
+double f32_other_us(const cigemmContext*, int64_t M, int64_t N, int64_t K, const float* A,
+                    int64_t lda, const float* B, int64_t ldb, const float* C, int64_t ldc,
+                    const BiasAct* ba);
 bool launch_f32_mfma(cigemmContext*, int64_t M, int64_t N, int64_t K, const float* A,
                      int64_t lda, const float* B, int64_t ldb, float* C, int64_t ldc,
                      const BiasAct* ba = nullptr);

@@ -15,13 +15,11 @@ static bool f32_tile_ok(int64_t M, int64_t N, int64_t K, const float* A, int64_t
          ((uintptr_t)C & 15) == 0 && !(ba && ba->bias && ((uintptr_t)ba->bias & 15));
 }
 
-bool launch_f32_mfma(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const float* A,
-                     int64_t lda, const float* B, int64_t ldb, float* C, int64_t ldc,
-                     const BiasAct* ba) {
-  if (!f32_tile_ok(M, N, K, A, lda, B, ldb, C, ldc, ba)) return false;
+// Whether a call that the tile kernel takes is the small kernel's.
+static bool aligned_is_small(const cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const float* A,
+                             int64_t lda, const float* B, int64_t ldb) {
   const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
   const bool one_round = ((M + 255) / 256) * ((N + tile::BN - 1) / tile::BN) <= cus;
-  bool small = false;
   if (f32_small_shape_ok(M, N, K, A, lda)) {
     // Both costs in units of a quarter of one 256x256 tile's time per unit of k: the tile
     // plan's own figure against 0.115 per resident round of 32x32 tiles (2048^3: tile kernel
@@ -33,7 +31,7 @@ bool launch_f32_mfma(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const 
     // With a long K the tile kernel wins whenever its tiles fit one round: it can split K over
     // the idle compute units (512 x 512 x 4096: 33 us against 55 us; 1024^3: 31 against 32;
     // 512^3: 17 against 9; 960 x 3584 x 3584: 222 against 298).
-    small = small_cost < tile_cost && !(K >= 2048 && one_round);
+    return small_cost < tile_cost && !(K >= 2048 && one_round);
   } else if (f32_small_any_ok(M, N, K)) {
     // A K of whole 16-byte pieces that is no multiple of 8: by the small kernel's estimate against
     // the planner's + 4 us, or against what the launches of several rounds are estimated at.  Over
@@ -52,11 +50,37 @@ bool launch_f32_mfma(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const 
       // loop: 81708 x 356 x 12 38.3 us, estimated 48.0, small kernel 54.4)
       if (K <= 16) tile_us *= 0.73;
     }
-    small = any::f32_small_us(M, N, K, cus, f32_small_b16(N, B, ldb), false) < tile_us;
+    return any::f32_small_us(M, N, K, cus, f32_small_b16(N, B, ldb), false) < tile_us;
   }
-  if (!small) return launch_f32_tile(ctx, M, N, K, A, lda, B, ldb, C, ldc, ba);
+  return false;
+}
+
+bool launch_f32_mfma(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const float* A,
+                     int64_t lda, const float* B, int64_t ldb, float* C, int64_t ldc,
+                     const BiasAct* ba) {
+  if (!f32_tile_ok(M, N, K, A, lda, B, ldb, C, ldc, ba)) return false;
+  if (!aligned_is_small(ctx, M, N, K, A, lda, B, ldb))
+    return launch_f32_tile(ctx, M, N, K, A, lda, B, ldb, C, ldc, ba);
   launch_f32_small(ctx, M, N, K, A, lda, B, ldb, C, ldc, ba);
   return true;
+}
+
+double f32_other_us(const cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const float* A,
+                    int64_t lda, const float* B, int64_t ldb, const float* C, int64_t ldc,
+                    const BiasAct* ba) {
+  const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+  const size_t room = ctx->workspace ? ctx->ws_partial_bytes : 0;
+  const any::Problem p{M, N, K * 4, 4, 4, false, false, false};
+  const double small =
+      f32_small_any_ok(M, N, K) ? any::f32_small_us(M, N, K, cus, f32_small_b16(N, B, ldb),
+                                                    f32_small_is_narrow(M, N, K, A, lda))
+                                : 1e30;
+  if (f32_tile_ok(M, N, K, A, lda, B, ldb, C, ldc, ba))
+    return aligned_is_small(ctx, M, N, K, A, lda, B, ldb)
+               ? small
+               : any::other_us(any::COST_F32, p, true, cus, room);
+  const double other = any::other_us(any::COST_F32, p, false, cus, room);
+  return small < other ? small : other;
 }
 
 bool launch_f32_tile(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const float* A,

@@ -1,4 +1,4 @@
-// GEMM of a small output: 32 x 64 tiles, one workgroup each, whose four waves share out k.
+// GEMM of a small output: 32 x 64 tiles (fp32: 32 x 32), one workgroup each, whose four waves share out k.
 //
 // What bounds these calls is latency: the launch, one trip to memory, what one compute unit can take
 // from its L2 while most of the others have nothing to do (about 100 KB per us), and, where K is cut,
@@ -8,13 +8,16 @@
 // 6.5, 48 x 4096 x 3776 13.6 -> 10.5, 678 x 128 x 6284 13.9 -> 9.5; int8 N x K 365 x 96 x 853 13.6 ->
 // 6.0, K x N 1066 x 320 x 3264 13.3 -> 9.8, 107 x 6208 x 2576 15.7 -> 13.0; the 341 of 760 random sizes
 // that came here (M 1..40000, N 16..16384, K 64..16384) 1.33 times as fast (geometric mean), 4 of them
-// 3..6 % slower.
+// 3..6 % slower.  fp32 (against the tile kernel and the register-loaded small kernel): 95 x 896 x 1344
+// 17.1 -> 7.8, 22 x 19 x 7616 24.2 -> 8.4, 5812 x 8 x 5568 149 -> 28.6; of 350 random sizes the 163 that
+// came here 1.91 times as fast, one 11 % slower; the error against 64 bits 1.71e-7 from 2.01e-7
+// (geometric mean over 112 products), at most 3.8e-7 from 6.1e-7.
 //
 // Workgroup = 256 lanes = 4 waves.  Wave w takes the 128-byte pieces w, w + 4, ... of k (64 halves,
 // 128 int8, 32 floats), each through its own LDS slots -- no barrier before the waves' sums meet --:
 // A [32 rows][128 B] and B one of [64 n][128 B] (N x K), [64 k][128 B] (K x N, 16-bit), [128 k][64 B]
-// (int8), [32 k][256 B] (fp32), moved by LDS-DMA with the bank swizzle on the global side.  Up to
-// SLOTS pieces of a wave are in flight (144 KiB a workgroup); with more workgroups than units one
+// (int8), [32 k][128 B] (fp32), moved by LDS-DMA with the bank swizzle on the global side.  Up to
+// MAX_SLOTS pieces of a wave are in flight (144 or 128 KiB a workgroup); with more workgroups than units one
 // piece per wave, so that three workgroups share a unit.  The four sums meet in LDS in wave order.
 //
 // K ranges: the grid has `splits` workgroups per tile.  Each stores its sums to the workspace with
@@ -35,15 +38,22 @@ namespace cig {
 namespace kwaves {
 namespace {
 
-constexpr int A_BYTES = TM * PB, B_BYTES = TN * PB;
-constexpr int SLOT_BYTES = A_BYTES + B_BYTES;    // 12 KiB
-constexpr int PER = SLOT_BYTES / 1024;           // DMA instructions per piece
-constexpr int SUM_LD = TN + 4;                   // floats per row of a wave's sums in LDS
-static_assert(TM * SUM_LD * 4 <= SLOT_BYTES, "a wave's sums fit its first slot");
+// Tiles of 32 NT columns: fp32, whose matrix instructions take 64 cycles, 32, the others 64.
+template <int BMODE>
+struct Geo {
+  static constexpr int NT = BMODE == tile::B_KN32 ? 1 : 2;
+  static constexpr int TN = 32 * NT;
+  static constexpr int A_BYTES = TM * PB, B_BYTES = TN * PB;
+  static constexpr int SLOT_BYTES = A_BYTES + B_BYTES;  // 8 or 12 KiB
+  static constexpr int PER = SLOT_BYTES / 1024;         // DMA instructions per piece
+  static constexpr int MAX_SLOTS = NT == 1 ? 4 : 3;     // pieces of a wave in flight
+  static constexpr int SUM_LD = TN + 4;                 // floats per row of a wave's sums in LDS
+  static_assert(TM * SUM_LD * 4 <= SLOT_BYTES, "a wave's sums fit its first slot");
+};
 
-// B piece: DMA instruction q (0..7) fills 1 KiB; lane l fetches the 16 bytes at dma_src from the
-// tile's origin (`last` = last valid row (N x K) or 16-byte chunk of a row (K x N)).  READS LDS reads
-// give the fragment of 32 columns and k-step kk (0..3).
+// B piece: DMA instruction q fills 1 KiB; lane l fetches the 16 bytes at dma_src from the tile's
+// origin (`last` = last valid row (N x K) or 16-byte chunk of a row (K x N)).  frag: the fragment of the
+// 32 columns from n0, k-step kk (0..3).
 template <int BMODE>
 struct BPiece;
 
@@ -105,9 +115,33 @@ struct BPiece<tile::B_KN8> {
   }
 };
 
+// [32 k][32 n] floats.  A read takes 32 columns of two rows k and k + 4, each half of the banks: row k
+// sits at k ^ (bit 2 of k), so that the two have different parities.
+template <>
+struct BPiece<tile::B_KN32> {
+  static constexpr int CHUNKS = 8;
+  static __device__ __forceinline__ int row(int k) { return k ^ ((k >> 2) & 1); }  // (its own inverse)
+  static __device__ __forceinline__ int off(int k, int c) { return row(k) * 128 + (c << 4); }
+  static __device__ __forceinline__ uint32_t dma_src(int q, int l, int64_t ld, int last) {
+    const int k = row(8 * q + (l >> 3)), c = l & 7;
+    return (uint32_t)((int64_t)k * ld + ((c < last ? c : last) << 4));
+  }
+  static __device__ __forceinline__ u32x4 frag(const char* sb, int, int kk, int l) {
+    u32x4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      v[e] = *reinterpret_cast<const uint32_t*>(sb + row(8 * kk + 4 * (l >> 5) + e) * 128 + (l & 31) * 4);
+    return v;
+  }
+};
+
 // vmcnt(rem * PER): at most `rem` whole pieces still in flight
+template <int PER>
 __device__ __forceinline__ void wait_pieces(int rem) {
-  if (rem >= 2)
+  static_assert(3 * PER < 64, "vmcnt is a 6-bit counter");
+  if (rem >= 3)
+    __builtin_amdgcn_s_waitcnt(0x0f70 | ((3 * PER) & 15) | (((3 * PER) >> 4) << 14));
+  else if (rem == 2)
     __builtin_amdgcn_s_waitcnt(0x0f70 | ((2 * PER) & 15) | (((2 * PER) >> 4) << 14));
   else if (rem == 1)
     __builtin_amdgcn_s_waitcnt(0x0f70 | (PER & 15) | ((PER >> 4) << 14));
@@ -123,7 +157,7 @@ __device__ __forceinline__ const char* uniform(const char* p) {
   return (const char*)((uint64_t)hi << 32 | lo);
 }
 
-// lda, ldb in bytes; slots: pieces of a wave in flight (1..3).  `tail`: the last 1..128 bytes of k
+// lda, ldb in bytes; slots: pieces of a wave in flight (1..MAX_SLOTS).  `tail`: the last 1..128 bytes of k
 // go through registers.  grid.x = tiles_m * tiles_n * splits; range r covers the bytes
 // [r * range_bytes, (r + 1) * range_bytes) of k, the last one what is left; range_bytes is a whole
 // number of pieces whenever there is more than one range.
@@ -135,6 +169,10 @@ __global__ __launch_bounds__(256, 3) void kwaves_kernel(
   typedef typename Math::acc_t acc_t;
   typedef typename Math::scalar_t scalar_t;
   typedef BPiece<BMODE> BT;
+  typedef Geo<BMODE> G;
+  constexpr int NT = G::NT, TN = G::TN, A_BYTES = G::A_BYTES, SLOT_BYTES = G::SLOT_BYTES;
+  constexpr int NB = 4 * NT;  // DMA instructions of a B piece
+  constexpr int SUM_LD = G::SUM_LD;
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   __shared__ int is_last;
   const int t = threadIdx.x, l = t & 63;
@@ -172,7 +210,7 @@ __global__ __launch_bounds__(256, 3) void kwaves_kernel(
   const int a_last = (int)(M - 1 - m0 < TM - 1 ? M - 1 - m0 : TM - 1);
   const int n_left = (int)(N - n0 < TN ? N - n0 : TN);
   const int b_last = BMODE == tile::B_NK ? n_left - 1 : (n_left * Math::ELEM_BYTES + 15) / 16 - 1;
-  uint32_t a_voff[4], b_voff[8];
+  uint32_t a_voff[4], b_voff[NB];
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     const int r = 8 * q + (l >> 3);
@@ -180,7 +218,7 @@ __global__ __launch_bounds__(256, 3) void kwaves_kernel(
                            (((l & 7) ^ tile::pair_swz(r)) << 4));
   }
 #pragma unroll
-  for (int q = 0; q < 8; ++q) b_voff[q] = BT::dma_src(q, l, ldb, b_last);
+  for (int q = 0; q < NB; ++q) b_voff[q] = BT::dma_src(q, l, ldb, b_last);
   char* const own = lds + w * slots * SLOT_BYTES;  // this wave's slots
   const uint32_t own_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)own;
   auto dma16 = [&](const char* from, uint32_t voff, uint32_t lds_dst) {
@@ -196,41 +234,49 @@ __global__ __launch_bounds__(256, 3) void kwaves_kernel(
     const char* const b_src = b_tile + (int64_t)p * b_step;
     const uint32_t dst = own_base + slot * SLOT_BYTES;
 #pragma unroll
-    for (int q = 0; q < 8; ++q) dma16(b_src, b_voff[q], dst + A_BYTES + q * 1024);
+    for (int q = 0; q < NB; ++q) dma16(b_src, b_voff[q], dst + A_BYTES + q * 1024);
 #pragma unroll
     for (int q = 0; q < 4; ++q) dma16(a_src, a_voff[q], dst + q * 1024);
   };
 
-  acc_t acc[2];
+  acc_t acc[NT];
 #pragma unroll
-  for (int j = 0; j < 2; ++j)
+  for (int j = 0; j < NT; ++j)
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[j][e] = 0;
   struct Frags {
-    u32x4 a[4], b[4][2];
+    u32x4 a[4], b[4][NT];
   };
   auto read = [&](Frags& f, const char* sa) {
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {
       f.a[kk] = *reinterpret_cast<const u32x4*>(sa + tile::pair_off(l & 31, 2 * kk + (l >> 5)));
 #pragma unroll
-      for (int j = 0; j < 2; ++j) f.b[kk][j] = BT::frag(sa + A_BYTES, 32 * j, kk, l);
+      for (int j = 0; j < NT; ++j) f.b[kk][j] = BT::frag(sa + A_BYTES, 32 * j, kk, l);
     }
   };
   auto multiply = [&](const Frags& f) {
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) acc[j] = Math::mfma(f.b[kk][j], f.a[kk], acc[j]);
+      for (int j = 0; j < NT; ++j) {
+        if constexpr (Math::SUBSTEPS == 1) {
+          acc[j] = Math::mfma(f.b[kk][j], f.a[kk], acc[j]);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            acc[j] = Math::mfma(Math::afrag(f.b[kk][j], e), Math::afrag(f.a[kk], e), acc[j]);
+        }
+      }
   };
 
 #pragma unroll
-  for (int i = 0; i < 3; ++i)
+  for (int i = 0; i < G::MAX_SLOTS; ++i)
     if (i < slots && i < mine) issue(i, i);
   int slot = 0;
   for (int i = 0; i < mine; ++i) {
     const int rem = mine - 1 - i < slots - 1 ? mine - 1 - i : slots - 1;
-    wait_pieces(rem);
+    wait_pieces<G::PER>(rem);
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
     Frags f;
@@ -254,14 +300,14 @@ __global__ __launch_bounds__(256, 3) void kwaves_kernel(
     const int64_t lda_e = lda / Math::ELEM_BYTES, ldb_e = ldb / Math::ELEM_BYTES;
     const int64_t k0 = (int64_t)pieces * PB / Math::ELEM_BYTES, k_end = k_here / Math::ELEM_BYTES;
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    u32x4 ta[4], tb[8];
+    u32x4 ta[4], tb[NB];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int c = l + 64 * q;
       ta[q] = tile::load_piece(Ae, lda_e, m0 + (c >> 3), M, k0 + (c & 7) * CE, k_end);
     }
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
+    for (int q = 0; q < NB; ++q) {
       const int c = l + 64 * q;
       if constexpr (BMODE == tile::B_NK)
         tb[q] = tile::load_piece(Be, ldb_e, n0 + (c >> 3), N, k0 + (c & 7) * CE, k_end);
@@ -275,7 +321,7 @@ __global__ __launch_bounds__(256, 3) void kwaves_kernel(
           tile::trim_piece<elem_t>(ta[q], m0 + (c >> 3), M, k0 + (c & 7) * CE, k_end);
     }
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
+    for (int q = 0; q < NB; ++q) {
       const int c = l + 64 * q;
       if constexpr (BMODE == tile::B_NK)
         *reinterpret_cast<u32x4*>(own + A_BYTES + BT::off(c >> 3, c & 7)) =
@@ -291,23 +337,24 @@ __global__ __launch_bounds__(256, 3) void kwaves_kernel(
     multiply(f);
   }
 
-  // The waves' sums, each in its wave's first slot, meet in wave order: thread t holds quads
-  // (t / 16, 4 (t % 16)) and (t / 16 + 16, ..).  acc[j][4q + e] = C[l % 32][32 j + 8 q + 4 g + e].
+  // The waves' sums, each in its wave's first slot, meet in wave order: thread t holds NT quads of
+  // columns 4 (t % QPR).., rows t / QPR + h * ROWS.  acc[j][4q + e] = C[l % 32][32 j + 8 q + 4 g + e].
   typedef __attribute__((ext_vector_type(4))) scalar_t quad_t;
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's fragments are in registers
 #pragma unroll
-  for (int j = 0; j < 2; ++j)
+  for (int j = 0; j < NT; ++j)
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const quad_t v = {acc[j][4 * q], acc[j][4 * q + 1], acc[j][4 * q + 2], acc[j][4 * q + 3]};
       *reinterpret_cast<quad_t*>(own + ((l & 31) * SUM_LD + 32 * j + 8 * q + 4 * (l >> 5)) * 4) = v;
     }
   __syncthreads();
-  const int orow = t >> 4, ocol = (t & 15) * 4;
-  scalar_t sum[2][4];
+  constexpr int QPR = TN / 4, ROWS = 256 / QPR;
+  const int orow = t / QPR, ocol = (t % QPR) * 4;
+  scalar_t sum[NT][4];
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const char* at = lds + ((orow + 16 * h) * SUM_LD + ocol) * 4;
+  for (int h = 0; h < NT; ++h) {
+    const char* at = lds + ((orow + ROWS * h) * SUM_LD + ocol) * 4;
     quad_t s = *reinterpret_cast<const quad_t*>(at);
 #pragma unroll
     for (int ww = 1; ww < WAVES; ++ww)
@@ -317,12 +364,12 @@ __global__ __launch_bounds__(256, 3) void kwaves_kernel(
   }
 
   if (splits > 1) {
-    // word x (0..3) of thread t at x * 256 + t of the range's 8 KiB
-    constexpr int WORDS = 4 * 256;
+    // word x of thread t at x * 256 + t of the range's 4 NT KiB
+    constexpr int NX = 2 * NT, WORDS = NX * 256;
     const int tile_id = tn * tiles_m + tm;
     uint64_t* const tile_part = partials + (int64_t)tile_id * splits * WORDS + t;
 #pragma unroll
-    for (int x = 0; x < 4; ++x) {
+    for (int x = 0; x < NX; ++x) {
       const uint64_t lo = __builtin_bit_cast(uint32_t, sum[x / 2][x % 2 * 2]);
       const uint64_t hi = __builtin_bit_cast(uint32_t, sum[x / 2][x % 2 * 2 + 1]);
       __hip_atomic_store(tile_part + (int64_t)range * WORDS + x * 256, lo | hi << 32,
@@ -338,17 +385,17 @@ __global__ __launch_bounds__(256, 3) void kwaves_kernel(
     __syncthreads();
     if (!is_last) return;
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int h = 0; h < NT; ++h)
 #pragma unroll
       for (int e = 0; e < 4; ++e) sum[h][e] = 0;
     // (the loads of eight ranges are issued back to back before the first addition waits)
     for (int r0 = 0; r0 < splits; r0 += 8) {
-      uint64_t v[8][4];
+      uint64_t v[8][NX];
 #pragma unroll
       for (int b = 0; b < 8; ++b)
         if (r0 + b < splits) {
 #pragma unroll
-          for (int x = 0; x < 4; ++x)
+          for (int x = 0; x < NX; ++x)
             v[b][x] = __hip_atomic_load(tile_part + (int64_t)(r0 + b) * WORDS + x * 256,
                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
@@ -356,7 +403,7 @@ __global__ __launch_bounds__(256, 3) void kwaves_kernel(
       for (int b = 0; b < 8; ++b)
         if (r0 + b < splits) {
 #pragma unroll
-          for (int x = 0; x < 4; ++x) {
+          for (int x = 0; x < NX; ++x) {
             sum[x / 2][x % 2 * 2] += __builtin_bit_cast(scalar_t, (uint32_t)v[b][x]);
             sum[x / 2][x % 2 * 2 + 1] += __builtin_bit_cast(scalar_t, (uint32_t)(v[b][x] >> 32));
           }
@@ -366,8 +413,8 @@ __global__ __launch_bounds__(256, 3) void kwaves_kernel(
   }
 
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int64_t r = m0 + orow + 16 * h, c = n0 + ocol;
+  for (int h = 0; h < NT; ++h) {
+    const int64_t r = m0 + orow + ROWS * h, c = n0 + ocol;
     if (r < M && c < N) tile::store_quad_any(epi, r, c, N, sum[h]);
   }
 }
@@ -380,21 +427,22 @@ bool is_whole(int64_t K_bytes, int64_t n_bytes, bool b_nk) {
 template <typename Math, int BMODE, typename Epi>
 void launch(cigemmContext* ctx, Plan plan, int64_t M, int64_t N, int64_t K_bytes, const void* A,
             int64_t lda_bytes, const void* B, int64_t ldb_bytes, const Epi& epi) {
+  typedef Geo<BMODE> G;
   auto kern = kwaves_kernel<Math, BMODE, Epi>;
   static std::atomic<uint64_t> lds_set{0};
-  if (!ensure_dynamic_lds(ctx, (const void*)kern, WAVES * 3 * SLOT_BYTES, lds_set)) return;
-  const int tiles_m = (int)((M + TM - 1) / TM), tiles_n = (int)((N + TN - 1) / TN);
+  if (!ensure_dynamic_lds(ctx, (const void*)kern, WAVES * G::MAX_SLOTS * G::SLOT_BYTES, lds_set)) return;
+  const int tiles_m = (int)((M + TM - 1) / TM), tiles_n = (int)((N + G::TN - 1) / G::TN);
   int64_t range_stages = 0;
   const int splits = tile::k_ranges(K_bytes, plan.splits, &range_stages);
   const int64_t range_bytes = splits > 1 ? range_stages * tile::KB : K_bytes;
   const bool whole = is_whole(K_bytes, N * Math::ELEM_BYTES, BMODE == tile::B_NK);
   const int64_t wgs = (int64_t)tiles_m * tiles_n * splits;
   const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
-  const int slots = wgs <= cus ? 3 : 1;
+  const int slots = wgs <= cus ? G::MAX_SLOTS : 1;
   ctx->last_tile_rows = TM;
   ctx->last_k_splits = splits;
   ctx->last_waves = WAVES;
-  hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(256), WAVES * slots * SLOT_BYTES, ctx->stream,
+  hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(256), WAVES * slots * G::SLOT_BYTES, ctx->stream,
                      (int)M, (int)N, tiles_m, tiles_n, splits, (int)range_bytes, (int)K_bytes,
                      whole ? 0 : 1, slots, static_cast<const char*>(A), lda_bytes,
                      static_cast<const char*>(B), ldb_bytes, epi,
@@ -424,6 +472,16 @@ Plan plan_of(cigemmContext* ctx, bool ok, const Cost& cost, const any::Cost& oth
   if (ctx->force_tile_rows) return Plan{0};
   return choose(cost, other, p, is_whole(p.K_bytes, p.N * p.elem, b_nk), aligned,
                 ctx->num_cus > 0 ? ctx->num_cus : 256, room, ctx->ws_counter_bytes);
+}
+
+void launch_f32(cigemmContext* ctx, Plan plan, int64_t M, int64_t N, int64_t K, const float* A,
+                int64_t lda, const float* B, int64_t ldb, float* C, int64_t ldc, const BiasAct* ba) {
+  if (ba)
+    launch<tile::MathF32, tile::B_KN32>(ctx, plan, M, N, K * 4, A, lda * 4, B, ldb * 4,
+                                        EpiBiasActAnyF32x4{C, ldc, ba->bias, ba->relu});
+  else
+    launch<tile::MathF32, tile::B_KN32>(ctx, plan, M, N, K * 4, A, lda * 4, B, ldb * 4,
+                                        EpiStoreF32x4{C, ldc});
 }
 
 template <int BMODE>
@@ -461,6 +519,35 @@ bool launch_kwaves_16(cigemmContext* ctx, bool bf16, int64_t M, int64_t N, int64
     kwaves::launch<tile::MathF16, tile::B_KN16>(ctx, p, M, N, K * 2, A, lda * 2, B, ldb * 2,
                                                 EpiStore16x4<F16>{C, ldc});
   kwaves::set_name(ctx, bf16 ? "bf16" : "f16", 64, "", !aligned);
+  return true;
+}
+
+bool launch_kwaves_f32(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const float* A,
+                       int64_t lda, const float* B, int64_t ldb, float* C, int64_t ldc,
+                       const BiasAct* ba) {
+  const size_t room = ctx->workspace ? ctx->ws_partial_bytes : 0;
+  kwaves::Plan p{1};
+  if (!any::tile_ok(M, N, K, 4, lda, ldb, true) || ctx->force_kwaves < 0 ||
+      !kwaves::fits(M, N, p, room, ctx->ws_counter_bytes, kwaves::TN_F32))
+    return false;
+  if (ctx->force_kwaves > 0) {
+    if (kwaves::fits(M, N, kwaves::Plan{ctx->force_kwaves}, room, ctx->ws_counter_bytes, kwaves::TN_F32))
+      p.splits = ctx->force_kwaves;
+  } else {
+    // (a plan of another kernel is imposed; up to 16 columns and K = 512 the small kernel's 16-column
+    // form streams as fast: 20000 x 10 x 512 11.5 against 11.7 us, 2145 x 15 x 320 5.5 against 6.1)
+    if (ctx->force_tile_rows || (K <= 512 && f32_small_is_narrow(M, N, K, A, lda))) return false;
+    double est = 0;
+    p = kwaves::best_f32(M, N, K, ctx->num_cus > 0 ? ctx->num_cus : 256, room, ctx->ws_counter_bytes,
+                         &est);
+    if (!p.splits || est >= f32_other_us(ctx, M, N, K, A, lda, B, ldb, C, ldc, ba)) return false;
+  }
+  kwaves::launch_f32(ctx, p, M, N, K, A, lda, B, ldb, C, ldc, ba);
+  // (one family with the register-loaded small kernel: 32 x 32 tiles, k split over four waves)
+  snprintf(ctx->kernel_name, sizeof(ctx->kernel_name), "f32_mfma_%ssmall_32x32_ksplit4%s%s",
+           f32_small_shape_ok(M, N, K, A, lda) ? "" : "any_", ba ? "_bias_act" : "",
+           ctx->last_k_splits > 1 ? "_splitk" : "");
+  ctx->last_kernel = ctx->kernel_name;
   return true;
 }
 

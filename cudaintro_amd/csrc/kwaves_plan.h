@@ -11,16 +11,17 @@ struct Plan {
   int splits;  // K ranges; 0: no plan
 };
 
-constexpr int TM = 32, TN = 64, PB = 128;  // output tile; bytes of k per piece
+constexpr int TM = 32, TN = 64, PB = 128;  // output tile (fp32: 32 columns); bytes of k per piece
 constexpr int WAVES = 4;
 
 // The plan's grid fits a launch, and its partial sums and arrival counters their parts of the
 // workspace.
-inline bool fits(int64_t M, int64_t N, Plan p, size_t partial_bytes, size_t counter_bytes) {
-  const int64_t tiles = any::div_up(M, TM) * any::div_up(N, TN);
+inline bool fits(int64_t M, int64_t N, Plan p, size_t partial_bytes, size_t counter_bytes,
+                 int tn = TN) {
+  const int64_t tiles = any::div_up(M, TM) * any::div_up(N, tn);
   if (tiles > 2147483647LL / p.splits) return false;
   return p.splits == 1 || (tiles <= (int64_t)(counter_bytes / 4) &&
-                           tiles * p.splits * TM * TN * 4 <= (int64_t)partial_bytes);
+                           tiles * p.splits * TM * tn * 4 <= (int64_t)partial_bytes);
 }
 
 // us: a call's start, then per piece of the workgroups that share the fullest compute unit (what the
@@ -78,6 +79,55 @@ inline Plan choose(const Cost& c, const any::Cost& other, const any::Problem& p,
   // (beyond one round the two estimates have to differ by more than they usually err)
   if (tiles > cus) est *= 1.1;
   return est < any::other_us(other, p, aligned, cus, partial_bytes) ? b : Plan{0};
+}
+
+// ---- fp32: tiles of 32 x 32 ---------------------------------------------------------------------
+// us: `start`, then per piece of the busiest wave of a unit (its 16 matrix instructions: the unit's
+// workgroups one after the other) and of a workgroup's busiest wave, per piece on average, per
+// workgroup of a unit, operand bytes, K ranges and the tail.  Fitted to the kernel timed at 420 sizes
+// (M 1..6000, N 4..8192, K 16..8192, log-uniform) x up to 8 numbers of ranges; rms error 7 %.
+struct CostF32 {
+  double start, unit_piece, wave_piece, load, unit_tile, in_mb, split, part_mb, tail;
+};
+constexpr CostF32 COST_F32{4.58, 0.341, 0.140, 0.0441, 0.123, 0.0160, 0.816, 0.107, 0.375};
+constexpr int TN_F32 = 32;
+// No range of k is longer than 64 pieces (2048 floats, 512 for each wave to add up): a long K keeps
+// the rounding of the shorter sums it has on the tile kernel, and the ranges cost 0.8 us.
+constexpr int MAX_RANGE_BYTES_F32 = 64 * PB;
+
+inline double us_f32(int64_t M, int64_t N, int64_t K, int cus, int splits) {
+  const CostF32& c = COST_F32;
+  int64_t stages = 0;
+  const int sp = tile::k_ranges(K * 4, splits, &stages);
+  const int64_t pieces = any::div_up(stages, 2), wave = any::div_up(pieces, WAVES);
+  const int64_t wgs = any::div_up(M, TM) * any::div_up(N, TN_F32) * sp, per = any::div_up(wgs, cus);
+  double t = c.start + (double)(per * wave) * c.unit_piece + (double)wave * c.wave_piece +
+             (double)wgs / cus * (double)pieces * c.load + (double)per * c.unit_tile +
+             (double)(M + N) * (double)K * 4e-6 * c.in_mb + (K % 32 || N % 4 ? c.tail : 0.0);
+  if (sp > 1) t += c.split + (double)M * (double)N * 4e-6 * sp * c.part_mb;
+  return t;
+}
+
+// The plan with the lowest estimate, which goes to *est; no plan (0) for a K of no more than two pieces,
+// more tiles than four a unit, a K of more ranges than 16, or operands beyond the 256 MB cache, whose
+// stream the 256-column tiles keep up better (39 x 9664 x 9984 130 us against 116).
+inline Plan best_f32(int64_t M, int64_t N, int64_t K, int cus, size_t partial_bytes,
+                     size_t counter_bytes, double* est) {
+  const int64_t tiles = any::div_up(M, TM) * any::div_up(N, TN_F32), K_bytes = 4 * K;
+  const int64_t least = any::div_up(K_bytes, MAX_RANGE_BYTES_F32);
+  *est = 1e30;
+  Plan b{0};
+  if (K_bytes <= 2 * PB || tiles > 4 * (int64_t)cus || (M + N) * K_bytes > 256000000) return b;
+  for (int64_t sp = least; sp <= 16; ++sp) {
+    if (sp > least && (K_bytes / sp < 1024 || tiles * sp > 4 * (int64_t)cus)) break;
+    if (!fits(M, N, Plan{(int)sp}, partial_bytes, counter_bytes, TN_F32)) break;
+    const double t = us_f32(M, N, K, cus, (int)sp);
+    if (t < *est) *est = t, b = Plan{(int)sp};
+  }
+  // (beyond a round and a half the estimates have to differ by more than they err: 127 x 7360 x 4032
+  // 79 us here against 70 on the tile kernel, estimated equal)
+  if (2 * tiles > 3 * (int64_t)cus) *est *= 1.12;
+  return b;
 }
 
 }  // namespace kwaves

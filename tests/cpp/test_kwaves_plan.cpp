@@ -35,6 +35,28 @@ int main() {
             }
             ++(plan.splits ? taken : refused);
           }
+  // fp32: the same, no range longer than 8 KiB of k
+  for (long long M : Ms)
+    for (long long N : Ns)
+      for (long long K : {16LL, 64LL, 65LL, 1000LL, 2048LL, 2049LL, 30000LL, 40000LL, 500000000LL})
+        for (size_t room : {(size_t)0, (size_t)1 << 20, (size_t)64 << 20}) {
+          double est = 0;
+          const size_t counters = 4096;
+          const kwaves::Plan plan = kwaves::best_f32(M, N, K, 256, room, counters, &est);
+          const long long tiles = any::div_up(M, 32) * any::div_up(N, 32);
+          int64_t stages = 0;
+          const int ranges = tile::k_ranges(4 * K, plan.splits, &stages);
+          bool ok = !((K <= 64 || tiles > 1024 || K > 32768) && plan.splits) && plan.splits <= 16;
+          if (plan.splits) ok = ok && est > 4.0 && est < 1e6 && stages * 64 <= 8192 + 128;
+          if (plan.splits > 1)
+            ok = ok && stages % 2 == 0 && (ranges - 1) * stages * 64 < 4 * K &&
+                 tiles * plan.splits * 4096 <= (long long)room && tiles * 4 <= (long long)counters;
+          if (!ok) {
+            std::printf("FAILED fp32 %lld %lld %lld room %zu: %d ranges\n", M, N, K, room, plan.splits);
+            return 1;
+          }
+          ++(plan.splits ? taken : refused);
+        }
   if (taken < 100 || refused < 100) return std::printf("FAILED: %d taken, %d refused\n", taken, refused), 1;
   std::printf("kwaves plan OK\n");
   return 0;

@@ -1,4 +1,4 @@
-"""The kernel of small outputs (32 x 64 tiles, k shared out to four waves, K ranges joined inside the
+"""The kernel of small outputs (32 x 64 tiles, fp32 32 x 32, k shared out to four waves, K ranges joined inside the
 kernel) at the sizes where it can go wrong: M and N around its tiles, K around its 128-byte pieces (all
 of K in the separately multiplied tail, fewer pieces than waves, more than its slots hold, a tail of one
 element up to a whole piece, in every wave), one and several K ranges, aligned and unaligned operands.  Operand
@@ -14,7 +14,7 @@ from gpu_util import bits
 from test_gpu_mfma_any import VALS, embed
 
 pytestmark = pytest.mark.gpu
-BYTES = {"bf16": 2, "f16": 2, "i8_kn": 1, "i8_nk": 1}
+BYTES = {"bf16": 2, "f16": 2, "f32": 4, "i8_kn": 1, "i8_nk": 1}
 SHAPES = [  # M, N, aligned
     (33, 136, True), (129, 260, True), (200, 384, True), (65, 64, True),
     (64, 127, False), (130, 193, False), (257, 33, False),
@@ -33,6 +33,7 @@ def test_kwaves(handle, torch_gpu, oracle, rng, kind):
     torch = torch_gpu
     int8 = kind.startswith("i8")
     layout = ci.B_NK if kind == "i8_nk" else ci.B_KN
+    name = "small_32x32_ksplit4" if kind == "f32" else "kwaves_32x64"
     host = lambda t: bits(torch, t) if t.element_size() == 2 else t.contiguous().cpu().numpy()  # noqa: E731
     for M, N, aligned in SHAPES:
         for K in sizes_of_k(BYTES[kind], aligned):
@@ -44,10 +45,11 @@ def test_kwaves(handle, torch_gpu, oracle, rng, kind):
             else:
                 A, B = rng.choice(VALS, size=(M, K)), rng.choice(VALS, size=(K, N))
                 ref = oracle.gemm_f32(A, B)
-                dt = odt = {"bf16": torch.bfloat16, "f16": torch.float16}[kind]
+                dt = odt = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[kind]
                 pad = float("nan")
-                narrow = {"bf16": oracle.f32_to_bf16, "f16": oracle.f32_to_f16}[kind]
-                A, B, ref = narrow(A).view(np.int16), narrow(B).view(np.int16), narrow(ref)
+                narrow = {"bf16": oracle.f32_to_bf16, "f16": oracle.f32_to_f16}.get(kind)
+                if narrow:
+                    A, B, ref = narrow(A).view(np.int16), narrow(B).view(np.int16), narrow(ref)
             # rows of whole 16-byte pieces at offset 0, or everything off by an element
             step = 16 // BYTES[kind]
             off, fill = (0, lambda c, e: -c % e) if aligned else (1, lambda c, e: 3)
@@ -69,23 +71,29 @@ def test_kwaves(handle, torch_gpu, oracle, rng, kind):
                             handle.gemm_i8_i32(a, b, layout, out=out)
                         else:
                             getattr(handle, "gemm_" + kind)(a, b, out=out)
-                        assert "kwaves_32x64" in handle.last_kernel, handle.last_kernel
+                        assert name in handle.last_kernel, handle.last_kernel
+                        assert handle.last_plan[0] == 32    # (0: the register-loaded fp32 kernel)
                         what = f"{handle.last_kernel} {handle.last_plan} M={M} N={N} K={K}"
                         np.testing.assert_array_equal(host(out), ref, err_msg=what)
                         assert (host(flat)[guard] == sentinel).all(), what
                     if int8:
                         sa = rng.uniform(1e-3, 5e-2, M).astype(np.float32)
                         sb = rng.uniform(1e-3, 5e-2, N).astype(np.float32)
-                        for name, ot in (("f32", ci.OUT_F32), ("bf16", ci.OUT_BF16)):
+                        for out_name, ot in (("f32", ci.OUT_F32), ("bf16", ci.OUT_BF16)):
                             y = handle.gemm_i8_dequant(a, b, torch.from_numpy(sa).cuda(),
                                                        torch.from_numpy(sb).cuda(), layout, ot)
-                            assert "kwaves_32x64" in handle.last_kernel, handle.last_kernel
+                            assert name in handle.last_kernel, handle.last_kernel
                             np.testing.assert_array_equal(
-                                host(y), oracle.dequant(ref, sa, sb, out_dtype=name, sa_per_row=M > 1,
+                                host(y), oracle.dequant(ref, sa, sb, out_dtype=out_name, sa_per_row=M > 1,
                                                         sb_per_col=True), err_msg=what)
                             y = handle.gemm_i8_dequant(a, b, torch.from_numpy(sa[:1]).cuda(),
                                                        torch.from_numpy(sb[:1]).cuda(), layout, ot)
                             np.testing.assert_array_equal(
-                                host(y), oracle.dequant(ref, sa[:1], sb[:1], out_dtype=name), err_msg=what)
+                                host(y), oracle.dequant(ref, sa[:1], sb[:1], out_dtype=out_name), err_msg=what)
+                    elif kind == "f32":
+                        bias = rng.choice(VALS, size=N)
+                        y = handle.linear_f32(a, b, torch.from_numpy(bias).cuda(), ci.ACT_RELU)
+                        assert name in handle.last_kernel, handle.last_kernel
+                        np.testing.assert_array_equal(host(y), oracle.linear_f32(A, B, bias, True), err_msg=what)
                 finally:
                     probe.force_kwaves_plan(handle, 0)
