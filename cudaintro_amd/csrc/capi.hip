@@ -260,6 +260,21 @@ static bool any_i8(cigemmHandle_t h, int64_t M, int64_t N, int64_t K, const int8
          launch_mfma_any_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq);
 }
 
+// A call whose last few columns are the kernel of small outputs' (kwaves_rest_columns): `main(n1)`
+// runs the first n1, `rest(n1)` the others.  False, with nothing launched, where there is no such plan.
+extern "C++" {
+template <typename Main, typename Rest>
+static bool rest_columns(cigemmHandle_t h, int64_t M, int64_t N, int64_t K_bytes, bool f32, Main main,
+                         Rest rest) {
+  const int64_t n1 = kwaves_rest_columns(h, M, N, K_bytes, f32);
+  if (!n1 || !rest(n1) || !main(n1)) return false;
+  char first[sizeof(h->kernel_name)];
+  snprintf(first, sizeof(first), "%s", h->last_kernel);
+  name_rest_columns(h, first);
+  return true;
+}
+}  // extern "C++"
+
 // fp32 dispatch.  DEFAULT: one of the two aligned MFMA kernels when the shape allows, else one of
 // those that take any (the scalar kernel only if no tile grid fits a launch).
 // Returns false when a selected family refuses the call.
@@ -282,6 +297,18 @@ static bool dispatch_f32(cigemmHandle_t h, int64_t M, int64_t N, int64_t K, cons
       return true;
     default:
       if (!launch_kwaves_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba) &&
+          !rest_columns(
+              h, M, N, K * 4, true,
+              [&](int64_t n1) {
+                return launch_f32_mfma(h, M, n1, K, A, lda, B, ldb, C, ldc, ba) ||
+                       any_f32(h, M, n1, K, A, lda, B, ldb, C, ldc, ba);
+              },
+              [&](int64_t n1) {
+                BiasAct shifted{};
+                if (ba) shifted = BiasAct{ba->bias ? ba->bias + n1 : nullptr, ba->relu};
+                return launch_kwaves_f32(h, M, N - n1, K, A, lda, B + n1, ldb, C + n1, ldc,
+                                         ba ? &shifted : nullptr, true);
+              }) &&
           !launch_f32_mfma(h, M, N, K, A, lda, B, ldb, C, ldc, ba) &&
           !any_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba))
         launch_generic_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba);
@@ -333,6 +360,15 @@ static cigemmStatus_t gemm16(cigemmHandle_t h, const char* name, bool bf16, int6
       // neither that nor the tile kernel takes (odd N, unaligned rows) stays on the matrix cores
       if (!launch_skinny_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc) &&
           !launch_kwaves_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc) &&
+          !rest_columns(
+              h, M, N, K * 2, false,
+              [&](int64_t n1) {
+                return launch_16b_mfma(h, bf16, M, n1, K, A, lda, B, ldb, C, ldc) ||
+                       any_16(h, bf16, M, n1, K, A, lda, B, ldb, C, ldc);
+              },
+              [&](int64_t n1) {
+                return launch_kwaves_16(h, bf16, M, N - n1, K, A, lda, B + n1, ldb, C + n1, ldc, true);
+              }) &&
           !launch_16b_mfma(h, bf16, M, N, K, A, lda, B, ldb, C, ldc) &&
           !any_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc))
         launch_generic_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc);
@@ -370,6 +406,23 @@ static cigemmStatus_t gemm_i8(cigemmHandle_t h, const char* name, int64_t M, int
     default:
       if (!launch_skinny_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq) &&
           !launch_kwaves_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq) &&
+          !((!dq || !dq->acc_out) &&
+            rest_columns(
+                h, M, N, K, false,
+                [&](int64_t n1) {
+                  return launch_i8_mfma(h, M, n1, K, A, lda, B, ldb, b_nk, C, ldc, dq) ||
+                         any_i8(h, M, n1, K, A, lda, B, ldb, b_nk, C, ldc, dq);
+                },
+                [&](int64_t n1) {
+                  DequantArgs shifted{};
+                  if (dq) {
+                    shifted = *dq;
+                    shifted.out = static_cast<char*>(dq->out) + n1 * (dq->out_bf16 ? 2 : 4);
+                    if (dq->sb_vec) shifted.sb = dq->sb + n1;
+                  }
+                  return launch_kwaves_i8(h, M, N - n1, K, A, lda, B + (b_nk ? n1 * ldb : n1), ldb, b_nk,
+                                          C ? C + n1 : nullptr, ldc, dq ? &shifted : nullptr, true);
+                })) &&
           !launch_i8_mfma(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq) &&
           !any_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq))
         launch_generic_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq);

@@ -252,14 +252,23 @@ bool launch_tile_any_i8(cigemmContext*, int64_t M, int64_t N, int64_t K, const i
                         int64_t lda, const int8_t* B, int64_t ldb, bool b_nk, int32_t* C,
                         int64_t ldc, const DequantArgs* dq, tile::SmallPlan plan);
 // gemm_kwaves.hip: 32 x 64 tiles, k shared out to the waves; any size and alignment.  False, with
-// nothing launched, where another kernel is estimated to be faster.
+// nothing launched, where another kernel is estimated to be faster.  `rest`: the call is the last few
+// columns of a wider one (kwaves_rest_columns said so): taken without an estimate, and B has whole
+// 16-byte pieces in front of the first of them.
 bool launch_kwaves_16(cigemmContext*, bool bf16, int64_t M, int64_t N, int64_t K, const uint16_t* A,
-                      int64_t lda, const uint16_t* B, int64_t ldb, uint16_t* C, int64_t ldc);
+                      int64_t lda, const uint16_t* B, int64_t ldb, uint16_t* C, int64_t ldc,
+                      bool rest = false);
 bool launch_kwaves_f32(cigemmContext*, int64_t M, int64_t N, int64_t K, const float* A, int64_t lda,
-                       const float* B, int64_t ldb, float* C, int64_t ldc, const BiasAct* ba);
+                       const float* B, int64_t ldb, float* C, int64_t ldc, const BiasAct* ba,
+                       bool rest = false);
 bool launch_kwaves_i8(cigemmContext*, int64_t M, int64_t N, int64_t K, const int8_t* A, int64_t lda,
                       const int8_t* B, int64_t ldb, bool b_nk, int32_t* C, int64_t ldc,
-                      const DequantArgs* dq);
+                      const DequantArgs* dq, bool rest = false);
+// Columns of the full rounds of 256-row tiles where those and a few columns more (at most 64, on 32-row
+// tiles) cover the output best; 0: no such plan.
+int64_t kwaves_rest_columns(const cigemmContext*, int64_t M, int64_t N, int64_t K_bytes, bool f32);
+// the kernel's name after such a pair of calls: "<first>+<tile of the rest>"
+void name_rest_columns(cigemmContext*, const char* first);
 void launch_generic_16(cigemmContext*, bool bf16, int64_t M, int64_t N, int64_t K,
                        const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb,
                        uint16_t* C, int64_t ldc);

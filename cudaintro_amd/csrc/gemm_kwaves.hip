@@ -460,7 +460,7 @@ void set_name(cigemmContext* ctx, const char* dtype, int k_elems, const char* su
 
 // `ok`: the kernel can run the call; `aligned`: the tile kernel's aligned form can.
 Plan plan_of(cigemmContext* ctx, bool ok, const Cost& cost, const any::Cost& other,
-             const any::Problem& p, bool aligned, bool b_nk) {
+             const any::Problem& p, bool aligned, bool b_nk, bool rest) {
   const size_t room = ctx->workspace ? ctx->ws_partial_bytes : 0;
   if (!ok || ctx->force_kwaves < 0 || !fits(p.M, p.N, Plan{1}, room, ctx->ws_counter_bytes))
     return Plan{0};
@@ -470,6 +470,10 @@ Plan plan_of(cigemmContext* ctx, bool ok, const Cost& cost, const any::Cost& oth
   }
   // (a plan of another kernel is imposed)
   if (ctx->force_tile_rows) return Plan{0};
+  if (rest) {
+    double est = 0;
+    return best(cost, p, false, ctx->num_cus > 0 ? ctx->num_cus : 256, room, ctx->ws_counter_bytes, &est);
+  }
   return choose(cost, other, p, is_whole(p.K_bytes, p.N * p.elem, b_nk), aligned,
                 ctx->num_cus > 0 ? ctx->num_cus : 256, room, ctx->ws_counter_bytes);
 }
@@ -505,12 +509,12 @@ void launch_i8_layout(cigemmContext* ctx, Plan plan, int64_t M, int64_t N, int64
 
 bool launch_kwaves_16(cigemmContext* ctx, bool bf16, int64_t M, int64_t N, int64_t K,
                       const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb, uint16_t* C,
-                      int64_t ldc) {
+                      int64_t ldc, bool rest) {
   const bool aligned = tile_16_ok(M, N, K, A, lda, B, ldb, C, ldc);
   const any::Problem call{M, N, K * 2, 2, 2, false, any::rows_apart(A, lda * 2),
                           any::rows_apart(B, ldb * 2)};
-  const kwaves::Plan p = kwaves::plan_of(ctx, any::tile_ok(M, N, K, 2, lda, ldb, true),
-                                         kwaves::COST_16, any::COST_16, call, aligned, false);
+  const kwaves::Plan p = kwaves::plan_of(ctx, any::tile_ok(M, rest ? 64 : N, K, 2, lda, ldb, true),
+                                         kwaves::COST_16, any::COST_16, call, aligned, false, rest);
   if (!p.splits) return false;
   if (bf16)
     kwaves::launch<tile::MathBF16, tile::B_KN16>(ctx, p, M, N, K * 2, A, lda * 2, B, ldb * 2,
@@ -524,10 +528,10 @@ bool launch_kwaves_16(cigemmContext* ctx, bool bf16, int64_t M, int64_t N, int64
 
 bool launch_kwaves_f32(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const float* A,
                        int64_t lda, const float* B, int64_t ldb, float* C, int64_t ldc,
-                       const BiasAct* ba) {
+                       const BiasAct* ba, bool rest) {
   const size_t room = ctx->workspace ? ctx->ws_partial_bytes : 0;
   kwaves::Plan p{1};
-  if (!any::tile_ok(M, N, K, 4, lda, ldb, true) || ctx->force_kwaves < 0 ||
+  if (!any::tile_ok(M, rest ? 64 : N, K, 4, lda, ldb, true) || ctx->force_kwaves < 0 ||
       !kwaves::fits(M, N, p, room, ctx->ws_counter_bytes, kwaves::TN_F32))
     return false;
   if (ctx->force_kwaves > 0) {
@@ -536,11 +540,11 @@ bool launch_kwaves_f32(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, cons
   } else {
     // (a plan of another kernel is imposed; up to 16 columns and K = 512 the small kernel's 16-column
     // form streams as fast: 20000 x 10 x 512 11.5 against 11.7 us, 2145 x 15 x 320 5.5 against 6.1)
-    if (ctx->force_tile_rows || (K <= 512 && f32_small_is_narrow(M, N, K, A, lda))) return false;
+    if (ctx->force_tile_rows || (!rest && K <= 512 && f32_small_is_narrow(M, N, K, A, lda))) return false;
     double est = 0;
     p = kwaves::best_f32(M, N, K, ctx->num_cus > 0 ? ctx->num_cus : 256, room, ctx->ws_counter_bytes,
                          &est);
-    if (!p.splits || est >= f32_other_us(ctx, M, N, K, A, lda, B, ldb, C, ldc, ba)) return false;
+    if (!p.splits || (!rest && est >= f32_other_us(ctx, M, N, K, A, lda, B, ldb, C, ldc, ba))) return false;
   }
   kwaves::launch_f32(ctx, p, M, N, K, A, lda, B, ldb, C, ldc, ba);
   // (one family with the register-loaded small kernel: 32 x 32 tiles, k split over four waves)
@@ -554,14 +558,14 @@ bool launch_kwaves_f32(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, cons
 // (the accumulator dump is left to the other kernels)
 bool launch_kwaves_i8(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const int8_t* A,
                       int64_t lda, const int8_t* B, int64_t ldb, bool b_nk, int32_t* C, int64_t ldc,
-                      const DequantArgs* dq) {
+                      const DequantArgs* dq, bool rest) {
   const bool aligned = tile::i8_tile_ok(M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq);
   const any::Problem call{M, N, K, 1, dq && dq->out_bf16 ? 2 : 4, dq != nullptr,
                           any::rows_apart(A, lda), any::rows_apart(B, ldb)};
   const kwaves::Plan p = kwaves::plan_of(
-      ctx, any::tile_ok(M, N, K, 1, lda, ldb, !b_nk) && !(dq && dq->acc_out),
+      ctx, any::tile_ok(M, rest ? 64 : N, K, 1, lda, ldb, !b_nk) && !(dq && dq->acc_out),
       b_nk ? kwaves::COST_I8_NK : kwaves::COST_I8_KN, b_nk ? any::COST_I8_NK : any::COST_I8_KN, call,
-      aligned, b_nk);
+      aligned, b_nk, rest);
   if (!p.splits) return false;
   if (b_nk)
     kwaves::launch_i8_layout<tile::B_NK>(ctx, p, M, N, K, A, lda, B, ldb, C, ldc, dq);
@@ -571,6 +575,32 @@ bool launch_kwaves_i8(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const
                    dq ? (b_nk ? "_nk_dequant" : "_kn_dequant") : (b_nk ? "_nk" : "_kn"),
                    !aligned);
   return true;
+}
+
+int64_t kwaves_rest_columns(const cigemmContext* ctx, int64_t M, int64_t N, int64_t K_bytes, bool f32) {
+  // A rest of up to 64 columns costs the tile kernel a column of 256-column tiles, a quarter of them
+  // or less used; here 32-row tiles of 32 or 64 columns.  fp32 4095 x 4097 x 4099, one column: 63 us of
+  // 64-row tiles over four K ranges and 5 of reduction (977 us the call, 930 here); bf16 4096 x 4104 x 4096
+  // 124 -> 115, int8 2048 x 8200 x 1024 36.7 -> 32.1; 17 such sizes 1.06 times as fast, none slower.
+  const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+  if (ctx->force_tile_rows || ctx->force_kwaves || K_bytes <= 3 * kwaves::PB ||
+      any::div_up(M, tile::BM) * any::div_up(N, tile::BN) <= cus)
+    return 0;
+  int rows = 0;
+  const tile::RoundsPlan r = f32 ? tile::plan_rounds32(M, N, cus, &rows)
+                                 : tile::plan_rounds(M, N, cus, tile::TILE_UNITS);
+  const int64_t rest = N - r.first_cols;
+  if (!r.first_cols || rest > 64) return 0;
+  const int64_t tiles = any::div_up(M, kwaves::TM) * any::div_up(rest, f32 ? kwaves::TN_F32 : kwaves::TN);
+  return tiles <= 3 * (int64_t)cus ? r.first_cols : 0;
+}
+
+void name_rest_columns(cigemmContext* ctx, const char* first) {
+  char name[sizeof(ctx->kernel_name)];
+  snprintf(name, sizeof(name), "%s+%dx%d", first, kwaves::TM,
+           strncmp(first, "f32", 3) ? kwaves::TN : kwaves::TN_F32);
+  memcpy(ctx->kernel_name, name, sizeof(name));
+  ctx->last_kernel = ctx->kernel_name;
 }
 
 }  // namespace cig

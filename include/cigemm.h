@@ -127,7 +127,8 @@ CIGEMM_API int cigemmGetVersion(void);
  * "_splitk" after such a name: the second launch ran as K ranges plus a reduction); the kernel of
  * small outputs "<type>_mfma_[any_]kwaves_32x64x<k per piece>_w4[_kn|_nk][_dequant]_splitk" (k is
  * always split, over its four waves at least), fp32 "f32_mfma_[any_]small_32x32_ksplit4[_bias_act]
- * [_splitk]".  Valid until the next GEMM call on the handle. */
+ * [_splitk]"; "+32x64" or "+32x32" behind any of these: the last few columns ran on that kernel.
+ * Valid until the next GEMM call on the handle. */
 CIGEMM_API const char* cigemmGetLastKernelName(cigemmHandle_t handle);
 
 /* Plan of the last successful GEMM call on this handle, for tests and profiles: rows of the
