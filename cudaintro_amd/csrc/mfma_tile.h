@@ -2,7 +2,8 @@
 //
 // Workgroup = 256 lanes = 4 waves (2 x 2) -- or, for N x K int8 weights with a 16-bit output and
 // for their 128-row tiles, 512 lanes = 8 waves (4 x 2) of half the height, two per SIMD, same data
-// flow, see launch_tile_256 / launch_tile_128 --; macro tile 256 (m) x 256 (n); k is consumed in
+// flow, see launch_tile_256 / launch_tile_128; fp32 has its 4 waves side by side, see
+// mfma_tile_kernel --; macro tile 256 (m) x 256 (n); k is consumed in
 // stages of 64 BYTES per row (32 halves, 64 int8 or 16 floats) = two MFMA k-steps.  Each wave
 // owns a 128 x 128 block = 4 x 4 MFMA tiles of 32 x 32 = 256 accumulators per lane (the AGPR
 // file); one wave per SIMD.  The tile height is a template parameter (MT = 4, 3, 2 or 1 row
@@ -625,7 +626,8 @@ __device__ __forceinline__ void store_tile(const Epi& epi, typename Math::acc_t 
 // Measured against the kernel that served these calls before (mfma_any_kernel: one 64-byte step
 // in flight between two barriers, every piece trimmed) and against aligned sizes: bf16 4096 x 4095
 // x 4096 264 -> 112 us (4096^3: 104), 8191 x 8192 at M = 2048 523 -> 219, at M = 1 31.5 -> 26.5;
-// int8 N x K 2048 x 8191 x 8191 342 -> 161; fp32 4095 x 4097 x 4099 1493 -> 981 (4096^3: 905).
+// int8 N x K 2048 x 8191 x 8191 342 -> 161; fp32 4095 x 4097 x 4099 1493 -> 981 (4096^3: 905; since the
+// remaining column runs elsewhere, see kwaves_rest_columns, 930).
 // What is left of the difference: a piece that is not 16-byte aligned takes the address path twice
 // (10 % per stage where one 16-bit operand is misaligned, 40 % where both int8 ones are), and so
 // do the stores of unaligned rows (10 us per 64 MiB).
@@ -1343,6 +1345,9 @@ void launch_tile_rows(cigemmContext* ctx, int rows, int64_t M, int64_t N, int64_
 
 // Runs one plan: tiles of `rows` rows; with more than one K range the ranges go over
 // blockIdx.y, partial sums to the workspace, then one reduction launch with the real epilogue.
+// (Joining them inside, by the last workgroup of a tile, is slower here: it takes the other ranges'
+// 64..256 KiB tiles alone, 70 KB per us, where the reduction launch has the whole chip: bf16
+// 256 x 8192 x 8192 51.4 -> 55.4 us, int8 K x N 385 x 1984 x 4938 16.8 -> 20.5.)
 // Returns true when it ran as such a pair of launches.
 template <typename Math, int BMODE, bool ANY = false, typename Epi>
 bool run_tile_plan(cigemmContext* ctx, int rows, int splits, int64_t M, int64_t N, int64_t K_bytes,
