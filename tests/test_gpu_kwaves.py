@@ -97,3 +97,31 @@ def test_kwaves(handle, torch_gpu, oracle, rng, kind):
                         np.testing.assert_array_equal(host(y), oracle.linear_f32(A, B, bias, True), err_msg=what)
                 finally:
                     probe.force_kwaves_plan(handle, 0)
+
+
+@pytest.mark.parametrize("kind,M,N,K", [("bf16", 52, 64, 4096), ("f32", 95, 96, 4099), ("bf16", 2048, 8200, 512)])
+def test_replayed_from_a_graph(torch_gpu, kind, M, N, K):
+    """K ranges and a remainder of columns recorded and replayed, eager calls of another size on the same handle
+    in between: every replay finds the counters at zero and gives the eager bits."""
+    torch = torch_gpu
+    dt = {"bf16": torch.bfloat16, "f32": torch.float32}[kind]
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    new = lambda r, c: torch.randn((r, c), generator=gen, device="cuda").to(dt)  # noqa: E731
+    a, b, a2, b2 = new(M, K), new(K, N), new(40, 2048), new(2048, 128)
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side), ci.Handle() as h:
+        gemm = getattr(h, "gemm_" + kind)
+        want, want2 = gemm(a, b), gemm(a2, b2)
+        gemm(a, b)
+        assert "kwaves" in h.last_kernel or "small_32x32" in h.last_kernel or "+32x64" in h.last_kernel
+        out = torch.zeros_like(want)
+        graph = torch.cuda.CUDAGraph()
+        side.synchronize()
+        with torch.cuda.graph(graph, stream=side):
+            gemm(a, b, out=out)
+        for _ in range(4):
+            out.zero_()
+            graph.replay()
+            assert torch.equal(gemm(a2, b2), want2)
+            side.synchronize()
+            assert torch.equal(out, want)
