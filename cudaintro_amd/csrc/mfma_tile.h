@@ -502,6 +502,11 @@ __device__ __forceinline__ void store_tile(const Epi& epi, typename Math::acc_t 
   const bool piece_half = OB == 2 && piece_col + 8 > N;
   const int64_t row_step = (intptr_t)epi.out_row(1) - (intptr_t)epi.out_row(0);  // bytes per row
   const bool interior = m0 + TILE_M <= M && n0 + BN <= N;  // (uniform)
+  // (uniform) Streaming stores: C is not read again by this kernel and should not evict A and B (ANY,
+  // on aligned rows, bf16 4096 x 4096 x 4095: 106 against 115 us).  Plain ones where the segments of a
+  // row begin inside a line, so that the L2 joins its two halves (ANY, unaligned rows, int8 -> int32
+  // 4096 x 4095 x 2047: 55 against 59 us); store_streams says where that is.
+  const bool stream = store_streams((intptr_t)epi.out_row(0), row_step, ANY, NT, TILE_M);
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
     const int64_t row0 = m0 + wm * 32 * MT + 32 * i;
@@ -540,16 +545,11 @@ __device__ __forceinline__ void store_tile(const Epi& epi, typename Math::acc_t 
     if constexpr (ANY) {
       constexpr int PE = 16 / OB;  // elements of a piece
       const int inside = (int)(N - piece_col);  // elements of this lane's piece inside the row
-      // (uniform) streaming stores where C's rows are aligned all the same: plain ones evict the
-      // operands (bf16 4096 x 4096 x 4095 106 against 115 us).  On unaligned rows the plain ones
-      // are the better, the L2 joins the two halves of a line (int8 -> int32 4096 x 4095 x 2047
-      // 55 against 59 us).
-      const bool rows_aligned = (((intptr_t)epi.out_row(0) | row_step) & 15) == 0;
 #pragma unroll
       for (int p = 0; p < NPASS; ++p)
         if (row0 + p * ROWS_PER_PASS + lane_row < M && inside >= PE) {
           char* dst = dst0 + p * ROWS_PER_PASS * row_step;
-          if (rows_aligned)
+          if (stream)
             __builtin_nontemporal_store(v[p], reinterpret_cast<u32x4*>(dst));
           else
             __builtin_memcpy(dst, &v[p], 16);
@@ -583,13 +583,18 @@ __device__ __forceinline__ void store_tile(const Epi& epi, typename Math::acc_t 
             }
           }
       }
+    } else if (interior && stream) {
+#pragma unroll
+      for (int p = 0; p < NPASS; ++p)
+        __builtin_nontemporal_store(v[p],
+                                    reinterpret_cast<u32x4*>(dst0 + p * ROWS_PER_PASS * row_step));
+      // (two branches that end in the same stores would be joined, and those are plain then)
+      if constexpr (NT == 2 && TILE_M > 64) asm volatile("" ::: "memory");
     } else if (interior) {
 #pragma unroll
       for (int p = 0; p < NPASS; ++p)
-        // streaming stores: C is not read again by this kernel and should not evict A / B
-        __builtin_nontemporal_store(v[p],
-                                    reinterpret_cast<u32x4*>(dst0 + p * ROWS_PER_PASS * row_step));
-    } else {
+        *reinterpret_cast<u32x4*>(dst0 + p * ROWS_PER_PASS * row_step) = v[p];
+    } else if (stream) {
 #pragma unroll
       for (int p = 0; p < NPASS; ++p) {
         char* dst = dst0 + p * ROWS_PER_PASS * row_step;
@@ -600,6 +605,12 @@ __device__ __forceinline__ void store_tile(const Epi& epi, typename Math::acc_t 
             __builtin_nontemporal_store(v[p], reinterpret_cast<u32x4*>(dst));
         }
       }
+      if constexpr (NT == 2 && TILE_M > 64) asm volatile("" ::: "memory");
+    } else {
+#pragma unroll
+      for (int p = 0; p < NPASS; ++p)
+        if (row0 + p * ROWS_PER_PASS + lane_row < M && piece_in)
+          *reinterpret_cast<u32x4*>(dst0 + p * ROWS_PER_PASS * row_step) = v[p];
     }
   }
 }

@@ -84,6 +84,14 @@ static void check_plans() {
   // tile heights of plans of several rounds
   CHECK(best_mt(8192, 8192, 256) == 4, "8192^2: %d", best_mt(8192, 8192, 256));
   CHECK(best_mt(2048, 11008, 256) == 3, "2048 x 11008: %d", best_mt(2048, 11008, 256));
+  // which rows of C the epilogue streams: whole lines for fp32's waves of 64 columns, whole pieces else
+  CHECK(store_streams(4096, 4 * 4096, false, 2, 256) && !store_streams(4096, 4 * 4100, false, 2, 96) &&
+        !store_streams(4096 + 64, 4 * 4096, false, 2, 256) && !store_streams(4096, 4 * 4100, true, 2, 128) &&
+        store_streams(4096, 4 * 4100, false, 2, 64) && !store_streams(4096, 4 * 4097, true, 2, 64),
+        "rows of fp32 tiles");
+  CHECK(store_streams(4096, 2 * 4104, false, 4, 256) && store_streams(4096, 2 * 4104, true, 4, 256) &&
+        !store_streams(4096, 2 * 4095, true, 4, 64) && !store_streams(4098, 2 * 4096, true, 4, 128),
+        "rows of the other types' tiles");
   // fp32 pays by the row: short tiles where they waste fewer rounds
   CHECK(best_mt(5120, 4096, 256, nullptr, TILE_UNITS_F32) == 1, "fp32 5120 x 4096");
   CHECK(best_mt(8192, 6144, 256, nullptr, TILE_UNITS_F32) == 4, "fp32 8192 x 6144");

@@ -79,3 +79,28 @@ def test_cross_workgroup_exchange_uses_agent_scope_accesses():
         assert re.search(r"global_load_dwordx2 .* sc1", body), name
         assert re.search(r"global_atomic_(add|swap)", body), name
     assert seen >= 12
+
+
+@pytest.mark.skipif(HIPCC is None, reason="hipcc not installed")
+def test_fp32_tiles_have_both_kinds_of_stores():
+    """The fp32 tile kernel stores rows of whole lines with streaming stores and others with plain ones
+    (tile_plan.h, store_streams; tiles of 64 rows stream all).  The compiler may join two branches that
+    end in the same stores, and the joined ones are plain: half of the 16-byte stores of each instance
+    must carry the nt bit (64 rows: all)."""
+    with tempfile.TemporaryDirectory() as d:
+        out = os.path.join(d, "f32.s")
+        subprocess.run([HIPCC, *FLAGS, os.path.join(CSRC, "gemm_f32.hip"), "-o", out], check=True,
+                       stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
+        text = open(out).read()
+    seen = 0
+    for body in re.split(r"\n(?=_Z\w+:)", text):
+        name = body.split(":", 1)[0]
+        if "mfma_tile_kernelINS0_7MathF32E" not in name or ":" not in body:
+            continue
+        stores = re.findall(r"global_store_dwordx4 .*", body.split(".Lfunc_end")[0])
+        if not stores:
+            continue
+        seen += 1
+        tall = "MathF32ELi3ELi4ELi2E" not in name
+        assert (1 + tall) * sum(" nt" in s for s in stores) == len(stores), (name, len(stores))
+    assert seen >= 42      # seven heights x (partial sums, plain, four epilogues)

@@ -41,3 +41,33 @@ def test_heights(handle, torch_gpu, oracle, rng, rows, aligned):
                         np.testing.assert_array_equal(y.cpu().numpy(), oracle.linear_f32(A, B, bias, True), err_msg=what)
                 finally:
                     probe.force_tile_plan(handle, 0)
+
+
+@pytest.mark.parametrize("rows", [64, 96, 256])
+@pytest.mark.parametrize("kind", ["aligned", "any"])
+def test_rows_that_begin_inside_a_line(handle, torch_gpu, rng, kind, rows):
+    """The epilogue's two kinds of stores (tile_plan.h, store_streams): rows of C that begin with a line and
+    rows that begin inside one, by the leading dimension and by the pointer, whole tiles and ragged
+    ones; K ranges too (their partial sums have rows of N).  Sums are exact: bit for bit."""
+    torch = torch_gpu
+    for M, N in ((256, 512), (300, 512), (256, 516), (300, 516), (257, 740)):
+        if kind == "any":
+            N += 1
+        A, B = (torch.from_numpy(rng.choice(VALS, size=s)).cuda() for s in ((M, 208), (208, N)))
+        ref = (A.double() @ B.double()).float()
+        for off, ld in ((0, -(-N // 32) * 32), (16, -(-N // 32) * 32), (0, -(-N // 4) * 4 + 4), (4, -(-N // 4) * 4 + 4)):
+            flat = torch.empty(off + M * ld, device="cuda")
+            out = flat[off:].view(M, ld)[:, :N]
+            for ranges in (1, 3):
+                probe.force_tile_plan(handle, rows, ranges)
+                try:
+                    with handle.algo(ci.ALGO_TILE if kind == "aligned" else ci.ALGO_MFMA_ANY):
+                        flat.fill_(7)
+                        handle.gemm_f32(A, B, out=out)
+                        what = f"{handle.last_kernel} {M} {N} {off} {ld}"
+                        assert f"{rows}x256x16" in handle.last_kernel, what
+                        assert torch.equal(out, ref), what
+                        out.fill_(7)
+                        assert bool((flat == 7).all()), what
+                finally:
+                    probe.force_tile_plan(handle, 0)
