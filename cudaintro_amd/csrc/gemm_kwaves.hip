@@ -587,7 +587,7 @@ int64_t kwaves_rest_columns(const cigemmContext* ctx, int64_t M, int64_t N, int6
       any::div_up(M, tile::BM) * any::div_up(N, tile::BN) <= cus)
     return 0;
   int rows = 0;
-  const tile::RoundsPlan r = f32 ? tile::plan_rounds32(M, N, cus, &rows)
+  const tile::RoundsPlan r = f32 ? tile::plan_rounds32(M, N, K_bytes, cus, &rows)
                                  : tile::plan_rounds(M, N, cus, tile::TILE_UNITS);
   const int64_t rest = N - r.first_cols;
   if (!r.first_cols || rest > 64) return 0;

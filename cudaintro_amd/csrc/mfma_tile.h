@@ -1430,7 +1430,7 @@ bool launch_tile(cigemmContext* ctx, int64_t M, int64_t N, int64_t K_bytes, cons
   RoundsPlan rounds;
   int rows = 0;
   if constexpr (BMODE == B_KN32) {
-    rounds = plan_rounds32(M, N, cus, &rows);
+    rounds = plan_rounds32(M, N, K_bytes, cus, &rows);
   } else {
     rounds = plan_rounds(M, N, cus, TILE_UNITS);
     rows = 64 * rounds.mt;

@@ -243,12 +243,13 @@ inline RoundsPlan plan_rounds(int64_t M, int64_t N, int cus, TileUnits units) {
 // (4095 x 4097 x 4099: 17th column of tiles 63 us + 5 for the reduction, a quarter of a 64-row round
 // is 60).  us before -> here: 20000 x 512 x 784 143.5 (210 tiles of 192 rows) -> 130.3 (250 of 160, one
 // round), 3000^3 503 (192) -> 422 (160), 7000 x 4096 x 4096 1604 (64) -> 1588 (224).
-// A second launch of more than 64 columns costs 0.4 units beside its tiles (its ramp, its epilogue, the
-// units that wait for the first one's last tiles): 136 sizes where both plans were timed, K 64..4096,
-// against the faster plan of each: 0.16 % slower on average, without that price 2.6 % (2111 x 8128 x 192
-// 74.5 us in two launches, 65.5 in one of 96-row tiles; 2609 x 8160 x 64 47.6 and 43.9; 3188 x 7040 x 192
-// 89.0 and 85.4).  Up to 64 columns end sooner, here or in kwaves_rest_columns.
-inline RoundsPlan plan_rounds32(int64_t M, int64_t N, int cus, int* rows) {
+// A second launch of more than 64 columns costs 0.35 units and 1 us beside its tiles (its ramp, its
+// epilogue, the units that wait for the first one's last tiles; below K = 64, where nothing was timed,
+// 0.48 units): 136 sizes where both plans were timed, K 64..4096, against the faster plan of each: 0.13 % slower on average, without that
+// price 2.6 % (2111 x 8128 x 192 74.5 us in two launches, 65.5 in one of 96-row tiles; 2609 x 8160 x 64
+// 47.6 and 43.9; 3188 x 7040 x 192 89.0 and 85.4).  Up to 64 columns end sooner, here or in
+// kwaves_rest_columns.
+inline RoundsPlan plan_rounds32(int64_t M, int64_t N, int64_t K_bytes, int cus, int* rows) {
   constexpr TileUnits u = TILE_UNITS_F32;
   const int64_t tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   double best = 1e30;
@@ -263,7 +264,10 @@ inline RoundsPlan plan_rounds32(int64_t M, int64_t N, int cus, int* rows) {
   if (full_cols <= 0 || full_cols >= tiles_n) return RoundsPlan{*rows / 64, 0};
   double rest = 0;
   const int mt2 = best_mt(M, N - full_cols * BN, cus, &rest, u);
-  const double second = N - full_cols * BN > 64 ? 0.4 : 0.0;
+  // (us of a unit: 64 rows of a tile over all stages of k)
+  const double unit_us = STAGE_COST_KN32.per_64_rows_us * (double)((K_bytes + KB - 1) / KB);
+  const double price = unit_us > 2.5 ? 0.35 + 1.0 / unit_us : 0.48;
+  const double second = N - full_cols * BN > 64 ? price : 0.0;
   if (tiles_m * (tiles_n - full_cols) <= cus) {
     const double share =
         0.05 + (double)((M + 63) / 64 * (tiles_n - full_cols)) / cus * tile_cost_units(1, u);

@@ -84,14 +84,17 @@ static void check_plans() {
   // tile heights of plans of several rounds
   CHECK(best_mt(8192, 8192, 256) == 4, "8192^2: %d", best_mt(8192, 8192, 256));
   CHECK(best_mt(2048, 11008, 256) == 3, "2048 x 11008: %d", best_mt(2048, 11008, 256));
-  // fp32 in two launches: where the second one is worth its price
+  // fp32 in two launches (K in bytes): where the second one is worth its price
   int rows = 0;
-  CHECK(plan_rounds32(2609, 8160, 256, &rows).first_cols == 0 && rows == 192, "2609 x 8160");
-  CHECK(plan_rounds32(3188, 7040, 256, &rows).first_cols == 0, "3188 x 7040");
-  CHECK(plan_rounds32(2111, 8128, 256, &rows).first_cols == 0 && rows == 96, "2111 x 8128");
-  CHECK(plan_rounds32(3580, 5888, 256, &rows).first_cols > 0, "3580 x 5888");
-  CHECK(plan_rounds32(4095, 4097, 256, &rows).first_cols == 4096, "4095 x 4097");
-  CHECK(plan_rounds32(4095, 4353, 256, &rows).first_cols == 4096, "4095 x 4353");
+  CHECK(plan_rounds32(2609, 8160, 4 * 64, 256, &rows).first_cols == 0 && rows == 192, "2609 x 8160 x 64");
+  CHECK(plan_rounds32(8176, 4288, 4 * 64, 256, &rows).first_cols == 0 && rows == 192, "8176 x 4288 x 64");
+  CHECK(plan_rounds32(3188, 7040, 4 * 192, 256, &rows).first_cols == 0, "3188 x 7040 x 192");
+  CHECK(plan_rounds32(2111, 8128, 4 * 192, 256, &rows).first_cols == 0 && rows == 96, "2111 x 8128 x 192");
+  CHECK(plan_rounds32(3580, 5888, 4 * 768, 256, &rows).first_cols > 0, "3580 x 5888 x 768");
+  for (int64_t K : {5, 1025, 4099}) {
+    CHECK(plan_rounds32(4095, 4097, 4 * K, 256, &rows).first_cols == 4096, "4095 x 4097");
+    CHECK(plan_rounds32(4095, 4353, 4 * K, 256, &rows).first_cols == 4096, "4095 x 4353");
+  }
   // which rows of C the epilogue streams: whole lines for fp32's waves of 64 columns, whole pieces else
   CHECK(store_streams(4096, 4 * 4096, false, 2, 256) && !store_streams(4096, 4 * 4100, false, 2, 96) &&
         !store_streams(4096 + 64, 4 * 4096, false, 2, 256) && !store_streams(4096, 4 * 4100, true, 2, 128) &&
