@@ -82,12 +82,19 @@ inline tile::SmallPlan tile_plan(const Cost& c, const Problem& p, int cus, size_
                           p.K_bytes * p.N);
 }
 
-// One launch of the tile form (and the reduction behind it): N columns on tiles of 64 mt rows.
-inline double tile_launch_us(const Cost& c, const Problem& p, int64_t N, int cus, tile::SmallPlan plan) {
-  const int mt = plan.mt;
+// Rows of the tiles that the launcher runs `plan` of N columns with: fp32 may have a height between.
+inline int tile_rows(const Cost& c, const Problem& p, int64_t N, int cus, tile::SmallPlan plan) {
+  return p.elem == 4 ? tile::plan_small_rows32(cus, p.M, N, p.K_bytes, p.out_bytes, c.sc, p.K_bytes * N,
+                                               plan)
+                     : 64 * plan.mt;
+}
+
+// One launch of the tile form (and the reduction behind it): N columns on tiles of `rows` rows.
+inline double tile_launch_us(const Cost& c, const Problem& p, int64_t N, int cus, int rows, int splits) {
+  const double mt = rows / 64.0;
   int64_t stages = 0;
-  const int sp = tile::k_ranges(p.K_bytes, plan.splits, &stages);
-  const double rounds = (double)div_up(div_up(p.M, 64 * mt) * div_up(N, tile::BN) * sp, cus);
+  const int sp = tile::k_ranges(p.K_bytes, splits, &stages);
+  const double rounds = (double)div_up(div_up(p.M, rows) * div_up(N, tile::BN) * sp, cus);
   const double apart = (p.a_apart ? mt : 0) + (p.b_apart ? 4 : 0);
   const double mn = (double)p.M * (double)N * 1e-6;
   double us = rounds * ((double)stages * (c.t_stage + c.t_stage_64_rows * mt + c.t_apart * apart) +
@@ -104,15 +111,22 @@ inline double tile_launch_us(const Cost& c, const Problem& p, int64_t N, int cus
 inline double tile_us(const Cost& c, const Problem& p, int cus, size_t partial_bytes,
                       tile::SmallPlan plan) {
   const double us = c.t_start + (p.dequant ? c.t_dequant : 0.0);
-  if (plan.mt) return us + tile_launch_us(c, p, p.N, cus, plan);
-  const tile::RoundsPlan r = tile::plan_rounds(p.M, p.N, cus, c.units);
-  if (!r.first_cols) return us + tile_launch_us(c, p, p.N, cus, tile::SmallPlan{r.mt, 1});
+  if (plan.mt) return us + tile_launch_us(c, p, p.N, cus, tile_rows(c, p, p.N, cus, plan), plan.splits);
+  int rows = 0;
+  tile::RoundsPlan r;
+  if (p.elem == 4) {
+    r = tile::plan_rounds32(p.M, p.N, p.K_bytes, cus, &rows);
+  } else {
+    r = tile::plan_rounds(p.M, p.N, cus, c.units);
+    rows = 64 * r.mt;
+  }
+  if (!r.first_cols) return us + tile_launch_us(c, p, p.N, cus, rows, 1);
   Problem rest = p;
   rest.N = p.N - r.first_cols;
-  tile::SmallPlan second = tile_plan(c, rest, cus, partial_bytes);
-  if (!second.mt) second = tile::SmallPlan{r.mt, 1};
-  return us + tile_launch_us(c, p, r.first_cols, cus, tile::SmallPlan{4, 1}) +
-         tile_launch_us(c, rest, rest.N, cus, second);
+  const tile::SmallPlan second = tile_plan(c, rest, cus, partial_bytes);
+  return us + tile_launch_us(c, p, r.first_cols, cus, 256, 1) +
+         tile_launch_us(c, rest, rest.N, cus,
+                        second.mt ? tile_rows(c, rest, rest.N, cus, second) : 64 * r.mt, second.splits);
 }
 
 // K ranges of the register-staged kernel (tiles of 128 x 128, steps of 64 bytes of k) for a problem

@@ -25,7 +25,7 @@ static bool aligned_is_small(const cigemmContext* ctx, int64_t M, int64_t N, int
     // plan's own figure against 0.115 per resident round of 32x32 tiles (2048^3: tile kernel
     // 157 us, small kernel 225 us; 1024^3: 74 us against 33 us; 512^3: 38 us against 8 us).
     double tile_cost = 0;
-    tile::best_mt(M, N, cus, &tile_cost);
+    tile::best_rows32(M, N, cus, tile::TILE_UNITS, &tile_cost);
     const double tiles32 = (double)((M + 31) / 32) * (double)((N + 31) / 32);
     const double small_cost = 0.115 * (tiles32 > cus ? tiles32 / cus : 1.0);
     // With a long K the tile kernel wins whenever its tiles fit one round: it can split K over
@@ -41,7 +41,9 @@ static bool aligned_is_small(const cigemmContext* ctx, int64_t M, int64_t N, int
     const size_t room = ctx->workspace ? ctx->ws_partial_bytes : 0;
     double tile_us = 0;
     if (one_round) {
-      tile::plan_small(cus, room, M, N, K * 4, 4, tile::STAGE_COST_KN32, K * 4 * N, &tile_us);
+      const tile::SmallPlan plan =
+          tile::plan_small(cus, room, M, N, K * 4, 4, tile::STAGE_COST_KN32, K * 4 * N);
+      tile::plan_small_rows32(cus, M, N, K * 4, 4, tile::STAGE_COST_KN32, K * 4 * N, plan, &tile_us);
       tile_us += 4.0;
     } else {
       tile_us = any::tile_us(any::COST_F32, any::Problem{M, N, K * 4, 4, 4, false, false, false}, cus,

@@ -154,9 +154,10 @@ inline SmallPlan plan_small(int cus, size_t partial_bytes, int64_t M, int64_t N,
 
 // fp32, whose tiles may have any multiple of 32 rows: the height for `plan`'s number of K ranges that
 // the same estimate likes best, among the plan's own and all that lie between the multiples of 64.
-// (96 x 4096 x 4096: 96 rows in place of 128.)
+// (83 x 6752 x 4352: 96 rows in place of 128.)  `est_us`, if given, receives that height's estimate.
 inline int plan_small_rows32(int cus, int64_t M, int64_t N, int64_t K_bytes,
-                             int out_bytes, StageCost sc, int64_t b_bytes, SmallPlan plan) {
+                             int out_bytes, StageCost sc, int64_t b_bytes, SmallPlan plan,
+                             double* est_us = nullptr) {
   const bool streamed = b_bytes > (16LL << 20);
   if (cus <= 0) cus = 256;
   int64_t range_stages = 0;
@@ -169,6 +170,7 @@ inline int plan_small_rows32(int cus, int64_t M, int64_t N, int64_t K_bytes,
         plan_us_rows(M, N, K_bytes, out_bytes, sc, streamed, cus, rows, sp, range_stages);
     if (us < best_us) best_us = us, best = rows;
   }
+  if (est_us) *est_us = best_us;
   return best;
 }
 
@@ -238,7 +240,20 @@ inline RoundsPlan plan_rounds(int64_t M, int64_t N, int cus, TileUnits units) {
   return r;
 }
 
-// fp32: the same with every multiple of 32 rows (but 32) for the single launch, whose height goes to
+// The height of a single launch of fp32 tiles: best_mt's choice among every multiple of 32 rows but 32.
+inline int best_rows32(int64_t M, int64_t N, int cus, TileUnits u, double* cost) {
+  const int64_t tiles_n = (N + BN - 1) / BN;
+  int best = 0;
+  *cost = 1e30;
+  for (int rows = 256; rows >= 64; rows -= 32) {
+    const int64_t tiles = (M + rows - 1) / rows * tiles_n;
+    const double c = (double)((tiles + cus - 1) / cus) * (u.fixed + u.per_64_rows * rows / 64);
+    if (c < *cost) *cost = c, best = rows;
+  }
+  return best;
+}
+
+// fp32: plan_rounds with every multiple of 32 rows (but 32) for the single launch, whose height goes to
 // *rows; the second launch, which may split K, priced by the share of the chip its 64-row tiles take
 // (4095 x 4097 x 4099: 17th column of tiles 63 us + 5 for the reduction, a quarter of a 64-row round
 // is 60).  us before -> here: 20000 x 512 x 784 143.5 (210 tiles of 192 rows) -> 130.3 (250 of 160, one
@@ -252,12 +267,8 @@ inline RoundsPlan plan_rounds(int64_t M, int64_t N, int cus, TileUnits units) {
 inline RoundsPlan plan_rounds32(int64_t M, int64_t N, int64_t K_bytes, int cus, int* rows) {
   constexpr TileUnits u = TILE_UNITS_F32;
   const int64_t tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-  double best = 1e30;
-  for (int r = 256; r >= 64; r -= 32) {
-    const int64_t tiles = (M + r - 1) / r * tiles_n;
-    const double cost = (double)((tiles + cus - 1) / cus) * (u.fixed + u.per_64_rows * r / 64);
-    if (cost < best) best = cost, *rows = r;
-  }
+  double best = 0;
+  *rows = best_rows32(M, N, cus, u, &best);
   if (tiles_m > cus) return RoundsPlan{*rows / 64, 0};
   const int64_t cols_per_round = cus / tiles_m;
   const int64_t full_cols = tiles_n / cols_per_round * cols_per_round;

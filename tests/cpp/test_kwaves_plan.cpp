@@ -57,6 +57,28 @@ int main() {
           }
           ++(plan.splits ? taken : refused);
         }
+  // What fp32's estimate is compared with has the tile kernel's own heights: 96 and 160 rows here, where
+  // this kernel is the slower one (us: K, here, there).
+  const struct { long long M, N, K; double here, there; } other[] = {
+      {67, 5568, 3392, 41.5, 38.9}, {68, 5696, 4416, 50.0, 47.1}, {86, 6848, 5568, 76.2, 69.3},
+      {94, 8704, 2240, 44.5, 41.5}, {74, 6528, 8320, 102.5, 91.7}};
+  const size_t room = (size_t)64 << 20;
+  for (const auto& o : other) {
+    double est = 0;
+    kwaves::best_f32(o.M, o.N, o.K, 256, room, 65536, &est);
+    const any::Problem p{o.M, o.N, 4 * o.K, 4, 4, false, false, false};
+    const double there = any::other_us(any::COST_F32, p, true, 256, room);
+    if (est <= there)
+      return std::printf("FAILED fp32 %lld %lld %lld: %.1f here, %.1f there\n", o.M, o.N, o.K, est, there), 1;
+  }
+  // and its times: one round of 160-row tiles (130 us), three of 160 rows (420)
+  const struct { long long M, N, K; double us; } times[] = {{20000, 512, 784, 130}, {3000, 3000, 3000, 420}};
+  for (const auto& o : times) {
+    const any::Problem p{o.M, o.N, 4 * o.K, 4, 4, false, false, false};
+    const double us = any::other_us(any::COST_F32, p, true, 256, room);
+    if (us < 0.93 * o.us || us > 1.07 * o.us)
+      return std::printf("FAILED fp32 %lld %lld %lld: %.1f us\n", o.M, o.N, o.K, us), 1;
+  }
   if (taken < 100 || refused < 100) return std::printf("FAILED: %d taken, %d refused\n", taken, refused), 1;
   std::printf("kwaves plan OK\n");
   return 0;
