@@ -61,7 +61,11 @@ int main() {
   // this kernel is the slower one (us: K, here, there).
   const struct { long long M, N, K; double here, there; } other[] = {
       {67, 5568, 3392, 41.5, 38.9}, {68, 5696, 4416, 50.0, 47.1}, {86, 6848, 5568, 76.2, 69.3},
-      {94, 8704, 2240, 44.5, 41.5}, {74, 6528, 8320, 102.5, 91.7}};
+      {94, 8704, 2240, 44.5, 41.5}, {74, 6528, 8320, 102.5, 91.7},
+      // two row tiles and more over a long stream of B, and many tiles
+      {36, 5016, 7040, 59.5, 44.5}, {47, 11228, 4608, 85.0, 66.8}, {48, 11328, 3904, 72.9, 59.4},
+      {54, 9920, 2496, 42.6, 35.4}, {104, 2048, 10176, 61.0, 47.6}, {467, 768, 7936, 64.4, 56.1},
+      {420, 704, 7616, 56.2, 46.1}};
   const size_t room = (size_t)64 << 20;
   for (const auto& o : other) {
     double est = 0;
@@ -69,6 +73,17 @@ int main() {
     const any::Problem p{o.M, o.N, 4 * o.K, 4, 4, false, false, false};
     const double there = any::other_us(any::COST_F32, p, true, 256, room);
     if (est <= there)
+      return std::printf("FAILED fp32 %lld %lld %lld: %.1f here, %.1f there\n", o.M, o.N, o.K, est, there), 1;
+  }
+  // while these stay here
+  const struct { long long M, N, K; double here, there; } kept[] = {
+      {42, 6144, 2816, 22.9, 26.4}, {1, 5120, 7472, 39.1, 44.6}, {17, 9216, 3776, 38.5, 40.5}, {95, 896, 1344, 7.8, 17.1}};
+  for (const auto& o : kept) {
+    double est = 0;
+    kwaves::best_f32(o.M, o.N, o.K, 256, room, 65536, &est);
+    const any::Problem p{o.M, o.N, 4 * o.K, 4, 4, false, false, false};
+    const double there = any::other_us(any::COST_F32, p, true, 256, room);
+    if (est >= there)
       return std::printf("FAILED fp32 %lld %lld %lld: %.1f here, %.1f there\n", o.M, o.N, o.K, est, there), 1;
   }
   // and its times: one round of 160-row tiles (130 us), three of 160 rows (420)
