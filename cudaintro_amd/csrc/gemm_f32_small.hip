@@ -14,7 +14,7 @@
 // 512^3 gives 256 workgroups instead of the 16 of the 64x256 tile.  Outputs of at most 16
 // columns have a form of their own below.
 //
-// K beyond a few blocks, and few tiles, are the LDS-DMA form's (gemm_kwaves.hip, same tile, same names):
+// K beyond a few blocks, and few tiles, are the LDS-DMA form's (gemm_kwaves.hip, same tile):
 // this one has a chain of loads to wait for, that one all of a wave's in flight.
 //
 // Ragged M and N: loads past the edge re-read the last valid row / column, stores are

@@ -547,10 +547,8 @@ bool launch_kwaves_f32(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, cons
     if (!p.splits || (!rest && est >= f32_other_us(ctx, M, N, K, A, lda, B, ldb, C, ldc, ba))) return false;
   }
   kwaves::launch_f32(ctx, p, M, N, K, A, lda, B, ldb, C, ldc, ba);
-  // (one family with the register-loaded small kernel: 32 x 32 tiles, k split over four waves)
-  snprintf(ctx->kernel_name, sizeof(ctx->kernel_name), "f32_mfma_%ssmall_32x32_ksplit4%s%s",
-           f32_small_shape_ok(M, N, K, A, lda) ? "" : "any_", ba ? "_bias_act" : "",
-           ctx->last_k_splits > 1 ? "_splitk" : "");
+  snprintf(ctx->kernel_name, sizeof(ctx->kernel_name), "f32_mfma_%ssmall_kwaves_32x32x32_w4%s_splitk",
+           f32_small_shape_ok(M, N, K, A, lda) ? "" : "any_", ba ? "_bias_act" : "");
   ctx->last_kernel = ctx->kernel_name;
   return true;
 }

@@ -126,13 +126,15 @@ CIGEMM_API int cigemmGetVersion(void);
  * ring4_nk_dequant" when two launches of different tile heights covered the columns (a
  * "_splitk" after such a name: the second launch ran as K ranges plus a reduction); the kernel of
  * small outputs "<type>_mfma_[any_]kwaves_32x64x<k per piece>_w4[_kn|_nk][_dequant]_splitk" (k is
- * always split, over its four waves at least), fp32 "f32_mfma_[any_]small_32x32_ksplit4[_bias_act]
- * [_splitk]"; "+32x64" or "+32x32" behind any of these: the last few columns ran on that kernel.
+ * always split, over its four waves at least), fp32 "f32_mfma_[any_]small_kwaves_32x32x32_w4[_bias_act]
+ * _splitk" (its register-loaded sibling: "f32_mfma_[any_]small_32x32_ksplit4[_bias_act]"); "+32x64" or
+ * "+32x32" behind any of these: the last few columns ran on that kernel.
  * Valid until the next GEMM call on the handle. */
 CIGEMM_API const char* cigemmGetLastKernelName(cigemmHandle_t handle);
 
 /* Plan of the last successful GEMM call on this handle, for tests and profiles: rows of the
- * output tile (256, 192, 128 or 64; with two launches, of the second; 32 for the kernel of small
+ * output tile (256, 192, 128 or 64, fp32 also 224, 160 and 96; 32 for the kernel of small outputs; with
+ * two launches, of the second, but of the first where the last few columns ran on the kernel of small
  * outputs) and number of K ranges (one workgroup each) when the LDS-tiled matrix-core kernel or the
  * kernel of small outputs ran, 0 and 0 when another family did.  Either pointer
  * may be null.  No counterpart in the reference: cuBLAS does not report its heuristics'

@@ -255,8 +255,12 @@ def test_default_choice_by_shape(handle, torch_gpu):
     assert "x256x16_w" in kernel_for(2048, 2048, 2048)
     assert "x256x16_w" in kernel_for(4096, 4096, 64)
     assert "x256x16_w" in kernel_for(20000, 512, 784)
-    assert kernel_for(512, 512, 4096).endswith("_splitk")      # long K: tile kernel, K split
-    assert kernel_for(256, 1024, 8192).endswith("_splitk")
+    # long K: the kernel of small outputs, or tiles, K split
+    assert kernel_for(512, 512, 4096) == "f32_mfma_small_kwaves_32x32x32_w4_splitk"
+    assert kernel_for(256, 1024, 8192) == "f32_mfma_small_kwaves_32x32x32_w4_splitk"
+    assert kernel_for(77, 91, 4099) == "f32_mfma_any_small_kwaves_32x32x32_w4_splitk"
+    for shape in ((256, 4096, 4096), (128, 4096, 8192)):
+        assert re.fullmatch(r"f32_mfma_\d+x256x16_w4_ring4_splitk", kernel_for(*shape)), handle.last_kernel
     assert kernel_for(77, 91, 300) == "f32_mfma_any_small_32x32_ksplit4"
     assert re.match(r"f32_mfma_any_[0-9+]+x256x16_w4_ring4", kernel_for(2049, 2047, 1025))
 

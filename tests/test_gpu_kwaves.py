@@ -33,7 +33,7 @@ def test_kwaves(handle, torch_gpu, oracle, rng, kind):
     torch = torch_gpu
     int8 = kind.startswith("i8")
     layout = ci.B_NK if kind == "i8_nk" else ci.B_KN
-    name = "small_32x32_ksplit4" if kind == "f32" else "kwaves_32x64"
+    name = "small_kwaves_32x32x32" if kind == "f32" else "kwaves_32x64"
     host = lambda t: bits(torch, t) if t.element_size() == 2 else t.contiguous().cpu().numpy()  # noqa: E731
     for M, N, aligned in SHAPES:
         for K in sizes_of_k(BYTES[kind], aligned):
@@ -113,7 +113,10 @@ def test_replayed_from_a_graph(torch_gpu, kind, M, N, K):
         gemm = getattr(h, "gemm_" + kind)
         want, want2 = gemm(a, b), gemm(a2, b2)
         gemm(a, b)
-        assert "kwaves" in h.last_kernel or "small_32x32" in h.last_kernel or "+32x64" in h.last_kernel
+        if N > 256:
+            assert h.last_kernel.endswith("+32x64"), h.last_kernel
+        else:
+            assert "kwaves" in h.last_kernel and h.last_plan[0] == 32 and h.last_plan[1] > 1, (h.last_kernel, h.last_plan)
         out = torch.zeros_like(want)
         graph = torch.cuda.CUDAGraph()
         side.synchronize()
