@@ -128,3 +128,66 @@ def test_replayed_from_a_graph(torch_gpu, kind, M, N, K):
             assert torch.equal(gemm(a2, b2), want2)
             side.synchronize()
             assert torch.equal(out, want)
+
+
+# (M, N of 16-bit and int8, N of fp32, whole pieces of k, K ranges imposed, regime): a wave has more pieces than
+# slots, so that a slot is filled again while others are in flight; more workgroups than units, so that
+# its one slot is; more than eight ranges, which the last workgroup adds up in groups of eight.
+REGIMES = [
+    (33, 136, 72, 40, 1, "ring"), (65, 200, 136, 53, 2, "ring"),
+    (520, 1040, 1040, 9, 1, "one slot"), (520, 1040, 520, 22, 2, "one slot"), (545, 1100, 1100, 17, 1, "one slot"),
+    (64, 136, 72, 18, 9, "ranges"), (33, 72, 40, 31, 16, "ranges"), (70, 200, 104, 45, 12, "ranges"),
+]
+
+
+@pytest.mark.parametrize("M,n,n32,pieces,ranges,regime", REGIMES)
+@pytest.mark.parametrize("kind", list(BYTES))
+def test_regimes(handle, torch_gpu, rng, kind, M, n, n32, pieces, ranges, regime):
+    """Every regime is asked for by its definition (slots, pieces of a wave, ranges), with and without a tail of
+    k, aligned and off by an element.  Reference: torch in 64 bits on operands whose sums are exact in 32."""
+    torch = torch_gpu
+    int8 = kind.startswith("i8")
+    layout = ci.B_NK if kind == "i8_nk" else ci.B_KN
+    dt = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}.get(kind, torch.int8)
+    odt = torch.int32 if int8 else dt
+    units = torch.cuda.get_device_properties(0).multi_processor_count
+    stage, N, tn, max_slots = 128 // BYTES[kind], n32 if kind == "f32" else n, 32 if kind == "f32" else 64, \
+        4 if kind == "f32" else 3
+    for tail, off in ((0, 0), (0, 1), (1, 1), (stage - 1, 1), (stage // 8, 0)):
+        # (one piece less where a tail follows: `ranges` ranges of an even number of 64-byte stages)
+        K = (pieces - (tail > 0)) * stage + tail
+
+        def operand(r, c):
+            src = rng.integers(-127, 128, size=(r, c), dtype=np.int8) if int8 else rng.choice(VALS, size=(r, c))
+            ld = c + (-c % 16 if off == 0 else 3)
+            flat = torch.full((off + r * ld,), 127 if int8 else float("nan"), dtype=dt, device="cuda")
+            view = flat[off:].view(r, ld)[:, :c]
+            view.copy_(torch.from_numpy(src).cuda())
+            return view
+        a = operand(M, K)
+        b = operand(N, K) if kind == "i8_nk" else operand(K, N)
+        ref = (a.double() @ (b.t() if kind == "i8_nk" else b).double().contiguous()).to(odt)
+        ld = N + (-N % 16 if off == 0 else 3)
+        flat = torch.empty(off + M * ld, dtype=odt, device="cuda")
+        out = flat[off:].view(M, ld)[:, :N]
+        probe.force_kwaves_plan(handle, ranges)
+        try:
+            for _ in range(2):
+                flat.fill_(7)
+                if int8:
+                    handle.gemm_i8_i32(a, b, layout, out=out)
+                else:
+                    getattr(handle, "gemm_" + kind)(a, b, out=out)
+                what = f"{handle.last_kernel} {handle.last_plan} {M} {N} {K}"
+                assert "kwaves_32x" in handle.last_kernel and handle.last_plan[0] == 32, what
+                got = handle.last_plan[1]
+                workgroups = -(-M // 32) * -(-N // tn) * got
+                of_a_wave = -(-(-(-K // stage) // got) // 4)
+                assert {"ring": workgroups <= units and of_a_wave > max_slots,
+                        "one slot": workgroups > units and of_a_wave > 1,
+                        "ranges": got > 8 and got == ranges}[regime], (what, workgroups, of_a_wave)
+                assert torch.equal(out, ref), what
+                out.fill_(7)
+                assert bool((flat == 7).all()), what
+        finally:
+            probe.force_kwaves_plan(handle, 0)
