@@ -29,12 +29,21 @@ inline bool fits(int64_t M, int64_t N, Plan p, size_t partial_bytes, size_t coun
 // that unit; pieces the address path takes apart, operand bytes, and for K ranges their meeting and
 // the bytes of their sums.  Fitted to the kernel timed at 320 sizes of each layout (M 17..3000, N and
 // K 64..16384, log-uniform, 40 % of the widths odd) x up to 8 numbers of ranges; rms error 9..12 %.
+// Long streams of k, where that is too low: the estimate has to win by 30 % (N x K) or 10 % (K x N) there.
+// N x K: 65 to 768 columns whose k is no whole pieces, once a unit takes more than 8000 bytes of k for all
+// of its workgroups (787 x 392 x 15048 29.8 us here, 22.1 on the tile kernel; 8748 x 72 x 6000 35.4 and
+// 26.5; with whole pieces 387 x 1066 x 12416 16.7 and 20.8).  K x N: rows of more than 128 bytes, ranges of more
+// than `long_range` bytes that at least half of the units have (bf16 904 x 276 x 3896 17.6 and 14.1, 757 x
+// 570 x 3856 18.3 and 15.9; of narrower outputs int8 3615 x 99 x 5552 16.2 and 20.3).  Of 11468 random
+// sizes taken before, most of them with 120..768 tiles, 637 were more than 3 % slower here than without
+// this kernel, 195 of those taken now; 56 that were more than 3 % faster are taken no longer.
 struct Cost {
   double start, unit_piece, load, unit_tile, apart, in_mb, split, part_mb, tail, dequant;
+  double long_range;  // bytes; 0: N x K
 };
-constexpr Cost COST_16{3.95, 0.0849, 0.0562, 0.0155, 0.0202, 0.0664, 1.46, 0.130, 1.05, 0.0};
-constexpr Cost COST_I8_KN{4.31, 0.0907, 0.103, 0.0, 0.0342, 0.0608, 1.32, 0.0941, 0.365, 0.692};
-constexpr Cost COST_I8_NK{4.47, 0.0708, 0.0599, 0.0990, 0.0299, 0.0759, 1.09, 0.163, 0.552, 0.717};
+constexpr Cost COST_16{3.95, 0.0849, 0.0562, 0.0155, 0.0202, 0.0664, 1.46, 0.130, 1.05, 0.0, 7000};
+constexpr Cost COST_I8_KN{4.31, 0.0907, 0.103, 0.0, 0.0342, 0.0608, 1.32, 0.0941, 0.365, 0.692, 5000};
+constexpr Cost COST_I8_NK{4.47, 0.0708, 0.0599, 0.0990, 0.0299, 0.0759, 1.09, 0.163, 0.552, 0.717, 0};
 
 // `whole`: no tail (k and the rows of a K x N operand are whole pieces)
 inline double us(const Cost& c, const any::Problem& p, bool whole, int cus, int splits) {
@@ -78,6 +87,14 @@ inline Plan choose(const Cost& c, const any::Cost& other, const any::Problem& p,
   const Plan b = best(c, p, whole, cus, partial_bytes, counter_bytes, &est);
   // (beyond one round the two estimates have to differ by more than they usually err)
   if (tiles > cus) est *= 1.1;
+  int64_t stages = 0;
+  const int sp = tile::k_ranges(p.K_bytes, b.splits, &stages);
+  const double range = (double)p.K_bytes / sp;
+  if (c.long_range > 0) {
+    if (p.N * p.elem > PB && 2 * tiles > cus && range > c.long_range) est *= 1.1;
+  } else if (!whole && p.N > TN && p.N <= 768 && (double)any::div_up(tiles * sp, cus) * range > 8000.0) {
+    est *= 1.3;
+  }
   return est < any::other_us(other, p, aligned, cus, partial_bytes) ? b : Plan{0};
 }
 

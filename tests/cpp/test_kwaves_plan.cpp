@@ -94,6 +94,25 @@ int main() {
     if (us < 0.93 * o.us || us > 1.07 * o.us)
       return std::printf("FAILED fp32 %lld %lld %lld: %.1f us\n", o.M, o.N, o.K, us), 1;
   }
+  // 16-bit and int8: long streams of k that the tile kernel is the faster for, and some that stay here
+  const struct { int elem; bool nk; long long M, N, K; double here, there; } streams[] = {
+      {1, true, 787, 392, 15048, 29.8, 22.1}, {1, true, 8672, 128, 6088, 36.2, 27.6},
+      {1, true, 2234, 144, 12464, 25.4, 19.4}, {2, false, 904, 276, 3896, 17.6, 14.1},
+      {2, false, 1337, 232, 3944, 17.9, 15.0}, {2, false, 757, 570, 3856, 18.3, 15.9},
+      {1, false, 77, 3112, 5408, 16.3, 14.0},
+      {2, false, 50, 7648, 3264, 12.5, 16.0}, {2, false, 112, 3776, 2888, 11.6, 14.0}, {1, true, 285, 4384, 3200, 14.2, 18.7},
+      {1, true, 61, 9352, 4096, 12.4, 15.6}};
+  for (const auto& o : streams) {
+    const any::Problem p{o.M, o.N, o.K * o.elem, o.elem, o.elem == 2 ? 2 : 4, false, false, false};
+    const bool whole = p.K_bytes % 128 == 0 && (o.nk || o.N * o.elem % 16 == 0);
+    const bool aligned = p.K_bytes % 16 == 0 && o.N * (o.nk ? p.out_bytes : o.elem) % 16 == 0;
+    const kwaves::Cost& c =
+        o.elem == 2 ? kwaves::COST_16 : o.nk ? kwaves::COST_I8_NK : kwaves::COST_I8_KN;
+    const any::Cost& other = o.elem == 2 ? any::COST_16 : o.nk ? any::COST_I8_NK : any::COST_I8_KN;
+    const bool taken_here = kwaves::choose(c, other, p, whole, aligned, 256, room, 65536).splits > 0;
+    if (taken_here != (o.here < o.there))
+      return std::printf("FAILED %lld x %lld x %lld: %.1f us here, %.1f there\n", o.M, o.N, o.K, o.here, o.there), 1;
+  }
   if (taken < 100 || refused < 100) return std::printf("FAILED: %d taken, %d refused\n", taken, refused), 1;
   std::printf("kwaves plan OK\n");
   return 0;
