@@ -142,14 +142,14 @@ inline Plan best_f32(int64_t M, int64_t N, int64_t K, int cus, size_t partial_by
     if (t < *est) *est = t, b = Plan{(int)sp};
   }
   // Where the estimate is too low, it has to be below the other by more.  Row tiles that share a B beyond
-  // what the L2s keep: 20 % from 128 MB of operands on (36 x 5016 x 7040 estimated 46 us, took 60; 45 on
-  // the tile kernel).  Four to seven workgroups a unit, of which three are resident: 12 % (467 x 768 x 7936
+  // what the L2s keep: 20 % from 128 MB of it on (36 x 5016 x 7040 estimated 46 us, took 60; 45 on the
+  // tile kernel; a long A is no such stream: 15963 x 8 x 1146 16.7 us here, 22.4 register-loaded).  Four to seven workgroups a unit, of which three are resident: 12 % (467 x 768 x 7936
   // 64 us, tile kernel 56), but for outputs of up to 128 columns, which the other kernels pad (7250 x 64 x
   // 5935 76 us here, 115 there).  Beyond a round and a half: 12 % (127 x 7360 x 4032 79 and 70, estimated
   // equal).  Of 1094 sizes around these lines that were taken before, 313 were more than 3 % slower here
   // than on the other kernels (the worst 29 %), 38 of those taken now; the choice is 0.6 % off the faster
   // kernel on average, 3.9 % before.
-  const double mb = (double)(M + N) * (double)K_bytes * 1e-6;
+  const double mb = (double)N * (double)K_bytes * 1e-6;
   if (M > TM && mb > 48.0) *est *= 1.0 + 0.2 * any::at_most((mb - 48.0) / 80.0, 1.0);
   if (tiles * b.splits > 4 * (int64_t)cus && tiles * b.splits <= 7 * (int64_t)cus && N > 128) *est *= 1.12;
   if (2 * tiles > 3 * (int64_t)cus) *est *= 1.12;

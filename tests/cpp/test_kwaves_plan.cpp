@@ -77,7 +77,8 @@ int main() {
   }
   // while these stay here
   const struct { long long M, N, K; double here, there; } kept[] = {
-      {42, 6144, 2816, 22.9, 26.4}, {1, 5120, 7472, 39.1, 44.6}, {17, 9216, 3776, 38.5, 40.5}, {95, 896, 1344, 7.8, 17.1}};
+      {42, 6144, 2816, 22.9, 26.4}, {1, 5120, 7472, 39.1, 44.6}, {17, 9216, 3776, 38.5, 40.5}, {95, 896, 1344, 7.8, 17.1},
+      {1995, 352, 12280, 185.1, 206.3}, {1708, 344, 13816, 191.2, 204.6}};  // (the long stream is A)
   for (const auto& o : kept) {
     double est = 0;
     kwaves::best_f32(o.M, o.N, o.K, 256, room, 65536, &est);
