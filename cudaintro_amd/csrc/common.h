@@ -264,8 +264,8 @@ bool launch_kwaves_f32(cigemmContext*, int64_t M, int64_t N, int64_t K, const fl
 bool launch_kwaves_i8(cigemmContext*, int64_t M, int64_t N, int64_t K, const int8_t* A, int64_t lda,
                       const int8_t* B, int64_t ldb, bool b_nk, int32_t* C, int64_t ldc,
                       const DequantArgs* dq, bool rest = false);
-// Columns of the full rounds of 256-row tiles where those and a few columns more (at most 64, on 32-row
-// tiles) cover the output best; 0: no such plan.
+// Columns of the full rounds of 256-row tiles where the tile kernel would run the rest, at most 64 columns,
+// as a launch of its own: those are the kernel of small outputs'; 0: no such plan.
 int64_t kwaves_rest_columns(const cigemmContext*, int64_t M, int64_t N, int64_t K_bytes, bool f32);
 // the kernel's name after such a pair of calls: "<first>+<tile of the rest>"
 void name_rest_columns(cigemmContext*, const char* first);

@@ -4,14 +4,14 @@
 // from its L2 while most of the others have nothing to do (about 100 KB per us), and, where K is cut,
 // the meeting of the ranges.  A 64 x 256 tile of mfma_tile.h makes one unit fetch 320 rows of K; here
 // it fetches 96, on four to eight times as many units, and the ranges meet inside the kernel.  us a
-// call, there -> here: bf16 33 x 250 x 333 6.98 -> 5.83 (the host's own pace), 52 x 64 x 2048 9.0 ->
+// call, there -> here: bf16 33 x 250 x 333 7.0 -> 5.3..6.0 (the host's own pace), 52 x 64 x 2048 9.0 ->
 // 6.5, 48 x 4096 x 3776 13.6 -> 10.5, 678 x 128 x 6284 13.9 -> 9.5; int8 N x K 365 x 96 x 853 13.6 ->
-// 6.0, K x N 1066 x 320 x 3264 13.3 -> 9.8, 107 x 6208 x 2576 15.7 -> 13.0; the 341 of 760 random sizes
-// that came here (M 1..40000, N 16..16384, K 64..16384) 1.33 times as fast (geometric mean), 4 of them
-// 3..6 % slower.  fp32 (against the tile kernel and the register-loaded small kernel): 95 x 896 x 1344
-// 17.1 -> 7.8, 22 x 19 x 7616 24.2 -> 8.4, 5812 x 8 x 5568 149 -> 28.6; of 350 random sizes the 163 that
-// came here 1.91 times as fast, one 11 % slower; the error against 64 bits 1.71e-7 from 2.01e-7
-// (geometric mean over 112 products), at most 3.8e-7 from 6.1e-7.
+// 6.0, K x N 1066 x 320 x 3264 13.3 -> 9.8, 107 x 6208 x 2576 15.7 -> 13.0; 3080 random calls that came
+// here (M 17..40000, N 8..16384, K 64..16384) 1.45 times as fast (geometric mean of the kernels inside a
+// graph), 18 of them more than 3 % slower, the worst 16 %.  fp32 (against the tile kernel and the
+// register-loaded small kernel): 95 x 896 x 1344 17.1 -> 7.8, 22 x 19 x 7616 24.2 -> 8.4, 5812 x 8 x 5568
+// 149 -> 28.6; of 5072 calls that came here 53 more than 3 % slower, the worst 27 %; the error against 64
+// bits 1.71e-7 from 2.01e-7 (geometric mean over 112 products), at most 3.8e-7 from 6.1e-7.
 //
 // Workgroup = 256 lanes = 4 waves.  Wave w takes the 128-byte pieces w, w + 4, ... of k (64 halves,
 // 128 int8, 32 floats), each through its own LDS slots -- no barrier before the waves' sums meet --:

@@ -258,11 +258,11 @@ inline int best_rows32(int64_t M, int64_t N, int cus, TileUnits u, double* cost)
 // (4095 x 4097 x 4099: 17th column of tiles 63 us + 5 for the reduction, a quarter of a 64-row round
 // is 60).  us before -> here: 20000 x 512 x 784 143.5 (210 tiles of 192 rows) -> 130.3 (250 of 160, one
 // round), 3000^3 503 (192) -> 422 (160), 7000 x 4096 x 4096 1604 (64) -> 1588 (224).
-// A second launch of more than 64 columns costs 0.35 units and 1 us beside its tiles (its ramp, its
-// epilogue, the units that wait for the first one's last tiles; below K = 64, where nothing was timed,
-// 0.48 units): 136 sizes where both plans were timed, K 64..4096, against the faster plan of each: 0.13 % slower on average, without that
-// price 2.6 % (2111 x 8128 x 192 74.5 us in two launches, 65.5 in one of 96-row tiles; 2609 x 8160 x 64
-// 47.6 and 43.9; 3188 x 7040 x 192 89.0 and 85.4).  Up to 64 columns end sooner, here or in
+// A second launch of more than 64 columns costs 0.35 units and 1 us beside its tiles: its ramp, its epilogue,
+// the units that wait for the first one's last tiles (0.48 units below K = 64, where nothing was timed).
+// 136 sizes where both plans were timed, K 64..4096, against the faster plan of each: 0.13 % slower on
+// average, without that price 2.6 % (2111 x 8128 x 192 74.5 us in two launches, 65.5 in one of 96-row tiles;
+// 2609 x 8160 x 64 47.6 and 43.9; 3188 x 7040 x 192 89.0 and 85.4).  Up to 64 columns end sooner, here or in
 // kwaves_rest_columns.
 inline RoundsPlan plan_rounds32(int64_t M, int64_t N, int64_t K_bytes, int cus, int* rows) {
   constexpr TileUnits u = TILE_UNITS_F32;
