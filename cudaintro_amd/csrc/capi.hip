@@ -94,6 +94,8 @@ cigemmStatus_t cigemmCreate(cigemmHandle_t* handle) {
   ctx->force_tile_splits = 0;
   ctx->force_kwaves = 0;
   ctx->force_any_kernel = ANY_BY_SHAPE;
+  ctx->force_split_rows = 0;
+  ctx->force_split_ranges = 0;
   ctx->workspace = nullptr;
   if (hipMalloc(&ctx->workspace,
                 ctx->ws_partial_bytes + ctx->ws_counter_bytes + ctx->ws_swap_bytes) != hipSuccess ||
@@ -296,7 +298,8 @@ static bool dispatch_f32(cigemmHandle_t h, int64_t M, int64_t N, int64_t K, cons
       launch_generic_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba);
       return true;
     default:
-      if (!launch_kwaves_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba) &&
+      if (!launch_f32_split(h, M, N, K, A, lda, B, ldb, C, ldc, ba) &&
+          !launch_kwaves_f32(h, M, N, K, A, lda, B, ldb, C, ldc, ba) &&
           !rest_columns(
               h, M, N, K * 4, true,
               [&](int64_t n1) {

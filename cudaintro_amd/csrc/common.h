@@ -51,6 +51,10 @@ struct cigemmContext {
   // Test aid, set through the probe library only: which kernel serves a call that
   // CIGEMM_ALGO_MFMA_ANY selects: AnyKernel.
   int force_any_kernel;
+  // The same for the fp32 tiles on the bf16 matrix instructions: rows and K ranges imposed on every call
+  // they take, -1 keeps them out of every call, 0 = the library chooses.
+  int force_split_rows;
+  int force_split_ranges;
   char last_error[256];
 };
 
@@ -282,13 +286,24 @@ void launch_generic_i8(cigemmContext*, int64_t M, int64_t N, int64_t K, const in
 bool launch_f32_tile(cigemmContext*, int64_t M, int64_t N, int64_t K, const float* A,
                      int64_t lda, const float* B, int64_t ldb, float* C, int64_t ldc,
                      const BiasAct* ba = nullptr);
-// what the call is estimated to take on the kernel that DEFAULT would choose without gemm_kwaves.hip
-double f32_other_us(const cigemmContext*, int64_t M, int64_t N, int64_t K, const float* A,
-                    int64_t lda, const float* B, int64_t ldb, const float* C, int64_t ldc,
-                    const BiasAct* ba);
+// What the call is estimated to take on the kernel that DEFAULT would choose without gemm_kwaves.hip and
+// gemm_f32_split.hip, and the longest sum of k that kernel adds up in a row.
+struct F32Other {
+  double us;
+  int64_t sum_length;
+};
+F32Other f32_other(const cigemmContext*, int64_t M, int64_t N, int64_t K, const float* A,
+                   int64_t lda, const float* B, int64_t ldb, const float* C, int64_t ldc,
+                   const BiasAct* ba);
+bool f32_tile_ok(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, const float* B, int64_t ldb,
+                 const float* C, int64_t ldc, const BiasAct* ba);
 bool launch_f32_mfma(cigemmContext*, int64_t M, int64_t N, int64_t K, const float* A,
                      int64_t lda, const float* B, int64_t ldb, float* C, int64_t ldc,
                      const BiasAct* ba = nullptr);
+// gemm_f32_split.hip: 256-column tiles on the bf16 matrix instructions.  False without launching where
+// the call is not theirs, or another kernel is estimated to be as fast.
+bool launch_f32_split(cigemmContext*, int64_t M, int64_t N, int64_t K, const float* A, int64_t lda,
+                      const float* B, int64_t ldb, float* C, int64_t ldc, const BiasAct* ba);
 // gemm_f32_small.hip: 32x32 tile per workgroup, k split over the waves.
 bool f32_small_shape_ok(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda);
 // any K, any alignment of A: the sizes alone

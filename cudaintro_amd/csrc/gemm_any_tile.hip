@@ -63,7 +63,7 @@ bool launch_tile_any_f32(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, co
                EpiBiasActAnyF32x4{C, ldc, ba->bias, ba->relu}, plan)
          : tile::launch_tile<tile::MathF32, tile::B_KN32, true>(ctx, M, N, K * 4, A, lda * 4, B,
                                                                 ldb * 4, EpiStoreF32x4{C, ldc}, plan);
-  set_tile_kernel_name(ctx, "f32", 16, ba ? "_bias_act" : "", split, true);
+  set_tile_kernel_name(ctx, "f32", 16, ba ? "_32x32x2_bias_act" : "_32x32x2", split, true);
   return true;
 }
 

@@ -8,7 +8,7 @@
 
 namespace cig {
 
-static bool f32_tile_ok(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda,
+bool f32_tile_ok(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda,
                         const float* B, int64_t ldb, const float* C, int64_t ldc,
                         const BiasAct* ba) {
   return tile::tile_shape_ok(M, N, K, 4, A, lda, B, ldb, true) && ldc % 4 == 0 &&
@@ -67,22 +67,31 @@ bool launch_f32_mfma(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const 
   return true;
 }
 
-double f32_other_us(const cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const float* A,
-                    int64_t lda, const float* B, int64_t ldb, const float* C, int64_t ldc,
-                    const BiasAct* ba) {
+F32Other f32_other(const cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const float* A,
+                   int64_t lda, const float* B, int64_t ldb, const float* C, int64_t ldc,
+                   const BiasAct* ba) {
   const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
   const size_t room = ctx->workspace ? ctx->ws_partial_bytes : 0;
   const any::Problem p{M, N, K * 4, 4, 4, false, false, false};
-  const double small =
+  const F32Other small{
       f32_small_any_ok(M, N, K) ? any::f32_small_us(M, N, K, cus, f32_small_b16(N, B, ldb),
                                                     f32_small_is_narrow(M, N, K, A, lda))
-                                : 1e30;
-  if (f32_tile_ok(M, N, K, A, lda, B, ldb, C, ldc, ba))
-    return aligned_is_small(ctx, M, N, K, A, lda, B, ldb)
-               ? small
-               : any::other_us(any::COST_F32, p, true, cus, room);
-  const double other = any::other_us(any::COST_F32, p, false, cus, room);
-  return small < other ? small : other;
+                                : 1e30,
+      any::div_up(K, 4)};
+  if (f32_tile_ok(M, N, K, A, lda, B, ldb, C, ldc, ba)) {
+    if (aligned_is_small(ctx, M, N, K, A, lda, B, ldb)) return small;
+    tile::SmallPlan plan{0, 1};
+    if (any::div_up(M, tile::BM) * any::div_up(N, tile::BN) <= cus)
+      plan = tile::plan_small(cus, room, M, N, K * 4, 4, any::COST_F32.sc, K * 4 * N);
+    return F32Other{any::tile_us(any::COST_F32, p, cus, room, plan), K / plan.splits};
+  }
+  const tile::SmallPlan plan = any::tile_plan(any::COST_F32, p, cus, room);
+  const double tile = any::tile_us(any::COST_F32, p, cus, room, plan);
+  const double staged = any::staged_us(any::COST_F32, p, cus, room);
+  int64_t steps = 0;
+  const F32Other other = staged < tile ? F32Other{staged, K / any::staged_ranges(p, cus, room, &steps)}
+                                       : F32Other{tile, K / plan.splits};
+  return small.us < other.us ? small : other;
 }
 
 bool launch_f32_tile(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const float* A,
@@ -92,7 +101,7 @@ bool launch_f32_tile(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const 
   if (!ba) {
     const bool split = tile::launch_tile<tile::MathF32, tile::B_KN32>(
         ctx, M, N, K * 4, A, lda * 4, B, ldb * 4, EpiStoreF32x4{C, ldc});
-    set_tile_kernel_name(ctx, "f32", 16, "", split);
+    set_tile_kernel_name(ctx, "f32", 16, "_32x32x2", split);
     return true;
   }
   bool split = false;
@@ -105,7 +114,7 @@ bool launch_f32_tile(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const 
     if (ba->relu) CIG_BA(false, true); else CIG_BA(false, false);
   }
 #undef CIG_BA
-  set_tile_kernel_name(ctx, "f32", 16, "_bias_act", split);
+  set_tile_kernel_name(ctx, "f32", 16, "_32x32x2_bias_act", split);
   return true;
 }
 

@@ -544,7 +544,7 @@ bool launch_kwaves_f32(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, cons
     double est = 0;
     p = kwaves::best_f32(M, N, K, ctx->num_cus > 0 ? ctx->num_cus : 256, room, ctx->ws_counter_bytes,
                          &est);
-    if (!p.splits || (!rest && est >= f32_other_us(ctx, M, N, K, A, lda, B, ldb, C, ldc, ba))) return false;
+    if (!p.splits || (!rest && est >= f32_other(ctx, M, N, K, A, lda, B, ldb, C, ldc, ba).us)) return false;
   }
   kwaves::launch_f32(ctx, p, M, N, K, A, lda, B, ldb, C, ldc, ba);
   snprintf(ctx->kernel_name, sizeof(ctx->kernel_name), "f32_mfma_%ssmall_kwaves_32x32x32_w4%s_splitk",

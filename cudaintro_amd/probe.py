@@ -33,6 +33,7 @@ SIGNATURES = {
     "cigemm_probe_force_tile_plan": (_ci, [_vp, _ci, _ci]),
     "cigemm_probe_force_kwaves_plan": (_ci, [_vp, _ci]),
     "cigemm_probe_force_any_kernel": (_ci, [_vp, _ci]),
+    "cigemm_probe_force_f32_split": (_ci, [_vp, _ci, _ci]),
 }
 
 
@@ -174,6 +175,13 @@ def force_kwaves_plan(h: Handle, k_ranges: int):
     hands the choice back."""
     _check(h, load_library().cigemm_probe_force_kwaves_plan(h.raw, k_ranges),
            "cigemm_probe_force_kwaves_plan")
+
+
+def force_f32_split(h: Handle, tile_rows: int, k_ranges: int = 1):
+    """The same for the fp32 tiles on the bf16 matrix instructions; tile_rows = -1 keeps them out of the
+    handle's calls, 0 hands the choice back."""
+    _check(h, load_library().cigemm_probe_force_f32_split(h.raw, tile_rows, k_ranges),
+           "cigemm_probe_force_f32_split")
 
 
 ANY_BY_SHAPE, ANY_REGISTER_STAGED, ANY_F32_SMALL, ANY_TILE = 0, 1, 2, 3

@@ -1,0 +1,181 @@
+"""fp32 tiles on the bf16 matrix instructions (every operand as the exact sum of three bf16 numbers): each
+height with one and several K ranges at the edges of tiles, stages and column pairs, operands whose second
+and third parts matter, and what the three parts cannot hold (infinities, NaN, the largest and the smallest
+magnitudes), which the kernel computes once more in fp32.  NaN padding around the operands, the output in
+a sentinel-filled buffer."""
+import numpy as np
+import pytest
+
+import cudaintro_amd as ci
+from cudaintro_amd import probe
+from test_gpu_mfma_any import embed
+
+pytestmark = pytest.mark.gpu
+
+ROWS = (64, 96, 128, 160, 192, 224, 256)
+
+
+@pytest.fixture(autouse=True)
+def hand_back(handle):
+    yield
+    probe.force_f32_split(handle, 0)
+
+
+def run(handle, torch, A, B, rows, ranges, off, pad, bias=None):
+    """The product (or the layer with ReLU) on embedded operands; checks the guard around the output."""
+    M, N = A.shape[0], B.shape[1]
+    _, a = embed(torch, A, torch.float32, off, pad, float("nan"))
+    _, b = embed(torch, B, torch.float32, off, pad, float("nan"))
+    flat, out = embed(torch, np.zeros((M, N), np.float32), torch.float32, off, pad, 0)
+    probe.force_f32_split(handle, rows, ranges)
+    flat.fill_(7)
+    if bias is None:
+        handle.gemm_f32(a, b, out=out)
+    else:
+        handle.linear_f32(a, b, torch.from_numpy(bias).cuda(), ci.ACT_RELU, out=out)
+    what = f"{handle.last_kernel} {M}x{N}x{A.shape[1]} ranges {ranges}"
+    assert f"{rows}x256x16_w4" in handle.last_kernel and "32x32x2" not in handle.last_kernel, what
+    got = out.cpu().numpy().copy()
+    out.fill_(7)
+    assert bool((flat == 7).all()), what
+    return got, what
+
+
+@pytest.mark.parametrize("rows", ROWS)
+def test_exact_sums(handle, torch_gpu, rng, rows):
+    """Integers of 12 bits times small ones: two parts of one operand, every sum exact."""
+    for M in (1, rows - 1, rows + 33):
+        for N in (2, 255, 257, 258, 300):
+            for K in (17, 31, 32, 33, 48, 49, 113, 160, 400):
+                wide = rng.integers(-2048, 2049, size=(M, K)).astype(np.float32)
+                small = rng.integers(-2, 3, size=(K, N)).astype(np.float32)
+                off, pad = (0, 4) if K % 2 == 0 else (1, 3)
+                for ranges in (1, 3):
+                    got, what = run(handle, torch_gpu, wide, small, rows, ranges, off, pad)
+                    np.testing.assert_array_equal(got, wide.astype(np.float64) @ small, err_msg=what)
+                small, wide = (rng.integers(-2, 3, size=(M, K)).astype(np.float32),
+                               rng.integers(-2048, 2049, size=(K, N)).astype(np.float32))
+                bias = rng.integers(-9, 9, size=N).astype(np.float32)
+                got, what = run(handle, torch_gpu, small, wide, rows, 1, off, pad, bias)
+                np.testing.assert_array_equal(got, np.maximum(small.astype(np.float64) @ wide + bias, 0), err_msg=what)
+
+
+@pytest.mark.parametrize("rows", ROWS)
+def test_one_hot_operands_select_all_24_bits(handle, torch_gpu, rng, rows):
+    M, N, K = rows + 5, 267, 93
+    X = rng.normal(size=(M, K)).astype(np.float32)
+    take = rng.integers(0, K, size=N)
+    W = np.zeros((K, N), np.float32)
+    W[take, np.arange(N)] = 1
+    got, what = run(handle, torch_gpu, X, W, rows, 1, 1, 3)
+    np.testing.assert_array_equal(got, X[:, take], err_msg=what)
+    Y = rng.normal(size=(K, N)).astype(np.float32)
+    take = rng.integers(0, K, size=M)
+    S = np.zeros((M, K), np.float32)
+    S[np.arange(M), take] = 1
+    got, what = run(handle, torch_gpu, S, Y, rows, 2, 0, 4)
+    np.testing.assert_array_equal(got, Y[take], err_msg=what)
+
+
+@pytest.mark.parametrize("rows", ROWS)
+@pytest.mark.parametrize("kind", ["symmetric", "positive", "wide"])
+def test_no_further_from_64_bits_than_the_fp32_instructions(handle, torch_gpu, rng, rows, kind):
+    """The same call on the tiles of v_mfma_f32_32x32x2_f32 is the measure, error by sum of magnitudes, over
+    131072 outputs; 1 % for the draw."""
+    torch = torch_gpu
+    M, N = 256, 512
+    for K in (64, 700, 4096):
+        draw = {"symmetric": lambda s: rng.uniform(-1, 1, s), "positive": lambda s: rng.uniform(0, 1, s),
+                "wide": lambda s: rng.normal(size=s) * np.exp(3 * rng.normal(size=s))}[kind]
+        A, B = draw((M, K)).astype(np.float32), draw((K, N)).astype(np.float32)
+        ref = A.astype(np.float64) @ B.astype(np.float64)
+        got, what = run(handle, torch, A, B, rows, 1, 0, 0)
+        probe.force_f32_split(handle, 0)
+        probe.force_tile_plan(handle, 256, 1)
+        try:
+            with handle.algo(ci.ALGO_TILE):
+                old = handle.gemm_f32(torch.from_numpy(A).cuda(), torch.from_numpy(B).cuda()).cpu().numpy()
+                assert "32x32x2" in handle.last_kernel
+        finally:
+            probe.force_tile_plan(handle, 0)
+        size = np.abs(A.astype(np.float64)) @ np.abs(B.astype(np.float64))
+        err, err_old = np.linalg.norm((got - ref) / size), np.linalg.norm((old - ref) / size)
+        assert err <= 1.01 * err_old, (what, err / err_old)
+
+
+@pytest.mark.parametrize("rows", ROWS)
+def test_infinities_nan_and_extreme_magnitudes(handle, torch_gpu, rng, rows):
+    """One value in the last row / column block of A or B, everything else ordinary: the rows and columns
+    it reaches are those of float64 rounded to fp32, NaN and the sign of infinity included."""
+    M, N, K = rows + 3, 270, 75
+    big = np.float32(np.finfo(np.float32).max)
+    for value in (np.inf, -np.inf, np.nan, big, -big, np.float32(2.0 ** -120), np.float32(2.0 ** -145)):
+        for where in ("A", "B"):
+            A = rng.choice([-1.0, 0.5, 1.0], size=(M, K)).astype(np.float32)
+            B = rng.choice([-1.0, 0.5, 1.0], size=(K, N)).astype(np.float32)
+            if abs(value) < 1:      # alone in its row (column), so that nothing larger hides it
+                if where == "A":
+                    A[M - 1] = 0
+                else:
+                    B[:, N - 1] = 0
+            if where == "A":
+                A[M - 1, 40] = value
+            else:
+                B[40, N - 1] = value
+            for ranges in (1, 2):
+                got, what = run(handle, torch_gpu, A, B, rows, ranges, 0, 0)
+                with np.errstate(all="ignore"):
+                    ref = (A.astype(np.float64) @ B.astype(np.float64)).astype(np.float32)
+                np.testing.assert_allclose(got, ref, rtol=2e-6, atol=0, err_msg=f"{what} {value} in {where}")
+
+
+def test_tiny_values_anywhere_are_not_lost(handle, torch_gpu, rng):
+    """Rows of subnormal size times large columns: relative precision as of ordinary values."""
+    M, N, K = 200, 300, 130
+    A = (rng.uniform(0.5, 1, size=(M, K)) * 2.0 ** -122).astype(np.float32)
+    B = (rng.uniform(0.5, 1, size=(K, N)) * 2.0 ** 100).astype(np.float32)
+    ref = A.astype(np.float64) @ B.astype(np.float64)
+    for rows in (64, 160, 256):
+        got, what = run(handle, torch_gpu, A, B, rows, 1, 0, 0)
+        np.testing.assert_allclose(got, ref, rtol=1e-6, err_msg=what)
+
+
+def test_default_takes_it_where_it_pays_and_graphs_replay(handle, torch_gpu, rng):
+    """The library's own choice on a size of two launches, one of K ranges and one with the remaining column
+    on the kernel of small outputs, recorded and replayed with other work between."""
+    torch = torch_gpu
+    sizes = ((1142, 2560, 661), (152, 4096, 2208), (1030, 2817, 515))
+    ops = [(torch.rand((M, K), device="cuda") - 0.5, torch.rand((K, N), device="cuda") - 0.5,
+            torch.empty((M, N), device="cuda")) for M, N, K in sizes]
+    side = torch.cuda.Stream()
+    h = ci.Handle(stream=side)
+
+    def sequence():
+        names = []
+        for a, b, out in ops:
+            h.gemm_f32(a, b, out=out)
+            names.append(h.last_kernel)
+        return names
+
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        names = sequence()
+    side.synchronize()
+    assert all("x256x16_w4" in n and "32x32x2" not in n for n in names), names
+    eager = [o[2].clone() for o in ops]
+    for (a, b, _), got in zip(ops, eager):
+        ref = a.double() @ b.double()
+        assert float((got - ref).abs().max()) <= 1e-5 * float(ref.pow(2).mean().sqrt()) * 4
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        sequence()
+    for _ in range(3):
+        for o in ops:
+            o[2].fill_(float("nan"))
+        handle.gemm_f32(ops[1][0], ops[1][1])
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for o, e in zip(ops, eager):
+            assert torch.equal(o[2], e)
+    h.close()
