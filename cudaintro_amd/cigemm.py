@@ -117,6 +117,34 @@ def _torch():
     return torch
 
 
+_entries = None
+
+
+def _native():
+    """The binding of the hot calls in native code (``csrc/binding.cpp``), built beside the library."""
+    _torch()  # (it is linked against torch's own libraries)
+    try:
+        from . import _binding
+    except ImportError as e:
+        raise FileNotFoundError(f"{os.path.join(_HERE, '_binding.so')} is not built or does not load ({e}); run "
+                                "`python -c 'import __graft_entry__ as g; g.build()'`") from e
+    return _binding
+
+
+def _native_entries():
+    """The attributes of a :class:`Handle` that its hot calls use: the binding's functions (``_n_``) and the
+    library's entry points as addresses (``_p_``); looked up once."""
+    global _entries
+    if _entries is None:
+        native, lib = _native(), load_library()
+        _entries = {f"_n_{name}": getattr(native, name)
+                    for name in ("gemm", "linear_f32", "gemm_i8_i32", "gemm_i8_dequant", "quantize_rows_i8")}
+        for name in ("gemm_f32", "gemm_f16", "gemm_bf16", "linear_f32", "gemm_i8_i32", "gemm_i8_dequant",
+                     "quantize_rows_i8"):
+            _entries[f"_p_{name}"] = C.cast(getattr(lib, f"cigemm_{name}"), _vp).value
+    return _entries
+
+
 def gemm_bf16_static(A, B, out=None, stream=None):
     """``cigemm_gemm_bf16_static``: the decode-shape bf16 GEMM without a handle and without any
     allocation inside the library (``out`` is allocated here, by torch, when not given)."""
@@ -162,12 +190,15 @@ class Handle:
                                                       torch.int8)
         s = torch.cuda.current_stream() if stream is None else stream
         self.set_stream(s.cuda_stream)
+        self._address = h.value  # the handle, for the native binding
+        self.__dict__.update(_native_entries())
 
     # -- plumbing ---------------------------------------------------------------------------
     def close(self):
         if getattr(self, "_h", None):
             self.lib.cigemmDestroy(self._h)
             self._h = None
+            self._address = 0  # (a null handle: the library answers NOT_INITIALIZED)
 
     def __del__(self):
         try:
@@ -237,27 +268,38 @@ class Handle:
     def _ld(t):
         return _mat(t)[2]
 
-    # A small product takes as long as the host needs to issue it (fp32 512^3: 6.55 us a call, 5.80
-    # since), so each call asks a tensor for its shape, strides and address once and looks nothing
-    # else up.
+    # A small product takes as long as the host needs to issue it, so a call with its output given goes
+    # through the native binding (us a call at the host's pace, in Python -> there: fp32 3 x 277 x 64
+    # 5.1 -> 2.9, bf16 33 x 250 x 333 5.6 -> 3.1, quantizer and int8 product 2 x 5376 x 128 10.4 -> 5.7); what that does not
+    # take (-1) and calls that allocate are done here.
     def _gemm(self, fn, name, A, B, out, out_dtype):
         M, K, lda = _mat(A)
         K2, N, ldb = _mat(B)
         assert K == K2
         if out is None:
             out = _torch().empty((M, N), dtype=out_dtype, device=A.device)
-        st = fn(self._h, M, N, K, A.data_ptr(), lda, B.data_ptr(), ldb, out.data_ptr(), _mat(out)[2])
-        if st:
-            self._check(st, name)
+        self._check(fn(self._h, M, N, K, A.data_ptr(), lda, B.data_ptr(), ldb, out.data_ptr(), _mat(out)[2]), name)
         return out
 
     def gemm_f32(self, A, B, out=None):
+        if out is not None:
+            st = self._n_gemm(self._p_gemm_f32, self._address, 0, A, B, out)
+            if st == 0:
+                return out
+            if st > 0:
+                self._check(st, "cigemm_gemm_f32")
         f32 = self._f32
         assert A.dtype == f32 and B.dtype == f32
         return self._gemm(self.lib.cigemm_gemm_f32, "cigemm_gemm_f32", A, B, out, f32)
 
     def linear_f32(self, X, W, bias=None, act=ACT_NONE, out=None):
         """out = act(bias + X @ W) with W stored K x N (input-major)."""
+        if out is not None:
+            st = self._n_linear_f32(self._p_linear_f32, self._address, X, W, bias, act, out)
+            if st == 0:
+                return out
+            if st > 0:
+                self._check(st, "cigemm_linear_f32")
         f32 = self._f32
         assert X.dtype == f32 and W.dtype == f32
         M, K, ldx = _mat(X)
@@ -273,6 +315,12 @@ class Handle:
         return out
 
     def gemm_f16(self, A, B, out=None):
+        if out is not None:
+            st = self._n_gemm(self._p_gemm_f16, self._address, 1, A, B, out)
+            if st == 0:
+                return out
+            if st > 0:
+                self._check(st, "cigemm_gemm_f16")
         f16 = self._f16
         assert A.dtype == f16 and B.dtype == f16
         return self._gemm(self.lib.cigemm_gemm_f16, "cigemm_gemm_f16", A, B, out, f16)
@@ -302,11 +350,23 @@ class Handle:
         return Cm
 
     def gemm_bf16(self, A, B, out=None):
+        if out is not None:
+            st = self._n_gemm(self._p_gemm_bf16, self._address, 2, A, B, out)
+            if st == 0:
+                return out
+            if st > 0:
+                self._check(st, "cigemm_gemm_bf16")
         bf16 = self._bf16
         assert A.dtype == bf16 and B.dtype == bf16
         return self._gemm(self.lib.cigemm_gemm_bf16, "cigemm_gemm_bf16", A, B, out, bf16)
 
     def gemm_i8_i32(self, A, B, b_layout=B_KN, out=None):
+        if out is not None:
+            st = self._n_gemm_i8_i32(self._p_gemm_i8_i32, self._address, A, B, b_layout, out)
+            if st == 0:
+                return out
+            if st > 0:
+                self._check(st, "cigemm_gemm_i8_i32")
         assert A.dtype == self._i8 and B.dtype == self._i8
         M, K, lda = _mat(A)
         K2, N, ldb = _mat(B)
@@ -326,6 +386,12 @@ class Handle:
                         dump_acc=False):
         """Returns ``out`` or ``(out, acc)`` when ``dump_acc``.  A scale tensor with one
         element is per-tensor, otherwise per-row (A) / per-column (B)."""
+        if out is not None and not dump_acc:
+            st = self._n_gemm_i8_dequant(self._p_gemm_i8_dequant, self._address, A, B, scale_a, scale_b, b_layout, out_type, out)
+            if st == 0:
+                return out
+            if st > 0:
+                self._check(st, "cigemm_gemm_i8_dequant")
         f32 = self._f32
         M, K, lda = _mat(A)
         K2, N, ldb = _mat(B)
@@ -363,6 +429,13 @@ class Handle:
         return out
 
     def quantize_rows_i8(self, x, out=None):
+        if out is not None:
+            q, s = out
+            st = self._n_quantize_rows_i8(self._p_quantize_rows_i8, self._address, x, q, s)
+            if st == 0:
+                return q, s
+            if st > 0:
+                self._check(st, "cigemm_quantize_rows_i8")
         assert x.dtype == self._f32 and x.dim() == 2
         rows, cols, ldx = _mat(x)
         if out is None:

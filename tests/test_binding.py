@@ -1,0 +1,110 @@
+"""The native binding of the hot calls (csrc/binding.cpp) without a GPU: the entry points it is given are
+Python callbacks that record their arguments, over every order and stride the Python code takes, against
+what that computes; what that refuses is refused."""
+import ctypes as C
+
+import pytest
+import torch
+
+import cudaintro_amd as ci
+from cudaintro_amd import cigemm
+
+native = cigemm._native()
+HANDLE = 0x1230
+
+
+class Entry:
+    """A C function of the prototype of `name` that records its arguments and returns `status`."""
+
+    def __init__(self, name, status=0):
+        res, args = cigemm.SIGNATURES[name]
+        self.calls = []
+
+        def body(*a):
+            self.calls.append(a)
+            return status
+        self._keep = C.CFUNCTYPE(res, *args)(body)
+        self.address = C.cast(self._keep, C.c_void_p).value
+
+
+def matrices(rows, cols, dtype):
+    """The same matrix shape in every form: packed, a column block, a row step, one row, offset."""
+    big = torch.zeros((2 * rows + 1, cols + 5), dtype=dtype)
+    yield torch.zeros((rows, cols), dtype=dtype)
+    yield big[:rows, 3:3 + cols]
+    yield big[1:1 + 2 * rows:2, :cols]
+    yield torch.zeros((1, cols), dtype=dtype).expand(rows, cols)      # every row the same one
+    if cols == 1:
+        yield torch.zeros((1, rows), dtype=dtype).t()                 # a single column of any stride
+
+
+def expect(t):
+    rows, cols, ld = cigemm._mat(t)
+    return rows, cols, ld, t.data_ptr() or None
+
+
+@pytest.mark.parametrize("code,dtype", [(0, torch.float32), (1, torch.float16), (2, torch.bfloat16)])
+def test_gemm(code, dtype):
+    fn = Entry("cigemm_gemm_f32")
+    for M, K, N in ((3, 5, 7), (1, 4, 1), (4, 1, 6), (2, 0, 3), (0, 2, 2)):
+        for A in matrices(M, K, dtype):
+            for B in matrices(K, N, dtype):
+                for out in matrices(M, N, torch.float32):
+                    assert native.gemm(fn.address, HANDLE, code, A, B, out) == 0
+                    (m, k, lda, a), (_, n, ldb, b), (_, _, ldc, c) = expect(A), expect(B), expect(out)
+                    assert fn.calls.pop() == (HANDLE, m, n, k, a, lda, b, ldb, c, ldc)
+    assert native.gemm(Entry("cigemm_gemm_f32", 13).address, HANDLE, code, A, B, out) == 13
+
+
+def test_refused_as_before():
+    fn = Entry("cigemm_gemm_f32")
+    A, B, out = torch.zeros(3, 5), torch.zeros(5, 7), torch.zeros(3, 7)
+    for bad in ((A.double(), B, out), (A, B.half(), out), (A, torch.zeros(4, 7), out), (A.t().contiguous().t(), B, out),
+                (A, torch.zeros(7, 5).t(), out), (A, B, torch.zeros(7, 3).t()), (A, B, torch.zeros(21)),
+                (torch.zeros(5), B, out), (torch.zeros(1, 3, 5), B, out)):
+        with pytest.raises(AssertionError):
+            native.gemm(fn.address, HANDLE, 0, *bad)
+
+    class Sub(torch.Tensor):
+        pass
+    for odd in ((A.numpy(), B, out), (A, B.as_subclass(Sub), out), (A, B, None)):
+        assert native.gemm(fn.address, HANDLE, 0, *odd) == -1      # (left to the Python code)
+    assert native.gemm(fn.address, HANDLE, 0, torch.nn.Parameter(A), B, out) == 0
+    with pytest.raises(TypeError):
+        native.gemm(fn.address, HANDLE, 0, A, B)
+    assert len(fn.calls) == 1
+
+
+def test_linear_int8_quantizer():
+    fn = Entry("cigemm_linear_f32")
+    X, W, out = torch.zeros(3, 5), torch.zeros(5, 7), torch.zeros(3, 7)
+    bias = torch.zeros(7)
+    for b in (None, bias):
+        assert native.linear_f32(fn.address, HANDLE, X, W, b, ci.ACT_RELU, out) == 0
+        assert fn.calls.pop() == (HANDLE, 3, 7, 5, X.data_ptr(), 5, W.data_ptr(), 7, b.data_ptr() if b is not None else None,
+                                  int(ci.ACT_RELU), out.data_ptr(), 7)
+    for b in (torch.zeros(6), bias.double()):
+        with pytest.raises(AssertionError):
+            native.linear_f32(fn.address, HANDLE, X, W, b, 0, out)
+
+    A, sa, sb = torch.zeros((3, 5), dtype=torch.int8), torch.zeros(3), torch.zeros(1)
+    f32, f16 = Entry("cigemm_gemm_i8_i32"), Entry("cigemm_gemm_i8_dequant")
+    for layout, B in ((ci.B_KN, torch.zeros((5, 7), dtype=torch.int8)), (ci.B_NK, torch.zeros((7, 5), dtype=torch.int8))):
+        acc, y = torch.zeros((3, 7), dtype=torch.int32), torch.zeros((3, 7), dtype=torch.bfloat16)
+        assert native.gemm_i8_i32(f32.address, HANDLE, A, B, layout, acc) == 0
+        assert f32.calls.pop() == (HANDLE, 3, 7, 5, A.data_ptr(), 5, B.data_ptr(), B.stride(0), int(layout), acc.data_ptr(), 7)
+        assert native.gemm_i8_dequant(f16.address, HANDLE, A, B, sa, sb, layout, ci.OUT_BF16, y) == 0
+        assert f16.calls.pop() == (HANDLE, 3, 7, 5, A.data_ptr(), 5, B.data_ptr(), B.stride(0), int(layout), sa.data_ptr(),
+                                   int(ci.SCALE_VECTOR), sb.data_ptr(), int(ci.SCALE_TENSOR), y.data_ptr(),
+                                   int(ci.OUT_BF16), 7, None, 0)
+        for bad in ((sa[:2], sb), (sa, torch.zeros(3)), (sa.double(), sb)):
+            with pytest.raises(AssertionError):
+                native.gemm_i8_dequant(f16.address, HANDLE, A, B, *bad, layout, ci.OUT_BF16, y)
+
+    q = Entry("cigemm_quantize_rows_i8")
+    x, xq, sx = torch.zeros(3, 9)[:, 2:7], torch.zeros((3, 5), dtype=torch.int8), torch.zeros(3)
+    assert native.quantize_rows_i8(q.address, HANDLE, x, xq, sx) == 0
+    assert q.calls.pop() == (HANDLE, 3, 5, x.data_ptr(), 9, xq.data_ptr(), 5, sx.data_ptr())
+    for bad in ((x.double(), xq, sx), (x, xq[:2], sx), (x, xq.int(), sx), (x, xq, sx.double())):
+        with pytest.raises(AssertionError):
+            native.quantize_rows_i8(q.address, HANDLE, *bad)
