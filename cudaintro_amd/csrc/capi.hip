@@ -96,6 +96,7 @@ cigemmStatus_t cigemmCreate(cigemmHandle_t* handle) {
   ctx->force_any_kernel = ANY_BY_SHAPE;
   ctx->force_split_rows = 0;
   ctx->force_split_ranges = 0;
+  ctx->force_panel_rows = 0;
   ctx->workspace = nullptr;
   if (hipMalloc(&ctx->workspace,
                 ctx->ws_partial_bytes + ctx->ws_counter_bytes + ctx->ws_swap_bytes) != hipSuccess ||
@@ -363,6 +364,7 @@ static cigemmStatus_t gemm16(cigemmHandle_t h, const char* name, bool bf16, int6
       // neither that nor the tile kernel takes (odd N, unaligned rows) stays on the matrix cores
       if (!launch_skinny_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc) &&
           !launch_kwaves_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc) &&
+          !launch_panel_16(h, bf16, M, N, K, A, lda, B, ldb, C, ldc) &&
           !rest_columns(
               h, M, N, K * 2, false,
               [&](int64_t n1) {
@@ -409,6 +411,7 @@ static cigemmStatus_t gemm_i8(cigemmHandle_t h, const char* name, int64_t M, int
     default:
       if (!launch_skinny_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq) &&
           !launch_kwaves_i8(h, M, N, K, A, lda, B, ldb, b_nk, C, ldc, dq) &&
+          !(b_nk && launch_panel_i8_nk(h, M, N, K, A, lda, B, ldb, C, ldc, dq)) &&
           !((!dq || !dq->acc_out) &&
             rest_columns(
                 h, M, N, K, false,

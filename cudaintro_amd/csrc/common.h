@@ -55,6 +55,8 @@ struct cigemmContext {
   // they take, -1 keeps them out of every call, 0 = the library chooses.
   int force_split_rows;
   int force_split_ranges;
+  // The same for gemm_panel.hip: tiles of force_panel_rows rows (< 0: never).
+  int force_panel_rows;
   char last_error[256];
 };
 
@@ -270,6 +272,12 @@ bool launch_kwaves_i8(cigemmContext*, int64_t M, int64_t N, int64_t K, const int
                       const DequantArgs* dq, bool rest = false);
 // Columns of the full rounds of 256-row tiles where the tile kernel would run the rest, at most 64 columns,
 // as a launch of its own: those are the kernel of small outputs'; 0: no such plan.
+// gemm_panel.hip: one round of tiles of 64 or 128 rows x 64 columns, the aligned tile kernel's operands.
+// False, with nothing launched, where the call is left to the other kernels.
+bool launch_panel_16(cigemmContext*, bool bf16, int64_t M, int64_t N, int64_t K, const uint16_t* A,
+                     int64_t lda, const uint16_t* B, int64_t ldb, uint16_t* C, int64_t ldc);
+bool launch_panel_i8_nk(cigemmContext*, int64_t M, int64_t N, int64_t K, const int8_t* A, int64_t lda,
+                        const int8_t* B, int64_t ldb, int32_t* C, int64_t ldc, const DequantArgs* dq);
 int64_t kwaves_rest_columns(const cigemmContext*, int64_t M, int64_t N, int64_t K_bytes, bool f32);
 // the kernel's name after such a pair of calls: "<first>+<tile of the rest>"
 void name_rest_columns(cigemmContext*, const char* first);

@@ -500,3 +500,11 @@ extern "C" cigemmStatus_t cigemm_probe_force_f32_split(cigemmHandle_t h, int til
   h->force_split_ranges = tile_rows > 0 ? k_ranges : 0;
   return CIGEMM_STATUS_SUCCESS;
 }
+
+extern "C" cigemmStatus_t cigemm_probe_force_panel_rows(cigemmHandle_t h, int tile_rows) {
+  if (!h || h->magic != kCtxMagic) return CIGEMM_STATUS_NOT_INITIALIZED;
+  if (tile_rows < -1 || (tile_rows > 0 && tile_rows != 64 && tile_rows != 128))
+    return fail(h, CIGEMM_STATUS_INVALID_VALUE, "cigemm_probe_force_panel_rows: tile_rows %d", tile_rows);
+  h->force_panel_rows = tile_rows;
+  return CIGEMM_STATUS_SUCCESS;
+}

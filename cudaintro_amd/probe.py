@@ -34,6 +34,7 @@ SIGNATURES = {
     "cigemm_probe_force_kwaves_plan": (_ci, [_vp, _ci]),
     "cigemm_probe_force_any_kernel": (_ci, [_vp, _ci]),
     "cigemm_probe_force_f32_split": (_ci, [_vp, _ci, _ci]),
+    "cigemm_probe_force_panel_rows": (_ci, [_vp, _ci]),
 }
 
 
@@ -182,6 +183,12 @@ def force_f32_split(h: Handle, tile_rows: int, k_ranges: int = 1):
     handle's calls, 0 hands the choice back."""
     _check(h, load_library().cigemm_probe_force_f32_split(h.raw, tile_rows, k_ranges),
            "cigemm_probe_force_f32_split")
+
+
+def force_panel_rows(h: Handle, tile_rows: int):
+    """The same for the kernel of batches (tiles of 64 or 128 rows x 64 columns); tile_rows = -1 keeps it out
+    of the handle's calls, 0 hands the choice back."""
+    _check(h, load_library().cigemm_probe_force_panel_rows(h.raw, tile_rows), "cigemm_probe_force_panel_rows")
 
 
 ANY_BY_SHAPE, ANY_REGISTER_STAGED, ANY_F32_SMALL, ANY_TILE = 0, 1, 2, 3

@@ -150,6 +150,10 @@ CIGEMM_API cigemmStatus_t cigemm_probe_force_any_kernel(cigemmHandle_t handle, i
  * keeps them out of every call, 0 hands the choice back to the library. */
 CIGEMM_API cigemmStatus_t cigemm_probe_force_f32_split(cigemmHandle_t handle, int tile_rows, int k_ranges);
 
+/* The same for the kernel of batches (gemm_panel.hip): rows of a tile (64 or 128) of the handle's following
+ * 16-bit and N x K int8 calls under CIGEMM_ALGO_DEFAULT (those it takes). */
+CIGEMM_API cigemmStatus_t cigemm_probe_force_panel_rows(cigemmHandle_t handle, int tile_rows);
+
 #ifdef __cplusplus
 }
 #endif

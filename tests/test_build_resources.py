@@ -18,7 +18,7 @@ FLAGS = ["-O3", "-std=c++17", "--offload-arch=gfx950", "-fvisibility=hidden", "-
 
 
 FILES = ("gemm_16b.hip", "gemm_i8.hip", "gemm_f32.hip", "gemm_any_tile.hip", "gemm_skinny.hip", "gemm_kwaves.hip",
-         "gemm_f32_small.hip", "probe.hip", "probe_paired.hip")
+         "gemm_panel.hip", "gemm_f32_small.hip", "probe.hip", "probe_paired.hip")
 
 
 @pytest.fixture(scope="module")
@@ -59,6 +59,7 @@ def test_hot_kernels_do_not_spill(assembly):
     spills = {k: v for text in assembly.values() for k, v in spill_counts(text).items()}
     assert len(spills) > 60          # every template instance was seen
     assert sum("kwaves_kernelINS" in k for k in spills) >= 10
+    assert sum("panel_kernel" in k for k in spills) == 10
     assert sum("mfma_tile_kernelINS0_7MathF32E" in k for k in spills) >= 63    # seven heights, both forms
     for name, n in spills.items():
         if re.search(r"EpiDequantX4ILb[01]ELb1", name):
