@@ -1,15 +1,17 @@
 // GEMM of a batch of rows on tiles of 64 or 128 rows x 64 columns, one round of them, all of k in one workgroup.
 //
-// What bounds these calls: a compute unit takes about 50 KB/us of operands, whatever is in flight and however many
-// units do (256 x 8192 x 8192 on half of the units takes as long for a stage as on all), and, where K is cut to
-// fill the chip with 256-column tiles, the partial sums and the launch that adds them up (5 to 8 us).  Tiles of 64
-// columns fill it with whole k: 4 x 64 tiles of 64 rows serve 256 x 4096 where mfma_tile.h has 64 tiles and cuts
-// k in four.  Wider outputs or longer k are that kernel's, whose 256 columns share each fetch of A.  us, there ->
-// here: bf16 229 x 2752 x 1984 17.4 -> 11.9, 1097 x 1664 x 1664 19.0 -> 13.6, 113 x 14464 x 2624 29.0 -> 22.9; int8
-// 256 x 4096 x 4096 17.3 -> 12.7, 512 x 4096 x 4096 22.8 -> 17.0, 584 x 2752 x 2944 21.1 -> 12.9.
+// What bounds these calls: a compute unit takes 50 to 55 KB/us of operands here (112 where every line is in its L2:
+// lines that come from memory hold up those behind them), also with half of the units at work; and, where k is cut
+// to fill the chip with 256-column tiles, the partial sums and the launch that adds them up (5 to 8 us).  Tiles
+// of 64 columns fill it with whole k: 4 x 64 tiles of 64 rows serve 256 x 4096 where mfma_tile.h has 64 tiles
+// and cuts k in four.  Wider outputs or longer k are that kernel's, whose 256 columns share each fetch of A.  us,
+// there -> here: bf16 229 x 2752 x 1984 17.4 -> 11.9, 1097 x 1664 x 1664 19.0 -> 13.6, 113 x 14464 x 2624 29.0 ->
+// 22.9; int8 with scales 256 x 4096 x 4096 17.3 -> 12.7, 512 x 4096 x 4096 22.8 -> 17.0.
 // Tried and not kept: K ranges joined inside (by the tile's last workgroup; a few calls gained), tiles of 256 rows
 // (256 x 8192 x 8192 over two ranges 59.7 us, 51.7 on the tile kernel), K x N int8 (whose 64-byte rows are half
-// lines: as fast as the tile kernel at best).
+// lines: as fast as the tile kernel at best), a ring of 10 for 64 rows (no difference), workgroups that begin at
+// different stages (none), waves that move only A or only B through rings of their own (256 x 4096 x 4096 21.7 ->
+// 28.2).
 //
 // Workgroup = 512 lanes = 8 waves, 2 (rows) x 4 (k): a stage is 128 bytes of k (64 halves, 128 int8), of which
 // each wave multiplies one k-step of 32 MT rows x 64 columns.  Stages of A [rows][128 B] and B ([64 n][128 B] or

@@ -31,7 +31,8 @@ inline double us(const Cost& c, const any::Problem& p, int cus, int rows) {
 // 6000 the other one is often too high (int8 150 x 7040 x 10560 estimated 46 us there, took 38, here 47), and this
 // one has to be 10 % below it.  Of some 2000 random calls that the tile kernel served with k up to 6000 bytes, 179
 // 16-bit and 101 int8 ones are taken: 1.13 and 1.24 times as fast (geometric mean), 271 of them by more than 3 %,
-// one more than 3 % slower (f16 67 x 13936 x 2544: 27.2 us, 23.9 there).
+// one more than 3 % slower (f16 67 x 13936 x 2544: 27.2 us, 23.9 there).  Of 316 taken among random sizes timed
+// afterwards, 1.13 (16-bit) and 1.20 (int8) times as fast, five are 4 to 8 % slower.
 inline int choose(const Cost& c, const any::Cost& other, const any::Problem& p, int cus, size_t partial_bytes) {
   if (p.M <= 32 || p.M > 2048 || p.N < 256 || p.K_bytes < 1536) return 0;
   int rows = 0;
