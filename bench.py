@@ -37,10 +37,10 @@ PEAK_HBM_GBS = 8000.0
 
 
 def fp32_peak(kernel):
-    """What bounds an fp32 call: the fp32 matrix instructions, or a sixth of the bf16 ones' rate (the
-    256-column tiles multiply with six bf16 instructions in place of one)."""
+    """What bounds an fp32 call: the fp32 matrix instructions, or an eighth of the bf16 ones' rate (the
+    256-column tiles on bf16 parts multiply with eight bf16 instructions for 16 of k)."""
     tiles = "x256x16" in kernel and "32x32x2" not in kernel
-    return PEAK_16BIT_TFLOPS / 6 if tiles else PEAK_FP32_MATRIX_TFLOPS
+    return PEAK_16BIT_TFLOPS / 8 if tiles else PEAK_FP32_MATRIX_TFLOPS
 
 
 def log(*a):

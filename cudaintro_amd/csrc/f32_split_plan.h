@@ -7,7 +7,7 @@ namespace cig {
 namespace split32 {
 
 struct Plan {
-  int rows;          // of a tile: 64, 96 .. 256; 0: no plan
+  int rows;          // of a tile: 64, 96 or 128; 0: no plan
   int ranges;        // of K
   int64_t first_cols;  // > 0: these columns first, unsplit, on tiles of first_rows; the others by the above
   int first_rows;
@@ -37,16 +37,15 @@ inline bool ok(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb) {
 }
 
 // us of one launch.  A stage of a round of workgroups: a part of its own and a part that grows with the
-// units at work (the chip's power limit); a round: ramp and epilogue; the output and the operands by
-// the MB, the reduction behind K ranges.  Fitted to 6600 timed plans of 1000 sizes (M 16..20000, N 16..
-// 16384, K 17..16384, log-uniform, up to 1.4e11 operations): rms error 5 %; the plan it likes best is 0.5 %
+// units at work (the chip's power limit); a round: ramp and epilogue; the operands by the MB, the
+// reduction behind K ranges.  Fitted to 35092 timed plans of 10198 sizes (M 16..20000, N 16..16384, K
+// 17..16384, log-uniform, up to 1.4e11 operations): rms error 4 %; the plan it likes best is 0.2 %
 // slower than the best one timed, on average.
 struct Cost {
   double stage, stage_chip, round;
 };
-constexpr Cost COST[7] = {{0.647, 0.131, 4.52}, {0.696, 0.225, 5.38}, {0.852, 0.274, 6.44}, {1.038, 0.386, 6.59},
-                          {1.117, 0.467, 7.72}, {1.292, 0.499, 8.22}, {1.419, 0.561, 9.36}};
-constexpr double START_US = 2.54, OUT_MB = 0.0523, IN_MB = 0.0141, REDUCE_US = 2.65, REDUCE_MB = 0.155;
+constexpr Cost COST[3] = {{0.554, 0.379, 5.25}, {0.670, 0.523, 6.32}, {0.807, 0.648, 7.51}};
+constexpr double START_US = 2.47, IN_MB = 0.0174, REDUCE_US = 1.26, REDUCE_MB = 0.153;
 constexpr Cost cost_of(int rows) { return COST[rows / 32 - 2]; }
 
 inline double launch_us(int64_t M, int64_t N, int64_t K, int cus, int rows, int ranges) {
@@ -57,22 +56,23 @@ inline double launch_us(int64_t M, int64_t N, int64_t K, int cus, int rows, int 
   const double stages = (double)range_k / 16 + 1, mn = (double)M * (double)N * 4e-6;
   double us = START_US + (double)(tiles / cus) * (stages * (c.stage + c.stage_chip) + c.round);
   if (tiles % cus) us += stages * (c.stage + c.stage_chip * (double)(tiles % cus) / cus) + c.round;
-  us += OUT_MB * mn * sp + IN_MB * (double)(M + N) * (double)K * 4e-6;
+  us += IN_MB * (double)(M + N) * (double)K * 4e-6;
   if (sp > 1) us += REDUCE_US + REDUCE_MB * mn * (sp + 1);
   return us;
 }
 
-// The longest sum of k that a result may be made of, as the fp32 instructions add it up, where the tiles
-// of this height are to round no more: with one running sum of a block (above 128 rows) their error is 0.75
-// to 0.93 of the fp32 instructions', with two 0.32 to 0.4, and it grows with the square root of the length.
-constexpr int64_t range_limit(int rows, int64_t sum_length) { return rows > 128 ? sum_length : 6 * sum_length; }
+// The longest sum of k that a result may be made of, where the other kernel adds up `sum_length`.  Of equally long
+// sums the error here is at most 0.71 times the fp32 instructions' (0.83 and 1.00 where two products or one
+// make the result, whose errors do not grow); that of positive operands grows with the length (over K in one
+// sum, against the fp32 instructions over six ranges of it: 1.7 to 4.3 times).
+constexpr int64_t range_limit(int64_t sum_length) { return sum_length + sum_length / 4; }
 
 // The best single launch; `sum_length`: of the kernel this one takes the place of.
 inline Plan best_launch(int64_t M, int64_t N, int64_t K, int64_t sum_length, int cus, size_t partial_bytes,
                         double* est) {
   Plan best{0, 1, 0, 0};
   *est = 1e30;
-  for (int rows = 64; rows <= 256; rows += 32) {
+  for (int rows = 64; rows <= 128; rows += 32) {
     if (rows > 64 && rows - 32 >= M) break;  // a lower height already covers M
     const int64_t tiles = any::div_up(M, rows) * any::div_up(N, tile::BN);
     int last = 0;
@@ -84,7 +84,7 @@ inline Plan best_launch(int64_t M, int64_t N, int64_t K, int64_t sum_length, int
         break;
       if (sp == last) continue;
       last = sp;
-      if (range_k > range_limit(rows, sum_length)) continue;
+      if (range_k > range_limit(sum_length)) continue;
       const double us = launch_us(M, N, K, cus, rows, sp);
       if (us < *est) *est = us, best = Plan{rows, sp, 0, 0};
     }
@@ -97,9 +97,9 @@ inline Plan best(int64_t M, int64_t N, int64_t K, int64_t sum_length, int cus, s
                  double* est) {
   Plan b = best_launch(M, N, K, sum_length, cus, partial_bytes, est);
   const int64_t tiles_n = any::div_up(N, tile::BN);
-  for (int rows = 96; rows <= 256; rows += 32) {
+  for (int rows = 96; rows <= 128; rows += 32) {
     const int64_t tiles_m = any::div_up(M, rows);
-    if (tiles_m > cus || K > range_limit(rows, sum_length)) continue;
+    if (tiles_m > cus || K > range_limit(sum_length)) continue;
     const int64_t per_round = cus / tiles_m, cols = tiles_n / per_round * per_round;
     if (cols <= 0 || cols >= tiles_n) continue;
     const double first = launch_us(M, cols * tile::BN, K, cus, rows, 1);

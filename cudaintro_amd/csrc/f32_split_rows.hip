@@ -1,5 +1,5 @@
-// The fp32 tiles on the bf16 matrix instructions of one height (CIG_SPLIT_ROWS and the shape it stands for,
-// given on the compiler's command line: a file each, since a kernel takes ten seconds to compile).
+// The fp32 tiles on the bf16 matrix instructions of one height (CIG_SPLIT_ROWS, given on the compiler's
+// command line: a file each, since a kernel takes ten seconds to compile).
 #include "epilogues.h"
 #include "f32_split_tile.h"
 
@@ -9,9 +9,9 @@ namespace split32 {
 template <int ROWS, typename Epi>
 void launch(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, int64_t range_k, int ranges, const float* A,
             int64_t lda, const float* B, int64_t ldb, const Epi& epi) {
-  typedef tile::SplitTile<CIG_SPLIT_SHAPE> S;
+  typedef tile::SplitTile<ROWS / 32> S;
   static_assert(S::TILE_M == ROWS, "");
-  auto kern = tile::f32_split_kernel<CIG_SPLIT_SHAPE, true, Epi>;
+  auto kern = tile::f32_split_kernel<ROWS / 32, Epi>;
   static std::atomic<uint64_t> lds_set{0};
   if (!ensure_dynamic_lds(ctx, (const void*)kern, S::LDS_BYTES, lds_set)) return;
   const int tiles_m = (int)((M + ROWS - 1) / ROWS), tiles_n = (int)((N + tile::BN - 1) / tile::BN);

@@ -1,37 +1,38 @@
 // fp32 GEMM tiles on the bf16 matrix instructions, every operand held exactly.
 //
 // An fp32 number of 24 bits is the sum of three bf16 numbers of 8: h = bf16(x), m = bf16(x - h), l = x - h -
-// m, every difference exact.  a b is then h h' + (h m' + m h') + (m m' + h l' + l h') and three products
-// below 2^-24 of it, which are left out: six v_mfma_f32_32x32x16_bf16 in place of eight v_mfma_f32_32x32x2_f32
-// for 16 of k, 192 cycles in place of 512, sums in fp32 as before.  The error against 64 bits is smaller than the fp32
-// instructions', which round twice per instruction and product pair (65536 outputs at
-// K = 64, 512 and 4096 each, symmetric, positive and wide-ranging operands): 0.75 to 0.93 of it with one running sum of a
-// block, 0.32 to 0.4 with a second one for the five smaller products (tiles of up to 128 rows, where the
-// registers allow it).  The host takes the tiles only where no sum gets longer by more than that
-// (f32_split_plan.h, range_limit).
+// m, every difference exact.  a b is then h h' + (h m' + m h') + (m m' + h l' + l h') + (m l' + l m') and l l', below
+// 2^-32 of it, which is left out: eight v_mfma_f32_32x32x16_bf16 in place of eight v_mfma_f32_32x32x2_f32
+// for 16 of k, 256 cycles in place of 512, sums in fp32 as before.
+// h h' has a running sum of its own, the seven smaller products another, and the two meet at the end: a rounding of
+// the large sum for eight of k, where the fp32 instruction rounds for each one.  Error against 64 bits, by the
+// fp32 instructions' on the same operands (131072 outputs each, K = 64, 1024 and 4096): 0.30 to 0.33 for dense
+// operands, 0.32 to 0.83 for rows with 2 nonzero values up to 60 % of them, and where one product makes the result
+// the same to four digits (at most 0.51 units in the last place, 0.50 there).  With one running sum that ratio is 0.75 to
+// 0.87 for dense operands but up to 2.0 for sparse ones (each of the products rounds the sum, where the fp32
+// instruction adds zeros), and without m l' + l m' a lone product is off by up to 0.91 units: neither is kept,
+// though tiles of 256 rows, whose registers hold one sum only, take 743 us for 4096^3, and six products 668 here.
+// The host takes the tiles only where no sum gets longer by more than the rest allows (f32_split_plan.h,
+// range_limit).
 //
 // What three parts cannot hold: infinities and NaN (x - h is NaN), magnitudes that bf16 rounds to infinity,
 // and below 2^-110, where the last part falls short of bf16's subnormals.  A workgroup that met a nonzero
 // value below 2^-110 or got a result that is not finite computes its tile once more with the fp32
 // instructions, straight from memory (slow, about twice the tile's time, and only there).
 //
-// Workgroup = 256 lanes = 4 waves, tile of 64 .. 256 rows x 256 columns, stages of 16 k.  Values go from
+// Workgroup = 256 lanes = 4 waves, tile of 64, 96 or 128 rows x 256 columns, stages of 16 k.  Values go from
 // memory to registers (8 k of one row of A; 8 k of two columns of B, so that the matrix instruction's
 // order of B needs no transposing read), are split there, once per workgroup, and written to LDS as the three parts in fragment
 // order ([32 rows][16 k] blocks of 1 KiB, a lane's 16 bytes in one read, rows permuted so that reads and
 // writes meet no bank conflict).  Any alignment: nothing here needs more than the elements'.
 // One barrier a stage, behind the first matrix instructions; the parts of stage s + 2 are written under the
-// multiplies of stage s, whose own fragments were read in the stage before; loads are one (tiles above 128
-// rows, whose stages take long) or two stages ahead of the splitting.  The order of the slots (one matrix
-// instruction, its share of the splitting, at most a read, a write and a load) is pinned.
+// multiplies of stage s, whose own fragments were read in the stage before; loads are two stages ahead of the
+// splitting.  The order of the slots (one matrix instruction, its share of the splitting, at most a read, a write and a
+// load) is pinned.
 //
-// What bounds it: the chip's power.  4096^3 in us, all 256 units at work, tiles of 128 rows: matrix
-// instructions and fragment reads alone 605, with the loads 682, with the splitting 743, with the writes
-// 782; the main loop's 2134 cycles a stage (1560 without splitting and loads) are the same with one
-// workgroup, the clock falls from 2.3 to 1.4 GHz.  Hence the 256-row tile: two thirds of the loads, splits,
-// writes and reads per product, 3100 cycles for twice the work.  fp32 instructions -> here, one process, us: 4096^3 905
-// -> 579, 8192 x 2048 x 4096 909 -> 575, 4095 x 4097 x 4099 931 -> 606, 20000 x 512 x 784 117 -> 87, 2049 x 2047
-// x 1025 94.6 -> 63.3, 256 x 8192 x 8192 240 -> 181, 2048^3 118 -> 100.
+// What bounds it: the chip's power.  The main loop takes the same cycles with one workgroup and with all units at
+// work, the clock falls from 2.3 to 1.4 GHz.  fp32 instructions -> here, one process, us: 4096^3 898 -> 762, 4095 x 4097 x 4099
+// 928 -> 793, 256 x 8192 x 8192 239 -> 219.
 #pragma once
 
 #include "mfma_tile.h"
@@ -45,30 +46,27 @@ __device__ __forceinline__ void each_of(F&& f, std::integer_sequence<int, I...>)
   (f(std::integral_constant<int, I>{}), ...);
 }
 
-// MT x NT blocks of 32 x 32 a wave, WM rows of 4 / WM waves, SUMS running sums a block.
-template <int MT, int NT, int WM, int SUMS>
+// MT x NT blocks of 32 x 32 a wave, the waves side by side.
+template <int MT>
 struct SplitTile {
-  static constexpr int WN = 4 / WM;
-  static constexpr int TILE_M = 32 * MT * WM;
-  static_assert(32 * NT * WN == BN, "tiles are 256 columns wide");
+  static constexpr int NT = BN / 4 / 32;
+  static constexpr int TILE_M = 32 * MT;
+  static_assert(MT >= 2 && MT <= 4, "two sums of a block fill the accumulator registers at 128 rows");
   static constexpr int KS = 16;                       // k of a stage: one matrix instruction's
-  static constexpr int A_BLOCKS = TILE_M > 128 ? 8 : 4, B_BLOCKS = 8;
+  static constexpr int A_BLOCKS = 4, B_BLOCKS = 8;    // (A's are fetched and split as of 128 rows)
   static constexpr int BLOCK = 1024;                  // 32 rows (columns) x 16 k of one part
   static constexpr int A_BYTES = 3 * A_BLOCKS * BLOCK, SLOT = A_BYTES + 3 * B_BLOCKS * BLOCK;
-  static constexpr int RING = TILE_M > 128 ? 3 : 4;
+  static constexpr int RING = 4;
   static constexpr int LDS_BYTES = RING * SLOT + 16;
-  static constexpr int MFMAS = 6 * MT * NT;           // per stage and wave
-  static constexpr int DEPTH = TILE_M > 128 ? 1 : 2;  // stages whose values wait in registers
-  // (an odd number of row blocks leaves the next stage's first fragments in the other registers)
-  static constexpr int TRIP = DEPTH == 2 || MT % 2 ? 2 : 1;  // stages of a trip of the main loop
-  static constexpr int A_TASKS = A_BLOCKS / 4, TASKS = 2 + A_TASKS;
+  static constexpr int PRODUCTS = 8;
+  static constexpr int MFMAS = PRODUCTS * MT * NT;    // per stage and wave
+  static constexpr int TASKS = 3;                     // groups of 8 elements a lane splits per stage: B, B, A
 };
 
 // The running sums of an output block.
-template <int SUMS>
 struct MathSplit {
   struct acc_t {
-    f32x16 part[SUMS];
+    f32x16 part[2];  // of h h' and of the smaller products
     __device__ __forceinline__ float operator[](int e) const { return part[0][e]; }
   };
 };
@@ -87,7 +85,7 @@ struct EpiChecked : Epi {
   }
 };
 
-template <int MT, int NT, int WM, int SUMS, bool ANY, typename Epi>
+template <int MT, typename Epi>
 __global__ __launch_bounds__(256, 1) void f32_split_kernel(int M, int N, int K_total, int range_k,
                                                            int tiles_m, int tiles_n,
                                                            const float* __restrict__ A, int64_t lda,
@@ -99,11 +97,11 @@ __global__ __launch_bounds__(256, 1) void f32_split_kernel(int M, int N, int K_t
   A += k_from;
   B += (int64_t)k_from * ldb;
   const Epi epi = epilogue_of_split(epi_all, (int)blockIdx.y);
-  typedef SplitTile<MT, NT, WM, SUMS> S;
+  typedef SplitTile<MT> S;
+  constexpr int NT = S::NT;
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int t = threadIdx.x, l = t & 63;
   const int w = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int wm = w / S::WN, wn = w % S::WN;
   volatile int* const vote = reinterpret_cast<volatile int*>(lds + S::RING * S::SLOT);
   if (t == 0) *vote = 0;
   int tm, tn;
@@ -116,21 +114,17 @@ __global__ __launch_bounds__(256, 1) void f32_split_kernel(int M, int N, int K_t
   // A: 8 k of a row.  B: 8 k of two columns (a wave 8 rows of k x 128 columns).  The last 1..16 of k
   // come first, element by element.
   const int full = (K - 1) / S::KS, tail = K - full * S::KS;
-  // (the tail, and with two stages a trip one of zeros where their number is odd)
-  const int first = S::TRIP == 2 && full % 2 == 0 ? 2 : 1;
+  // (the tail, and one of zeros where their number is odd: two stages a trip of the main loop)
+  const int first = full % 2 == 0 ? 2 : 1;
   const int stages = full + first;
   const int a_half = t & 1, a_row = t >> 1;
   const int b_half = w & 1, b_col = 128 * (w >> 1) + 2 * l;
   const int b_left = N - n0 < BN ? (int)(N - n0) : BN;  // columns of the tile
   const int b_back = b_left == 1 ? 1 : 0;
-  uint32_t a_voff[S::A_TASKS], b_voff[8];
+  uint32_t a_voff, b_voff[8];
   {
     const int64_t last = M - 1 - m0;
-#pragma unroll
-    for (int q = 0; q < S::A_TASKS; ++q) {
-      const int64_t r = 128 * q + a_row;
-      a_voff[q] = (uint32_t)((r < last ? r : last) * lda * 4) + a_half * 32;
-    }
+    a_voff = (uint32_t)((a_row < last ? a_row : last) * lda * 4) + a_half * 32;
     // (columns past N - 2 fetch the last two: what no row holds is read nowhere)
     const int64_t c = b_col < b_left - 2 ? b_col : b_left - 2;
 #pragma unroll
@@ -147,9 +141,8 @@ __global__ __launch_bounds__(256, 1) void f32_split_kernel(int M, int N, int K_t
     a_next += to_load > 0 ? 64 : 0;
     b_next += to_load > 0 ? b_step : 0;
   };
-  // groups of 8 elements a lane splits per stage: B, B, A (, A)
   typedef float raw_t[S::TASKS][8];
-  raw_t raw[S::DEPTH];
+  raw_t raw[2];
   // (a lane offset the compiler may not widen outside the loop: scalar base + 32 bits is one instruction)
   auto load_b = [&](raw_t& x, int j) {
     uint32_t v = b_voff[j];
@@ -159,31 +152,28 @@ __global__ __launch_bounds__(256, 1) void f32_split_kernel(int M, int N, int K_t
     x[0][j] = q[0];
     x[1][j] = q[1];
   };
-  auto load_a = [&](raw_t& x, int task, int half) {
-    uint32_t v = a_voff[task - 2];
+  auto load_a = [&](raw_t& x, int half) {
+    uint32_t v = a_voff;
     asm volatile("" : "+v"(v));
     f32x4 q;
     __builtin_memcpy(&q, a_next + v + 16 * half, 16);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) x[task][4 * half + e] = q[e];
+    for (int e = 0; e < 4; ++e) x[2][4 * half + e] = q[e];
   };
   auto load_stage = [&](raw_t& x) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) load_b(x, j);
 #pragma unroll
-    for (int q = 0; q < 2 * S::A_TASKS; ++q) load_a(x, 2 + q / 2, q % 2);
+    for (int q = 0; q < 2; ++q) load_a(x, q);
     advance();
   };
   auto load_tail = [&](raw_t& x, int valid) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const int ka = a_half * 8 + j, kb = b_half * 8 + j;
-#pragma unroll
-      for (int q = 0; q < S::A_TASKS; ++q) {
-        const float a = *reinterpret_cast<const float*>(a_tile + (a_voff[q] - a_half * 32) +
-                                                        (int64_t)(ka < valid ? full * 16 + ka : K - 1) * 4);
-        x[2 + q][j] = ka < valid ? a : 0.0f;
-      }
+      const float a = *reinterpret_cast<const float*>(a_tile + (a_voff - a_half * 32) +
+                                                      (int64_t)(ka < valid ? full * 16 + ka : K - 1) * 4);
+      x[2][j] = ka < valid ? a : 0.0f;
       const float* row = reinterpret_cast<const float*>(
           b_tile + (int64_t)(kb < valid ? full * 16 + kb : K - 1) * ldb * 4 + b_voff[0]);
       const float b0 = row[0], b1 = row[1];
@@ -194,9 +184,9 @@ __global__ __launch_bounds__(256, 1) void f32_split_kernel(int M, int N, int K_t
 
   // ---- splitting -----------------------------------------------------------------------------
   const int r32 = l & 31;
-  const uint32_t rd_a = wm * MT * S::BLOCK + (l >> 5) * 512 + ((r32 ^ ((l >> 5) << 2)) << 4);
+  const uint32_t rd_a = (l >> 5) * 512 + ((r32 ^ ((l >> 5) << 2)) << 4);
   const uint32_t rd_b =
-      S::A_BYTES + wn * NT * S::BLOCK + (l >> 5) * 512 + (((r32 >> 1) ^ (r32 & 1 ? 20 : 0)) << 4);
+      S::A_BYTES + w * NT * S::BLOCK + (l >> 5) * 512 + (((r32 >> 1) ^ (r32 & 1 ? 20 : 0)) << 4);
   const uint32_t wr_a = (a_row >> 5) * S::BLOCK + a_half * 512 + (((a_row & 31) ^ (a_half << 2)) << 4);
   uint32_t wr_b[2];
 #pragma unroll
@@ -223,7 +213,7 @@ __global__ __launch_bounds__(256, 1) void f32_split_kernel(int M, int N, int K_t
   };
   auto put = [&](uint32_t slot, int task, int plane, u32x4 v) {
     const uint32_t at = task < 2 ? wr_b[task] + plane * S::B_BLOCKS * S::BLOCK
-                                 : wr_a + ((task - 2) * 4 + plane * S::A_BLOCKS) * S::BLOCK;
+                                 : wr_a + plane * S::A_BLOCKS * S::BLOCK;
     *reinterpret_cast<u32x4*>(lds + slot + at) = v;
   };
   u32x4 part;
@@ -254,20 +244,16 @@ __global__ __launch_bounds__(256, 1) void f32_split_kernel(int M, int N, int K_t
 
   // ---- prologue ------------------------------------------------------------------------------
   load_tail(raw[0], tail);
-  raw_t& second = raw[S::DEPTH - 1];
-  if constexpr (S::DEPTH == 1) split_stage(raw[0], 0);
-  if (first > 1) load_tail(second, 0); else load_stage(second);
-  if constexpr (S::DEPTH == 2) {
-    split_stage(raw[0], 0);
-    load_stage(raw[0]);
-  }
-  split_stage(second, S::SLOT);
-  load_stage(second);
+  if (first > 1) load_tail(raw[1], 0); else load_stage(raw[1]);
+  split_stage(raw[0], 0);
+  load_stage(raw[0]);
+  split_stage(raw[1], S::SLOT);
+  load_stage(raw[1]);
   barrier();
 
-  typename MathSplit<SUMS>::acc_t acc[MT][NT];
+  MathSplit::acc_t acc[MT][NT];
 #pragma unroll
-  for (int c = 0; c < SUMS; ++c)
+  for (int c = 0; c < 2; ++c)
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -292,24 +278,24 @@ __global__ __launch_bounds__(256, 1) void f32_split_kernel(int M, int N, int K_t
   // One stage: MFMAS slots of one matrix instruction and a handful of others.  `now` is multiplied,
   // `next` the stage after it, `to` the one after that, which the splitting fills.
   auto stage = [&](uint32_t now, uint32_t next, uint32_t to, auto u_) {
-    constexpr int CUR = decltype(u_)::value, RAW = CUR % S::DEPTH;
+    constexpr int CUR = decltype(u_)::value, P = S::PRODUCTS;
     constexpr int STEPS = 12 * S::TASKS, SPLIT_SLOTS = S::MFMAS - 2, BARRIER_SLOT = 1;
     // (nothing is written before the barrier behind which every wave is done with the stage before)
     static_assert(5 * SPLIT_SLOTS / STEPS > BARRIER_SLOT, "");
-    // part products, smallest first: (a part, b part).  The B fragments of the next stage replace
+    // part products, h h' last: (a part, b part).  The B fragments of the next stage replace
     // this one's in the last row block, each part behind its last use.
-    constexpr int PB[6] = {2, 1, 1, 0, 0, 0}, PA[6] = {0, 1, 0, 2, 1, 0};
+    constexpr int PB[P] = {2, 2, 1, 1, 1, 0, 0, 0}, PA[P] = {1, 0, 2, 1, 0, 2, 1, 0};
 #pragma unroll
-    for (int c = 0; c < SUMS; ++c)
+    for (int c = 0; c < 2; ++c)
 #pragma unroll
       for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j) asm volatile("" : "+a"(acc[i][j].part[c]));
     each_of([&](auto slot_) {
       constexpr int slot = decltype(slot_)::value;
-      constexpr int i = slot / (6 * NT), in_row = slot % (6 * NT), p = in_row / NT, j = in_row % NT;
+      constexpr int i = slot / (P * NT), in_row = slot % (P * NT), p = in_row / NT, j = in_row % NT;
       constexpr int fi = (i + CUR * MT) & 1;
-      f32x16& c = acc[i][j].part[SUMS == 2 && p < 5 ? SUMS - 1 : 0];
+      f32x16& c = acc[i][j].part[p < P - 1 ? 1 : 0];
       c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fb[PB[p]][j]),
                                                   __builtin_bit_cast(bf16x8, fa[fi][PA[p]]), c, 0, 0, 0);
       // fragments of the next row block, or of the next stage's first
@@ -317,25 +303,23 @@ __global__ __launch_bounds__(256, 1) void f32_split_kernel(int M, int N, int K_t
         constexpr int pl = (in_row - 3) / 2;
         fa[fi ^ 1][pl] = i + 1 < MT ? read_a(now, pl, i + 1) : read_a(next, pl, 0);
       }
-      if constexpr (i == MT - 1 && (p == 0 || p == 2 || p == 5)) {
-        constexpr int pl = p == 0 ? 2 : p == 2 ? 1 : 0;
+      if constexpr (i == MT - 1 && (p == 1 || p == 4 || p == 7)) {
+        constexpr int pl = p == 1 ? 2 : p == 4 ? 1 : 0;
         fb[pl][j] = read_b(next, pl, j);
       }
       each_of([&](auto step_) {
         constexpr int step = decltype(step_)::value;
-        if constexpr (step * SPLIT_SLOTS / STEPS == slot) split_step(raw[RAW], to, step / 12, step % 12);
+        if constexpr (step * SPLIT_SLOTS / STEPS == slot) split_step(raw[CUR], to, step / 12, step % 12);
       }, std::make_integer_sequence<int, STEPS>{});
       // the raw values of a later stage, into the registers the tasks have left
       constexpr int B_FROM = 24 * SPLIT_SLOTS / STEPS + 1, B_SPAN = 11 * SPLIT_SLOTS / STEPS;
       each_of([&](auto k_) {
         constexpr int k = decltype(k_)::value;
-        if constexpr (slot == B_FROM + k * B_SPAN / 8) load_b(raw[RAW], k);
+        if constexpr (slot == B_FROM + k * B_SPAN / 8) load_b(raw[CUR], k);
       }, std::make_integer_sequence<int, 8>{});
-      each_of([&](auto q_) {
-        constexpr int q = decltype(q_)::value, done = (12 * (3 + q) * SPLIT_SLOTS - 1) / STEPS + 1;
-        if constexpr (slot == done) load_a(raw[RAW], 2 + q, 0);
-        if constexpr (slot == done + 1) load_a(raw[RAW], 2 + q, 1);
-      }, std::make_integer_sequence<int, S::A_TASKS>{});
+      constexpr int A_FROM = (12 * S::TASKS * SPLIT_SLOTS - 1) / STEPS + 1;
+      if constexpr (slot == A_FROM) load_a(raw[CUR], 0);
+      if constexpr (slot == A_FROM + 1) load_a(raw[CUR], 1);
       if constexpr (slot == S::MFMAS - 1) advance();
       if constexpr (slot == BARRIER_SLOT) barrier();
       __builtin_amdgcn_sched_barrier(0);
@@ -345,57 +329,31 @@ __global__ __launch_bounds__(256, 1) void f32_split_kernel(int M, int N, int K_t
   uint32_t slot0 = 0, slot1 = S::SLOT, slot2 = 2 * S::SLOT, slot3 = (S::RING - 1) * S::SLOT;
   int s = 0;
   do {
-    if constexpr (S::RING == 3) {
-      each_of([&](auto u_) {
-        stage(slot0, slot1, slot2, u_);
-        const uint32_t was = slot0;
-        slot0 = slot1;
-        slot1 = slot2;
-        slot2 = was;
-      }, std::make_integer_sequence<int, S::TRIP>{});
-    } else {
-      stage(slot0, slot1, slot2, std::integral_constant<int, 0>{});
-      stage(slot1, slot2, slot3, std::integral_constant<int, 1>{});
-      const uint32_t was0 = slot0, was1 = slot1;
-      slot0 = slot2;
-      slot1 = slot3;
-      slot2 = was0;
-      slot3 = was1;
-    }
-    s += S::TRIP;
+    stage(slot0, slot1, slot2, std::integral_constant<int, 0>{});
+    stage(slot1, slot2, slot3, std::integral_constant<int, 1>{});
+    const uint32_t was0 = slot0, was1 = slot1;
+    slot0 = slot2;
+    slot1 = slot3;
+    slot2 = was0;
+    slot3 = was1;
+    s += 2;
   } while (s < stages);
 
   // ---- results -------------------------------------------------------------------------------
   // (one block at a time, kept where the matrix instructions left it: all of them in vector registers
   // at once would not fit)
-  if constexpr (SUMS == 2) {
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
+  for (int i = 0; i < MT; ++i)
 #pragma unroll
-      for (int j = 0; j < NT; ++j) {
-        acc[i][j].part[0] += acc[i][j].part[SUMS - 1];
-        asm volatile("" : "+a"(acc[i][j].part[0]));
-        __builtin_amdgcn_sched_barrier(0);
-      }
-  }
-  if constexpr (SUMS == 1) {
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-      for (int j = 0; j < NT; ++j) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          float v = acc[i][j].part[0][e];
-          asm volatile("" : "+a"(v));
-          acc[i][j].part[0][e] = v;
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-  }
+    for (int j = 0; j < NT; ++j) {
+      acc[i][j].part[0] += acc[i][j].part[1];
+      asm volatile("" : "+a"(acc[i][j].part[0]));
+      __builtin_amdgcn_sched_barrier(0);
+    }
   float check = 0.0f;  // NaN once a result was not finite
   __syncthreads();     // (every wave is past its last fragment read: store_tile uses the ring)
-  store_tile<MathSplit<SUMS>, MT, 4, S::TILE_M, ANY, NT>(EpiChecked<Epi>{epi, check}, acc, lds, w, wm, wn, m0,
-                                                         n0, M, N, 0.0f, 0.0f);
+  store_tile<MathSplit, MT, 4, S::TILE_M, true, NT>(EpiChecked<Epi>{epi, check}, acc, lds, w, 0, w, m0, n0, M,
+                                                    N, 0.0f, 0.0f);
   // ---- what the split cannot hold: the tile once more, in fp32 ---------------------------------
   if (check != 0.0f || least < (17u << 24) - 1) *vote = 1;
   __syncthreads();
@@ -410,12 +368,12 @@ __global__ __launch_bounds__(256, 1) void f32_split_kernel(int M, int N, int K_t
   int64_t ar[MT], bcol[NT];
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
-    const int64_t r = wm * 32 * MT + 32 * i + (l & 31), last = M - 1 - m0;
+    const int64_t r = 32 * i + (l & 31), last = M - 1 - m0;
     ar[i] = (m0 + (r < last ? r : last)) * lda;
   }
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
-    const int64_t c = n0 + wn * 32 * NT + 32 * j + (l & 31);
+    const int64_t c = n0 + w * 32 * NT + 32 * j + (l & 31);
     bcol[j] = c < N ? c : N - 1;
   }
   for (int k0 = 0; k0 < K; k0 += 2) {
@@ -435,7 +393,7 @@ __global__ __launch_bounds__(256, 1) void f32_split_kernel(int M, int N, int K_t
       for (int j = 0; j < NT; ++j)
         sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(bv[j], av[i], sum[i][j], 0, 0, 0);
   }
-  store_tile<MathF32, MT, 4, S::TILE_M, ANY, NT>(epi, sum, lds, w, wm, wn, m0, n0, M, N, 0.0f, 0.0f);
+  store_tile<MathF32, MT, 4, S::TILE_M, true, NT>(epi, sum, lds, w, 0, w, m0, n0, M, N, 0.0f, 0.0f);
 }
 
 }  // namespace tile

@@ -21,7 +21,7 @@ void launch_rows(cigemmContext* ctx, int rows, int64_t M, int64_t N, int64_t K, 
 #define CIG_ROWS(R) \
   case R: return split32::launch<R>(ctx, M, N, K, range_k, ranges, A, lda, B, ldb, epi)
   switch (rows) {
-    CIG_ROWS(64); CIG_ROWS(96); CIG_ROWS(160); CIG_ROWS(192); CIG_ROWS(224); CIG_ROWS(256);
+    CIG_ROWS(64); CIG_ROWS(96);
     default: return split32::launch<128>(ctx, M, N, K, range_k, ranges, A, lda, B, ldb, epi);
   }
 #undef CIG_ROWS
@@ -68,18 +68,59 @@ void launch_plan(cigemmContext* ctx, const split32::Plan& plan, bool any, int64_
   const bool split =
       ba ? run_plan(ctx, plan, M, N, K, A, lda, B, ldb, EpiBiasActAnyF32x4{C, ldc, ba->bias, ba->relu})
          : run_plan(ctx, plan, M, N, K, A, lda, B, ldb, EpiStoreF32x4{C, ldc});
-  auto ring = [](int rows) { return rows > 128 ? 3 : 4; };
-  char rows[32], rings[32];
-  if (ctx->first_tile_rows) {
+  const bool two = ctx->first_tile_rows != 0;
+  char rows[32];
+  if (two)
     snprintf(rows, sizeof(rows), "%d+%d", ctx->first_tile_rows, ctx->last_tile_rows);
-    snprintf(rings, sizeof(rings), "w4+w4_ring%d+%d", ring(ctx->first_tile_rows), ring(ctx->last_tile_rows));
-  } else {
+  else
     snprintf(rows, sizeof(rows), "%d", ctx->last_tile_rows);
-    snprintf(rings, sizeof(rings), "w4_ring%d", ring(ctx->last_tile_rows));
-  }
-  snprintf(ctx->kernel_name, sizeof(ctx->kernel_name), "f32_mfma_%s%sx256x16_%s%s%s", any ? "any_" : "", rows, rings,
-           ba ? "_bias_act" : "", split ? "_splitk" : "");
+  snprintf(ctx->kernel_name, sizeof(ctx->kernel_name), "f32_mfma_%s%sx256x16_%s_ring4%s%s", any ? "any_" : "", rows,
+           two ? "w4+w4" : "w4", ba ? "_bias_act" : "", split ? "_splitk" : "");
   ctx->last_kernel = ctx->kernel_name;
+}
+
+// What CIGEMM_ALGO_DEFAULT does with a call: `plan.rows` = 0 leaves it to the other kernels; `rest`: so many of the
+// last columns by the kernel of small outputs, the others by the plan.
+struct Choice {
+  split32::Plan plan;
+  int64_t rest;
+};
+
+// The two estimates err by 4 and 11 %.  Asked to be 8 % below, this kernel is taken for 1985 of 10154 random sizes
+// (M 16..20000, N 16..16384, K 17..16384, one launch), 1.13 times as fast (geometric mean), 14 of them more than 3 %
+// slower, and the choice is 0.6 % off the faster kernel on average (0.3 % and 44 sizes at 5 %).
+constexpr double MARGIN = 0.92;
+
+Choice choose(const cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, const float* B,
+              int64_t ldb, const float* C, int64_t ldc, const BiasAct* ba) {
+  const Choice none{split32::Plan{0, 1, 0, 0}, 0};
+  // A tile of up to 64 rows streams a long B more slowly than estimated (62 x 12032 x 7744 117 us, fp32
+  // instructions 107).  Below 3e8 products the estimates took three of 1962 sizes, none of them
+  // faster here, and they are host time.
+  if (M <= 64 || (double)M * (double)N * (double)K < 3e8) return none;
+  const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+  const size_t room = ctx->workspace ? ctx->ws_partial_bytes : 0;
+  // the kernel that serves the call otherwise
+  const F32Other other = f32_other(ctx, M, N, K, A, lda, B, ldb, C, ldc, ba);
+  double us = 0;
+  // (the kernel of small outputs' calls stay there: of its short sums only K in many ranges here is an equal,
+  // and one of 900 such sizes was more than 3 % faster)
+  if (any::tile_ok(M, N, K, 4, lda, ldb, true) && !(K <= 512 && f32_small_is_narrow(M, N, K, A, lda)) &&
+      kwaves::best_f32(M, N, K, cus, room, ctx->ws_counter_bytes, &us).splits && us < other.us)
+    return none;
+  const split32::Plan plan = split32::best(M, N, K, other.sum_length, cus, room, &us);
+  // Up to 64 columns beyond whole tiles: the kernel of small outputs (4095 x 4097 x 4099 793 us;
+  // the 4097th column as tiles over 8 ranges of K would take 50).
+  const int64_t rest = N % tile::BN, n1 = N - rest;
+  if (rest && rest <= 64 && n1) {
+    double main_us = 0, rest_us = 0;
+    const split32::Plan main = split32::best(M, n1, K, other.sum_length, cus, room, &main_us);
+    const kwaves::Plan p = kwaves::best_f32(M, rest, K, cus, room, ctx->ws_counter_bytes, &rest_us);
+    if (main.rows && p.splits && main_us + rest_us < us && main_us + rest_us < MARGIN * other.us)
+      return Choice{main, rest};
+  }
+  if (!plan.rows || us >= MARGIN * other.us) return none;
+  return Choice{plan, 0};
 }
 
 }  // namespace
@@ -95,47 +136,21 @@ bool launch_f32_split(cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const
   }
   // (a plan of another kernel is imposed)
   if (ctx->force_tile_rows || ctx->force_kwaves) return false;
-  // Below this no plan here was the faster one by more than 2 % (1000 sizes), and the estimates are host time.
-  if ((double)M * (double)N * (double)K < 1.5e8) return false;
-  const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
-  const size_t room = ctx->workspace ? ctx->ws_partial_bytes : 0;
-  // the kernel that serves the call otherwise
-  F32Other other = f32_other(ctx, M, N, K, A, lda, B, ldb, C, ldc, ba);
-  if (any::tile_ok(M, N, K, 4, lda, ldb, true) && !(K <= 512 && f32_small_is_narrow(M, N, K, A, lda))) {
-    double us = 0;
-    const kwaves::Plan p = kwaves::best_f32(M, N, K, cus, room, ctx->ws_counter_bytes, &us);
-    // (its tiles one a unit at most: two of 207 such sizes were more than 3 % faster here, by 6 and 14 %)
-    if (p.splits && us < other.us) {
-      if (any::div_up(M, kwaves::TM) * any::div_up(N, kwaves::TN_F32) <= cus) return false;
-      other = F32Other{us, any::div_up(any::div_up(K, p.splits), kwaves::WAVES)};
-    }
+  const Choice c = choose(ctx, M, N, K, A, lda, B, ldb, C, ldc, ba);
+  if (!c.plan.rows) return false;
+  if (!c.rest) {
+    launch_plan(ctx, c.plan, any, M, N, K, A, lda, B, ldb, C, ldc, ba);
+    return true;
   }
-  double us = 0;
-  split32::Plan plan = split32::best(M, N, K, other.sum_length, cus, room, &us);
-  // Up to 64 columns beyond whole tiles: the kernel of small outputs (4095 x 4097 x 4099 606 us;
-  // the 4097th column as tiles of 128 rows over 8 ranges of K would take 50).
-  const int64_t rest = N % tile::BN, n1 = N - rest;
-  if (rest && rest <= 64 && n1) {
-    double main_us = 0, rest_us = 0;
-    const split32::Plan main = split32::best(M, n1, K, other.sum_length, cus, room, &main_us);
-    const kwaves::Plan p = kwaves::best_f32(M, rest, K, cus, room, ctx->ws_counter_bytes, &rest_us);
-    BiasAct shifted{};
-    if (ba) shifted = BiasAct{ba->bias ? ba->bias + n1 : nullptr, ba->relu};
-    if (main.rows && p.splits && main_us + rest_us < us && main_us + rest_us < 0.92 * other.us &&
-        launch_kwaves_f32(ctx, M, rest, K, A, lda, B + n1, ldb, C + n1, ldc, ba ? &shifted : nullptr, true)) {
-      launch_plan(ctx, main, any, M, n1, K, A, lda, B, ldb, C, ldc, ba);
-      char first[sizeof(ctx->kernel_name)];
-      snprintf(first, sizeof(first), "%s", ctx->last_kernel);
-      name_rest_columns(ctx, first);
-      return true;
-    }
-  }
-  // The two estimates err by 5 and 11 %.  Asked to be 8 % below, this one is taken for 400 of 864 sizes of
-  // which 7 were slower by more than 3 %, and the choice is 0.3 % off the faster kernel on average (0.3 and
-  // 20 sizes without, 0.8 at 15 %).  A tile of up to 64 rows streams a long B more slowly than estimated
-  // (50 x 3200 x 7296 33.0 us, 29.3 on the kernel of small outputs).
-  if (!plan.rows || us >= (M <= 64 ? 0.83 : 0.92) * other.us) return false;
-  launch_plan(ctx, plan, any, M, N, K, A, lda, B, ldb, C, ldc, ba);
+  const int64_t n1 = N - c.rest;
+  BiasAct shifted{};
+  if (ba) shifted = BiasAct{ba->bias ? ba->bias + n1 : nullptr, ba->relu};
+  if (!launch_kwaves_f32(ctx, M, c.rest, K, A, lda, B + n1, ldb, C + n1, ldc, ba ? &shifted : nullptr, true))
+    return false;
+  launch_plan(ctx, c.plan, any, M, n1, K, A, lda, B, ldb, C, ldc, ba);
+  char first[sizeof(ctx->kernel_name)];
+  snprintf(first, sizeof(first), "%s", ctx->last_kernel);
+  name_rest_columns(ctx, first);
   return true;
 }
 

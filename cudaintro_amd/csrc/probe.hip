@@ -492,7 +492,7 @@ extern "C" cigemmStatus_t cigemm_probe_force_any_kernel(cigemmHandle_t h, int ke
 
 extern "C" cigemmStatus_t cigemm_probe_force_f32_split(cigemmHandle_t h, int tile_rows, int k_ranges) {
   if (!h || h->magic != kCtxMagic) return CIGEMM_STATUS_NOT_INITIALIZED;
-  if (tile_rows < -1 || (tile_rows > 0 && (tile_rows % 32 || tile_rows < 64 || tile_rows > 256 || k_ranges < 1 ||
+  if (tile_rows < -1 || (tile_rows > 0 && (tile_rows % 32 || tile_rows < 64 || tile_rows > 128 || k_ranges < 1 ||
                                            k_ranges > 64)))
     return fail(h, CIGEMM_STATUS_INVALID_VALUE, "cigemm_probe_force_f32_split: tile_rows %d, k_ranges %d", tile_rows,
                 k_ranges);

@@ -145,7 +145,7 @@ CIGEMM_API cigemmStatus_t cigemm_probe_force_kwaves_plan(cigemmHandle_t handle, 
  * The other algorithms choose as ever. */
 CIGEMM_API cigemmStatus_t cigemm_probe_force_any_kernel(cigemmHandle_t handle, int kernel);
 
-/* The same for the fp32 tiles on the bf16 matrix instructions: rows (64 to 256, a multiple of 32) and K
+/* The same for the fp32 tiles on the bf16 matrix instructions: rows (64, 96 or 128) and K
  * ranges of the handle's following fp32 calls under CIGEMM_ALGO_DEFAULT (those they take).  tile_rows = -1
  * keeps them out of every call, 0 hands the choice back to the library. */
 CIGEMM_API cigemmStatus_t cigemm_probe_force_f32_split(cigemmHandle_t handle, int tile_rows, int k_ranges);

@@ -10,8 +10,8 @@ using namespace cig;
 static bool launch_ok(long long M, long long N, long long K, int rows, int wanted, long long length, size_t room) {
   int64_t range_k = 0;
   const int ranges = split32::k_ranges(K, wanted, &range_k);
-  bool ok = rows >= 64 && rows <= 256 && rows % 32 == 0 && ranges >= 1 && ranges <= wanted &&
-            range_k <= split32::range_limit(rows, length);
+  bool ok = rows >= 64 && rows <= 128 && rows % 32 == 0 && ranges >= 1 && ranges <= wanted &&
+            range_k <= length + length / 4;
   if (ranges == 1) return ok && range_k == K;
   const long long last = K - (ranges - 1) * range_k;
   return ok && range_k % 16 == 0 && range_k >= 32 && last >= 17 && last <= range_k &&
@@ -40,7 +40,7 @@ int main() {
             if (p.first_cols)
               ok = ok && p.first_cols % 256 == 0 && p.first_cols > 0 && p.first_cols < N &&
                    launch_ok(M, p.first_cols, K, p.first_rows, 1, length, room);
-            // unsplit two-sum tiles always may, with the whole K as the other kernel's sum
+            // (with the whole K as the other kernel's sum one range always may)
             if (length == K) ok = ok && p.rows;
             if (!ok) {
               std::printf("FAILED %lld %lld %lld length %lld room %zu: rows %d ranges %d first %lld x %d\n", M, N, K,

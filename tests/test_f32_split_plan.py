@@ -21,19 +21,17 @@ def test_plan(tmp_path):
 
 
 @pytest.mark.skipif(HIPCC is None, reason="hipcc not installed")
-@pytest.mark.parametrize("rows", [128, 256])
+@pytest.mark.parametrize("rows", [64, 96, 128])
 def test_main_loop_does_not_spill(tmp_path, rows):
     """The running sums fill the accumulator registers: the main loop must neither move them nor go to
     scratch memory."""
-    make = open(os.path.join(CSRC, "Makefile")).read()
-    shape = re.search(rf"^SPLIT_{rows}\s*:= (\S+)", make, re.M)[1]
     asm = tmp_path / "split.s"
-    subprocess.run([HIPCC, *FLAGS, f"-DCIG_SPLIT_ROWS={rows}", f"-DCIG_SPLIT_SHAPE={shape}",
-                    os.path.join(CSRC, "f32_split_rows.hip"), "-o", str(asm)], check=True, stderr=subprocess.DEVNULL)
+    subprocess.run([HIPCC, *FLAGS, f"-DCIG_SPLIT_ROWS={rows}", os.path.join(CSRC, "f32_split_rows.hip"), "-o", str(asm)],
+                   check=True, stderr=subprocess.DEVNULL)
     text = asm.read_text()
     spills = spill_counts(text)
-    assert len(spills) == 3 and max(spills.values()) <= 12, spills   # (256 rows: in the epilogue)
-    loops = [b for b in re.split(r"\n(?=\.LBB)", text) if b.count("v_mfma_f32_32x32x16_bf16") >= 96]
+    assert len(spills) == 3 and not any(spills.values()), spills
+    loops = [b for b in re.split(r"\n(?=\.LBB)", text) if b.count("v_mfma_f32_32x32x16_bf16") >= rows]
     assert len(loops) == 3
     for body in loops:
         body = body[:body.rindex("v_mfma_f32_32x32x16_bf16")]

@@ -3,6 +3,8 @@ height with one and several K ranges at the edges of tiles, stages and column pa
 and third parts matter, and what the three parts cannot hold (infinities, NaN, the largest and the smallest
 magnitudes), which the kernel computes once more in fp32.  NaN padding around the operands, the output in
 a sentinel-filled buffer."""
+import re
+
 import numpy as np
 import pytest
 
@@ -12,7 +14,7 @@ from test_gpu_mfma_any import embed
 
 pytestmark = pytest.mark.gpu
 
-ROWS = (64, 96, 128, 160, 192, 224, 256)
+ROWS = (64, 96, 128)
 
 
 @pytest.fixture(autouse=True)
@@ -77,30 +79,91 @@ def test_one_hot_operands_select_all_24_bits(handle, torch_gpu, rng, rows):
     np.testing.assert_array_equal(got, Y[take], err_msg=what)
 
 
+def on_fp32_instructions(handle, torch, A, B, ranges=1):
+    """The same call on the tiles of v_mfma_f32_32x32x2_f32."""
+    probe.force_f32_split(handle, 0)
+    probe.force_tile_plan(handle, 256, ranges)
+    try:
+        with handle.algo(ci.ALGO_TILE):
+            out = handle.gemm_f32(torch.from_numpy(A).cuda(), torch.from_numpy(B).cuda()).cpu().numpy()
+            assert "32x32x2" in handle.last_kernel and handle.last_plan == (256, ranges)
+    finally:
+        probe.force_tile_plan(handle, 0)
+    return out
+
+
+def nonzeros(rng, M, K, count):
+    """Rows of `count` values at random places, zero elsewhere."""
+    A = np.zeros((M, K), np.float32)
+    for row in A:
+        row[rng.choice(K, count, replace=False)] = rng.uniform(-1, 1, count)
+    return A
+
+
 @pytest.mark.parametrize("rows", ROWS)
-@pytest.mark.parametrize("kind", ["symmetric", "positive", "wide"])
+@pytest.mark.parametrize("kind", ["symmetric", "positive", "wide", "half zeros", "fifth", "8", "2", "dominating"])
 def test_no_further_from_64_bits_than_the_fp32_instructions(handle, torch_gpu, rng, rows, kind):
     """The same call on the tiles of v_mfma_f32_32x32x2_f32 is the measure, error by sum of magnitudes, over
     131072 outputs; 1 % for the draw."""
     torch = torch_gpu
     M, N = 256, 512
     for K in (64, 700, 4096):
-        draw = {"symmetric": lambda s: rng.uniform(-1, 1, s), "positive": lambda s: rng.uniform(0, 1, s),
-                "wide": lambda s: rng.normal(size=s) * np.exp(3 * rng.normal(size=s))}[kind]
+        draw = {"positive": lambda s: rng.uniform(0, 1, s),
+                "wide": lambda s: rng.normal(size=s) * np.exp(3 * rng.normal(size=s))}.get(
+                    kind, lambda s: rng.uniform(-1, 1, s))
         A, B = draw((M, K)).astype(np.float32), draw((K, N)).astype(np.float32)
+        count = {"half zeros": K // 2, "fifth": K // 5, "8": 8, "2": 2}.get(kind)
+        if count:
+            A = nonzeros(rng, M, K, count)
+        if kind == "dominating":
+            A[:, 1:] *= np.float32(2.0 ** -14)
         ref = A.astype(np.float64) @ B.astype(np.float64)
         got, what = run(handle, torch, A, B, rows, 1, 0, 0)
-        probe.force_f32_split(handle, 0)
-        probe.force_tile_plan(handle, 256, 1)
-        try:
-            with handle.algo(ci.ALGO_TILE):
-                old = handle.gemm_f32(torch.from_numpy(A).cuda(), torch.from_numpy(B).cuda()).cpu().numpy()
-                assert "32x32x2" in handle.last_kernel
-        finally:
-            probe.force_tile_plan(handle, 0)
+        old = on_fp32_instructions(handle, torch, A, B)
         size = np.abs(A.astype(np.float64)) @ np.abs(B.astype(np.float64))
         err, err_old = np.linalg.norm((got - ref) / size), np.linalg.norm((old - ref) / size)
         assert err <= 1.01 * err_old, (what, err / err_old)
+
+
+@pytest.mark.parametrize("rows", ROWS)
+def test_a_lone_product_is_rounded_once(handle, torch_gpu, rng, rows):
+    """Scaled permutations and diagonals of 24-bit factors.  The large part product is exact, and the sum of the seven
+    smaller ones, below 2^-7 of it, is rounded seven times: 0.5 + 7 * 2^-8 units in the last place at most.
+    The root mean square is that of a rounding, as the fp32 instructions', to 0.1 %."""
+    torch = torch_gpu
+    M, N, K = 2 * rows + 5, 512, 256
+    for ranges in (1, 2):
+        diagonal = np.zeros((K, N), np.float32)
+        cols = rng.permutation(N)
+        diagonal[np.arange(N) % K, cols] = rng.uniform(1, 4, N)
+        X = rng.normal(size=(M, K)).astype(np.float32)
+        for A, B in ((X, diagonal), (nonzeros(rng, M, K, 1), rng.normal(size=(K, N)).astype(np.float32))):
+            got, what = run(handle, torch, A, B, rows, ranges, 1, 3)
+            ref = A.astype(np.float64) @ B.astype(np.float64)          # one product of 48 bits: exact
+            ulp = np.exp2(np.floor(np.log2(np.abs(ref))) - 23)
+            off = np.abs(got - ref) / ulp
+            old = np.abs(ref.astype(np.float32) - ref) / ulp
+            assert off.max() <= 0.5 + 7 * 2.0 ** -8, (what, off.max())
+            assert np.sqrt((off ** 2).mean()) <= 1.001 * np.sqrt((old ** 2).mean()), what
+
+
+@pytest.mark.parametrize("M,N,K", [(256, 4096, 4096), (700, 3000, 1000), (2048, 2048, 2048)])
+def test_sums_get_no_longer_than_the_kernels_it_takes_the_place_of(handle, torch_gpu, M, N, K):
+    """Positive operands, whose error grows with the length of a sum: the library's own choice against what serves
+    the call without these tiles."""
+    torch = torch_gpu
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    for zeros in (0.0, 0.8):
+        A, B = torch.rand((M, K), generator=gen, device="cuda"), torch.rand((K, N), generator=gen, device="cuda")
+        A *= torch.rand((M, K), generator=gen, device="cuda") >= zeros
+        ref = A.double() @ B.double()
+        got = handle.gemm_f32(A, B)
+        assert "x256x16_w4" in handle.last_kernel and "32x32x2" not in handle.last_kernel, handle.last_kernel
+        probe.force_f32_split(handle, -1)
+        old = handle.gemm_f32(A, B)
+        assert "x256x16_w4" not in handle.last_kernel or "32x32x2" in handle.last_kernel
+        probe.force_f32_split(handle, 0)
+        assert float((got - ref).norm()) <= 1.01 * float((old - ref).norm()), zeros
 
 
 @pytest.mark.parametrize("rows", ROWS)
@@ -135,25 +198,30 @@ def test_tiny_values_anywhere_are_not_lost(handle, torch_gpu, rng):
     A = (rng.uniform(0.5, 1, size=(M, K)) * 2.0 ** -122).astype(np.float32)
     B = (rng.uniform(0.5, 1, size=(K, N)) * 2.0 ** 100).astype(np.float32)
     ref = A.astype(np.float64) @ B.astype(np.float64)
-    for rows in (64, 160, 256):
+    for rows in ROWS:
         got, what = run(handle, torch_gpu, A, B, rows, 1, 0, 0)
         np.testing.assert_allclose(got, ref, rtol=1e-6, err_msg=what)
 
 
 def test_default_takes_it_where_it_pays_and_graphs_replay(handle, torch_gpu, rng):
-    """The library's own choice on a size of two launches, one of K ranges and one with the remaining column
-    on the kernel of small outputs, recorded and replayed with other work between."""
+    """The library's own choice on a size of two launches, one of K ranges and two (one a layer with bias) with the
+    remaining column on the kernel of small outputs, recorded and replayed with other work between."""
     torch = torch_gpu
-    sizes = ((1142, 2560, 661), (152, 4096, 2208), (1030, 2817, 515))
-    ops = [(torch.rand((M, K), device="cuda") - 0.5, torch.rand((K, N), device="cuda") - 0.5,
-            torch.empty((M, N), device="cuda")) for M, N, K in sizes]
+    draw = lambda *s: torch.rand(s, device="cuda") - 0.5  # noqa: E731
+    sizes = ((1300, 6000, 1500, None), (256, 4096, 4096, None), (4095, 4097, 1031, None), (4095, 4097, 1031, draw(4097)))
+    plans = (r"f32_mfma_128\+64x256x16_w4\+w4_ring4_splitk", r"f32_mfma_128x256x16_w4_ring4_splitk",
+             r"f32_mfma_any_128x256x16_w4_ring4\+32x32", r"f32_mfma_any_128x256x16_w4_ring4_bias_act\+32x32")
+    ops = [(draw(M, K), draw(K, N), torch.empty((M, N), device="cuda"), bias) for M, N, K, bias in sizes]
     side = torch.cuda.Stream()
     h = ci.Handle(stream=side)
 
     def sequence():
         names = []
-        for a, b, out in ops:
-            h.gemm_f32(a, b, out=out)
+        for a, b, out, bias in ops:
+            if bias is None:
+                h.gemm_f32(a, b, out=out)
+            else:
+                h.linear_f32(a, b, bias, ci.ACT_RELU, out=out)
             names.append(h.last_kernel)
         return names
 
@@ -161,11 +229,15 @@ def test_default_takes_it_where_it_pays_and_graphs_replay(handle, torch_gpu, rng
     with torch.cuda.stream(side):
         names = sequence()
     side.synchronize()
-    assert all("x256x16_w4" in n and "32x32x2" not in n for n in names), names
+    for name, plan in zip(names, plans):
+        assert re.fullmatch(plan, name), (name, plan)
     eager = [o[2].clone() for o in ops]
-    for (a, b, _), got in zip(ops, eager):
+    for (a, b, _, bias), got in zip(ops, eager):
         ref = a.double() @ b.double()
-        assert float((got - ref).abs().max()) <= 1e-5 * float(ref.pow(2).mean().sqrt()) * 4
+        bound = 1e-5 * float(ref.pow(2).mean().sqrt()) * 4
+        if bias is not None:
+            ref = (ref + bias).clamp_min(0)
+        assert float((got - ref).abs().max()) <= bound
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph, stream=side):
         sequence()
