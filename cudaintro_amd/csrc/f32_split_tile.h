@@ -16,9 +16,13 @@
 // range_limit).
 //
 // What three parts cannot hold: infinities and NaN (x - h is NaN), magnitudes that bf16 rounds to infinity,
-// and below 2^-110, where the last part falls short of bf16's subnormals.  A workgroup that met a nonzero
-// value below 2^-110 or got a result that is not finite computes its tile once more with the fp32
-// instructions, straight from memory (slow, about twice the tile's time, and only there).
+// and below 2^-110, where the last part falls short of bf16's subnormals: there up to 2^-134 of the value is lost, and
+// of a result K 2^-133 times the largest magnitude of the tile's operands.  A workgroup that got a result that is not
+// finite, or met such small values and got a result of which that would be more than 2^-34, computes its tile
+// once more with the fp32 instructions, straight from memory, on top of the first pass.  (So a small value among
+// ordinary ones, the tail of a softmax or a decayed weight, changes nothing, unless a row or column of the
+// tile gives zero or next to it.)  us, 4096^3 with a value in every
+// 64th row: 1e-35 813 (809 without; every tile again 2283), NaN 2014 (fp32 instructions 905).
 //
 // Workgroup = 256 lanes = 4 waves, tile of 64, 96 or 128 rows x 256 columns, stages of 16 k.  Values go from
 // memory to registers (8 k of one row of A; 8 k of two columns of B, so that the matrix instruction's
@@ -31,8 +35,8 @@
 // load) is pinned.
 //
 // What bounds it: the chip's power.  The main loop takes the same cycles with one workgroup and with all units at
-// work, the clock falls from 2.3 to 1.4 GHz.  fp32 instructions -> here, one process, us: 4096^3 898 -> 762, 4095 x 4097 x 4099
-// 928 -> 793, 256 x 8192 x 8192 239 -> 219.
+// work, the clock falls from 2.3 to 1.4 GHz.  fp32 instructions -> here, one process, us: 4096^3 905 -> 809, 4095 x 4097 x 4099
+// 930 -> 838, 256 x 8192 x 8192 244 -> 226.
 #pragma once
 
 #include "mfma_tile.h"
@@ -70,17 +74,19 @@ struct MathSplit {
     __device__ __forceinline__ float operator[](int e) const { return part[0][e]; }
   };
 };
-// An epilogue that also notes whether any value was infinite or not a number.
+// An epilogue that also notes whether any value was infinite or not a number, and the smallest magnitude.
 template <typename Epi>
 struct EpiChecked : Epi {
-  float& check;
-  __device__ __forceinline__ EpiChecked(const Epi& e, float& c) : Epi(e), check(c) {}
+  float &check, &smallest;
+  __device__ __forceinline__ EpiChecked(const Epi& e, float& c, float& s) : Epi(e), check(c), smallest(s) {}
   template <typename R, typename C>
   __device__ __forceinline__ u32x4 pack(R r, C c, float v0, float v1, float v2, float v3) const {
     check = __builtin_fmaf(v0, 0.0f, check);
     check = __builtin_fmaf(v1, 0.0f, check);
     check = __builtin_fmaf(v2, 0.0f, check);
     check = __builtin_fmaf(v3, 0.0f, check);
+    smallest = __builtin_fminf(__builtin_fminf(smallest, __builtin_fabsf(v0)), __builtin_fabsf(v1));
+    smallest = __builtin_fminf(__builtin_fminf(smallest, __builtin_fabsf(v2)), __builtin_fabsf(v3));
     return Epi::pack(r, c, v0, v1, v2, v3);
   }
 };
@@ -102,8 +108,9 @@ __global__ __launch_bounds__(256, 1) void f32_split_kernel(int M, int N, int K_t
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int t = threadIdx.x, l = t & 63;
   const int w = __builtin_amdgcn_readfirstlane(t >> 6);
-  volatile int* const vote = reinterpret_cast<volatile int*>(lds + S::RING * S::SLOT);
-  if (t == 0) *vote = 0;
+  // the workgroup's: results not finite, values below 2^-110 met, largest operand, smallest result (bits)
+  uint32_t* const vote = reinterpret_cast<uint32_t*>(lds + S::RING * S::SLOT);
+  if (t < 4) vote[t] = t < 3 ? 0 : 0x7f800000;
   int tm, tn;
   tile_of_workgroup(tiles_m, tiles_n, tm, tn);
   tm = __builtin_amdgcn_readfirstlane(tm);
@@ -123,7 +130,8 @@ __global__ __launch_bounds__(256, 1) void f32_split_kernel(int M, int N, int K_t
   const int b_back = b_left == 1 ? 1 : 0;
   uint32_t a_voff, b_voff[8];
   {
-    const int64_t last = M - 1 - m0;
+    // (rows past the tile's re-read its last one)
+    const int64_t last = M - m0 < S::TILE_M ? M - m0 - 1 : S::TILE_M - 1;
     a_voff = (uint32_t)((a_row < last ? a_row : last) * lda * 4) + a_half * 32;
     // (columns past N - 2 fetch the last two: what no row holds is read nowhere)
     const int64_t c = b_col < b_left - 2 ? b_col : b_left - 2;
@@ -199,16 +207,18 @@ __global__ __launch_bounds__(256, 1) void f32_split_kernel(int M, int N, int K_t
     wr_b[1] = even;
   }
   uint32_t least = 0xffffffffu;
+  float most = 0.0f;
   auto part_of = [&](const float (&x)[8], int i) { return f32x2_to_bf16_bits(x[2 * i], x[2 * i + 1]); };
   auto rest_of = [&](float (&x)[8], uint32_t h, int i) {
     x[2 * i] -= __builtin_bit_cast(float, h << 16);
     x[2 * i + 1] -= __builtin_bit_cast(float, h & 0xffff0000u);
   };
-  // (twice the magnitude's bits less one: zero comes out largest)
+  // smallest nonzero magnitude (twice its bits less one: zero comes out largest) and largest one
   auto watch = [&](const float (&x)[8], int i) {
     uint32_t u, v;
-    asm volatile("v_lshl_add_u32 %1, %3, 1, -1\n\tv_lshl_add_u32 %2, %4, 1, -1\n\tv_min3_u32 %0, %0, %1, %2"
-                 : "+v"(least), "=&v"(u), "=&v"(v)
+    asm volatile("v_lshl_add_u32 %2, %4, 1, -1\n\tv_lshl_add_u32 %3, %5, 1, -1\n\tv_min3_u32 %0, %0, %2, %3\n\t"
+                 "v_max3_f32 %1, %1, |%4|, |%5|"
+                 : "+v"(least), "+v"(most), "=&v"(u), "=&v"(v)
                  : "v"(x[2 * i]), "v"(x[2 * i + 1]));
   };
   auto put = [&](uint32_t slot, int task, int plane, u32x4 v) {
@@ -351,13 +361,23 @@ __global__ __launch_bounds__(256, 1) void f32_split_kernel(int M, int N, int K_t
       __builtin_amdgcn_sched_barrier(0);
     }
   float check = 0.0f;  // NaN once a result was not finite
+  float smallest = __builtin_inff();
   __syncthreads();     // (every wave is past its last fragment read: store_tile uses the ring)
-  store_tile<MathSplit, MT, 4, S::TILE_M, true, NT>(EpiChecked<Epi>{epi, check}, acc, lds, w, 0, w, m0, n0, M,
-                                                    N, 0.0f, 0.0f);
+  store_tile<MathSplit, MT, 4, S::TILE_M, true, NT>(EpiChecked<Epi>{epi, check, smallest}, acc, lds, w, 0, w, m0, n0,
+                                                    M, N, 0.0f, 0.0f);
   // ---- what the split cannot hold: the tile once more, in fp32 ---------------------------------
-  if (check != 0.0f || least < (17u << 24) - 1) *vote = 1;
+  if (check != 0.0f) vote[0] = 1;
+  if (least < (17u << 24) - 1) vote[1] = 1;
   __syncthreads();
-  if (!__builtin_amdgcn_readfirstlane(*vote)) return;
+  if (!__builtin_amdgcn_readfirstlane(vote[0])) {
+    if (!__builtin_amdgcn_readfirstlane(vote[1])) return;
+    atomicMax(&vote[2], __builtin_bit_cast(uint32_t, most));
+    atomicMin(&vote[3], __builtin_bit_cast(uint32_t, smallest));
+    __syncthreads();
+    const float largest_operand = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(vote[2]));
+    const float smallest_result = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(vote[3]));
+    if (smallest_result >= (float)K * 0x1p-99f * largest_operand) return;
+  }
   f32x16 sum[MT][NT];
 #pragma unroll
   for (int i = 0; i < MT; ++i)
@@ -365,34 +385,58 @@ __global__ __launch_bounds__(256, 1) void f32_split_kernel(int M, int N, int K_t
     for (int j = 0; j < NT; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) sum[i][j][e] = 0.0f;
-  int64_t ar[MT], bcol[NT];
+  const float *arow[MT], *bcol[NT];
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
     const int64_t r = 32 * i + (l & 31), last = M - 1 - m0;
-    ar[i] = (m0 + (r < last ? r : last)) * lda;
+    arow[i] = A + (m0 + (r < last ? r : last)) * lda;
   }
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
     const int64_t c = n0 + w * 32 * NT + 32 * j + (l & 31);
-    bcol[j] = c < N ? c : N - 1;
+    bcol[j] = B + (c < N ? c : N - 1);
   }
-  for (int k0 = 0; k0 < K; k0 += 2) {
-    const int k = k0 + (l >> 5), kc = k < K ? k : K - 1;
-    float av[MT], bv[NT];
+  // Eight of k at a time, a lane 4 in a row; the next ones are fetched under the multiplies (2048 cycles for 128
+  // rows).  The last 1..8 of k element by element.
+  struct Eight {
+    float a[MT][4], b[NT][4];
+  };
+  auto fetch = [&](Eight& x, int k) {
 #pragma unroll
-    for (int i = 0; i < MT; ++i) av[i] = A[ar[i] + kc];
+    for (int i = 0; i < MT; ++i) __builtin_memcpy(x.a[i], arow[i] + k, 16);
 #pragma unroll
-    for (int j = 0; j < NT; ++j) bv[j] = B[kc * ldb + bcol[j]];
+    for (int j = 0; j < NT; ++j)
 #pragma unroll
-    for (int i = 0; i < MT; ++i) av[i] = k < K ? av[i] : 0.0f;
+      for (int e = 0; e < 4; ++e) x.b[j][e] = bcol[j][(int64_t)(k + e) * ldb];
+  };
+  auto multiply = [&](const Eight& x) {
 #pragma unroll
-    for (int j = 0; j < NT; ++j) bv[j] = k < K ? bv[j] : 0.0f;
+    for (int e = 0; e < 4; ++e)
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
+      for (int i = 0; i < MT; ++i)
 #pragma unroll
-      for (int j = 0; j < NT; ++j)
-        sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(bv[j], av[i], sum[i][j], 0, 0, 0);
+        for (int j = 0; j < NT; ++j)
+          sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x.b[j][e], x.a[i][e], sum[i][j], 0, 0, 0);
+  };
+  const int eights = (K - 1) / 8, k_lane = 4 * (l >> 5);  // (K is 17 at least)
+  Eight x, next;
+  fetch(x, k_lane);
+  for (int g = 0; g < eights; ++g) {
+    fetch(next, 8 * (g + 1 < eights ? g + 1 : g) + k_lane);
+    __builtin_amdgcn_sched_barrier(0);  // (the loads stay in front of the multiplies)
+    multiply(x);
+    __builtin_amdgcn_sched_barrier(0);
+    x = next;
   }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int k = 8 * eights + k_lane + e, kc = k < K ? k : K - 1;
+#pragma unroll
+    for (int i = 0; i < MT; ++i) x.a[i][e] = k < K ? arow[i][kc] : 0.0f;
+#pragma unroll
+    for (int j = 0; j < NT; ++j) x.b[j][e] = k < K ? bcol[j][(int64_t)kc * ldb] : 0.0f;
+  }
+  multiply(x);
   store_tile<MathF32, MT, 4, S::TILE_M, true, NT>(epi, sum, lds, w, 0, w, m0, n0, M, N, 0.0f, 0.0f);
 }
 

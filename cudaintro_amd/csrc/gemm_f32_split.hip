@@ -109,7 +109,7 @@ Choice choose(const cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const f
       kwaves::best_f32(M, N, K, cus, room, ctx->ws_counter_bytes, &us).splits && us < other.us)
     return none;
   const split32::Plan plan = split32::best(M, N, K, other.sum_length, cus, room, &us);
-  // Up to 64 columns beyond whole tiles: the kernel of small outputs (4095 x 4097 x 4099 793 us;
+  // Up to 64 columns beyond whole tiles: the kernel of small outputs (4095 x 4097 x 4099 838 us;
   // the 4097th column as tiles over 8 ranges of K would take 50).
   const int64_t rest = N % tile::BN, n1 = N - rest;
   if (rest && rest <= 64 && n1) {

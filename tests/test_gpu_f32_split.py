@@ -147,6 +147,50 @@ def test_a_lone_product_is_rounded_once(handle, torch_gpu, rng, rows):
             assert np.sqrt((off ** 2).mean()) <= 1.001 * np.sqrt((old ** 2).mean()), what
 
 
+@pytest.mark.parametrize("rows", ROWS)
+def test_tiny_values_beside_ordinary_ones_cost_nothing(handle, torch_gpu, rng, rows):
+    """Values below 2^-110 that no result can show (a softmax's tail): bit for bit the product with zeros in their
+    place, which a tile computed once more in fp32 is not (shown by a NaN in one row)."""
+    torch = torch_gpu
+    M, N, K = 2 * rows + 5, 300, 203
+    X, Y = rng.normal(size=(M, K)).astype(np.float32), rng.normal(size=(K, N)).astype(np.float32)
+    bias = rng.normal(size=N).astype(np.float32)
+    tiny = np.array([1e-34, -1e-35, 1e-42, -1e-45], np.float32)
+    for ranges, b in ((1, None), (2, None), (1, bias)):
+        for where in ("A", "B"):
+            A, B, zeros = X.copy(), Y.copy(), [X.copy(), Y.copy()]
+            T, Z = (A, zeros[0]) if where == "A" else (B, zeros[1])
+            at = rng.integers(0, T.size, 400)
+            T.flat[at], Z.flat[at] = tiny[rng.integers(0, 4, 400)], 0
+            got, what = run(handle, torch, A, B, rows, ranges, 1, 3, b)
+            want, _ = run(handle, torch, *zeros, rows, ranges, 1, 3, b)
+            np.testing.assert_array_equal(got, want, err_msg=f"{what} {where}")
+    again = X.copy()
+    again[3] = np.nan
+    got, _ = run(handle, torch, again, Y, rows, 1, 1, 3)
+    want, _ = run(handle, torch, X, Y, rows, 1, 1, 3)
+    assert (got[:rows] != want[:rows]).mean() > 0.1 and (got[rows:] == want[rows:]).all()
+
+
+@pytest.mark.parametrize("rows", ROWS)
+def test_only_the_tile_that_loses_something_is_computed_again(handle, torch_gpu, rng, rows):
+    """A row of zeros in the first tile of rows (results that any loss would be large beside), tiny values in the
+    second: the first one's other rows keep their bits."""
+    torch = torch_gpu
+    M, N, K = 3 * rows, 260, 150
+    A, B = rng.normal(size=(M, K)).astype(np.float32), rng.normal(size=(K, N)).astype(np.float32)
+    A[5] = 0
+    want, _ = run(handle, torch, A, B, rows, 1, 0, 4)
+    A[rows:2 * rows, 7] = 1e-36
+    got, what = run(handle, torch, A, B, rows, 1, 0, 4)
+    np.testing.assert_array_equal(got[:rows], want[:rows], err_msg=what)
+    # with a small row beside them, whose results the loss would show in: all of it, to fp32's precision
+    A[rows + 9] = (rng.uniform(0.5, 1, K) * 2.0 ** -125).astype(np.float32)
+    got, what = run(handle, torch, A, np.abs(B), rows, 1, 0, 4)
+    ref = A.astype(np.float64) @ np.abs(B).astype(np.float64)
+    np.testing.assert_allclose(got[rows + 9], ref[rows + 9], rtol=1e-5, err_msg=what)   # (2^-149 of some 2^-122)
+
+
 @pytest.mark.parametrize("M,N,K", [(256, 4096, 4096), (700, 3000, 1000), (2048, 2048, 2048)])
 def test_sums_get_no_longer_than_the_kernels_it_takes_the_place_of(handle, torch_gpu, M, N, K):
     """Positive operands, whose error grows with the length of a sum: the library's own choice against what serves
