@@ -216,7 +216,7 @@ def test_infinities_nan_and_extreme_magnitudes(handle, torch_gpu, rng, rows):
     it reaches are those of float64 rounded to fp32, NaN and the sign of infinity included."""
     M, N, K = rows + 3, 270, 75
     big = np.float32(np.finfo(np.float32).max)
-    for value in (np.inf, -np.inf, np.nan, big, -big, np.float32(2.0 ** -120), np.float32(2.0 ** -145)):
+    for value in (np.inf, -np.inf, np.nan, big, -big, np.float32(1.2345678 * 2.0 ** -120), np.float32(2.0 ** -145)):
         for where in ("A", "B"):
             A = rng.choice([-1.0, 0.5, 1.0], size=(M, K)).astype(np.float32)
             B = rng.choice([-1.0, 0.5, 1.0], size=(K, N)).astype(np.float32)
@@ -234,6 +234,43 @@ def test_infinities_nan_and_extreme_magnitudes(handle, torch_gpu, rng, rows):
                 with np.errstate(all="ignore"):
                     ref = (A.astype(np.float64) @ B.astype(np.float64)).astype(np.float32)
                 np.testing.assert_allclose(got, ref, rtol=2e-6, atol=0, err_msg=f"{what} {value} in {where}")
+
+
+@pytest.mark.parametrize("rows", ROWS)
+@pytest.mark.parametrize("exponent", [-100, -102, -103, -106, -109, -110, -111, -118, -126, -133])
+def test_lower_edge_of_the_parts(handle, torch_gpu, rng, rows, exponent):
+    """Factors of 24 bits around 2^-110, whose third part is a subnormal bf16 number or lost, selected by one power of two
+    of the other operand: bit for bit (2^100 scales nothing away)."""
+    M, N, K = rows + 3, 259, 70
+    scale = np.float32(2.0 ** 100)
+    X = (rng.uniform(1, 2, size=(M, K)) * rng.choice([-1, 1], size=(M, K)) * 2.0 ** exponent).astype(np.float32)
+    take = rng.integers(0, K, size=N)
+    W = np.zeros((K, N), np.float32)
+    W[take, np.arange(N)] = scale
+    got, what = run(handle, torch_gpu, X, W, rows, 1, 1, 3)
+    np.testing.assert_array_equal(got, X[:, take] * scale, err_msg=what)
+    Y = (rng.uniform(1, 2, size=(K, N)) * 2.0 ** exponent).astype(np.float32)
+    take = rng.integers(0, K, size=M)
+    S = np.zeros((M, K), np.float32)
+    S[np.arange(M), take] = -scale
+    got, what = run(handle, torch_gpu, S, Y, rows, 2, 0, 4)
+    np.testing.assert_array_equal(got, Y[take] * -scale, err_msg=what)
+
+
+@pytest.mark.parametrize("rows", ROWS)
+@pytest.mark.parametrize("exponent", [-108, -118, -122, -126, -130, -140])
+def test_products_of_ordinary_values_near_the_smallest_numbers(handle, torch_gpu, rng, rows, exponent):
+    """Lone products around 2^exponent, whose smaller part products are subnormal sums: as close as a product of
+    ordinary size (test_a_lone_product_is_rounded_once) plus eight roundings to 2^-149."""
+    M, N, K = rows + 3, 259, 70
+    half = exponent // 2
+    A = nonzeros(rng, M, K, 1)
+    A[A != 0] = rng.uniform(1, 2, M) * 2.0 ** half
+    B = (rng.uniform(1, 2, size=(K, N)) * 2.0 ** (exponent - half)).astype(np.float32)
+    got, what = run(handle, torch_gpu, A, B, rows, 1, 1, 3)
+    ref = A.astype(np.float64) @ B.astype(np.float64)
+    ulp = np.maximum(np.exp2(np.floor(np.log2(ref)) - 23), 2.0 ** -149)
+    assert (np.abs(got - ref) <= (0.5 + 7 * 2.0 ** -8) * ulp + 8 * 2.0 ** -150).all(), (what, np.max(np.abs(got - ref) / ulp))
 
 
 def test_tiny_values_anywhere_are_not_lost(handle, torch_gpu, rng):
