@@ -27,14 +27,16 @@ inline double us(const Cost& c, const any::Problem& p, int cus, int rows) {
 }
 
 // Rows of a tile, 0: no call of this kernel's.  One round of tiles only, and sizes inside the timed ones.  Below
-// 1536 bytes of k the estimates err too much (int8 641 x 2832 x 704 10.3 us here, 7.9 on the tile kernel); beyond
-// 6000 the other one is often too high (int8 150 x 7040 x 10560 estimated 46 us there, took 38, here 47), and this
-// one has to be 10 % below it.  Of some 2000 random calls that the tile kernel served with k up to 6000 bytes, 179
-// 16-bit and 101 int8 ones are taken: 1.13 and 1.24 times as fast (geometric mean), 271 of them by more than 3 %,
-// one more than 3 % slower (f16 67 x 13936 x 2544: 27.2 us, 23.9 there).  Of 316 taken among random sizes timed
-// afterwards, 1.13 (16-bit) and 1.20 (int8) times as fast, five are 4 to 8 % slower.
+// 1536 bytes of k the estimates err too much (int8 641 x 2832 x 704 10.3 us here, 7.9 on the tile kernel).  Beyond
+// 5000 this one is often too low and the other too high (bf16 1860 x 720 x 2768 estimated 20.5 and 21.5 us, took 24.5
+// and 21.3): it has to be 10 % below there, 2 % elsewhere.  Beyond 12000 no size timed was faster by more than the
+// estimate errs, and some far slower (int8 216 x 6464 x 13328 71 us, 54 there).  Of 2173 random calls with both
+// estimates near or in favour, each timed on both kernels in turn, 1626 are taken: 1.18 times as fast
+// (geometric mean), 1553 of them by more than 3 %, six more than 3 % slower (the worst 8 %); 32 were with one line
+// at 6000 and no margin below it.Of 1666 taken among as many random calls timed
+// afterwards 1.18 times as fast, four more than 3 % slower (the worst 10 %).
 inline int choose(const Cost& c, const any::Cost& other, const any::Problem& p, int cus, size_t partial_bytes) {
-  if (p.M <= 32 || p.M > 2048 || p.N < 256 || p.K_bytes < 1536) return 0;
+  if (p.M <= 32 || p.M > 2048 || p.N < 256 || p.K_bytes < 1536 || p.K_bytes > 12000) return 0;
   int rows = 0;
   double best = 1e30;
   for (int r : {64, 128}) {
@@ -43,7 +45,7 @@ inline int choose(const Cost& c, const any::Cost& other, const any::Problem& p, 
     const double t = us(c, p, cus, r);
     if (t < best) best = t, rows = r;
   }
-  if (p.K_bytes > 6000) best *= 1.1;
+  best *= p.K_bytes > 5000 ? 1.1 : 1.02;
   return rows && best < any::other_us(other, p, true, cus, partial_bytes) ? rows : 0;
 }
 
