@@ -64,19 +64,35 @@ inline double launch_us(int64_t M, int64_t N, int64_t K, int cus, int rows, int 
 // The longest sum of k that a result may be made of, where the other kernel adds up `sum_length`.  Of equally long
 // sums the error here is at most 0.71 times the fp32 instructions' (0.83 and 1.00 where two products or one
 // make the result, whose errors do not grow); that of positive operands grows with the length (over K in one
-// sum, against the fp32 instructions over six ranges of it: 1.7 to 4.3 times).
+// sum, against the fp32 instructions over six ranges of it: 1.7 to 4.3 times).  (Where the other kernel takes two
+// launches, its length is the first one's, which has most of the columns.)
 constexpr int64_t range_limit(int64_t sum_length) { return sum_length + sum_length / 4; }
 
-// The best single launch; `sum_length`: of the kernel this one takes the place of.
+// No single launch over these sizes takes less: the stages of all tiles spread evenly over the units, on the height
+// that needs least for a row, and the terms that no plan avoids.
+inline double least_us(int64_t M, int64_t N, int64_t K, int cus, int rows) {
+  const Cost c = cost_of(rows);
+  const double tiles = (double)(any::div_up(M, rows) * any::div_up(N, tile::BN));
+  return START_US + tiles * ((double)K / 16) / cus * (c.stage + c.stage_chip) + c.round +
+         IN_MB * (double)(M + N) * (double)K * 4e-6;
+}
+
+// The best single launch below `*est`, which it lowers; `sum_length`: of the kernel this one takes the place of.
+// What cannot be below it is not looked at: planning is host time (4000 random calls, M 1..8192, N and K 16..16384,
+// all of the choice: 0.31 us on average and 3.1 for one in a hundred with every plan, 0.16 and 1.6 now, most of it the
+// other kernels' estimates).
 inline Plan best_launch(int64_t M, int64_t N, int64_t K, int64_t sum_length, int cus, size_t partial_bytes,
                         double* est) {
   Plan best{0, 1, 0, 0};
-  *est = 1e30;
+  const int64_t limit = range_limit(sum_length);
+  const int fewest = (int)any::at_most((double)any::div_up(K, limit > 0 ? limit : 1), 33);
   for (int rows = 64; rows <= 128; rows += 32) {
     if (rows > 64 && rows - 32 >= M) break;  // a lower height already covers M
     const int64_t tiles = any::div_up(M, rows) * any::div_up(N, tile::BN);
+    const double least = least_us(M, N, K, cus, rows), mn = (double)M * (double)N * 4e-6;
     int last = 0;
-    for (int wanted = 1; wanted <= 32; ++wanted) {
+    for (int wanted = fewest > 1 ? fewest : 1; wanted <= 32; ++wanted) {
+      if (least + (wanted > 1 ? REDUCE_US + REDUCE_MB * mn * (last + 1) : 0.0) >= *est) break;
       int64_t range_k = 0;
       const int sp = k_ranges(K, wanted, &range_k);
       if (sp > 1 && (tiles * sp > 2 * (int64_t)cus || range_k < 64 ||
@@ -84,7 +100,7 @@ inline Plan best_launch(int64_t M, int64_t N, int64_t K, int64_t sum_length, int
         break;
       if (sp == last) continue;
       last = sp;
-      if (range_k > range_limit(sum_length)) continue;
+      if (range_k > limit) continue;
       const double us = launch_us(M, N, K, cus, rows, sp);
       if (us < *est) *est = us, best = Plan{rows, sp, 0, 0};
     }
@@ -92,7 +108,7 @@ inline Plan best_launch(int64_t M, int64_t N, int64_t K, int64_t sum_length, int
   return best;
 }
 
-// That, or the columns that fill whole rounds on one height and the others by themselves.
+// That, or the columns that fill whole rounds on one height and the others by themselves; `*est` as there.
 inline Plan best(int64_t M, int64_t N, int64_t K, int64_t sum_length, int cus, size_t partial_bytes,
                  double* est) {
   Plan b = best_launch(M, N, K, sum_length, cus, partial_bytes, est);
@@ -104,9 +120,9 @@ inline Plan best(int64_t M, int64_t N, int64_t K, int64_t sum_length, int cus, s
     if (cols <= 0 || cols >= tiles_n) continue;
     const double first = launch_us(M, cols * tile::BN, K, cus, rows, 1);
     if (first >= *est) continue;
-    double us = 0;
+    double us = *est - first;
     const Plan rest = best_launch(M, N - cols * tile::BN, K, sum_length, cus, partial_bytes, &us);
-    if (rest.rows && first + us < *est) *est = first + us, b = Plan{rest.rows, rest.ranges, cols * tile::BN, rows};
+    if (rest.rows) *est = first + us, b = Plan{rest.rows, rest.ranges, cols * tile::BN, rows};
   }
   return b;
 }

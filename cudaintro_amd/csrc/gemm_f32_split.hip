@@ -108,18 +108,19 @@ Choice choose(const cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const f
   if (any::tile_ok(M, N, K, 4, lda, ldb, true) && !(K <= 512 && f32_small_is_narrow(M, N, K, A, lda)) &&
       kwaves::best_f32(M, N, K, cus, room, ctx->ws_counter_bytes, &us).splits && us < other.us)
     return none;
+  us = MARGIN * other.us;
   const split32::Plan plan = split32::best(M, N, K, other.sum_length, cus, room, &us);
   // Up to 64 columns beyond whole tiles: the kernel of small outputs (4095 x 4097 x 4099 838 us;
   // the 4097th column as tiles over 8 ranges of K would take 50).
   const int64_t rest = N % tile::BN, n1 = N - rest;
   if (rest && rest <= 64 && n1) {
-    double main_us = 0, rest_us = 0;
-    const split32::Plan main = split32::best(M, n1, K, other.sum_length, cus, room, &main_us);
-    const kwaves::Plan p = kwaves::best_f32(M, rest, K, cus, room, ctx->ws_counter_bytes, &rest_us);
-    if (main.rows && p.splits && main_us + rest_us < us && main_us + rest_us < MARGIN * other.us)
-      return Choice{main, rest};
+    double rest_us = 0;
+    if (kwaves::best_f32(M, rest, K, cus, room, ctx->ws_counter_bytes, &rest_us).splits) {
+      us -= rest_us;
+      const split32::Plan main = split32::best(M, n1, K, other.sum_length, cus, room, &us);
+      if (main.rows) return Choice{main, rest};
+    }
   }
-  if (!plan.rows || us >= MARGIN * other.us) return none;
   return Choice{plan, 0};
 }
 

@@ -29,11 +29,11 @@ inline double us(const Cost& c, const any::Problem& p, int cus, int rows) {
 // Rows of a tile, 0: no call of this kernel's.  One round of tiles only, and sizes inside the timed ones.  Below
 // 1536 bytes of k the estimates err too much (int8 641 x 2832 x 704 10.3 us here, 7.9 on the tile kernel).  Beyond
 // 5000 this one is often too low and the other too high (bf16 1860 x 720 x 2768 estimated 20.5 and 21.5 us, took 24.5
-// and 21.3): it has to be 10 % below there, 2 % elsewhere.  Beyond 12000 no size timed was faster by more than the
-// estimate errs, and some far slower (int8 216 x 6464 x 13328 71 us, 54 there).  Of 2173 random calls with both
+// and 21.3): it has to be 10 % below there, 2 % elsewhere.  Beyond 12000 two of 22 calls
+// timed were faster by more than 3 % (5 and 7 %) and some far slower (int8 216 x 6464 x 13328 71 us, 54 there).  Of 2173 random calls with both
 // estimates near or in favour, each timed on both kernels in turn, 1626 are taken: 1.18 times as fast
 // (geometric mean), 1553 of them by more than 3 %, six more than 3 % slower (the worst 8 %); 32 were with one line
-// at 6000 and no margin below it.Of 1666 taken among as many random calls timed
+// at 6000 and no margin below it.  Of 1666 taken among as many random calls timed
 // afterwards 1.18 times as fast, four more than 3 % slower (the worst 10 %).
 inline int choose(const Cost& c, const any::Cost& other, const any::Problem& p, int cus, size_t partial_bytes) {
   if (p.M <= 32 || p.M > 2048 || p.N < 256 || p.K_bytes < 1536 || p.K_bytes > 12000) return 0;
