@@ -159,7 +159,7 @@ def gemm_bf16_static(A, B, out=None, stream=None):
     s = torch.cuda.current_stream() if stream is None else stream
     err = C.create_string_buffer(256)
     st = lib.cigemm_gemm_bf16_static(_vp(s.cuda_stream), M, N, K, A.data_ptr(), Handle._ld(A),
-                                     B.data_ptr(), Handle._ld(B), out.data_ptr(), Handle._ld(out),
+                                     B.data_ptr(), Handle._ld(B), out.data_ptr(), _out_ld(out, M, N, 2),
                                      err, len(err))
     if st != 0:
         raise CigemmError(st, err.value.decode(), "cigemm_gemm_bf16_static")
@@ -173,6 +173,13 @@ def _mat(t):
     rows, cols = t.shape
     assert cols <= 1 or s[1] == 1, "rows must be contiguous"
     return rows, cols, s[0] if rows > 1 else max(cols, s[0], 1)
+
+
+def _out_ld(t, M, N, itemsize):
+    """Leading dimension of an output with room for M x N elements of `itemsize` bytes."""
+    rows, cols, ld = _mat(t)
+    assert rows >= M and cols >= N and t.element_size() >= itemsize, "the output is too small"
+    return ld
 
 
 class Handle:
@@ -278,7 +285,8 @@ class Handle:
         assert K == K2
         if out is None:
             out = _torch().empty((M, N), dtype=out_dtype, device=A.device)
-        self._check(fn(self._h, M, N, K, A.data_ptr(), lda, B.data_ptr(), ldb, out.data_ptr(), _mat(out)[2]), name)
+        self._check(fn(self._h, M, N, K, A.data_ptr(), lda, B.data_ptr(), ldb, out.data_ptr(),
+                       _out_ld(out, M, N, A.element_size())), name)
         return out
 
     def gemm_f32(self, A, B, out=None):
@@ -304,12 +312,12 @@ class Handle:
         assert X.dtype == f32 and W.dtype == f32
         M, K, ldx = _mat(X)
         K2, N, ldw = _mat(W)
-        assert K == K2 and (bias is None or (bias.dtype == f32 and bias.numel() == N))
+        assert K == K2 and (bias is None or (bias.dtype == f32 and bias.numel() == N and bias.is_contiguous()))
         if out is None:
             out = _torch().empty((M, N), dtype=f32, device=X.device)
         st = self.lib.cigemm_linear_f32(self._h, M, N, K, X.data_ptr(), ldx, W.data_ptr(), ldw,
                                         bias.data_ptr() if bias is not None else None, act,
-                                        out.data_ptr(), _mat(out)[2])
+                                        out.data_ptr(), _out_ld(out, M, N, 4))
         if st:
             self._check(st, "cigemm_linear_f32")
         return out
@@ -377,7 +385,7 @@ class Handle:
             torch = _torch()
             out = torch.empty((M, N), dtype=torch.int32, device=A.device)
         st = self.lib.cigemm_gemm_i8_i32(self._h, M, N, K, A.data_ptr(), lda, B.data_ptr(), ldb,
-                                         b_layout, out.data_ptr(), _mat(out)[2])
+                                         b_layout, out.data_ptr(), _out_ld(out, M, N, 4))
         if st:
             self._check(st, "cigemm_gemm_i8_i32")
         return out
@@ -393,12 +401,14 @@ class Handle:
             if st > 0:
                 self._check(st, "cigemm_gemm_i8_dequant")
         f32 = self._f32
+        assert A.element_size() == 1 and B.element_size() == 1
         M, K, lda = _mat(A)
         K2, N, ldb = _mat(B)
         if b_layout == B_NK:
             K2, N = N, K2
         assert K == K2
         assert scale_a.dtype == f32 and scale_b.dtype == f32
+        assert scale_a.is_contiguous() and scale_b.is_contiguous()
         na, nb = scale_a.numel(), scale_b.numel()
         assert (na == 1 or na == M) and (nb == 1 or nb == N)
         if out is None:
@@ -411,7 +421,8 @@ class Handle:
         st = self.lib.cigemm_gemm_i8_dequant(
             self._h, M, N, K, A.data_ptr(), lda, B.data_ptr(), ldb, b_layout, scale_a.data_ptr(),
             SCALE_VECTOR if na > 1 else SCALE_TENSOR, scale_b.data_ptr(),
-            SCALE_VECTOR if nb > 1 else SCALE_TENSOR, out.data_ptr(), out_type, _mat(out)[2],
+            SCALE_VECTOR if nb > 1 else SCALE_TENSOR, out.data_ptr(), out_type,
+            _out_ld(out, M, N, 2 if out_type == OUT_BF16 else 4),
             acc.data_ptr() if dump_acc else None, N if dump_acc else 0)
         if st:
             self._check(st, "cigemm_gemm_i8_dequant")
@@ -445,6 +456,7 @@ class Handle:
         else:
             q, s = out
             assert q.dtype == self._i8 and q.shape == x.shape and s.dtype == self._f32
+            assert s.numel() >= rows and s.is_contiguous()
         st = self.lib.cigemm_quantize_rows_i8(self._h, rows, cols, x.data_ptr(), ldx, q.data_ptr(),
                                               _mat(q)[2], s.data_ptr())
         if st:

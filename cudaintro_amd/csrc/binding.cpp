@@ -36,6 +36,19 @@ bool matrix(PyObject* o, Mat* m) {
   return true;
 }
 
+// An output with room for rows x cols elements of `bytes`: more of any of them was always taken.
+bool output(PyObject* o, Mat* m, int64_t rows, int64_t cols, int64_t bytes) {
+  if (!matrix(o, m)) return false;
+  return (m->rows >= rows && m->cols >= cols && (int64_t)THPVariable_Unpack(o).element_size() >= bytes) ||
+         fail("the output is too small");
+}
+
+// A bias or the scales: the kernels read (write) numel elements in a row.
+bool dense(PyObject* o) { return THPVariable_Unpack(o).is_contiguous() || fail("contiguous vectors expected"); }
+
+// int8, or its bits in another type
+bool bytes(PyObject* o) { return THPVariable_Unpack(o).element_size() == 1 || fail("unexpected dtype"); }
+
 bool typed(PyObject* o, at::ScalarType type) {
   return THPVariable_Unpack(o).scalar_type() == type || fail("unexpected dtype");
 }
@@ -87,7 +100,7 @@ PyObject* gemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Mat A, B, C;
     if (!typed(a[3], type) || !typed(a[4], type) || !matrix(a[3], &A) || !matrix(a[4], &B)) return nullptr;
     if (A.cols != B.rows) return fail("inner dimensions differ"), nullptr;
-    if (!matrix(a[5], &C)) return nullptr;
+    if (!output(a[5], &C, A.rows, B.cols, code == 0 ? 4 : 2)) return nullptr;
     const auto fn = function<gemm_f32_fn>(a[0]);
     const cigemmHandle_t h = handle(a[1]);
     if (PyErr_Occurred()) return nullptr;
@@ -110,11 +123,11 @@ PyObject* linear_f32(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const float* bias = nullptr;
     if (has_bias) {
       const at::Tensor& b = THPVariable_Unpack(a[4]);
-      if (!typed(a[4], at::kFloat)) return nullptr;
+      if (!typed(a[4], at::kFloat) || !dense(a[4])) return nullptr;
       if (b.numel() != W.cols) return fail("one bias for each column expected"), nullptr;
       bias = static_cast<const float*>(b.data_ptr());
     }
-    if (!matrix(a[6], &C)) return nullptr;
+    if (!output(a[6], &C, X.rows, W.cols, 4)) return nullptr;
     const auto fn = function<decltype(&cigemm_linear_f32)>(a[0]);
     const cigemmHandle_t h = handle(a[1]);
     const long act = PyLong_AsLong(a[5]);
@@ -137,7 +150,7 @@ PyObject* gemm_i8_i32(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const long layout = PyLong_AsLong(a[4]);
     const bool nk = layout == CIGEMM_B_NK;
     if (A.cols != (nk ? B.cols : B.rows)) return fail("inner dimensions differ"), nullptr;
-    if (!matrix(a[5], &C)) return nullptr;
+    if (!output(a[5], &C, A.rows, nk ? B.rows : B.cols, 4)) return nullptr;
     const auto fn = function<decltype(&cigemm_gemm_i8_i32)>(a[0]);
     const cigemmHandle_t h = handle(a[1]);
     if (PyErr_Occurred()) return nullptr;
@@ -155,17 +168,17 @@ PyObject* gemm_i8_dequant(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
     if (!plain(a[2]) || !plain(a[3]) || !plain(a[4]) || !plain(a[5]) || !plain(a[8])) return PyLong_FromLong(-1);
     Mat A, B, C;
-    if (!matrix(a[2], &A) || !matrix(a[3], &B)) return nullptr;
+    if (!bytes(a[2]) || !bytes(a[3]) || !matrix(a[2], &A) || !matrix(a[3], &B)) return nullptr;
     const long layout = PyLong_AsLong(a[6]), out_type = PyLong_AsLong(a[7]);
     const bool nk = layout == CIGEMM_B_NK;
     const int64_t N = nk ? B.rows : B.cols;
     if (A.cols != (nk ? B.cols : B.rows)) return fail("inner dimensions differ"), nullptr;
-    if (!typed(a[4], at::kFloat) || !typed(a[5], at::kFloat)) return nullptr;
+    if (!typed(a[4], at::kFloat) || !typed(a[5], at::kFloat) || !dense(a[4]) || !dense(a[5])) return nullptr;
     const at::Tensor &sa = THPVariable_Unpack(a[4]), &sb = THPVariable_Unpack(a[5]);
     const int64_t na = sa.numel(), nb = sb.numel();
     if ((na != 1 && na != A.rows) || (nb != 1 && nb != N))
       return fail("one scale, or one for each row of A / column of C, expected"), nullptr;
-    if (!matrix(a[8], &C)) return nullptr;
+    if (!output(a[8], &C, A.rows, N, out_type == CIGEMM_OUT_BF16 ? 2 : 4)) return nullptr;
     const auto fn = function<decltype(&cigemm_gemm_i8_dequant)>(a[0]);
     const cigemmHandle_t h = handle(a[1]);
     if (PyErr_Occurred()) return nullptr;
@@ -187,9 +200,10 @@ PyObject* quantize_rows_i8(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!plain(a[2]) || !plain(a[3]) || !plain(a[4])) return PyLong_FromLong(-1);
     Mat x, q;
     if (!typed(a[2], at::kFloat) || !matrix(a[2], &x) || !typed(a[3], at::kChar) || !matrix(a[3], &q) ||
-        !typed(a[4], at::kFloat))
+        !typed(a[4], at::kFloat) || !dense(a[4]))
       return nullptr;
-    if (q.rows != x.rows || q.cols != x.cols) return fail("shapes differ"), nullptr;
+    if (q.rows != x.rows || q.cols != x.cols || THPVariable_Unpack(a[4]).numel() < x.rows)
+      return fail("shapes differ"), nullptr;
     const auto fn = function<decltype(&cigemm_quantize_rows_i8)>(a[0]);
     const cigemmHandle_t h = handle(a[1]);
     if (PyErr_Occurred()) return nullptr;

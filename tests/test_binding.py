@@ -108,3 +108,88 @@ def test_linear_int8_quantizer():
     for bad in ((x.double(), xq, sx), (x, xq[:2], sx), (x, xq.int(), sx), (x, xq, sx.double())):
         with pytest.raises(AssertionError):
             native.quantize_rows_i8(q.address, HANDLE, *bad)
+
+
+def test_what_would_be_written_or_read_past_its_end_is_refused():
+    """Outputs with too few rows, columns or bytes an element, scales and biases that are short or not dense; room to
+    spare is taken."""
+    i8 = torch.int8
+    e = Entry("cigemm_gemm_f32")
+    A, B = torch.zeros(3, 5), torch.zeros(5, 7)
+    small = (torch.zeros(2, 7), torch.zeros(3, 6), torch.zeros(3, 14)[:, 4:10], torch.zeros((3, 7), dtype=torch.float16),
+             torch.zeros(1, 21))
+    for out in small:
+        with pytest.raises(AssertionError):
+            native.gemm(e.address, HANDLE, 0, A, B, out)
+    with pytest.raises(AssertionError):
+        native.gemm(e.address, HANDLE, 2, A.bfloat16(), B.bfloat16(), torch.zeros((3, 7), dtype=i8))
+    for out in (torch.zeros(4, 7), torch.zeros(3, 9), torch.zeros((3, 7), dtype=torch.float64),
+                torch.zeros((3, 7), dtype=torch.int32)):
+        assert native.gemm(e.address, HANDLE, 0, A, B, out) == 0
+
+    e = Entry("cigemm_linear_f32")
+    for out in small:
+        with pytest.raises(AssertionError):
+            native.linear_f32(e.address, HANDLE, A, B, None, 0, out)
+    for bias in (torch.zeros(14)[::2], torch.zeros(1).expand(7)):
+        with pytest.raises(AssertionError):
+            native.linear_f32(e.address, HANDLE, A, B, bias, 0, torch.zeros(3, 7))
+    assert native.linear_f32(e.address, HANDLE, A, B, torch.zeros(1, 7), 0, torch.zeros(3, 7)) == 0
+
+    qa, sa, sb = torch.zeros((3, 5), dtype=i8), torch.zeros(3), torch.zeros(7)
+    e, d = Entry("cigemm_gemm_i8_i32"), Entry("cigemm_gemm_i8_dequant")
+    for layout, qb in ((ci.B_KN, torch.zeros((5, 7), dtype=i8)), (ci.B_NK, torch.zeros((7, 5), dtype=i8))):
+        for out in small:
+            with pytest.raises(AssertionError):
+                native.gemm_i8_i32(e.address, HANDLE, qa, qb, layout, out)
+            with pytest.raises(AssertionError):
+                native.gemm_i8_dequant(d.address, HANDLE, qa, qb, sa, sb, layout, ci.OUT_F32, out)
+        y = torch.zeros((3, 7), dtype=torch.bfloat16)
+        assert native.gemm_i8_dequant(d.address, HANDLE, qa, qb, sa, sb, layout, ci.OUT_BF16, y) == 0
+        assert native.gemm_i8_dequant(d.address, HANDLE, qa.view(torch.uint8), qb, sa, sb, layout, ci.OUT_BF16, y) == 0
+        for bad in ((qa.float(), qb, sa, sb), (qa, qb.half(), sa, sb), (qa, qb, torch.zeros(6)[::2], sb),
+                    (qa, qb, sa, torch.zeros(1).expand(7))):
+            with pytest.raises(AssertionError):
+                native.gemm_i8_dequant(d.address, HANDLE, *bad, layout, ci.OUT_BF16, y)
+
+    q = Entry("cigemm_quantize_rows_i8")
+    for s in (torch.zeros(2), torch.zeros(6)[::2], torch.zeros(1).expand(3)):
+        with pytest.raises(AssertionError):
+            native.quantize_rows_i8(q.address, HANDLE, A, qa, s)
+    assert native.quantize_rows_i8(q.address, HANDLE, A, qa, torch.zeros(4)) == 0
+
+
+def test_refused_by_the_python_code_too():
+    """The same calls where the native binding hands them back."""
+    class Reached(Exception):
+        pass
+
+    class Lib:
+        def __getattr__(self, name):
+            def call(*a):
+                raise Reached(name)
+            return call
+    h = object.__new__(ci.Handle)
+    h.lib, h._h, h._address = Lib(), None, 0
+    h._f32, h._bf16, h._f16, h._i8 = torch.float32, torch.bfloat16, torch.float16, torch.int8
+    for name in cigemm._native_entries():
+        setattr(h, name, (lambda *a: -1) if name.startswith("_n_") else 0)
+    i8 = torch.int8
+    A, B, C = torch.zeros(3, 5), torch.zeros(5, 7), torch.zeros(3, 7)
+    qa, qb, sa, sb = torch.zeros((3, 5), dtype=i8), torch.zeros((5, 7), dtype=i8), torch.zeros(3), torch.zeros(7)
+    taken = [lambda: h.gemm_f32(A, B, out=C), lambda: h.gemm_bf16(A.bfloat16(), B.bfloat16(), out=C),
+             lambda: h.linear_f32(A, B, sb, out=torch.zeros(5, 9)), lambda: h.gemm_i8_i32(qa, qb, out=C),
+             lambda: h.gemm_i8_dequant(qa, qb, sa, sb, out=C), lambda: h.quantize_rows_i8(A, out=(qa, sa))]
+    refused = [lambda: h.gemm_f32(A, B, out=torch.zeros(2, 7)), lambda: h.gemm_f32(A, B, out=C.half()),
+               lambda: h.gemm_f16(A.half(), B.half(), out=torch.zeros((3, 6), dtype=torch.float16)),
+               lambda: h.linear_f32(A, B, torch.zeros(14)[::2], out=C), lambda: h.linear_f32(A, B, sb, out=C.half()),
+               lambda: h.gemm_i8_i32(qa, qb, out=C.half()), lambda: h.gemm_i8_dequant(qa.float(), qb, sa, sb, out=C),
+               lambda: h.gemm_i8_dequant(qa, qb, sa, torch.zeros(1).expand(7), out=C),
+               lambda: h.gemm_i8_dequant(qa, qb, sa, sb, out=C.half()),
+               lambda: h.quantize_rows_i8(A, out=(qa, torch.zeros(2)))]
+    for call in taken:
+        with pytest.raises(Reached):
+            call()
+    for call in refused:
+        with pytest.raises(AssertionError):
+            call()
