@@ -102,7 +102,7 @@ def load_library():
     if not os.path.exists(_LIB):
         raise FileNotFoundError(
             f"{_LIB} is not built; run `python -c 'import __graft_entry__ as g; g.build()'` "
-            "or `make -C cudaintro_amd/csrc`.  There is no CPU fallback.")
+            "or `make -C cudaintro_amd/csrc all python`.  There is no CPU fallback.")
     lib = C.CDLL(_LIB)
     for name, (res, args) in SIGNATURES.items():
         fn = getattr(lib, name)

@@ -2,6 +2,9 @@
 Python callbacks that record their arguments, over every order and stride the Python code takes, against
 what that computes; what that refuses is refused."""
 import ctypes as C
+import os
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -11,6 +14,7 @@ from cudaintro_amd import cigemm
 
 native = cigemm._native()
 HANDLE = 0x1230
+CSRC = os.path.join(os.path.dirname(cigemm.__file__), "csrc")
 
 
 class Entry:
@@ -193,3 +197,17 @@ def test_refused_by_the_python_code_too():
     for call in refused:
         with pytest.raises(AssertionError):
             call()
+
+
+def test_the_libraries_and_the_driver_build_without_python(tmp_path):
+    """`make` asks no Python for anything; `make python` builds the module for the Python it is given."""
+    plan = lambda *a: subprocess.run(["make", "-n", "-B", "-C", CSRC, *a], capture_output=True, text=True)  # noqa: E731
+    asked = tmp_path / "asked"
+    python = tmp_path / "python"
+    python.write_text(f"#!/bin/sh\ntouch {asked}\nexec {sys.executable} \"$@\"\n")
+    python.chmod(0o755)
+    out = plan("all", f"PYTHON={python}")
+    assert out.returncode == 0 and "gemm_suite" in out.stdout and "binding" not in out.stdout and not asked.exists()
+    out = plan("python", f"PYTHON={python}")
+    assert out.returncode == 0 and "binding.cpp" in out.stdout and os.path.dirname(torch.__file__) in out.stdout
+    assert asked.exists() and "libcigemm" not in out.stdout
