@@ -124,7 +124,11 @@ CIGEMM_API int cigemmGetVersion(void);
  * "<type>_mfma_<tile rows>x256x<k per stage>_w<waves per workgroup>_ring4[_kn|_nk][_dequant]
  * [_bias_act][_splitk]", e.g. "bf16_mfma_256x256x32_w4_ring4", "i8_mfma_256+192x256x64_w8+w4_
  * ring4_nk_dequant" when two launches of different tile heights covered the columns (a
- * "_splitk" after such a name: the second launch ran as K ranges plus a reduction); the kernel of
+ * "_splitk" after such a name: the second launch ran as K ranges plus a reduction).  "any_" behind
+ * "_mfma_": the form that takes any alignment.  fp32 tiles come in two kinds: with "_32x32x2" behind
+ * "_ring4" on the fp32 matrix instructions, without it on the bf16 ones, an operand as three parts
+ * ("f32_mfma_128x256x16_w4_ring4").  The kernel of batches reports
+ * "<type>_mfma_panel_<tile rows>x64x<k per stage>_w8[_nk][_dequant]", the kernel of
  * small outputs "<type>_mfma_[any_]kwaves_32x64x<k per piece>_w4[_kn|_nk][_dequant]_splitk" (k is
  * always split, over its four waves at least), fp32 "f32_mfma_[any_]small_kwaves_32x32x32_w4[_bias_act]
  * _splitk" (its register-loaded sibling: "f32_mfma_[any_]small_32x32_ksplit4[_bias_act]"); "+32x64" or
@@ -133,10 +137,11 @@ CIGEMM_API int cigemmGetVersion(void);
 CIGEMM_API const char* cigemmGetLastKernelName(cigemmHandle_t handle);
 
 /* Plan of the last successful GEMM call on this handle, for tests and profiles: rows of the
- * output tile (256, 192, 128 or 64, fp32 also 224, 160 and 96; 32 for the kernel of small outputs; with
+ * output tile (256, 192, 128 or 64, fp32 also 224, 160 and 96; 128 or 64 for the kernel of batches; 32 for
+ * the kernel of small outputs; with
  * two launches, of the second, but of the first where the last few columns ran on the kernel of small
- * outputs) and number of K ranges (one workgroup each) when the LDS-tiled matrix-core kernel or the
- * kernel of small outputs ran, 0 and 0 when another family did.  Either pointer
+ * outputs) and number of K ranges (one workgroup each) when the LDS-tiled matrix-core kernel, the
+ * kernel of batches or that of small outputs ran, 0 and 0 when another family did.  Either pointer
  * may be null.  No counterpart in the reference: cuBLAS does not report its heuristics'
  * choice (quantization/GEMM_bf16.cu:51-56). */
 CIGEMM_API cigemmStatus_t cigemmGetLastPlan(cigemmHandle_t handle, int* tile_rows, int* k_splits);
@@ -165,7 +170,15 @@ CIGEMM_API cigemmStatus_t cigemmGetAlgo(cigemmHandle_t handle, cigemmAlgo_t* alg
 /* ---- GEMM: C[M x N] = A[M x K] . B[K x N], row-major ------------------------------- */
 
 /* Replaces cublasGemmEx(CUDA_R_32F x3, CUBLAS_COMPUTE_32F)
- * (quantization/GEMM_fp32.cu:49-54, 62-67).  fp32 inputs, fp32 products and sums. */
+ * (quantization/GEMM_fp32.cu:49-54, 62-67).  fp32 inputs and sums.  Products: those of the fp32
+ * matrix instructions, or, where CIGEMM_ALGO_DEFAULT estimates that to be faster (large calls),
+ * of the operands' three exact bf16 parts, eight of the nine part products, which lie within 2^-32 of
+ * the exact product.  The sums' error against 64 bits is no larger there, for dense operands a third;
+ * a result that is a single product is within 0.53 units in the last place (0.50 on the fp32
+ * instructions).  Infinities, NaN and subnormal
+ * numbers come out as with fp32 instructions.  CIGEMM_ALGO_TILE, SMALL and MFMA_ANY use the fp32
+ * instructions alone, CIGEMM_ALGO_GENERIC the CPU loop's order.  The same holds for
+ * cigemm_linear_f32. */
 CIGEMM_API cigemmStatus_t cigemm_gemm_f32(cigemmHandle_t handle, int64_t M, int64_t N,
                                           int64_t K, const float* A, int64_t lda,
                                           const float* B, int64_t ldb, float* C, int64_t ldc);
