@@ -295,10 +295,11 @@ bool launch_f32_tile(cigemmContext*, int64_t M, int64_t N, int64_t K, const floa
                      int64_t lda, const float* B, int64_t ldb, float* C, int64_t ldc,
                      const BiasAct* ba = nullptr);
 // What the call is estimated to take on the kernel that DEFAULT would choose without gemm_kwaves.hip and
-// gemm_f32_split.hip, and the longest sum of k that kernel adds up in a row.
+// gemm_f32_split.hip, the longest sum of k that kernel adds up in a row, and whether it is the small kernel.
 struct F32Other {
   double us;
   int64_t sum_length;
+  bool small;
 };
 F32Other f32_other(const cigemmContext*, int64_t M, int64_t N, int64_t K, const float* A,
                    int64_t lda, const float* B, int64_t ldb, const float* C, int64_t ldc,

@@ -77,20 +77,20 @@ F32Other f32_other(const cigemmContext* ctx, int64_t M, int64_t N, int64_t K, co
       f32_small_any_ok(M, N, K) ? any::f32_small_us(M, N, K, cus, f32_small_b16(N, B, ldb),
                                                     f32_small_is_narrow(M, N, K, A, lda))
                                 : 1e30,
-      any::div_up(K, 4)};
+      any::div_up(K, 4), true};
   if (f32_tile_ok(M, N, K, A, lda, B, ldb, C, ldc, ba)) {
     if (aligned_is_small(ctx, M, N, K, A, lda, B, ldb)) return small;
     tile::SmallPlan plan{0, 1};
     if (any::div_up(M, tile::BM) * any::div_up(N, tile::BN) <= cus)
       plan = tile::plan_small(cus, room, M, N, K * 4, 4, any::COST_F32.sc, K * 4 * N);
-    return F32Other{any::tile_us(any::COST_F32, p, cus, room, plan), K / plan.splits};
+    return F32Other{any::tile_us(any::COST_F32, p, cus, room, plan), K / plan.splits, false};
   }
   const tile::SmallPlan plan = any::tile_plan(any::COST_F32, p, cus, room);
   const double tile = any::tile_us(any::COST_F32, p, cus, room, plan);
   const double staged = any::staged_us(any::COST_F32, p, cus, room);
   int64_t steps = 0;
-  const F32Other other = staged < tile ? F32Other{staged, K / any::staged_ranges(p, cus, room, &steps)}
-                                       : F32Other{tile, K / plan.splits};
+  const F32Other other = staged < tile ? F32Other{staged, K / any::staged_ranges(p, cus, room, &steps), false}
+                                       : F32Other{tile, K / plan.splits, false};
   return small.us < other.us ? small : other;
 }
 

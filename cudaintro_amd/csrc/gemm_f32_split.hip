@@ -86,10 +86,12 @@ struct Choice {
   int64_t rest;
 };
 
-// The two estimates err by 4 and 11 %.  Asked to be 8 % below, this kernel is taken for 1985 of 10154 random sizes
-// (M 16..20000, N 16..16384, K 17..16384, one launch), 1.13 times as fast (geometric mean), 14 of them more than 3 %
-// slower, and the choice is 0.6 % off the faster kernel on average (0.3 % and 44 sizes at 5 %).
-constexpr double MARGIN = 0.92;
+// The two estimates err by 4 and 11 %: this one has to be 8 % below.  The small kernel's is up to 25 % too high for K
+// of 500 to 1000 (1454 x 896 x 704 26.5 us there, 31.5 here): 16 %.  Of 6203 random calls taken with 8 % everywhere (M
+// 65..20000, N 16..16384, K 17..16384, both kernels in turn) 40 were more than 3 % slower, 34 of them of
+// the small kernel's 299; 6132 are taken with both, 1.16 times as fast (geometric mean), nine more than 3 % slower
+// (the worst 6 %).
+constexpr double MARGIN = 0.92, MARGIN_SMALL = 0.84;
 
 Choice choose(const cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, const float* B,
               int64_t ldb, const float* C, int64_t ldc, const BiasAct* ba) {
@@ -108,7 +110,7 @@ Choice choose(const cigemmContext* ctx, int64_t M, int64_t N, int64_t K, const f
   if (any::tile_ok(M, N, K, 4, lda, ldb, true) && !(K <= 512 && f32_small_is_narrow(M, N, K, A, lda)) &&
       kwaves::best_f32(M, N, K, cus, room, ctx->ws_counter_bytes, &us).splits && us < other.us)
     return none;
-  us = MARGIN * other.us;
+  us = (other.small ? MARGIN_SMALL : MARGIN) * other.us;
   const split32::Plan plan = split32::best(M, N, K, other.sum_length, cus, room, &us);
   // Up to 64 columns beyond whole tiles: the kernel of small outputs (4095 x 4097 x 4099 838 us;
   // the 4097th column as tiles over 8 ranges of K would take 50).

@@ -191,7 +191,7 @@ def test_only_the_tile_that_loses_something_is_computed_again(handle, torch_gpu,
     np.testing.assert_allclose(got[rows + 9], ref[rows + 9], rtol=1e-5, err_msg=what)   # (2^-149 of some 2^-122)
 
 
-@pytest.mark.parametrize("M,N,K", [(256, 4096, 4096), (700, 3000, 1000), (2048, 2048, 2048)])
+@pytest.mark.parametrize("M,N,K", [(256, 4096, 4096), (700, 3000, 1600), (2048, 2048, 2048)])
 def test_sums_get_no_longer_than_the_kernels_it_takes_the_place_of(handle, torch_gpu, M, N, K):
     """Positive operands, whose error grows with the length of a sum: the library's own choice against what serves
     the call without these tiles."""
@@ -282,6 +282,14 @@ def test_tiny_values_anywhere_are_not_lost(handle, torch_gpu, rng):
     for rows in ROWS:
         got, what = run(handle, torch_gpu, A, B, rows, 1, 0, 0)
         np.testing.assert_allclose(got, ref, rtol=1e-6, err_msg=what)
+
+
+@pytest.mark.parametrize("M,N,K", [(1454, 896, 704), (537, 2560, 640), (660, 4096, 704), (50, 16000, 8000),
+                                   (20000, 512, 784)])
+def test_left_to_the_kernels_that_are_faster(handle, torch_gpu, M, N, K):
+    """us, there and here: 26.5 and 31.5, 25.1 and 28.9, 46.5 and 52.9; a long B on 64 rows; 115 and 119."""
+    handle.gemm_f32(torch_gpu.zeros((M, K), device="cuda"), torch_gpu.zeros((K, N), device="cuda"))
+    assert "x256x16_w4" not in handle.last_kernel or "32x32x2" in handle.last_kernel, handle.last_kernel
 
 
 def test_default_takes_it_where_it_pays_and_graphs_replay(handle, torch_gpu, rng):
