@@ -1,6 +1,6 @@
 // GEMM of a batch of rows on tiles of 64 or 128 rows x 64 columns, one round of them, all of k in one workgroup.
 //
-// What bounds these calls: a compute unit takes 50 to 55 KB/us of operands here (112 where every line is in its L2:
+// What bounds these calls: a compute unit takes 50 to 55 KB/us of operands here (111 where every line is in its L2:
 // lines that come from memory hold up those behind them), also with half of the units at work; and, where k is cut
 // to fill the chip with 256-column tiles, the partial sums and the launch that adds them up (5 to 8 us).  Tiles
 // of 64 columns fill it with whole k: 4 x 64 tiles of 64 rows serve 256 x 4096 where mfma_tile.h has 64 tiles
