@@ -11,7 +11,8 @@
 // block's 8 x 32 sub-tile as 64 x 16 bytes, passes it through a private 1 KiB of LDS (LDS
 // instructions are almost free next to MFMAs) and reads its four values back.
 //
-// 512^3 gives 256 workgroups instead of the 16 of the 64x256 tile.  Outputs of at most 16
+// 512^3 gives 256 workgroups instead of the 16 of the 64x256 tile; its 5.8 us a call are this kernel's chain of loads
+// (a wave's 16 blocks of k, four at a time), the host issues one in 2.9.  Outputs of at most 16
 // columns have a form of their own below.
 //
 // K beyond a few blocks, and few tiles, are the LDS-DMA form's (gemm_kwaves.hip, same tile):
